@@ -300,6 +300,47 @@ cam::SchedSpec sched_spec(int64_t rows, int64_t G, int64_t N, int64_t Kd, bool s
     return sp;
 }
 
+// One grouped GEMM behind its schedule (tiles) or its row counts (few rows per expert: no schedule is needed).
+// `rows` receives where the kernels after it find the row total.
+hipError_t run_grouped_gemm(cam::GemmArgs g, const int64_t *group_list, int cumulative, int64_t G, int64_t A,
+                            cam::SchedSpec sp, void *sched_ws, const int32_t **rows, hipStream_t s)
+{
+    int32_t *ws = (int32_t *)sched_ws;
+    *rows = ws;
+    if (g.epilogue != cam::kEpiInt32 && cam::stream_gemm_applies(A, g.N)) {
+        cam::StreamGemmArgs sa{};
+        sa.g = g;
+        sa.group_list = group_list;
+        sa.cumulative = cumulative;
+        sa.G = (int)G;
+        sa.max_rows = A;
+        sa.rows_out = ws;
+        return cam::launch_stream_gemm(sa, A, s);
+    }
+    sp.sched = ws;
+    const hipError_t e = cam::launch_build_sched(group_list, cumulative, (int)G, A, 1, &sp, s);
+    if (e != hipSuccess) {
+        return e;
+    }
+    g.sched = sp.sched;
+    return cam::launch_gemm(g, s);
+}
+
+// The GEMMs of a fused layer: per-expert counts from its plan, g.sched filled when the permute built schedules.  A token
+// names an expert once, so no expert has more than T rows.
+hipError_t layer_gemm(const cam::GemmArgs &g, const int64_t *counts, int E, int64_t A, int T, bool stream, hipStream_t s)
+{
+    if (!stream) {
+        return cam::launch_gemm(g, s);
+    }
+    cam::StreamGemmArgs sa{};
+    sa.g = g;
+    sa.group_list = counts;
+    sa.G = E;
+    sa.max_rows = A;
+    return cam::launch_stream_gemm(sa, T, s);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1539,19 +1580,15 @@ camStatus camGroupedMatmulSwigluQuantGetWorkspaceSize(const camTensor *x, const 
     int8_t *yq = (int8_t *)y->data;
     float *ys = (float *)yScale->data;
     auto run = [=](void *wsp, hipStream_t s) mutable -> hipError_t {
-        sp.sched = (int32_t *)((char *)wsp + o_sched);
         float *prod = (float *)((char *)wsp + o_prod);
-        hipError_t e = cam::launch_build_sched(gc.group_list, gc.cumulative, (int)gc.G, gc.A, 1, &sp, s);
-        if (e != hipSuccess) {
-            return e;
-        }
-        g.sched = sp.sched;
         g.out = prod;
-        e = cam::launch_gemm(g, s);
+        const int32_t *rows = nullptr;
+        const hipError_t e = run_grouped_gemm(g, gc.group_list, gc.cumulative, gc.G, gc.A, sp, (char *)wsp + o_sched,
+                                              &rows, s);
         if (e != hipSuccess) {
             return e;
         }
-        return cam::launch_requant(prod, gc.A, (int)I, sp.sched, yq, ys, s);
+        return cam::launch_requant(prod, gc.A, (int)I, rows, yq, ys, s);
     };
     return finish_phase1(kOpGmm1, c.off, run, workspaceSize, executor);
 }
@@ -1604,22 +1641,17 @@ camStatus camGroupedMatmulDequantGetWorkspaceSize(const camTensor *x, const camT
     g.out_fp16 = out->dtype == CAM_DT_FLOAT16;
     uint8_t *wire_out = (uint8_t *)out->data;
     auto run = [=](void *wsp, hipStream_t s) mutable -> hipError_t {
-        sp.sched = (int32_t *)((char *)wsp + o_sched);
-        hipError_t e = cam::launch_build_sched(gc.group_list, gc.cumulative, (int)gc.G, gc.A, 1, &sp, s);
-        if (e != hipSuccess) {
-            return e;
-        }
-        g.sched = sp.sched;
-        if (!wire) {
-            return cam::launch_gemm(g, s);
-        }
         uint16_t *rows = (uint16_t *)((char *)wsp + o_rows);
-        g.out = rows;
-        e = cam::launch_gemm(g, s);
-        if (e != hipSuccess) {
+        if (wire) {
+            g.out = rows;
+        }
+        const int32_t *total = nullptr;
+        const hipError_t e = run_grouped_gemm(g, gc.group_list, gc.cumulative, gc.G, gc.A, sp, (char *)wsp + o_sched,
+                                              &total, s);
+        if (e != hipSuccess || !wire) {
             return e;
         }
-        return cam::launch_comm_quant(rows, 0, gc.A, g.N, sp.sched + 1, wire_out, s);  // sched[1]: rows that exist
+        return cam::launch_comm_quant(rows, 0, gc.A, g.N, total + 1, wire_out, s);  // [1]: rows that exist
     };
     return finish_phase1(kOpGmm2, c.off, run, workspaceSize, executor);
 }
@@ -1815,6 +1847,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     uint16_t *outp = (uint16_t *)output->data;
     int64_t *etn = (int64_t *)expertTokenNums->data;
     const int iT = (int)T, iK = (int)K, iH = (int)H, iI = (int)I, iE = (int)Epr;
+    const bool stream = cam::stream_gemm_applies(A, 2 * I);
 
     auto run = [=](void *wsp, hipStream_t s) -> hipError_t {
         char *w = (char *)wsp;
@@ -1860,14 +1893,16 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         d.quant = 2;
         d.out = x1;
         d.scales = x1s;
-        // the plan has written the per-expert counts: spare workgroups of the permute build both schedules
-        d.sched.group_list = etn;
-        d.sched.cumulative = 0;
-        d.sched.G = iE;
-        d.sched.nspec = 2;
-        d.sched.max_rows = A;
-        d.sched.spec[0] = specs[0];
-        d.sched.spec[1] = specs[1];
+        if (!stream) {
+            // the plan has written the per-expert counts: spare workgroups of the permute build both schedules
+            d.sched.group_list = etn;
+            d.sched.cumulative = 0;
+            d.sched.G = iE;
+            d.sched.nspec = 2;
+            d.sched.max_rows = A;
+            d.sched.spec[0] = specs[0];
+            d.sched.spec[1] = specs[1];
+        }
         e = cam::launch_dispatch(d, s);
         if (e != hipSuccess) return e;
 
@@ -1884,9 +1919,9 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         g1.gate_up = 1;
         g1.epilogue = cam::kEpiSwiglu;
         g1.out = prod;
-        e = cam::launch_gemm(g1, s);
+        e = layer_gemm(g1, etn, iE, A, iT, stream, s);
         if (e != hipSuccess) return e;
-        e = cam::launch_requant(prod, A, iI, specs[0].sched, x2, x2s, s);
+        e = cam::launch_requant(prod, A, iI, stream ? meta : specs[0].sched, x2, x2s, s);  // [1] of both: rows that exist
         if (e != hipSuccess) return e;
 
         cam::GemmArgs g2{};
@@ -1903,7 +1938,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         g2.epilogue = cam::kEpiDequantBf16;
         g2.out = y;
         g2.out_fp16 = x_is_fp16;
-        e = cam::launch_gemm(g2, s);
+        e = layer_gemm(g2, etn, iE, A, iT, stream, s);
         if (e != hipSuccess) return e;
 
         cam::CombineArgs cb{};
@@ -2047,13 +2082,8 @@ camStatus camGroupedMatmulFp8GetWorkspaceSize(const camTensor *x, const camTenso
     const int64_t *gl = (const int64_t *)groupList->data;
     const int cumulative = groupListType == 0;
     auto run = [=](void *wsp, hipStream_t s) mutable -> hipError_t {
-        sp.sched = (int32_t *)((char *)wsp + o_sched);
-        hipError_t e = cam::launch_build_sched(gl, cumulative, (int)G, A, 1, &sp, s);
-        if (e != hipSuccess) {
-            return e;
-        }
-        g.sched = sp.sched;
-        return cam::launch_gemm(g, s);
+        const int32_t *total = nullptr;
+        return run_grouped_gemm(g, gl, cumulative, G, A, sp, (char *)wsp + o_sched, &total, s);
     };
     return finish_phase1(kOpGmmFp8, c.off, run, workspaceSize, executor);
 }
@@ -2175,6 +2205,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
     uint16_t *outp = (uint16_t *)output->data;
     int64_t *etn = (int64_t *)expertTokenNums->data;
     const int iT = (int)T, iK = (int)K, iE = (int)E, iH = (int)H, iI = (int)I;
+    const bool stream = cam::stream_gemm_applies(A, 2 * I);
 
     auto run = [=](void *wsp, hipStream_t s) -> hipError_t {
         char *w = (char *)wsp;
@@ -2220,13 +2251,15 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         d.quant = 3;
         d.out = x1;
         d.scales = (float *)x1s;
-        d.sched.group_list = etn;  // spare workgroups of the permute build both schedules
-        d.sched.cumulative = 0;
-        d.sched.G = iE;
-        d.sched.nspec = 2;
-        d.sched.max_rows = A;
-        d.sched.spec[0] = specs[0];
-        d.sched.spec[1] = specs[1];
+        if (!stream) {
+            d.sched.group_list = etn;  // spare workgroups of the permute build both schedules
+            d.sched.cumulative = 0;
+            d.sched.G = iE;
+            d.sched.nspec = 2;
+            d.sched.max_rows = A;
+            d.sched.spec[0] = specs[0];
+            d.sched.spec[1] = specs[1];
+        }
         e = cam::launch_dispatch(d, s);
         if (e != hipSuccess) return e;
 
@@ -2243,7 +2276,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         g1.epilogue = cam::kEpiSwigluFp8;  // the SwiGLU product leaves GMM1 quantised for GMM2
         g1.out = x2;
         g1.out_scale8 = x2s;
-        e = cam::launch_gemm(g1, s);
+        e = layer_gemm(g1, etn, iE, A, iT, stream, s);
         if (e != hipSuccess) return e;
 
         cam::GemmArgs g2{};
@@ -2258,7 +2291,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         g2.gate_up = 0;
         g2.epilogue = cam::kEpiDequantBf16;
         g2.out = y;
-        e = cam::launch_gemm(g2, s);
+        e = layer_gemm(g2, etn, iE, A, iT, stream, s);
         if (e != hipSuccess) return e;
 
         cam::CombineArgs cb{};

@@ -190,6 +190,19 @@ struct GemmArgs {
 };
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t stream);
 
+// The same GEMM for few rows per expert (stream_gemm.hip): takes the row counts instead of a schedule (g.sched is
+// not used) and leaves kEpiInt32 to launch_gemm.
+struct StreamGemmArgs {
+    GemmArgs g;
+    const int64_t *group_list;  // [G] cumulative rows or rows per expert
+    int cumulative, G;
+    long long max_rows;         // rows of the tensors
+    int32_t *rows_out;          // optional: [1] receives the total row count (where launch_requant looks for it)
+};
+bool stream_gemm_applies(int64_t rows, int64_t N);  // whether it is the faster form
+// rows_per_expert: the most rows one expert can have, as far as the host knows.
+hipError_t launch_stream_gemm(const StreamGemmArgs &a, int64_t rows_per_expert, hipStream_t stream);
+
 // fp32 SwiGLU products [rows,I] -> int8 + per-row scale.  sched_for_rows: optional schedule whose header holds
 // the number of valid rows.
 hipError_t launch_requant(const float *y, int64_t max_rows, int I, const int32_t *sched_for_rows, int8_t *q,

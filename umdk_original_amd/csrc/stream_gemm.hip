@@ -1,0 +1,707 @@
+// Grouped w8a8 / FP8 GEMM for experts with few rows: a weight stream with the matrix cores beside it.
+//
+// Same operands, results and epilogues as gemm.hip (the reference's GMM1 / GMM2, cited there); this kernel is for
+// launches whose experts have so few rows that the weights are all the time goes into.  What bounds it is the rate at
+// which weight bytes arrive: HBM as a whole (7.05 TB/s for 1.5 GB of these loads with nothing else in the kernel, 6.7 for
+// 240 MB), and one CU at about 50 GB/s whatever the number of loads in flight, so a launch on fewer than half the CUs is
+// bound by the CUs.  The tile kernel of gemm.hip hands out 512-column panels over the whole K: 48 of them for one token
+// of a 128-expert layer (H 4096, I 1536, top-8), i.e. 48 of 256 CUs at work.
+//
+// Measured, tile kernel -> this one: that token's GMM1 (101 MB) 55.8 -> 21 us and GMM2 24.7 -> 13 us; 16 tokens on 16
+// experts (H 7168, I 2048): 123 -> 76 us (6.2 TB/s) and 41.5 -> 39 us; 512 rows over 124 experts, GMM1 248 -> 237 us
+// (6.6 TB/s); 1024 rows, where both are at 6.3 TB/s, no difference.
+//
+// Design.
+//   * An item is one row tile (32 or 128 rows) of one expert x P groups of 64 packed weight columns, chosen by the host so
+//     that there are items for every CU.  The eight waves of a workgroup are P columns of S = 8 / P: the S waves of a
+//     column group take every S-th 64-byte step of its K, so a workgroup always has eight streams of 4 KB steps, and
+//     the sums of the S waves meet in LDS at the end (int32: exact in any order; FP8: fp32 sums added in wave order).
+//   * Every weight byte is needed by exactly one wave, so it goes from memory to that wave's registers, non-temporal,
+//     with no LDS and no barrier on its way.  Each wave keeps two steps (8 KB) in flight; four made no difference.  The
+//     ring of two steps runs across items: while the last steps of an item are multiplied the first ones of the next are
+//     already requested.
+//   * The activation rows of the item lie in LDS, as much of K at a time as a buffer holds, double-buffered by
+//     direct-to-LDS loads; a barrier per chunk, not per step.  Pieces of 16 bytes are placed with an XOR of the row so
+//     that the fragment reads are free of bank conflicts.  The matrix cores are not what it waits for (without the
+//     multiplications the decode layer's launches take the same time).
+//   * No schedule: every workgroup derives the item list from the per-expert row counts by itself (a prefix sum over
+//     at most 512 experts) and takes items in a fixed order.  All items of a launch stream the same number of bytes,
+//     so nothing has to be balanced, and no builder runs before the GEMM.
+#include <algorithm>
+
+#include "cam_device.h"
+#include "cam_kernels.h"
+#include "permute_device.h"
+#include "rank_device.h"
+#include "../../include/cam_expf_spec.h"
+
+namespace cam {
+
+namespace {
+
+constexpr int kSThreads = 512;
+constexpr int R = 2;                     // 64-byte K steps in flight per wave
+constexpr int kSMaxKb = 64;              // FP8: K blocks of 128 bytes (Kd <= 8192)
+
+__device__ __forceinline__ void lds_barrier()
+{
+    // LDS traffic of this wave is done, weight loads stay in flight (a __syncthreads would drain them)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <typename T>
+__device__ __forceinline__ unsigned lds_addr(const T *p)
+{
+    return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) T *)p;
+}
+
+// A wave-uniform address the compiler does not know to be one, as a scalar register pair.
+__device__ __forceinline__ unsigned long long scalar_address(const void *p)
+{
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// The same value, computed anew as far as the compiler can tell: keeps loop-invariant address arithmetic out of registers.
+__device__ __forceinline__ int opaque(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+template <bool FP8>
+struct SAcc {
+    typedef v16i v16;
+    typedef v4i v4;
+};
+template <>
+struct SAcc<true> {
+    typedef v16f v16;
+    typedef v4f v4;
+};
+
+struct StreamItem {     // wave-uniform
+    int g, row0, rows;  // expert, first row, rows of the tile (0: there is no such item)
+    int blk;            // block of P column groups
+    int ckb, nch;       // bytes of K per activation chunk, chunks
+    const int8_t *w;    // this wave's first weight piece: expert, column group
+    int wstep;          // bytes from one 64-byte K step to the next
+};
+
+template <int MF, bool FP8, int P>
+__global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel(StreamGemmArgs sa)
+{
+    typedef typename SAcc<FP8>::v16 acc16;
+    typedef typename SAcc<FP8>::v4 acc4;
+    constexpr int kABuf = MF == 1 ? 32768 : 65536;  // one of the two activation buffers
+    constexpr int kSLds = 2 * kABuf;
+    constexpr int NFR = MF == 1 ? 1 : 2;            // column fragments whose partial sums (32 KB each) fit a buffer
+    const GemmArgs &a = sa.g;
+    __shared__ __attribute__((aligned(1024))) int8_t lds[kSLds];
+    __shared__ int tile_start[kMaxExperts + 1];  // row tiles of the experts before
+    __shared__ int first_row[kMaxExperts + 1];
+    __shared__ int scan_s[kSThreads / kWave];
+    __shared__ int total_s;
+    // scales of the current and of the next item: int8 column (per group: 64, or 32 gate + 32 up) and row scales
+    __shared__ __attribute__((aligned(16))) float col_scale_s[2][FP8 ? 4 : P * 64];
+    __shared__ __attribute__((aligned(16))) float row_scale_s[2][FP8 ? 4 : 32 * MF];
+    __shared__ __attribute__((aligned(16))) uint8_t a_scale8_s[2][FP8 ? kSMaxKb * 32 * MF : 4];
+    __shared__ uint8_t w_scale8_s[FP8 ? 16 * kSMaxKb : 4];
+    __shared__ float rowmax_s[FP8 ? 8 * 32 : 1];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int G = sa.G;
+    constexpr int S = 8 / P;
+    const int p = wave & (P - 1);      // this wave's column group of the item
+    const int s = wave / P;            // and its share of K: steps s, s + S, ...
+    const int Kd = a.Kd, N = a.N;
+    const int KT = Kd >> 6;
+    const int ngroups = N >> 6;
+    const int blocks = (ngroups + P - 1) / P;
+    const int turns = (KT + S * R - 1) / (S * R);   // turns of the ring per item
+    constexpr int quantum = S * R > 4 ? 64 * S * R : 256;  // K bytes of one turn of all S waves
+    static_assert(NFR == 2 || S >= 4, "sums that pass one fragment at a time wait in registers for one block only");
+    static_assert(32 * MF * quantum <= kABuf, "a turn of a full tile has to fit an activation buffer");
+    const int kpad = (Kd + quantum - 1) / quantum * quantum;
+
+    // ---- the item list: rows, first row and row tiles of every expert (thread e: expert e)
+    {
+        int m0 = 0, rows = 0;
+        if (tid < G) {
+            const long long v = min(max(sa.group_list[tid], (int64_t)0), (int64_t)sa.max_rows);
+            if (sa.cumulative) {
+                m0 = tid == 0 ? 0 : (int)min(max(sa.group_list[tid - 1], (int64_t)0), (int64_t)sa.max_rows);
+                rows = max((int)v - m0, 0);
+            } else {
+                rows = (int)v;
+            }
+        }
+        if (!sa.cumulative) {
+            m0 = block_exclusive_scan<kSThreads / kWave>(rows, tid, scan_s, &total_s);
+            m0 = min(max(m0, 0), (int)sa.max_rows);
+            rows = min(rows, (int)sa.max_rows - m0);
+        }
+        const int tiles = (rows + 32 * MF - 1) / (32 * MF);
+        const int ts = block_exclusive_scan<kSThreads / kWave>(tiles, tid, scan_s, &total_s);
+        if (tid <= G) {
+            tile_start[tid] = ts;
+            first_row[tid] = m0;
+        }
+        if (tid == 0) {
+            tile_start[G] = total_s;   // (for G == 512, which no thread has)
+        }
+        __syncthreads();
+        if (sa.rows_out != nullptr && blockIdx.x == 0 && tid == G - 1) {
+            sa.rows_out[1] = m0 + rows;  // the rows the next kernel finds (the lists are ascending)
+        }
+        if (tid < G) {
+            // where the expert's rows end: kept in the slot after its first row's (experts are contiguous)
+            if (tid == G - 1) {
+                first_row[G] = m0 + rows;
+            }
+        }
+        __syncthreads();
+    }
+    const int n_items = tile_start[G] * blocks;
+
+    // Workgroup i runs on XCD i % 8.  Every XCD has an eighth of the list to itself and its workgroups walk through it side by
+    // side: the row tiles and column blocks of an expert meet in one L2 instead of being fetched by all eight (the decode
+    // layer's GMM1, 1024 rows over 128 experts: 261 -> 252 us; 512 rows over 16 experts with 32-row tiles: 110 -> 99 us).
+    const int xcd = (int)blockIdx.x & (kNumXcd - 1);
+    const int end_item = (int)((long long)n_items * (xcd + 1) / kNumXcd);
+    const int item_step = ((int)gridDim.x - xcd + kNumXcd - 1) / kNumXcd;
+    auto find_item = [&](int i) -> StreamItem {
+        StreamItem it;
+        it.g = 0; it.row0 = 0; it.rows = 0; it.blk = 0; it.ckb = quantum; it.nch = 1; it.w = nullptr; it.wstep = 0;
+        if (i >= end_item) {
+            return it;
+        }
+        const int q = i / blocks;      // a tile of the expert the item belongs to
+        int g = 0;                     // experts whose tiles all lie before
+        for (int base = 0; base < G; base += kWave) {
+            const int e = base + lane;
+            g += __popcll(__ballot(e < G && tile_start[min(e, G - 1) + 1] <= q));
+        }
+        g = __builtin_amdgcn_readfirstlane(min(g, G - 1));
+        const int ts = __builtin_amdgcn_readfirstlane(tile_start[g]);
+        const int tiles = __builtin_amdgcn_readfirstlane(tile_start[g + 1]) - ts;
+        const int fr = __builtin_amdgcn_readfirstlane(first_row[g]);
+        const int er = __builtin_amdgcn_readfirstlane(first_row[g + 1]);
+        const int local = i - ts * blocks;
+        int blk = local, j = 0;        // the row tiles of a column block side by side: they share its weights
+        if (tiles > 1) {
+            blk = local / tiles;
+            j = local - blk * tiles;
+        }
+        it.g = g;
+        it.blk = blk;
+        it.row0 = fr + j * 32 * MF;
+        it.rows = min(er - it.row0, 32 * MF);
+        const int fit = kABuf / max(it.rows, 1) / quantum * quantum;
+        it.ckb = min(max(fit, quantum), kpad);
+        it.nch = (Kd + it.ckb - 1) / it.ckb;
+        const int nw = min(blk * P + p, ngroups - 1);
+        const int b8 = nw >> 3;
+        it.wstep = min(8, ngroups - 8 * b8) * 4096;
+        const int8_t *wg = a.per_expert ? a.list.w[g] : a.w + (long long)g * Kd * N;
+        it.w = wg + (long long)b8 * 8 * Kd * 64 + (nw & 7) * 4096;
+        return it;
+    };
+
+    // ---- weights: step R q + r of this wave in ring[r]
+    v8i ring[R][2];  // [step][fragment]: .lo the first 32 K bytes of the step, .hi the second
+    // Buffer loads, because a wave requests steps that do not exist, too: past the end of its share of K and after the
+    // last item.  With zero records such a load is dropped on its way, without a branch around the requests: a branch
+    // would make the compiler wait for the younger of the two steps wherever it needs the older.
+    const int voff = lane * 16;
+    auto issue = [&](int r, const StreamItem &it, int q) {
+        const int t = s + (R * q + r) * S;
+        const bool there = it.rows > 0 && t < KT;
+        const __amdgpu_buffer_rsrc_t rsrc =
+            __builtin_amdgcn_make_buffer_rsrc((void *)it.w, 0, there ? 0x7fffffff : 0, 0x00020000);
+        const int soff = there ? t * it.wstep : 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const v4i piece = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff + j * 1024, soff, 2));
+            if (j < 2) {
+                ring[r][j].lo = piece;
+            } else {
+                ring[r][j - 2].hi = piece;
+            }
+        }
+    };
+
+    // ---- activations: chunk c of an item straight into LDS buffer `buf`.  16-byte piece i of the chunk (row i / pieces per
+    // row) lands at 16 i; which piece of its row that is follows from the XOR, so it is chosen on the global side.
+    auto load_a = [&](const StreamItem &it, int c, int buf) {
+        const int tid = opaque((int)threadIdx.x);
+        const int slots = it.ckb >> 4;
+        const float inv = 1.0f / (float)slots;
+        const int8_t *base = a.a + (long long)it.row0 * Kd;
+        for (int q = 0; q * kSThreads < it.rows * slots; ++q) {
+            const int idx = tid + q * kSThreads;
+            const int row = (int)(((float)idx + 0.5f) * inv);   // idx < 4096: exact
+            const int ls = (idx - row * slots) ^ (row & 15);
+            const unsigned off = (unsigned)(row * Kd + min(c * it.ckb + ls * 16, Kd - 16));
+            const unsigned dst = lds_addr(lds) + (unsigned)(buf * kABuf + (q * 8 + wave) * 1024);
+            if (row < it.rows) {
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                             :
+                             : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(scalar_address(base))
+                             : "memory", "m0");
+            }
+        }
+    };
+
+    // ---- scales of an item into set `set`, requested with the activations so that no epilogue waits for them.  (Loaded in
+    // the epilogue they wait behind the ring, which stands still meanwhile: 12 us of a 137 us launch of 1024 items.)
+    // int8: column and row scales straight to LDS.  FP8: the tile's rows of block scales as they lie in memory
+    // (a_scale8_s[row * KB + kb]; whole words straight to LDS), and 2 P rows of K blocks of the weight through registers.
+    constexpr int kWQ = FP8 ? 16 * kSMaxKb / kSThreads : 1;
+    uint8_t wreg[kWQ];
+    const int KB = Kd >> 7;
+    const bool words = (KB & 3) == 0;   // a row's scales are whole words
+    auto load_scales = [&](const StreamItem &it, int set) {
+        const int tid = opaque((int)threadIdx.x);
+        if (!FP8) {
+            const float *sg = a.per_expert ? a.list.s[it.g] : a.w_scale + (long long)it.g * N;
+            if (tid < P * 16) {
+                const int grp = min(it.blk * P + (tid >> 4), ngroups - 1);
+                const int c4 = (tid & 15) * 4;
+                const int col = a.gate_up ? grp * 32 + (c4 < 32 ? c4 : c4 - 32 + (N >> 1)) : grp * 64 + c4;
+                const unsigned dst = lds_addr(&col_scale_s[set][0]) + (unsigned)(wave * 1024);
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                             :
+                             : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"((unsigned)(col * 4)), "s"(scalar_address(sg))
+                             : "memory", "m0");
+            }
+            const int r = tid - 128;        // the waves from the third on: a row each lane
+            if (r >= 0 && r < it.rows) {
+                const unsigned dst = lds_addr(&row_scale_s[set][0]) + (unsigned)((wave - 2) * 256);
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                             :
+                             : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"((unsigned)(r * 4)), "s"(scalar_address(a.a_scale + it.row0))
+                             : "memory", "m0");
+            }
+            return;
+        }
+        if (words) {
+            const int n = it.rows * KB >> 2;
+            for (int q = 0; q * kSThreads < n; ++q) {
+                const int idx = tid + q * kSThreads;
+                if (idx < n) {
+                    const unsigned dst = lds_addr(&a_scale8_s[set][0]) + (unsigned)((q * 8 + wave) * 256);
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                                 :
+                                 : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"((unsigned)(idx * 4)), "s"(scalar_address(a.a_scale8 + (long long)it.row0 * KB))
+                                 : "memory", "m0");
+                }
+            }
+        }
+        const int nblk = N >> 7;
+        const float inv = 1.0f / (float)KB;
+#pragma unroll
+        for (int q = 0; q < kWQ; ++q) {
+            const int idx = tid + q * kSThreads;
+            const int gf = (int)(((float)idx + 0.5f) * inv);    // column group of the item * 2 + fragment
+            if (gf < 2 * P) {
+                const int grp = min(it.blk * P + (gf >> 1), ngroups - 1);
+                const int nf = gf & 1;
+                const int col = a.gate_up ? nf * (N / 2) + grp * 32 : grp * 64 + nf * 32;
+                wreg[q] = a.w_scale8[((long long)it.g * KB + (idx - gf * KB)) * nblk + (col >> 7)];
+            }
+        }
+    };
+    auto store_scales = [&](const StreamItem &it, int set) {
+        if (!FP8) {
+            return;
+        }
+        const int tid = opaque((int)threadIdx.x);
+        if (!words) {
+            for (int idx = tid; idx < it.rows * KB; idx += kSThreads) {
+                a_scale8_s[set][idx] = a.a_scale8[(long long)it.row0 * KB + idx];
+            }
+        }
+        const float inv = 1.0f / (float)KB;
+#pragma unroll
+        for (int q = 0; q < kWQ; ++q) {
+            const int idx = tid + q * kSThreads;
+            const int gf = (int)(((float)idx + 0.5f) * inv);
+            if (gf < 2 * P) {
+                w_scale8_s[gf * kSMaxKb + (idx - gf * KB)] = wreg[q];
+            }
+        }
+    };
+
+    // The youngest requests of a wave are its ring (4 pieces a step, younger than the activations): with no more than
+    // those outstanding, its share of the activations has landed.
+    auto a_landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * R) : "memory"); };
+
+    int set = 0;  // the set of scales in use, one per item in turn
+    int buf = 0;  // the activation buffer in use; chunks take turns, across items too
+    int item = (int)((long long)n_items * xcd / kNumXcd) + (int)blockIdx.x / kNumXcd;
+    StreamItem cur = find_item(item);
+    if (cur.rows <= 0) {
+        return;
+    }
+    load_a(cur, 0, 0);
+    load_scales(cur, 0);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        issue(r, cur, 0);
+    }
+    store_scales(cur, 0);
+    a_landed();
+    lds_barrier();
+
+    for (;;) {
+        item += item_step;
+        StreamItem nxt = find_item(item);
+        const bool more = nxt.rows > 0;
+
+        acc16 acc[MF][2];
+#pragma unroll
+        for (int mf = 0; mf < MF; ++mf) {
+#pragma unroll
+            for (int nf = 0; nf < 2; ++nf) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    acc[mf][nf][i] = 0;
+                }
+            }
+        }
+        int rowoff[MF];    // LDS offset of this lane's row of each fragment; rows that do not exist repeat the last
+        int rowx[MF];
+#pragma unroll
+        for (int mf = 0; mf < MF; ++mf) {
+            const int row = min(mf * 32 + (lane & 31), cur.rows - 1);
+            rowoff[mf] = row * cur.ckb;
+            rowx[mf] = row & 15;
+        }
+        const int half = lane >> 5;
+        const int turns_per_chunk = cur.ckb / (64 * S * R);
+
+        for (int c = 0; c < cur.nch; ++c) {
+            const bool last_chunk = c + 1 == cur.nch;
+            buf ^= c == 0 ? 0 : 1;
+            if (!last_chunk) {
+                load_a(cur, c + 1, buf ^ 1);
+            } else if (more) {
+                load_a(nxt, 0, buf ^ 1);
+                load_scales(nxt, set ^ 1);
+            }
+            const int8_t *abuf = lds + buf * kABuf;
+            const int q1 = min(turns, (c + 1) * turns_per_chunk);
+            const int t0 = c * (cur.ckb >> 6);
+            for (int q = c * turns_per_chunk; q < q1; ++q) {
+                const bool wrap = q + 1 == turns;
+                const StreamItem &src = wrap ? nxt : cur;
+                const int qn = wrap ? 0 : q + 1;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int t = s + (R * q + r) * S;
+                    if (t < KT) {
+                        const int slot = (t - t0) * 4 + half;
+                        const v8i(&bf)[2] = ring[r];
+                        int sw[2] = {0, 0};
+                        if (FP8) {
+                            sw[0] = w_scale8_s[(p * 2 + 0) * kSMaxKb + (t >> 1)];
+                            sw[1] = w_scale8_s[(p * 2 + 1) * kSMaxKb + (t >> 1)];
+                        }
+#pragma unroll
+                        for (int mf = 0; mf < MF; ++mf) {
+                            if (mf > 0 && mf * 32 >= cur.rows) {
+                                continue;
+                            }
+                            v8i af;
+                            af.lo = *(const v4i *)(abuf + rowoff[mf] + ((slot ^ rowx[mf]) << 4));
+                            af.hi = *(const v4i *)(abuf + rowoff[mf] + (((slot + 2) ^ rowx[mf]) << 4));
+                            if constexpr (FP8) {
+                                const int sx = a_scale8_s[set][min(mf * 32 + (lane & 31), cur.rows - 1) * KB + (t >> 1)];
+#pragma unroll
+                                for (int nf = 0; nf < 2; ++nf) {
+                                    acc[mf][nf] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[nf], af, acc[mf][nf], 0, 0,
+                                                                                                  0, sw[nf], 0, sx);
+                                }
+                            } else {
+#pragma unroll
+                                for (int nf = 0; nf < 2; ++nf) {
+                                    acc[mf][nf] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[nf].lo, af.lo, acc[mf][nf], 0, 0, 0);
+                                }
+#pragma unroll
+                                for (int nf = 0; nf < 2; ++nf) {
+                                    acc[mf][nf] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[nf].hi, af.hi, acc[mf][nf], 0, 0, 0);
+                                }
+                            }
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    issue(r, src, qn);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            a_landed();
+            lds_barrier();  // the chunk has been read, and the next one has landed
+        }
+
+        // ---- the S partial sums of a column group meet in LDS, in the buffer that was read last, 32 rows at a time and
+        // NFR column fragments at a time.  Register quad j of a fragment nf, lane l, is row l % 32, columns 8 j + 4 (l / 32)
+        // .. + 3; it goes to a 16-byte chunk whose row is XORed so that neither the writes nor the reads below meet in
+        // a bank.  Then eight lanes own a row (lane l: row l / 8 of a block of eight, piece l % 8), so that every row leaves in
+        // whole 128-byte lines, and the waves of the column group share the four blocks.
+        const int nw = cur.blk * P + p;
+        const bool live = nw < ngroups;
+        // (the compiler would keep every lane-dependent address below in registers through the whole K loop)
+        const int lane = opaque(tid) & (kWave - 1);
+        constexpr int BPW = S >= 4 ? 1 : 4 / S;   // blocks of eight rows per wave (the first four waves when S == 8)
+        const int piece = lane & 7;
+        const int I = N >> 1;
+        const bool swiglu = a.epilogue != kEpiDequantBf16;
+#pragma unroll
+        for (int mf = 0; mf < MF; ++mf) {
+            if (mf > 0 && mf * 32 >= cur.rows) {   // no such rows (cur.rows is the same in every wave)
+                continue;
+            }
+            acc4 lo, hi;   // SwiGLU: gate and up of columns 4 piece .. + 3; else columns 8 piece .. + 3 and + 4 .. + 7
+            v4f keep[BPW];   // kEpiSwigluFp8: the products until their block's maximum is known
+#pragma unroll
+            for (int n0 = 0; n0 < 2; n0 += NFR) {
+                if (mf + n0 > 0) {
+                    lds_barrier();  // the sums before these have been read
+                }
+                acc4 *const sums = (acc4 *)(lds + buf * kABuf);
+                {
+                    const int row = lane & 31, half2 = lane >> 5;
+                    if (mf * 32 + row < cur.rows) {
+#pragma unroll
+                        for (int nf = n0; nf < n0 + NFR; ++nf) {
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                sums[((wave * NFR + nf - n0) * 4 + j) * kWave + half2 * 32 + (row ^ ((2 * j + (half2 ^ nf)) << 1))] =
+                                    acc4{acc[mf][nf][4 * j], acc[mf][nf][4 * j + 1], acc[mf][nf][4 * j + 2], acc[mf][nf][4 * j + 3]};
+                            }
+                        }
+                    }
+                }
+                if (S > 1) {
+                    lds_barrier();
+                } else {
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // a wave reads what it wrote itself
+                }
+                auto read_sum = [&](int nf, int j, int half2, int row) -> acc4 {
+                    const acc4 *src = sums + ((p * NFR + nf - n0) * 4 + j) * kWave + half2 * 32 + (row ^ ((2 * j + (half2 ^ nf)) << 1));
+                    acc4 v = src[0];
+#pragma unroll
+                    for (int ss = 1; ss < S; ++ss) {
+                        v += src[ss * P * NFR * 4 * kWave];
+                    }
+                    return v;
+                };
+#pragma unroll
+                for (int b = 0; b < BPW; ++b) {
+                    const int row = (s * BPW + b) * 8 + (lane >> 3);
+                    if (s < 4 && live && mf * 32 + row < cur.rows) {
+                        if (swiglu) {
+                            if (NFR == 2 || n0 == 0) {
+                                lo = read_sum(0, piece >> 1, piece & 1, row);
+                            }
+                            if (NFR == 2 || n0 == 1) {
+                                hi = read_sum(1, piece >> 1, piece & 1, row);
+                            }
+                        } else if (NFR == 2 || (piece >> 2) == n0) {
+                            lo = read_sum(piece >> 2, piece & 3, 0, row);
+                            hi = read_sum(piece >> 2, piece & 3, 1, row);
+                        }
+                    }
+                    if (n0 + NFR < 2) {
+                        continue;   // one fragment at a time (a wave has one block then): the other is still to come
+                    }
+                        const int trow = mf * 32 + row;
+                        const long long grow = cur.row0 + trow;
+                        const bool mine = s < 4 && live && trow < cur.rows;
+                        const float xs = FP8 || !mine ? 1.0f : row_scale_s[set][trow];
+                        if (swiglu) {
+                            v4f y = {0.0f, 0.0f, 0.0f, 0.0f};
+                            float m = 0.0f;
+                            if (mine) {
+                                const v4f sgate = FP8 ? v4f{} : *(const v4f *)&col_scale_s[set][FP8 ? 0 : p * 64 + piece * 4];
+                                const v4f sup = FP8 ? v4f{} : *(const v4f *)&col_scale_s[set][FP8 ? 0 : p * 64 + 32 + piece * 4];
+        #pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    float tg, tu;
+                                    if constexpr (FP8) {
+                                        tg = lo[e];
+                                        tu = hi[e];
+                                    } else {
+                                        tg = __fmul_rn(__fmul_rn((float)lo[e], sgate[e]), xs);
+                                        tu = __fmul_rn(__fmul_rn((float)hi[e], sup[e]), xs);
+                                    }
+                                    y[e] = __fmul_rn(cam_silu_spec(tg), tu);
+                                    m = fmaxf(m, fabsf(y[e]));
+                                }
+                                if (a.epilogue == kEpiSwiglu) {
+                                    *(v4f *)((float *)a.out + grow * I + nw * 32 + piece * 4) = y;
+                                }
+                            }
+                            if constexpr (FP8 && P >= 4) {
+                                if (a.epilogue == kEpiSwigluFp8) {
+                                    keep[b] = y;
+                                    m = fmaxf(m, __shfl_xor(m, 1, kWave));
+                                    m = fmaxf(m, __shfl_xor(m, 2, kWave));
+                                    m = fmaxf(m, __shfl_xor(m, 4, kWave));
+                                    if (piece == 0 && s < 4) {
+                                        rowmax_s[p * 32 + row] = m;
+                                    }
+                                }
+                            }
+                        } else if (mine) {
+                            const int col = nw * 64 + piece * 8;
+                            const v4f w0 = FP8 ? v4f{} : *(const v4f *)&col_scale_s[set][FP8 ? 0 : p * 64 + piece * 8];
+                            const v4f w1 = FP8 ? v4f{} : *(const v4f *)&col_scale_s[set][FP8 ? 0 : p * 64 + piece * 8 + 4];
+                            float f[8];
+        #pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                if constexpr (FP8) {
+                                    f[e] = lo[e];
+                                    f[4 + e] = hi[e];
+                                } else {
+                                    f[e] = __fmul_rn(__fmul_rn((float)lo[e], w0[e]), xs);
+                                    f[4 + e] = __fmul_rn(__fmul_rn((float)hi[e], w1[e]), xs);
+                                }
+                            }
+                            v4u o;
+        #pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                o[e] = a.out_fp16 ? f32_to_fp16_bits(f[2 * e]) | (f32_to_fp16_bits(f[2 * e + 1]) << 16)
+                                                  : f32x2_to_bf16x2_bits(f[2 * e], f[2 * e + 1]);
+                            }
+                            *(v4u *)((uint16_t *)a.out + grow * N + col) = o;
+                        }
+                }
+            }
+            if constexpr (FP8 && P >= 4) {
+                if (a.epilogue == kEpiSwigluFp8) {
+                    // a block of 128 product columns is four neighbouring column groups (P is 4 or 8 here)
+                    lds_barrier();
+#pragma unroll
+                    for (int b = 0; b < BPW; ++b) {
+                        const int row = (s * BPW + b) * 8 + (lane >> 3);
+                        const long long grow = cur.row0 + mf * 32 + row;
+                        if (!live || mf * 32 + row >= cur.rows) {
+                            continue;
+                        }
+                        const float *rm = rowmax_s + (p & 4) * 32 + row;
+                        const int ex = fp8_block_scale_exp(fmaxf(fmaxf(rm[0], rm[32]), fmaxf(rm[64], rm[96])));
+                        const float f1 = exp2_int(-(ex / 2)), f2 = exp2_int(-(ex - ex / 2));
+                        int w = 0;
+                        w = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(__fmul_rn(keep[b][0], f1), f2),
+                                                            __fmul_rn(__fmul_rn(keep[b][1], f1), f2), w, false);
+                        w = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(__fmul_rn(keep[b][2], f1), f2),
+                                                            __fmul_rn(__fmul_rn(keep[b][3], f1), f2), w, true);
+                        *(int *)((uint8_t *)a.out + grow * I + nw * 32 + piece * 4) = w;
+                        if ((p & 3) == 0 && piece == 0) {
+                            a.out_scale8[grow * (I >> 7) + (nw >> 2)] = (uint8_t)(ex + 127);
+                        }
+                    }
+                    lds_barrier();  // rowmax_s is free again
+                }
+            }
+        }
+        if (!more) {
+            return;
+        }
+        store_scales(nxt, set ^ 1);
+        lds_barrier();  // the partial sums have been read, the next item's scales are in place
+        buf ^= 1;
+        set ^= 1;
+        cur = nxt;
+    }
+}
+
+template <int MF, bool FP8, int P>
+void launch_kernel(unsigned grid, hipStream_t stream, const StreamGemmArgs &sa)
+{
+    hipLaunchKernelGGL((stream_gemm_kernel<MF, FP8, P>), dim3(grid), dim3(kSThreads), 0, stream, sa);
+}
+
+template <bool FP8>
+void launch_variant(int mf, int P, unsigned grid, hipStream_t stream, const StreamGemmArgs &sa)
+{
+    if (mf == 1) {
+        P == 1 ? launch_kernel<1, FP8, 1>(grid, stream, sa) : launch_kernel<1, FP8, 2>(grid, stream, sa);
+    } else if (P == 2) {
+        launch_kernel<4, FP8, 2>(grid, stream, sa);
+    } else {
+        P == 4 ? launch_kernel<4, FP8, 4>(grid, stream, sa) : launch_kernel<4, FP8, 8>(grid, stream, sa);
+    }
+}
+
+}  // namespace
+
+// Rows x columns up to which the stream is the faster form: 64 rows per expert where the tile kernel has half as many
+// 512-column items as CUs, 32 where it has as many, 10 where it has three times as many (measured with the shapes of
+// DeepSeek-V3's, Qwen3's and smaller layers, 2 to 3072 rows; the two forms are within 5 % of each other along this line).
+bool stream_gemm_applies(int64_t rows, int64_t N)
+{
+    constexpr int64_t kMostRowsTimesColumns = 32ll * 512 * 256;
+    return rows > 0 && rows * N <= kMostRowsTimesColumns;
+}
+
+hipError_t launch_stream_gemm(const StreamGemmArgs &sa, int64_t rows_per_expert, hipStream_t stream)
+{
+    const GemmArgs &g = sa.g;
+    if (sa.group_list == nullptr || sa.G <= 0 || sa.G > kMaxExperts || sa.max_rows <= 0 || g.Kd % 128 != 0 || g.Kd < 128 ||
+        g.N % 64 != 0 || (g.gate_up && g.N % 128 != 0) || g.epilogue == kEpiInt32) {
+        return hipErrorInvalidValue;
+    }
+    if (g.fp8 && (g.N % 128 != 0 || (g.gate_up && g.N % 256 != 0) || g.Kd / 128 > kSMaxKb || g.per_expert ||
+                  g.a_scale8 == nullptr || g.w_scale8 == nullptr)) {
+        return hipErrorInvalidValue;
+    }
+    if (g.epilogue == kEpiSwigluFp8 && (!g.fp8 || !g.gate_up || g.out_scale8 == nullptr)) {
+        return hipErrorInvalidValue;
+    }
+    int cus = 0;
+    const hipError_t e = gemm_workgroups(&cus);
+    if (e != hipSuccess) {
+        return e;
+    }
+    // live experts at most, and the column groups they stream
+    const long long live = std::min<long long>(sa.G, sa.max_rows);
+    const long long groups = live * (g.N / 64);
+    const bool many = groups >= 6ll * cus;
+    // 32-row tiles, two workgroups per CU, while the stream is short: few column groups and no expert with more rows, or
+    // all tiles resident at once.  Otherwise 128-row tiles, so that an expert's weights are read once.
+    const bool quad = g.fp8 && g.gate_up;
+    const bool small = !quad &&
+                       ((rows_per_expert <= 32 && !many) || groups + sa.max_rows / 32 * (g.N / 64) <= 2ll * cus);
+    // Column groups per item: as few as it takes to give every CU work, then up to a megabyte of weights per item (an
+    // item's sums and stores interrupt its stream for about two microseconds).  kEpiSwigluFp8 needs the four groups
+    // of a 128-column block together, and the fp32 products of kEpiSwiglu are the same sums in the same order (quad).
+    int P = 2;
+    if (small) {
+        P = 2 * groups >= 3ll * cus ? 2 : 1;
+    } else if (many) {
+        P = 512ll * g.Kd <= (1 << 20) ? 8 : 4;
+    } else if (quad) {
+        P = 4;
+    }
+    const long long tiles = live + sa.max_rows / (small ? 32 : 128);
+    const long long items = tiles * ((g.N / 64 + P - 1) / P);
+    // a multiple of eight workgroups: every XCD takes an eighth of the items
+    const unsigned grid = (unsigned)((std::min<long long>(items, (small ? 2ll : 1ll) * cus) + kNumXcd - 1) / kNumXcd * kNumXcd);
+    if (g.fp8) {
+        launch_variant<true>(small ? 1 : 4, P, grid, stream, sa);
+    } else {
+        launch_variant<false>(small ? 1 : 4, P, grid, stream, sa);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace cam
