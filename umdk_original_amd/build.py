@@ -1,5 +1,6 @@
 """Builds libcam_mi355x.so (HIP kernels + C ABI) for gfx950 with hipcc, and libcam_torch_ops.so (the C++
-registration of torch.ops.umdk_cam_op_lib on top of that ABI) with the host compiler, both in-tree.
+registration of torch.ops.umdk_cam_op_lib on top of that ABI) and _cam_native.so (the Python module behind ops.py) with
+the host compiler, all in-tree.
 
 `python -m umdk_original_amd.build --timeline` builds a second library beside them, libcam_mi355x_timeline.so:
 the same sources with -DCAM_GEMM_TIMELINE, whose grouped-GEMM kernel stamps every tile of its schedule with
@@ -58,7 +59,7 @@ def build(verbose=False, timeline=False):
     if not timeline:
         build_calib(verbose)
         build_abi_consumer(verbose)
-        build_torch_ops(verbose)
+        build_torch_libraries(verbose)
     return out_path
 
 
@@ -91,28 +92,40 @@ def build_calib(verbose=False):
 
 
 TORCH_OPS_PATH = os.path.join(LIB_DIR, "libcam_torch_ops.so")
+NATIVE_PATH = os.path.join(LIB_DIR, "_cam_native.so")
 
 
-def build_torch_ops(verbose=False):
-    """The torch operator library: host C++ only (no device code), linked against torch and libcam_mi355x.so."""
+def _torch_cxx(source, output, libs, includes=()):
+    """The host compiler's command for a library against torch and libcam_mi355x.so (no device code)."""
     import torch
     from torch.utils import cpp_extension
     tdir = os.path.dirname(os.path.abspath(torch.__file__))
-    cxx = os.environ.get("CXX", "g++")
-    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
-    for inc in cpp_extension.include_paths() + ["/opt/rocm/include"]:
+    for inc in cpp_extension.include_paths() + ["/opt/rocm/include"] + list(includes):
         cmd += ["-I", inc]
-    cmd += [os.path.join(_CSRC, "torch_binding.cpp"), "-o", TORCH_OPS_PATH,
-            "-L", os.path.join(tdir, "lib"), "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_hip",
-            "-L", LIB_DIR, "-lcam_mi355x", "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + os.path.join(tdir, "lib")]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    if p.returncode != 0:
-        raise RuntimeError("building %s failed:\n%s" % (TORCH_OPS_PATH, p.stdout))
-    return TORCH_OPS_PATH
+    return cmd + [os.path.join(_CSRC, source), "-o", output, "-L", os.path.join(tdir, "lib"), "-ltorch", "-ltorch_cpu", "-lc10",
+                  "-lc10_hip", "-ltorch_hip"] + libs + ["-L", LIB_DIR, "-lcam_mi355x", "-Wl,-rpath,$ORIGIN",
+                                                        "-Wl,-rpath," + os.path.join(tdir, "lib")]
+
+
+def build_torch_libraries(verbose=False):
+    """The torch operator library and the Python module behind ops.py: host C++ only, linked against torch and
+    libcam_mi355x.so."""
+    import sysconfig
+    jobs = [(TORCH_OPS_PATH, _torch_cxx("torch_binding.cpp", TORCH_OPS_PATH, ["-lamdhip64"])),
+            (NATIVE_PATH, _torch_cxx("py_native.cpp", NATIVE_PATH, ["-ltorch_python", "-lamdhip64"],
+                                     [sysconfig.get_paths()["include"]]))]
+    procs = []
+    for path, cmd in jobs:
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        procs.append((path, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+    for path, p in procs:
+        out, _ = p.communicate()
+        if p.returncode != 0:
+            raise RuntimeError("building %s failed:\n%s" % (path, out))
 
 
 if __name__ == "__main__":

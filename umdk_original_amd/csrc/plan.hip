@@ -26,6 +26,12 @@ namespace {
 constexpr int kScanThreads = 1024;  // single-workgroup scan kernel (notify)
 constexpr int kGlobalThreads = 512; // phase 2: one thread per expert column
 
+// The per-expert counts may lie in host memory a CPU is watching (each count on its own): stored for the whole system.
+__device__ __forceinline__ void store_count(int64_t *p, int v)
+{
+    __hip_atomic_store(p, (int64_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Phase 1.  Workgroup b ranks the flat entries [b*chunk, (b+1)*chunk), chunk = IT*256 (rank_chunk), and
 // publishes the chunk's per-expert histogram in hist_out[b][*].
 template <typename IdT, int IT>
@@ -144,7 +150,7 @@ __global__ __launch_bounds__(kGlobalThreads) void plan_global_kernel(PlanArgs a,
         if (a.off) a.off[tid] = off;
         if (a.recv_off) a.recv_off[tid] = off;
         if (a.recv_count) a.recv_count[tid] = off + cnt;
-        if (a.tokens_per_expert) a.tokens_per_expert[tid] = cnt;
+        if (a.tokens_per_expert) store_count(a.tokens_per_expert + tid, cnt);
         if (a.group_list) a.group_list[tid] = (int64_t)off + cnt;
     }
     if (tid == 0 && a.total) {
@@ -201,7 +207,7 @@ __global__ __launch_bounds__(kLocalThreads) void plan_single_kernel(PlanArgs a)
             if (a.off) a.off[e] = o2[h];
             if (a.recv_off) a.recv_off[e] = o2[h];
             if (a.recv_count) a.recv_count[e] = o2[h] + c2[h];
-            if (a.tokens_per_expert) a.tokens_per_expert[e] = c2[h];
+            if (a.tokens_per_expert) store_count(a.tokens_per_expert + e, c2[h]);
             if (a.group_list) a.group_list[e] = (int64_t)o2[h] + c2[h];
         }
     }

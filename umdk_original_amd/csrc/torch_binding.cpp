@@ -22,9 +22,6 @@
 // and fused_deep_moe accepts only weights that live in such a storage: views of a packed tensor pass, a copy
 // made by clone() or to() does not (its bytes would still be packed, but nothing says so) and is refused with a
 // message instead of being multiplied as if it were row-major.
-#include <ATen/ATen.h>
-#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
-#include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 
@@ -33,40 +30,21 @@
 #include <unordered_map>
 #include <vector>
 
-#include "../../include/cam_mi355x.h"
+#include "torch_util.h"
 
 namespace {
 
-int32_t cam_dtype(const at::Tensor &t)
-{
-    switch (t.scalar_type()) {
-        case at::kFloat: return CAM_DT_FLOAT;
-        case at::kHalf: return CAM_DT_FLOAT16;
-        case at::kChar: return CAM_DT_INT8;
-        case at::kInt: return CAM_DT_INT32;
-        case at::kByte: return CAM_DT_UINT8;
-        case at::kLong: return CAM_DT_INT64;
-        case at::kBool: return CAM_DT_BOOL;
-        case at::kBFloat16: return CAM_DT_BF16;
-        case at::kFloat8_e4m3fn: return CAM_DT_FLOAT8_E4M3FN;
-        default: TORCH_CHECK(false, "umdk_cam_op_lib: unsupported dtype ", t.scalar_type());
-    }
-}
+using cam_torch::HostCounts;
+using cam_torch::new_empty;
+using cam_torch::Phase2;
 
 camTensor to_cam(const at::Tensor &t, int32_t format = CAM_FORMAT_ND)
 {
     TORCH_CHECK(t.is_cuda(), "umdk_cam_op_lib: tensors must live on a ROCm device (the CAM kernels have no CPU path)");
     TORCH_CHECK(t.dim() <= CAM_MAX_DIMS, "umdk_cam_op_lib: too many dimensions");
-    camTensor c{};
-    c.data = t.data_ptr();
-    c.dtype = cam_dtype(t);
-    c.ndim = (int32_t)t.dim();
-    for (int64_t d = 0; d < t.dim(); ++d) {
-        c.sizes[d] = t.size(d);
-        c.strides[d] = t.stride(d);
-    }
-    c.format = format;
-    return c;
+    const int32_t dtype = cam_torch::cam_dtype(t.scalar_type());
+    TORCH_CHECK(dtype >= 0, "umdk_cam_op_lib: unsupported dtype ", t.scalar_type());
+    return cam_torch::view_of(t, dtype, format);
 }
 
 // Views of a TensorList for the C ABI; keeps the camTensor structs alive.
@@ -93,17 +71,9 @@ void check(camStatus st, const char *op)
     TORCH_CHECK(st == CAM_OK, op, " failed with cam status ", (int)st, ": ", camGetRecentErrMsg());
 }
 
-typedef camStatus (*Phase2)(void *, uint64_t, camOpExecutor *, camStream_t);
-
-// Phase 2 of an operator whose phase 1 has produced (bytes, executor).
 void run_phase2(Phase2 fn, const char *op, uint64_t bytes, camOpExecutor *executor, const at::Tensor &like)
 {
-    // the workspace, the stream and the launches belong to the device the tensors live on
-    const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(like.device());
-    at::Tensor ws = at::empty({(int64_t)(bytes > 0 ? bytes : 1)}, like.options().dtype(at::kByte));
-    const camStatus st = fn(ws.data_ptr(), bytes, executor,
-                            (camStream_t)c10::hip::getCurrentHIPStream(like.device().index()).stream());
-    check(st, op);
+    check(cam_torch::launch(fn, bytes, executor, like), op);
 }
 
 // ---- storages that hold packed weights: StorageImpl -> (weak reference, gate/up pairing)
@@ -158,9 +128,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> get_dispatch_layout(const at::Ten
     TORCH_CHECK(topk_idx.is_contiguous(), "Assertion failed: topkIdx.is_contiguous()");
     TORCH_CHECK(num_experts > 0, "Assertion failed: numExperts > 0");
     const int64_t T = topk_idx.size(0), K = topk_idx.size(1);
-    at::Tensor per_expert = at::empty({num_experts}, topk_idx.options().dtype(at::kInt));
-    at::Tensor per_rank = at::empty({num_ranks}, topk_idx.options().dtype(at::kInt));
-    at::Tensor in_rank = at::empty({T, num_ranks}, topk_idx.options().dtype(at::kBool));
+    at::Tensor per_expert = new_empty({num_experts}, at::kInt, topk_idx);
+    at::Tensor per_rank = new_empty({num_ranks}, at::kInt, topk_idx);
+    at::Tensor in_rank = new_empty({T, num_ranks}, at::kBool, topk_idx);
     camTensor ci = to_cam(topk_idx), cr = to_cam(per_rank), ce = to_cam(per_expert), cb = to_cam(in_rank);
     uint64_t bytes = 0;
     camOpExecutor *ex = nullptr;
@@ -172,8 +142,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> get_dispatch_layout(const at::Ten
 
 // -> (expand_x [total,H], expand_idx int32 [3*total], recv_count int32 [E], num_recv_tokens_per_expert int64 on
 // the CPU), total = max(rows received, 1) as in the reference (moe_dispatch_prefill.cpp:161-167).  The row total
-// decides the output shapes, so 8 bytes come back to the host first (the reference brings two whole tensors back and
-// loops over them).  num_worst_tokens only enters the reference's globalBs (:154-155), which one rank does not need.
+// decides the output shapes, so the host waits for the counts per expert (the reference brings two whole tensors back
+// and loops over them).  num_worst_tokens only enters the reference's globalBs (:154-155), which one rank does not need.
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> moe_dispatch_prefill(
     const at::Tensor &x, const at::Tensor &topk_idx, const at::Tensor &topk_weights,
     const at::Tensor &num_tokens_per_rank, const at::Tensor &is_token_in_rank, const at::Tensor &num_tokens_per_expert,
@@ -208,25 +178,38 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> moe_dispatch_prefill(
     (void)num_worst_tokens;
     const int64_t T = x.size(0), H = x.size(1), K = topk_idx.size(1);
     const int64_t A = std::max<int64_t>(T * K, 1);
-    auto i32 = x.options().dtype(at::kInt);
-    at::Tensor recv_x = at::empty({A, H}, x.options());
-    at::Tensor expand_idx = at::empty({3 * A}, i32);
-    at::Tensor pos = at::empty({T, K}, i32);
-    at::Tensor recv_count = at::empty({E}, i32);
-    at::Tensor per_expert = at::empty({E / num_ranks}, x.options().dtype(at::kLong));
-    at::Tensor total = at::empty({1}, x.options().dtype(at::kLong));
-    camTensor cx = to_cam(x), ci = to_cam(topk_idx), crx = to_cam(recv_x), cidx = to_cam(expand_idx), cpos = to_cam(pos),
-              crc = to_cam(recv_count), cpe = to_cam(per_expert), ct = to_cam(total);
+    camTensor cx = to_cam(x), ci = to_cam(topk_idx);   // (checks that both are on the GPU)
+    at::Tensor recv_x = new_empty({A, H}, x.scalar_type(), x);
+    at::Tensor expand_idx = new_empty({3 * A}, at::kInt, x);
+    at::Tensor pos = new_empty({T, K}, at::kInt, x);
+    at::Tensor recv_count = new_empty({E}, at::kInt, x);
+    camTensor crx = to_cam(recv_x), cidx = to_cam(expand_idx), cpos = to_cam(pos), crc = to_cam(recv_count);
+    const int64_t per_rank = E / num_ranks;
+    TORCH_CHECK(per_rank <= HostCounts::kMost, "numExperts ", E, " outside (0, ", HostCounts::kMost, "]");
+    camTensor cpe{};   // the counts per expert, in host memory the plan kernel stores to
+    cpe.data = HostCounts::begin(per_rank);
+    cpe.dtype = CAM_DT_INT64;
+    cpe.ndim = 1;
+    cpe.sizes[0] = per_rank;
+    cpe.strides[0] = 1;
     uint64_t bytes = 0;
     camOpExecutor *ex = nullptr;
     check(camMoeDispatchPrefillGetWorkspaceSize(&cx, &ci, E, num_ranks, rank, 0, &crx, nullptr, &cidx, &cpos, nullptr,
-                                                nullptr, nullptr, &crc, &cpe, &ct, &bytes, &ex),
+                                                nullptr, nullptr, &crc, &cpe, nullptr, &bytes, &ex),
           "camMoeDispatchPrefill");
     run_phase2(camMoeDispatchPrefill, "camMoeDispatchPrefill", bytes, ex, x);
-    const int64_t n = std::max<int64_t>(total.item<int64_t>(), 1);  // the one host round trip: the shapes need it
-    recv_x = recv_x.narrow(0, 0, n);
-    expand_idx = expand_idx.narrow(0, 0, 3 * n);
-    return {recv_x, expand_idx, recv_count, per_expert.cpu()};
+    // the one thing the host waits for: the shapes need the row total
+    at::Tensor per_expert = HostCounts::wait(per_rank, x);
+    int64_t n = 0;
+    for (int64_t e = 0; e < per_rank; ++e) {
+        n += per_expert.data_ptr<int64_t>()[e];
+    }
+    n = std::max<int64_t>(n, 1);
+    if (n != A) {
+        recv_x = recv_x.narrow(0, 0, n);
+        expand_idx = expand_idx.narrow(0, 0, 3 * n);
+    }
+    return {recv_x, expand_idx, recv_count, per_expert};
 }
 
 at::Tensor moe_combine_prefill(const at::Tensor &x, const at::Tensor &topk_idx, const at::Tensor &topk_weights,
@@ -235,12 +218,13 @@ at::Tensor moe_combine_prefill(const at::Tensor &x, const at::Tensor &topk_idx, 
 {
     TORCH_CHECK(x.dim() == 2 && x.is_contiguous(), "Assertion failed: x.dim() == 2 and x.is_contiguous()");
     const int64_t T = topk_weights.size(0);
-    at::Tensor out = at::empty({T, x.size(1)}, x.options());
-    camTensor cx = to_cam(x), cs = to_cam(src_idx), ch = to_cam(send_head), cw = to_cam(topk_weights), co = to_cam(out);
-    std::string group(group_ep);
+    camTensor cx = to_cam(x);
+    at::Tensor out = new_empty({T, x.size(1)}, x.scalar_type(), x);
+    camTensor cs = to_cam(src_idx), ch = to_cam(send_head), cw = to_cam(topk_weights), co = to_cam(out);
+    const std::string group(group_ep);
     uint64_t bytes = 0;
     camOpExecutor *ex = nullptr;
-    check(camMoeCombineNormalGetWorkspaceSize(&cx, &cs, &ch, &cw, nullptr, group.data(), num_ranks, rank, group.data(), 1,
+    check(camMoeCombineNormalGetWorkspaceSize(&cx, &cs, &ch, &cw, nullptr, const_cast<char *>(group.c_str()), num_ranks, rank, const_cast<char *>(group.c_str()), 1,
                                               0, send_head.size(0), topk_idx.size(0) * num_ranks, &co, &bytes, &ex),
           "camMoeCombineNormal");
     run_phase2(camMoeCombineNormal, "camMoeCombineNormal", bytes, ex, x);
@@ -258,10 +242,11 @@ std::vector<at::Tensor> fused_deep_moe(const at::Tensor &x, const at::Tensor &ex
     TORCH_CHECK(x.dim() == 2, "x must be [bs, H]");
     require_packed(w1, true, "gmm1PermutedWeight");
     require_packed(w2, false, "gmm2Weight");
-    at::Tensor output = at::empty({x.size(0), x.size(1)}, x.options());
+    TORCH_CHECK(x.is_cuda(), "umdk_cam_op_lib: tensors must live on a ROCm device (the CAM kernels have no CPU path)");
+    at::Tensor output = new_empty({x.size(0), x.size(1)}, x.scalar_type(), x);
     const bool shared = ep_rank_id < shared_expert_rank_num;
     const int64_t local = shared ? 1 : moe_expert_num / std::max<int64_t>(ep_rank_size - shared_expert_rank_num, 1);
-    at::Tensor expert_token_nums = at::empty({local}, x.options().dtype(at::kLong));
+    at::Tensor expert_token_nums = new_empty({local}, at::kLong, x);
     camTensor cx = to_cam(x), ci = to_cam(expert_ids), cs = to_cam(expert_scales), co = to_cam(output),
               cn = to_cam(expert_token_nums);
     CamList l1(w1, CAM_FORMAT_MFMA_B), l1s(w1s, CAM_FORMAT_ND), l2(w2, CAM_FORMAT_MFMA_B), l2s(w2s, CAM_FORMAT_ND);
@@ -275,10 +260,10 @@ std::vector<at::Tensor> fused_deep_moe(const at::Tensor &x, const at::Tensor &ex
         cm = to_cam(*mask);
         pm = &cm;
     }
-    std::string group(group_ep);
+    const std::string group(group_ep);
     uint64_t bytes = 0;
     camOpExecutor *ex = nullptr;
-    check(camFusedDeepMoeGetWorkspaceSize(&cx, &ci, &l1.list, &l1s.list, &l2.list, &l2s.list, &cs, psm, pm, group.data(),
+    check(camFusedDeepMoeGetWorkspaceSize(&cx, &ci, &l1.list, &l1s.list, &l2.list, &l2s.list, &cs, psm, pm, const_cast<char *>(group.c_str()),
                                           ep_rank_size, ep_rank_id, moe_expert_num, shared_expert_num,
                                           shared_expert_rank_num, quant_mode, global_bs, &co, &cn, &bytes, &ex),
           "camFusedDeepMoe");
@@ -319,13 +304,16 @@ std::vector<at::Tensor> dispatch_shmem_outputs(const at::Tensor &x, const at::Te
     const int64_t bs = x.size(0), h = x.size(1), k = expert_ids.size(1);
     const int64_t rows = shared ? bs * ep_world_size / shared_expert_rank_num
                                 : bs * ep_world_size * std::min<int64_t>(per_rank, k);
-    auto ids = expert_ids.options();
-    return {at::empty({rows, h}, quant_mode == 2 ? x.options().dtype(at::kChar) : x.options()),
-            at::empty({rows}, x.options().dtype(at::kFloat)),
-            at::empty({bs * k}, ids),
-            at::empty({shared ? 1 : per_rank}, ids.dtype(at::kLong)),
-            at::empty({shared ? ep_world_size : ep_world_size * per_rank}, ids),
-            at::empty({tp_world_size}, ids)};
+    auto make = [](at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor &like) {
+        return like.is_cuda() ? new_empty(sizes, dtype, like) : at::empty(sizes, like.options().dtype(dtype));
+    };
+    const at::ScalarType id = expert_ids.scalar_type();
+    return {make({rows, h}, quant_mode == 2 ? at::kChar : x.scalar_type(), x),
+            make({rows}, at::kFloat, x),
+            make({bs * k}, id, expert_ids),
+            make({shared ? 1 : per_rank}, at::kLong, expert_ids),
+            make({shared ? ep_world_size : ep_world_size * per_rank}, id, expert_ids),
+            make({tp_world_size}, id, expert_ids)};
 }
 
 std::vector<at::Tensor> moe_dispatch_shmem(const at::Tensor &x, const at::Tensor &expert_ids,
@@ -376,8 +364,9 @@ at::Tensor moe_combine_shmem(const at::Tensor &expand_x, const at::Tensor &exper
                              int64_t group_list_type)
 {
     TORCH_CHECK(expand_x.dim() == 2 && expert_ids.dim() == 2, "expandX must be [A, H] and expertIds [bs, K]");
-    at::Tensor out = at::empty({expert_ids.size(0), expand_x.size(1)}, expand_x.options());
-    camTensor cx = to_cam(expand_x), ci = to_cam(expert_ids), ce = to_cam(expand_idx), cc = to_cam(ep_send_counts),
+    camTensor cx = to_cam(expand_x);
+    at::Tensor out = new_empty({expert_ids.size(0), expand_x.size(1)}, expand_x.scalar_type(), expand_x);
+    camTensor ci = to_cam(expert_ids), ce = to_cam(expand_idx), cc = to_cam(ep_send_counts),
               cw = to_cam(expert_scales), co = to_cam(out);
     camTensor t0{}, t1{}, t2{}, t3{}, t4{}, t5{};
     uint64_t bytes = 0;
@@ -406,6 +395,25 @@ at::Tensor moe_combine_shmem_meta(const at::Tensor &expand_x, const at::Tensor &
 // ---- autograd: forward = the operator below the autograd key, backward = one undefined gradient per input.
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
+
+// Whether a call takes part in a graph at all.  When it does not, which is every call of an inference program, the node and
+// its bookkeeping are skipped: the outputs are the same tensors without a grad_fn.
+bool wants_grad(const at::Tensor &t) { return t.defined() && t.requires_grad(); }
+bool wants_grad(const c10::optional<at::Tensor> &t) { return t.has_value() && wants_grad(*t); }
+bool wants_grad(at::TensorList ts)
+{
+    for (const at::Tensor &t : ts) {
+        if (wants_grad(t)) {
+            return true;
+        }
+    }
+    return false;
+}
+template <typename... Ts>
+bool in_graph(const Ts &...ts)
+{
+    return at::GradMode::is_enabled() && (wants_grad(ts) || ...);
+}
 
 template <int NumInputs>
 variable_list no_gradients()
@@ -493,11 +501,19 @@ std::vector<at::Tensor> fused_deep_moe_autograd(const at::Tensor &x, const at::T
                                                 int64_t a, int64_t b, int64_t c, int64_t d, int64_t e, int64_t f,
                                                 int64_t g)
 {
+    if (!in_graph(x, ids, w1, w1s, w2, w2s, es, smooth, mask)) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        return fused_deep_moe(x, ids, w1, w1s, w2, w2s, es, smooth, mask, group, a, b, c, d, e, f, g);
+    }
     return FusedDeepMoeFn::apply(x, ids, w1, w1s, w2, w2s, es, smooth, mask, group, a, b, c, d, e, f, g);
 }
 
 std::tuple<at::Tensor, at::Tensor, at::Tensor> get_dispatch_layout_autograd(const at::Tensor &idx, int64_t e, int64_t r)
 {
+    if (!in_graph(idx)) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        return get_dispatch_layout(idx, e, r);
+    }
     variable_list v = DispatchLayoutFn::apply(idx, e, r);
     return {v[0], v[1], v[2]};
 }
@@ -507,6 +523,10 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> moe_dispatch_prefill_
     const at::Tensor &in_rank, const at::Tensor &per_expert, int64_t worst, c10::string_view group, int64_t rank,
     int64_t ranks)
 {
+    if (!in_graph(x, idx, w, per_rank, in_rank, per_expert)) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        return moe_dispatch_prefill(x, idx, w, per_rank, in_rank, per_expert, worst, group, rank, ranks);
+    }
     variable_list v = DispatchPrefillFn::apply(x, idx, w, per_rank, in_rank, per_expert, worst, group, rank, ranks);
     return {v[0], v[1], v[2], v[3]};
 }
@@ -515,6 +535,10 @@ at::Tensor moe_combine_prefill_autograd(const at::Tensor &x, const at::Tensor &i
                                         const at::Tensor &src, const at::Tensor &head, c10::string_view group,
                                         int64_t rank, int64_t ranks)
 {
+    if (!in_graph(x, idx, w, src, head)) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        return moe_combine_prefill(x, idx, w, src, head, group, rank, ranks);
+    }
     return CombinePrefillFn::apply(x, idx, w, src, head, group, rank, ranks);
 }
 
@@ -524,6 +548,10 @@ std::vector<at::Tensor> moe_dispatch_shmem_autograd(const at::Tensor &x, const a
                                                     int64_t c, int64_t d, int64_t e, int64_t f, int64_t g, int64_t h,
                                                     int64_t i, int64_t j, int64_t k, int64_t l)
 {
+    if (!in_graph(x, ids, scales, mask)) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        return moe_dispatch_shmem(x, ids, scales, mask, a, b, c, d, e, f, g, h, i, j, k, l);
+    }
     return DispatchShmemFn::apply(x, ids, scales, mask, a, b, c, d, e, f, g, h, i, j, k, l);
 }
 
@@ -535,6 +563,10 @@ at::Tensor moe_combine_shmem_autograd(const at::Tensor &x, const at::Tensor &ids
                                       int64_t a, int64_t b, int64_t c, int64_t d, int64_t e, int64_t f, int64_t g,
                                       int64_t h, int64_t i, int64_t j, int64_t k, int64_t l, int64_t m)
 {
+    if (!in_graph(x, ids, eidx, counts, w, o0, o1, o2, o3, o4, o5)) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        return moe_combine_shmem(x, ids, eidx, counts, w, o0, o1, o2, o3, o4, o5, a, b, c, d, e, f, g, h, i, j, k, l, m);
+    }
     return CombineShmemFn::apply(x, ids, eidx, counts, w, o0, o1, o2, o3, o4, o5, a, b, c, d, e, f, g, h, i, j, k, l, m);
 }
 

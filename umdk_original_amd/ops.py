@@ -17,6 +17,7 @@ prepacked with `prepack_weight` (the reference needs `npu_format_cast(..., FRACT
 place); `moe_dispatch_prefill` takes an optional `quant_mode` keyword (the reference binding
 hard-codes 0 although its kernel supports dynamic quantisation).
 """
+import importlib.util
 import os
 import weakref
 
@@ -37,6 +38,23 @@ def _bind_assert(cond, what):
     # Counterpart of TORCH_BIND_ASSERT (src/cam/comm_operator/pybind/utils.h:15-38): throws.
     if not cond:
         raise RuntimeError("Assertion failed: " + what)
+
+
+_native_module = None
+
+
+def _native():
+    """The C++ module behind the operators below (csrc/py_native.cpp), loaded on first use."""
+    global _native_module
+    if _native_module is None:
+        path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_cam_native.so")
+        if not os.path.exists(path):
+            raise RuntimeError("%s is missing: build it with `python -m umdk_original_amd.build` "
+                               "(there is no CPU fallback)" % path)
+        spec = importlib.util.spec_from_file_location("_cam_native", path)
+        _native_module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(_native_module)
+    return _native_module
 
 
 def _require_gpu(t, name):
@@ -109,34 +127,9 @@ def moe_dispatch_fused(x, topk_idx, num_experts, quant_mode=0, num_rows=None, ra
     num_tokens_per_expert, send_offset, recv_count, num_recv_tokens_per_expert, total)
     """
     _require_gpu(x, "x")
-    T, H = x.shape
-    K = topk_idx.size(1)
-    A = max(int(T * K if num_rows is None else num_rows), 1)
-    dev = x.device
-    i32 = dict(dtype=torch.int32, device=dev)
-    if quant_mode == 4:   # block-scaled FP8: E4M3 rows, one E8M0 scale per row and 128 columns
-        rx = torch.empty((A, H), dtype=torch.float8_e4m3fn, device=dev)
-        rs = torch.empty((A, H // 128), dtype=torch.uint8, device=dev)
-    else:
-        rx = torch.empty((A, H), dtype=torch.int8 if quant_mode != 0 else x.dtype, device=dev)
-        rs = torch.empty(A, dtype=torch.float32, device=dev)
-    out = dict(
-        recv_x=rx,
-        recv_x_scales=rs,
-        expand_idx=torch.empty(3 * A, **i32),
-        send_token_idx=torch.empty((T, K), **i32),
-        slot_row=torch.empty((T, K), **i32),
-        num_tokens_per_expert=torch.empty(num_experts, **i32),
-        send_offset=torch.empty(num_experts, **i32),
-        recv_count=torch.empty(num_experts, **i32),
-        num_recv_tokens_per_expert=torch.empty(num_experts // max(num_ranks, 1), dtype=torch.int64, device=dev),
-        total=torch.empty(1, dtype=torch.int64, device=dev),
-    )
-    _lib.call("MoeDispatchPrefill", [x, topk_idx, num_experts, num_ranks, rank, quant_mode, out["recv_x"],
-                                     out["recv_x_scales"], out["expand_idx"], out["send_token_idx"], out["slot_row"],
-                                     out["num_tokens_per_expert"], out["send_offset"], out["recv_count"],
-                                     out["num_recv_tokens_per_expert"], out["total"]])
-    return out
+    # quant_mode 4 is block-scaled FP8: E4M3 rows, one E8M0 scale per row and 128 columns
+    return _native().moe_dispatch_fused(x, topk_idx, num_experts, quant_mode, -1 if num_rows is None else int(num_rows),
+                                        rank, num_ranks)
 
 
 def moe_dispatch_normal(x, topk_idx, send_offset, send_token_idx, recv_offset, recv_count, total_rows,
@@ -161,11 +154,11 @@ def moe_dispatch_prefill(x, topk_idx, topk_weights, num_tokens_per_rank, is_toke
     """-> (expand_x [total,H], expand_idx int32 [3*total], recv_count int32 [E],
            num_recv_tokens_per_expert int64 [E/R] on the CPU).
 
-    One launch (MoeDispatchPrefill) ranks, places and copies/quantises the rows.  The total row count
-    decides the output shapes, so one 8-byte device-to-host copy is made afterwards (the reference makes
-    two larger ones and runs the index arithmetic on the CPU).  With `num_worst_tokens` > 0 the outputs keep
-    that many rows instead, nothing is copied until the fourth return value is produced, and rows beyond the
-    true total are left unwritten (moe_combine_prefill ignores them: it stops at recv_count[-1]).
+    One operator (MoeDispatchPrefill) ranks, places and copies/quantises the rows.  The total row count
+    decides the output shapes, so the host waits until the plan kernel has stored the counts per expert, which it
+    does to host memory (the reference copies two tensors back and runs the index arithmetic on the CPU).  With
+    `num_worst_tokens` > 0 the outputs keep that many rows instead, and rows beyond the true total are left
+    unwritten (moe_combine_prefill ignores them: it stops at recv_count[-1]).
     """
     _bind_assert(is_token_in_rank.dtype == torch.bool, "isTokenInRank.scalar_type() == at::kBool")
     _bind_assert(num_tokens_per_expert.dtype == torch.int32, "numTokensPerExpert.scalar_type() == at::kInt")
@@ -192,18 +185,16 @@ def moe_dispatch_prefill(x, topk_idx, topk_weights, num_tokens_per_rank, is_toke
     _require_gpu(x, "x")
 
     worst = bool(num_worst_tokens and num_worst_tokens > 0)
-    d = moe_dispatch_fused(x, topk_idx, num_experts, quant_mode=quant_mode,
-                           num_rows=int(num_worst_tokens) if worst else None, rank=rank, num_ranks=num_ranks)
-    recv_x, scales, expand_idx = d["recv_x"], d["recv_x_scales"], d["expand_idx"]
+    recv_x, scales, expand_idx, recv_count, per_expert_cpu = _native().moe_dispatch_prefill(
+        x, topk_idx, num_experts, quant_mode, int(num_worst_tokens) if worst else -1, rank, num_ranks)
     if not worst:
         # The reference sizes expand_x by the true total (moe_dispatch_prefill.cpp:156-162); the rows were written
         # into worst-case buffers, so the results are prefix views of those and nothing is copied.
-        total = int(d["total"].item())
+        total = int(per_expert_cpu.sum())
         recv_x, scales, expand_idx = recv_x[:total], scales[:total], expand_idx[:3 * total]
-    per_expert_cpu = d["num_recv_tokens_per_expert"].cpu()
     if return_scales:
-        return recv_x, expand_idx, d["recv_count"], per_expert_cpu, scales
-    return recv_x, expand_idx, d["recv_count"], per_expert_cpu
+        return recv_x, expand_idx, recv_count, per_expert_cpu, scales
+    return recv_x, expand_idx, recv_count, per_expert_cpu
 
 
 def moe_combine_normal(recv_x, token_src_info, ep_recv_counts, topk_weights, group_ep="", rank=0, num_ranks=1,
@@ -239,7 +230,7 @@ def moe_combine_gather(recv_x, token_src_info, slot_row, topk_weights, out=None,
         h = recv_x.size(1) // 5 * 4 if recv_x.dtype == torch.int8 else recv_x.size(1)
         out = torch.empty((topk_weights.size(0), h),
                           dtype=torch.bfloat16 if recv_x.dtype == torch.int8 else recv_x.dtype, device=recv_x.device)
-    _lib.call("MoeCombineGather", [recv_x, token_src_info, slot_row, ep_recv_counts, topk_weights, shared_x, out])
+    _native().moe_combine_gather(recv_x, token_src_info, slot_row, ep_recv_counts, topk_weights, shared_x, out)
     return out
 
 
@@ -325,12 +316,7 @@ def grouped_matmul_swiglu_quant(x, x_scale, weight, weight_scale, group_list, gr
     """GMM1 stage: int8 [A,H] -> (int8 [A,I], fp32 [A])."""
     weight = _tag_list(weight if isinstance(weight, (list, tuple)) else [weight])
     weight_scale = list(weight_scale) if isinstance(weight_scale, (list, tuple)) else [weight_scale]
-    A = x.size(0)
-    I = weight[0].size(-1) // 2
-    y = torch.empty((A, I), dtype=torch.int8, device=x.device)
-    ys = torch.empty(A, dtype=torch.float32, device=x.device)
-    _lib.call("GroupedMatmulSwigluQuant", [x, x_scale, weight, weight_scale, group_list, group_list_type, y, ys])
-    return y, ys
+    return _native().grouped_matmul_swiglu_quant(x, x_scale, weight, weight_scale, group_list, group_list_type)
 
 
 def grouped_matmul_dequant(x, x_scale, weight, weight_scale, group_list, group_list_type=0, wire_rows=False,
@@ -344,7 +330,7 @@ def grouped_matmul_dequant(x, x_scale, weight, weight_scale, group_list, group_l
         out = torch.empty((x.size(0), n + n // 4), dtype=torch.int8, device=x.device)
     else:
         out = torch.empty((x.size(0), n), dtype=out_dtype, device=x.device)
-    _lib.call("GroupedMatmulDequant", [x, x_scale, weight, weight_scale, group_list, group_list_type, out])
+    _native().grouped_matmul_dequant(x, x_scale, weight, weight_scale, group_list, group_list_type, out)
     return out
 
 
@@ -375,8 +361,7 @@ def grouped_matmul_fp8(x, x_scale, weight, weight_scale, group_list, group_list_
         out = torch.empty((x.size(0), n // 2), dtype=torch.float32, device=x.device)
     else:
         out = torch.empty((x.size(0), n), dtype=out_dtype, device=x.device)
-    _lib.call("GroupedMatmulFp8", [x, x_scale, weight, weight_scale, 1 if gate_up else 0, group_list,
-                                   group_list_type, out, out_scale])
+    _native().grouped_matmul_fp8(x, x_scale, weight, weight_scale, gate_up, group_list, group_list_type, out, out_scale)
     return out if out_scale is None else (out, out_scale)
 
 
@@ -394,13 +379,8 @@ def fused_deep_moe_fp8(x, expert_ids, gmm1_weight, gmm1_weight_scale, gmm2_weigh
     """-> [output bf16 [bs,H], expertTokenNums int64 [experts]]."""
     _require_gpu(x, "x")
     _tag_list([gmm1_weight, gmm2_weight])
-    bs, h = x.shape
-    e = moe_expert_num or gmm1_weight.size(0)
-    output = torch.empty((bs, h), dtype=torch.bfloat16, device=x.device)
-    etn = torch.empty(e, dtype=torch.int64, device=x.device)
-    _lib.call("FusedDeepMoeFp8", [x, expert_ids, gmm1_weight, gmm1_weight_scale, gmm2_weight, gmm2_weight_scale,
-                                  expert_scales, x_active_mask, e, output, etn])
-    return [output, etn]
+    return _native().fused_deep_moe_fp8(x, expert_ids, gmm1_weight, gmm1_weight_scale, gmm2_weight, gmm2_weight_scale,
+                                        expert_scales, x_active_mask, moe_expert_num or gmm1_weight.size(0))
 
 
 def fused_deep_moe(x, expertIds, gmm1PermutedWeight, gmm1PermutedWeightScale, gmm2Weight, gmm2WeightScale,
@@ -408,18 +388,12 @@ def fused_deep_moe(x, expertIds, gmm1PermutedWeight, gmm1PermutedWeightScale, gm
                    moeExpertNum=0, sharedExpertNum=1, sharedExpertRankNum=0, quantMode=0, globalBs=0):
     """-> [output bf16 [bs,H], expertTokenNums int64 [local experts]]."""
     _require_gpu(x, "x")
-    bs, h = x.shape
-    output = torch.empty((bs, h), dtype=x.dtype, device=x.device)
     is_shared = epRankId < sharedExpertRankNum
     local_experts = 1 if is_shared else moeExpertNum // max(epRankSize - sharedExpertRankNum, 1)
-    expert_token_nums = torch.empty(local_experts, dtype=torch.int64, device=x.device)
-    w1 = _tag_list(gmm1PermutedWeight)
-    w2 = _tag_list(gmm2Weight)
-    _lib.call("FusedDeepMoe", [x, expertIds, w1, list(gmm1PermutedWeightScale), w2, list(gmm2WeightScale),
-                               expertScales, expertSmoothScales, xActiveMask, groupEp, epRankSize, epRankId,
-                               moeExpertNum, sharedExpertNum, sharedExpertRankNum, quantMode, globalBs, output,
-                               expert_token_nums])
-    return [output, expert_token_nums]
+    return _native().fused_deep_moe(x, expertIds, _tag_list(gmm1PermutedWeight), list(gmm1PermutedWeightScale),
+                                    _tag_list(gmm2Weight), list(gmm2WeightScale), expertScales, expertSmoothScales,
+                                    xActiveMask, groupEp or "", epRankSize, epRankId, moeExpertNum, sharedExpertNum,
+                                    sharedExpertRankNum, quantMode, globalBs, local_experts)
 
 
 # --------------------------------------------------------------------------------------------------
