@@ -949,12 +949,8 @@ camStatus camMoeDispatchPrefillGetWorkspaceSize(const camTensor *x, const camTen
         if (p.dst_row == nullptr) {
             p.dst_row = (int32_t *)((char *)ws + o_row);
         }
-        hipError_t e = cam::launch_plan(p, s);
-        if (e != hipSuccess) {
-            return e;
-        }
         d.dst_row = p.dst_row;
-        return cam::launch_dispatch(d, s);
+        return cam::launch_plan_dispatch(p, d, s);
     };
     return finish_phase1(kOpPrefill, c.off, run, workspaceSize, executor);
 }
@@ -1311,12 +1307,8 @@ camStatus camMoeDispatchShmemGetWorkspaceSize(const camTensor *x, const camTenso
     auto run = [p, d, o_hist, o_row](void *ws, hipStream_t s) mutable -> hipError_t {
         p.hist_ws = (int32_t *)((char *)ws + o_hist);
         p.dst_row = (int32_t *)((char *)ws + o_row);
-        hipError_t e = cam::launch_plan(p, s);
-        if (e != hipSuccess) {
-            return e;
-        }
         d.dst_row = p.dst_row;
-        return cam::launch_dispatch(d, s);
+        return cam::launch_plan_dispatch(p, d, s);
     };
     return finish_phase1(kOpDispShmem, c.off, run, workspaceSize, executor);
 }
@@ -1411,7 +1403,6 @@ camStatus camMoeCombineShmemGetWorkspaceSize(
     CAM_TRY(check_aligned(expandX, "expandX", 16));
     CAM_TRY(check_aligned(out, "out", 16));
     Carver c;
-    const uint64_t o_slot = c.take((uint64_t)T * K * 4);
     const uint64_t o_wire = wire ? c.take((uint64_t)A * (uint64_t)(H + H / 4)) : 0;
     cam::CombineArgs g{};
     g.y = (const uint16_t *)expandX->data;
@@ -1422,20 +1413,16 @@ camStatus camMoeCombineShmemGetWorkspaceSize(
     g.A = A;
     g.act_fp16 = expandX->dtype == CAM_DT_FLOAT16;
     g.out = (uint16_t *)out->data;
-    const int32_t *ids = (const int32_t *)expertIds->data;
-    const int32_t *eidx = (const int32_t *)expandIdx->data;
     const int32_t *counts = (const int32_t *)epSendCounts->data;
+    g.ids = (const int32_t *)expertIds->data;
+    g.expand_idx = (const int32_t *)expandIdx->data;
+    g.ep_send_counts = counts;
+    g.E = (int)moeExpertNum;
     const int iE = (int)moeExpertNum;
     auto run = [=](void *ws, hipStream_t s) mutable -> hipError_t {
-        int32_t *slot = (int32_t *)((char *)ws + o_slot);
-        hipError_t e = cam::launch_rows_from_counts(ids, eidx, counts, (int64_t)g.T * g.K, iE, g.A, slot, s);
-        if (e != hipSuccess) {
-            return e;
-        }
-        g.slot_row = slot;
         if (wire) {  // every row takes the int8 wire format on its way (moe_combine_shmem.h:567-592,755-773)
             uint8_t *rows = (uint8_t *)ws + o_wire;
-            e = cam::launch_comm_quant(g.y, g.act_fp16, g.A, g.H, counts + (iE - 1), rows, s);
+            const hipError_t e = cam::launch_comm_quant(g.y, g.act_fp16, g.A, g.H, counts + (iE - 1), rows, s);
             if (e != hipSuccess) {
                 return e;
             }
@@ -1878,8 +1865,6 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         cam::SchedSpec specs[2] = {sp1, sp2};  // both GEMM schedules come from the per-expert counts of the plan
         specs[0].sched = (int32_t *)(w + o_sched1);
         specs[1].sched = (int32_t *)(w + o_sched2);
-        e = cam::launch_plan(p, s);
-        if (e != hipSuccess) return e;
         cam::DispatchArgs d{};
         d.x = xp;
         d.x_is_fp16 = x_is_fp16;
@@ -1903,7 +1888,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
             d.sched.spec[0] = specs[0];
             d.sched.spec[1] = specs[1];
         }
-        e = cam::launch_dispatch(d, s);
+        e = cam::launch_plan_dispatch(p, d, s);
         if (e != hipSuccess) return e;
 
         cam::GemmArgs g1{};
@@ -2236,8 +2221,6 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         cam::SchedSpec specs[2] = {sp1, sp2};
         specs[0].sched = (int32_t *)(w + o_sched1);
         specs[1].sched = (int32_t *)(w + o_sched2);
-        e = cam::launch_plan(p, s);
-        if (e != hipSuccess) return e;
         cam::DispatchArgs d{};
         d.x = xp;
         d.x_is_fp16 = x_is_fp16;
@@ -2260,7 +2243,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
             d.sched.spec[0] = specs[0];
             d.sched.spec[1] = specs[1];
         }
-        e = cam::launch_dispatch(d, s);
+        e = cam::launch_plan_dispatch(p, d, s);
         if (e != hipSuccess) return e;
 
         cam::GemmArgs g1{};

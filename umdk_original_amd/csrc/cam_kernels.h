@@ -127,6 +127,8 @@ struct DispatchArgs {
     SchedBuild sched;
 };
 hipError_t launch_dispatch(const DispatchArgs &a, hipStream_t stream);
+// launch_plan, then launch_dispatch with a.dst_row == p.dst_row; for few ids both as one launch.
+hipError_t launch_plan_dispatch(const PlanArgs &p, const DispatchArgs &a, hipStream_t stream);
 
 // ---------------------------------------------------------------------------------------------
 // Combine.
@@ -138,6 +140,10 @@ struct CombineArgs {
     int wire_rows;            // rows are H int8 values + H/8 block scales of the activation type (launch_comm_quant's output)
     int act_fp16;             // rows and output are IEEE fp16 instead of bf16 (not with wire_rows)
     const int32_t *slot_row;  // [T,K] row of slot (t,k) (<0: skip)
+    // instead of slot_row, when ids is set: the row of slot i is (e ? ep_send_counts[e-1] : 0) + expand_idx[i] for
+    // e = ids[i] in [0,E), none otherwise
+    const int32_t *ids, *expand_idx, *ep_send_counts;
+    int E;
     const int32_t *src_info;  // optional: when set, slot_row entries are verified against the triples
     const float *w;           // [T,K]
     int T, K, H;
@@ -148,10 +154,6 @@ struct CombineArgs {
     uint16_t *out;            // [T,H]
 };
 hipError_t launch_combine(const CombineArgs &a, hipStream_t stream);
-// slot_row[i] = (e ? ep_send_counts[e-1] : 0) + expand_idx[i] for e = ids[i] in [0,E) and a row below A, else -1
-// (how the SHMEM combine finds the row of slot i: moe_combine_shmem.h:514-556,833-837).
-hipError_t launch_rows_from_counts(const int32_t *ids, const int32_t *expand_idx, const int32_t *ep_send_counts,
-                                   int64_t n, int E, int64_t A, int32_t *slot_row, hipStream_t stream);
 // bf16 rows [A,H] -> wire rows [A, H + H/4] bytes: per block of 8 columns int8 values and one bf16 scale.
 // row_limit: optional device scalar; rows >= *row_limit are left untouched.
 hipError_t launch_comm_quant(const uint16_t *y, int act_fp16, int64_t A, int H, const int32_t *row_limit, uint8_t *out,

@@ -48,23 +48,18 @@ __global__ void invert_src_info_kernel(const int32_t *src_info, long long A, con
     }
 }
 
-__global__ void rows_from_counts_kernel(const int32_t *__restrict__ ids, const int32_t *__restrict__ expand_idx,
-                                        const int32_t *__restrict__ ep_send_counts, long long n, int E, long long A,
-                                        int32_t *__restrict__ slot_row)
+// The row of slot (t,k), or -1: from the map, or, with a.ids, the way the SHMEM combine finds it
+// (moe_combine_shmem.h:514-556,833-837): the rows of the experts before the slot's, plus its rank within the expert.
+__device__ __forceinline__ long long row_of_slot(const CombineArgs &a, long long slot)
 {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) {
-        return;
+    if (a.ids == nullptr) {
+        return a.slot_row[slot];
     }
-    const int e = ids[i];
-    long long row = -1;
-    if (e >= 0 && e < E) {
-        row = (long long)(e == 0 ? 0 : ep_send_counts[e - 1]) + expand_idx[i];
-        if (row < 0 || row >= A) {
-            row = -1;
-        }
-    }
-    slot_row[i] = (int32_t)row;
+    // (no branch, so that the loads of a token's slots stay side by side)
+    const int e = a.ids[slot];
+    const int before = a.ep_send_counts[min(max(e - 1, 0), a.E - 1)];
+    const long long row = (long long)(e > 0 ? before : 0) + a.expand_idx[slot];
+    return e >= 0 && e < a.E ? row : -1;
 }
 
 // Rows of the activation type (ACT: 0 = bf16, 1 = IEEE fp16) -> wire rows, whose block scales are of that type
@@ -150,7 +145,7 @@ __global__ __launch_bounds__(kCombThreads) void combine_kernel(CombineArgs a, in
                 v[j] = v4u{0u, 0u, 0u, 0u};
                 if (k < a.K) {
                     const long long slot = (long long)t * a.K + k;
-                    const long long row = a.slot_row[slot];
+                    const long long row = row_of_slot(a, slot);
                     bool good = row >= 0 && row < rows;
                     if (good && a.src_info != nullptr) {
                         // The inverse map is not pre-cleared: accept a row only if it names this slot.
@@ -251,7 +246,7 @@ __global__ __launch_bounds__(kCombThreads) void combine_wire16_kernel(CombineArg
                 sc2[j] = 0u;
                 if (k < a.K) {
                     const long long slot = (long long)t * a.K + k;
-                    const long long row = a.slot_row[slot];
+                    const long long row = row_of_slot(a, slot);
                     bool good = row >= 0 && row < rows;
                     if (good && a.src_info != nullptr) {
                         good = a.src_info[3 * row + 1] == t && a.src_info[3 * row + 2] == k;
@@ -314,17 +309,6 @@ hipError_t launch_invert_src_info(const int32_t *src_info, int64_t A, const int3
     }
     hipLaunchKernelGGL(invert_src_info_kernel, dim3((unsigned)((A + 255) / 256)), dim3(256), 0, stream, src_info,
                        (long long)A, row_limit, T, K, slot_row);
-    return hipGetLastError();
-}
-
-hipError_t launch_rows_from_counts(const int32_t *ids, const int32_t *expand_idx, const int32_t *ep_send_counts,
-                                   int64_t n, int E, int64_t A, int32_t *slot_row, hipStream_t stream)
-{
-    if (n <= 0) {
-        return hipSuccess;
-    }
-    hipLaunchKernelGGL(rows_from_counts_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, ids,
-                       expand_idx, ep_send_counts, (long long)n, E, (long long)A, slot_row);
     return hipGetLastError();
 }
 

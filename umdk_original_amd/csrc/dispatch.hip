@@ -17,6 +17,7 @@
 #include "cam_device.h"
 #include "cam_kernels.h"
 #include "permute_device.h"
+#include "rank_device.h"
 #include "sched_device.h"
 
 namespace cam {
@@ -58,10 +59,10 @@ __global__ __launch_bounds__(kDispWaves * kWave, QUANT == 3 ? 3 : 4) void dispat
     if (t >= a.T) {
         return;
     }
-    TokenRow r;
+    WaveRow r;
     load_token_row(a.x, t, a.H, lane, r);
     if (QUANT != 0) {
-        quant_token_row<QUANT, ACT>(r);
+        quant_token_row<QUANT, ACT>(r, WaveMax());
     }
     for (int k = 0; k < a.K; ++k) {
         const long long row = dispatch_row(a, t, k);
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(kDispWaves * kWave) void dispatch_smooth_kernel(Dis
     if (t >= a.T) {
         return;
     }
-    TokenRow r;
+    WaveRow r;
     load_token_row(a.x, t, a.H, lane, r);
     for (int k = 0; k < a.K; ++k) {
         const long long row = dispatch_row(a, t, k);
@@ -91,12 +92,187 @@ __global__ __launch_bounds__(kDispWaves * kWave) void dispatch_smooth_kernel(Dis
         if (row < 0 || row >= a.A || e < 0 || e >= a.E) {
             continue;
         }
-        quant_token_row_smooth<ACT>(r, a.smooth + (long long)e * a.H, a.H, lane);
+        quant_token_row_smooth<ACT>(r, a.smooth + (long long)e * a.H, a.H, lane, WaveMax());
         store_token_row<2>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, lane);
     }
 }
 
+// Plan and permute in one launch, for id sequences short enough that every workgroup can look at all of them.
+// A workgroup per token.  While its row is on its way it finds where the row goes: the row of entry (t,k) is the number
+// of entries that name an earlier expert plus the number of earlier entries that name the same one, so a look at all
+// T * K ids (counted with ballots) gives the rows and the ranks of the K entries with no table, no scan and nothing to
+// wait for from another workgroup.  Workgroup 0 counts for the per-expert outputs.  With few tokens the latency of one
+// row is what the launch takes, so it is spread over sixteen waves (four from 257 tokens on) instead of one.
+// Launches: one token x 4096 to 128 experts, top-8: 3.5 + 7.4 us -> 5.9; 64 x 4096 FP8: 6.2 + 15.6 -> 7.4; 128 x 7168 to 256
+// experts: 6.1 + 9.8 -> 7.8.
+constexpr int kSmallIds = 2048;   // ids per launch
+template <typename IdT, int QUANT, int ACT, bool SMOOTH, int NT>
+__global__ __launch_bounds__(NT) void dispatch_small_kernel(PlanArgs p, DispatchArgs a)
+{
+    constexpr int kPer = kSmallIds / NT;   // ids per thread
+    constexpr int kWaves = NT / kWave;
+    __shared__ int counts[2][kMaxTopk][kWaves];  // entries before the expert's, earlier entries of it: per k and wave
+    __shared__ int row_s[kMaxTopk];
+    __shared__ float max_s[kWaves];
+    __shared__ int active_s;
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wave = tid >> 6;
+    const IdT *__restrict__ idx = (const IdT *)p.idx;
+    const int n_all = p.T * p.K;
+    const int E = p.E, K = p.K;
+
+    if (blockIdx.x == 0) {  // counts, offsets and totals
+        __shared__ int hist[kMaxExperts];
+        __shared__ int scan_s[kWaves];
+        __shared__ int total_s;
+        int id[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int j = tid + i * NT;
+            id[i] = j < n_all ? load_id(idx, j, E) : -1;
+        }
+        const int t_active = count_active(p.mask, p.T, tid, NT, &active_s);
+        for (int i = tid; i < kMaxExperts; i += NT) {
+            hist[i] = 0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            if (tid + i * NT < t_active * K && id[i] >= 0) {
+                atomicAdd(&hist[id[i]], 1);
+            }
+        }
+        __syncthreads();
+        write_expert_outputs<NT>(p, hist, t_active, tid, scan_s, &total_s);
+        return;
+    }
+
+    const int t = (int)blockIdx.x - 1;
+    GroupRow<NT> r;
+    load_token_row(a.x, t, a.H, tid, r);
+    int id[kPer];  // entries tid, tid + NT, ...; E where none
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int j = tid + i * NT;
+        id[i] = E;
+        if (i * NT < n_all && j < n_all) {
+            const int e = load_id(idx, j, E);
+            id[i] = e >= 0 ? e : E;
+        }
+    }
+    const int own_ids = lane < K ? load_id(idx, t * K + lane, E) : -1;  // lane k: the id of entry (t,k)
+    const int t_active = count_active(p.mask, p.T, tid, NT, &active_s);
+    const int n = t_active * K;
+    for (int k = 0; k < K; ++k) {
+        const int own = t * K + k;
+        const int e = __builtin_amdgcn_readlane(own_ids, k);
+        int before = 0, earlier = 0;
+        if (own < n && e >= 0) {
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                if (i * NT < n) {
+                    const int j = tid + i * NT;
+                    before += __popcll(__ballot(j < n && id[i] < e));
+                    earlier += __popcll(__ballot(j < own && id[i] == e));
+                }
+            }
+        }
+        if (lane == 0) {
+            counts[0][k][wave] = before;
+            counts[1][k][wave] = earlier;
+        }
+    }
+    if (QUANT != 0 && !SMOOTH) {
+        quant_token_row<QUANT, ACT>(r, GroupMax<NT>{max_s});
+    }
+    __syncthreads();
+    if (tid < K) {
+        const int own = t * K + tid;
+        int row = -1, rank = -1;
+        if (own < n && own_ids >= 0) {
+            rank = 0;
+            row = 0;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                row += counts[0][tid][w];
+                rank += counts[1][tid][w];
+            }
+            row += rank;
+        }
+        row_s[tid] = row;
+        p.pos[own] = rank;
+        if (p.dst_row != nullptr) {
+            p.dst_row[own] = row;
+        }
+    }
+    __syncthreads();
+    for (int k = 0; k < K; ++k) {
+        const int row = row_s[k];
+        if (row < 0 || row >= a.A) {
+            continue;
+        }
+        if constexpr (SMOOTH) {
+            const int e = __builtin_amdgcn_readlane(own_ids, k);
+            quant_token_row_smooth<ACT>(r, a.smooth + (long long)e * a.H, a.H, tid, GroupMax<NT>{max_s});
+        }
+        store_token_row<QUANT>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, tid);
+    }
+}
+
+template <typename IdT, int QUANT, bool SMOOTH, int NT>
+hipError_t launch_small_with(const PlanArgs &p, const DispatchArgs &a, hipStream_t stream)
+{
+    const dim3 grid((unsigned)p.T + 1), block(NT);
+    if (a.x_is_fp16 && QUANT != 0) {  // (a copy does not look at the format)
+        hipLaunchKernelGGL((dispatch_small_kernel<IdT, QUANT, 1, SMOOTH, NT>), grid, block, 0, stream, p, a);
+    } else {
+        hipLaunchKernelGGL((dispatch_small_kernel<IdT, QUANT, 0, SMOOTH, NT>), grid, block, 0, stream, p, a);
+    }
+    return hipGetLastError();
+}
+
+template <typename IdT, int QUANT, bool SMOOTH = false>
+hipError_t launch_small_as(const PlanArgs &p, const DispatchArgs &a, hipStream_t stream)
+{
+    // sixteen waves per token while every token has a CU of its own
+    return p.T <= 256 ? launch_small_with<IdT, QUANT, SMOOTH, 1024>(p, a, stream)
+                      : launch_small_with<IdT, QUANT, SMOOTH, 256>(p, a, stream);
+}
+
+template <typename IdT>
+hipError_t launch_small(const PlanArgs &p, const DispatchArgs &a, hipStream_t stream)
+{
+    if (a.smooth != nullptr) {
+        return launch_small_as<IdT, 2, true>(p, a, stream);
+    }
+    switch (a.quant) {
+        case 0: return launch_small_as<IdT, 0>(p, a, stream);
+        case 1: return launch_small_as<IdT, 1>(p, a, stream);
+        case 2: return launch_small_as<IdT, 2>(p, a, stream);
+        default: return launch_small_as<IdT, 3>(p, a, stream);
+    }
+}
+
 }  // namespace
+
+hipError_t launch_plan_dispatch(const PlanArgs &p, const DispatchArgs &a, hipStream_t stream)
+{
+    const long long n = (long long)p.T * p.K;
+    // One launch up to 2048 ids, where the permute builds no schedules (their builders need the plan's counts first)
+    if (n > 0 && n <= kSmallIds && a.sched.nspec == 0) {
+        if (a.H % 8 != 0 || a.H / 8 > kDispMaxChunks * kWave || (a.quant == 3 && a.H % 128 != 0) ||
+            (a.smooth != nullptr && a.quant != 2) || p.K > kMaxTopk || p.E > kMaxExperts) {
+            return hipErrorInvalidValue;
+        }
+        return p.idx_is64 ? launch_small<int64_t>(p, a, stream) : launch_small<int32_t>(p, a, stream);
+    }
+    const hipError_t e = launch_plan(p, stream);
+    if (e != hipSuccess) {
+        return e;
+    }
+    return launch_dispatch(a, stream);
+}
 
 hipError_t launch_dispatch(const DispatchArgs &a_in, hipStream_t stream)
 {

@@ -1,5 +1,5 @@
-// Device code shared by the permute kernels: one wavefront loads one token row, quantises it in
-// registers and stores it to any number of destination rows.
+// Device code shared by the permute kernels: a wavefront, or a workgroup where there are few tokens, loads one token row,
+// quantises it in registers and stores it to any number of destination rows.
 //
 // Reference semantics (paths relative to the reference tree):
 //   quant   src/cam/comm_operator/ascend_kernels/moe_dispatch_normal/op_kernel/moe_dispatch_normal.h:278-316
@@ -36,12 +36,41 @@ __device__ __forceinline__ float act_bits_to_f32(uint32_t bits16)
     return (float)__builtin_bit_cast(_Float16, (unsigned short)bits16);  // exact
 }
 
-// One token row held by a wavefront: lane l owns the 16-byte chunks l, l+64, ... of the row.
+// One token row held by kLanes threads (a wavefront or a workgroup): thread l owns the 16-byte chunks l, l + kLanes, ...
+template <int CHUNKS, int LANES>
 struct TokenRow {
-    v4u raw[kDispMaxChunks];
-    v2u q[kDispMaxChunks];
+    static constexpr int kChunks = CHUNKS, kLanes = LANES;
+    v4u raw[CHUNKS];
+    v2u q[CHUNKS];
     float scale_out;
-    uint32_t scale8[kDispMaxChunks];  // QUANT 3: E8M0 scale of the 128-column block chunk j of this lane lies in
+    uint32_t scale8[CHUNKS];  // QUANT 3: E8M0 scale of the 128-column block chunk j of this thread lies in
+};
+typedef TokenRow<kDispMaxChunks, kWave> WaveRow;
+template <int NT>
+using GroupRow = TokenRow<(kDispMaxChunks * kWave + NT - 1) / NT, NT>;  // a workgroup of NT threads
+
+// The maximum over the threads that hold a row.
+struct WaveMax {
+    __device__ __forceinline__ float operator()(float m) const { return wave_max(m); }
+};
+template <int NT>
+struct GroupMax {
+    float *slots;  // LDS, one per wave
+    __device__ __forceinline__ float operator()(float m) const
+    {
+        m = wave_max(m);
+        __syncthreads();  // the maxima before these have been read
+        if ((threadIdx.x & (kWave - 1)) == 0) {
+            slots[threadIdx.x >> 6] = m;
+        }
+        __syncthreads();
+        m = slots[0];
+#pragma unroll
+        for (int w = 1; w < NT / kWave; ++w) {
+            m = fmaxf(m, slots[w]);
+        }
+        return m;
+    }
 };
 
 // Exponent x of the smallest power of two 2^x with amax / 2^x <= 448 (amax = m * 2^e: e - 8, one more when
@@ -71,13 +100,14 @@ __device__ __forceinline__ float exp2_int(int x)
     return x >= -126 ? __uint_as_float((uint32_t)(x + 127) << 23) : __uint_as_float(0x00400000u);
 }
 
-__device__ __forceinline__ void load_token_row(const uint16_t *x, int t, int H, int lane, TokenRow &r)
+template <typename Row>
+__device__ __forceinline__ void load_token_row(const uint16_t *x, int t, int H, int lane, Row &r)
 {
     const int nch = H >> 3;  // 8 values per chunk
     const v4u *src = (const v4u *)(x + (long long)t * H);
 #pragma unroll
-    for (int j = 0; j < kDispMaxChunks; ++j) {
-        const int c = j * kWave + lane;
+    for (int j = 0; j < Row::kChunks; ++j) {
+        const int c = j * Row::kLanes + lane;
         r.raw[j] = v4u{0u, 0u, 0u, 0u};
         if (c < nch) {
             r.raw[j] = __builtin_nontemporal_load(src + c);
@@ -85,15 +115,15 @@ __device__ __forceinline__ void load_token_row(const uint16_t *x, int t, int H, 
     }
 }
 
-// FP8 with one scale per 128 columns.  Chunk c = 64 j + lane holds columns 8c .. 8c+7, so a block of 128
+// FP8 with one scale per 128 columns.  Chunk c = kLanes j + lane holds columns 8c .. 8c+7, so a block of 128
 // columns is the 16 chunks of lanes 16 q .. 16 q + 15 at one j: its largest magnitude is a maximum over a
 // quarter of the wave.  The scaled values lie within +-448, where the hardware conversion (round to nearest
 // even) needs no saturation.
-template <int ACT>
-__device__ __forceinline__ void quant_token_row_fp8(TokenRow &r)
+template <int ACT, typename Row>
+__device__ __forceinline__ void quant_token_row_fp8(Row &r)
 {
 #pragma unroll
-    for (int j = 0; j < kDispMaxChunks; ++j) {
+    for (int j = 0; j < Row::kChunks; ++j) {
         float x[8];
         float m = 0.0f;
 #pragma unroll
@@ -123,28 +153,28 @@ __device__ __forceinline__ void quant_token_row_fp8(TokenRow &r)
 }
 
 // QUANT 1: scale = 127 / (max|x| + 1e-12); QUANT 2: scale = 127 / max|x|, an all-zero row giving zeros and scale 0.
-template <int QUANT, int ACT>
-__device__ __forceinline__ void quant_token_row(TokenRow &r)
+template <int QUANT, int ACT, typename Row, typename Max>
+__device__ __forceinline__ void quant_token_row(Row &r, const Max &row_max)
 {
     if (QUANT == 3) {
-        quant_token_row_fp8<ACT>(r);
+        quant_token_row_fp8<ACT, Row>(r);
         return;
     }
     float m = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kDispMaxChunks; ++j) {
+    for (int j = 0; j < Row::kChunks; ++j) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             m = fmaxf(m, fabsf(act_bits_to_f32<ACT>(r.raw[j][i] & 0xffffu)));
             m = fmaxf(m, fabsf(act_bits_to_f32<ACT>(r.raw[j][i] >> 16)));
         }
     }
-    m = wave_max(m);
+    m = row_max(m);
     // Keep the row as its 16-bit words across the two passes: left alone, the compiler holds the 112 converted
     // floats of the maximum pass for the scaling pass (a shift each to redo) and the kernel needs a third more
     // registers.
 #pragma unroll
-    for (int j = 0; j < kDispMaxChunks; ++j) {
+    for (int j = 0; j < Row::kChunks; ++j) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             asm volatile("" : "+v"(r.raw[j][i]));
@@ -160,7 +190,7 @@ __device__ __forceinline__ void quant_token_row(TokenRow &r)
     }
     r.scale_out = zero_row ? 0.0f : __fdiv_rn(1.0f, s);
 #pragma unroll
-    for (int j = 0; j < kDispMaxChunks; ++j) {
+    for (int j = 0; j < Row::kChunks; ++j) {
         int v[8];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -174,14 +204,15 @@ __device__ __forceinline__ void quant_token_row(TokenRow &r)
 // Quantisation of one COPY of a token row under a per-expert smooth scale
 // (src/cam/comm_operator/ascend_kernels/moe_dispatch_shmem/op_kernel/moe_dispatch_shmem.h:693-733):
 // xf = float(x) * smooth[h] (one rounded multiply), then the no-epsilon variant on xf.  r.raw is left untouched.
-template <int ACT>
-__device__ __forceinline__ void quant_token_row_smooth(TokenRow &r, const float *__restrict__ smooth, int H, int lane)
+template <int ACT, typename Row, typename Max>
+__device__ __forceinline__ void quant_token_row_smooth(Row &r, const float *__restrict__ smooth, int H, int lane,
+                                                       const Max &row_max)
 {
     const int nch = H >> 3;
     float m = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kDispMaxChunks; ++j) {
-        const int c = j * kWave + lane;
+    for (int j = 0; j < Row::kChunks; ++j) {
+        const int c = j * Row::kLanes + lane;
         if (c < nch) {
             const v4f s0 = *(const v4f *)(smooth + c * 8);
             const v4f s1 = *(const v4f *)(smooth + c * 8 + 4);
@@ -193,13 +224,13 @@ __device__ __forceinline__ void quant_token_row_smooth(TokenRow &r, const float 
             }
         }
     }
-    m = wave_max(m);
+    m = row_max(m);
     const bool zero_row = m == 0.0f;
     const float s = zero_row ? 0.0f : __fdiv_rn(127.0f, m);
     r.scale_out = zero_row ? 0.0f : __fdiv_rn(1.0f, s);
 #pragma unroll
-    for (int j = 0; j < kDispMaxChunks; ++j) {
-        const int c = j * kWave + lane;
+    for (int j = 0; j < Row::kChunks; ++j) {
+        const int c = j * Row::kLanes + lane;
         int v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         if (c < nch) {
             const v4f s0 = *(const v4f *)(smooth + c * 8);
@@ -216,16 +247,16 @@ __device__ __forceinline__ void quant_token_row_smooth(TokenRow &r, const float 
 }
 
 // Stores the row (quantised or raw) to output row `row`, with its scale and triple.
-template <int QUANT>
-__device__ __forceinline__ void store_token_row(const TokenRow &r, void *out, float *scales, int32_t *src_info,
+template <int QUANT, typename Row>
+__device__ __forceinline__ void store_token_row(const Row &r, void *out, float *scales, int32_t *src_info,
                                                 int src_rank, long long row, int t, int k, int H, int lane)
 {
     const int nch = H >> 3;
     if (QUANT != 0) {
         v2u *dst = (v2u *)((int8_t *)out + row * H);
 #pragma unroll
-        for (int j = 0; j < kDispMaxChunks; ++j) {
-            const int c = j * kWave + lane;
+        for (int j = 0; j < Row::kChunks; ++j) {
+            const int c = j * Row::kLanes + lane;
             if (c < nch) {
                 __builtin_nontemporal_store(r.q[j], dst + c);
             }
@@ -233,20 +264,20 @@ __device__ __forceinline__ void store_token_row(const TokenRow &r, void *out, fl
     } else {
         v4u *dst = (v4u *)((uint16_t *)out + row * H);
 #pragma unroll
-        for (int j = 0; j < kDispMaxChunks; ++j) {
-            const int c = j * kWave + lane;
+        for (int j = 0; j < Row::kChunks; ++j) {
+            const int c = j * Row::kLanes + lane;
             if (c < nch) {
                 __builtin_nontemporal_store(r.raw[j], dst + c);
             }
         }
     }
     if (QUANT == 3) {
-        // one E8M0 byte per 128 columns, written by the first lane of each quarter of the wave
+        // one E8M0 byte per 128 columns, written by the first of its sixteen threads
         uint8_t *sc = (uint8_t *)scales + row * (H >> 7);
         if ((lane & 15) == 0) {
 #pragma unroll
-            for (int j = 0; j < kDispMaxChunks; ++j) {
-                const int c = j * kWave + lane;
+            for (int j = 0; j < Row::kChunks; ++j) {
+                const int c = j * Row::kLanes + lane;
                 if (c < nch) {
                     sc[c >> 4] = (uint8_t)r.scale8[j];
                 }

@@ -26,12 +26,6 @@ namespace {
 constexpr int kScanThreads = 1024;  // single-workgroup scan kernel (notify)
 constexpr int kGlobalThreads = 512; // phase 2: one thread per expert column
 
-// The per-expert counts may lie in host memory a CPU is watching (each count on its own): stored for the whole system.
-__device__ __forceinline__ void store_count(int64_t *p, int v)
-{
-    __hip_atomic_store(p, (int64_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // Phase 1.  Workgroup b ranks the flat entries [b*chunk, (b+1)*chunk), chunk = IT*256 (rank_chunk), and
 // publishes the chunk's per-expert histogram in hist_out[b][*].
 template <typename IdT, int IT>
@@ -177,7 +171,6 @@ __global__ __launch_bounds__(kLocalThreads) void plan_single_kernel(PlanArgs a)
 {
     __shared__ int hist[kLocalWaves * kMaxExperts];
     __shared__ int cnt_s[kMaxExperts];
-    __shared__ int off_s[kMaxExperts];
     __shared__ int scan_s[kLocalWaves];
     __shared__ int total_s;
     __shared__ int active_s;
@@ -189,48 +182,13 @@ __global__ __launch_bounds__(kLocalThreads) void plan_single_kernel(PlanArgs a)
     const long long n_all = (long long)a.T * a.K;
     rank_chunk<IdT, IT>(idx, 0, n, n_all, E, hist, a.pos, cnt_s);
     __syncthreads();  // cnt_s complete; the ranks in a.pos are visible to the whole workgroup
-    // thread i owns experts 2i and 2i+1
-    int c2[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        c2[h] = 2 * tid + h < E ? cnt_s[2 * tid + h] : 0;
-    }
-    const int pair_off = block_exclusive_scan<kLocalWaves>(c2[0] + c2[1], tid, scan_s, &total_s);
-    const int total = total_s;
-    const int o2[2] = {pair_off, pair_off + c2[0]};
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int e = 2 * tid + h;
-        if (e < E) {
-            off_s[e] = o2[h];
-            if (a.cnt) a.cnt[e] = c2[h];
-            if (a.off) a.off[e] = o2[h];
-            if (a.recv_off) a.recv_off[e] = o2[h];
-            if (a.recv_count) a.recv_count[e] = o2[h] + c2[h];
-            if (a.tokens_per_expert) store_count(a.tokens_per_expert + e, c2[h]);
-            if (a.group_list) a.group_list[e] = (int64_t)o2[h] + c2[h];
-        }
-    }
+    write_expert_outputs<kLocalThreads>(a, cnt_s, t_active, tid, scan_s, &total_s);  // (leaves the offsets in cnt_s)
     __syncthreads();
     if (a.dst_row != nullptr) {
         for (long long i = tid; i < n_all; i += kLocalThreads) {
             const int e = i < n ? load_id(idx, i, E) : -1;
-            a.dst_row[i] = e >= 0 ? off_s[e] + a.pos[i] : -1;
+            a.dst_row[i] = e >= 0 ? cnt_s[e] + a.pos[i] : -1;
         }
-    }
-    if (tid == 0 && a.total) {
-        a.total[0] = total;
-    }
-    if (a.per_rank_zero != nullptr) {
-        for (int r = tid; r < a.R; r += kLocalThreads) {
-            a.per_rank_zero[r] = 0;
-        }
-    }
-    if (tid == 0 && a.meta != nullptr) {
-        a.meta[0] = 0;
-        a.meta[1] = total;
-        a.meta[2] = t_active;
-        a.meta[3] = 0;
     }
 }
 

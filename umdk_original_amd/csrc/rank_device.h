@@ -71,6 +71,56 @@ __device__ __forceinline__ int count_active(const uint8_t *mask, int T, int tid,
     return *slot;
 }
 
+// The per-expert counts may lie in host memory a CPU is watching (each count on its own): stored for the whole system.
+__device__ __forceinline__ void store_count(int64_t *p, int v)
+{
+    __hip_atomic_store(p, (int64_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Everything the plan says about the experts, from their complete counts cnt[0..E) (LDS), by one workgroup of NT >= 256
+// threads; leaves the exclusive offsets in cnt.
+template <int NT>
+__device__ __forceinline__ void write_expert_outputs(const PlanArgs &a, int *cnt, int t_active, int tid, int *scan_s, int *total_s)
+{
+    // thread i owns experts 2i and 2i+1
+    const int E = a.E;
+    int c2[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        c2[h] = 2 * tid + h < E ? cnt[2 * tid + h] : 0;
+    }
+    const int pair_off = block_exclusive_scan<NT / kWave>(c2[0] + c2[1], tid, scan_s, total_s);
+    const int total = *total_s;
+    const int o2[2] = {pair_off, pair_off + c2[0]};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int e = 2 * tid + h;
+        if (e < E) {
+            cnt[e] = o2[h];
+            if (a.cnt) a.cnt[e] = c2[h];
+            if (a.off) a.off[e] = o2[h];
+            if (a.recv_off) a.recv_off[e] = o2[h];
+            if (a.recv_count) a.recv_count[e] = o2[h] + c2[h];
+            if (a.tokens_per_expert) store_count(a.tokens_per_expert + e, c2[h]);
+            if (a.group_list) a.group_list[e] = (int64_t)o2[h] + c2[h];
+        }
+    }
+    if (tid == 0 && a.total) {
+        a.total[0] = total;
+    }
+    if (a.per_rank_zero != nullptr) {
+        for (int r = tid; r < a.R; r += NT) {
+            a.per_rank_zero[r] = 0;
+        }
+    }
+    if (tid == 0 && a.meta != nullptr) {
+        a.meta[0] = 0;
+        a.meta[1] = total;
+        a.meta[2] = t_active;
+        a.meta[3] = 0;
+    }
+}
+
 // Ranks the chunk of flat entries [b*IT*256, (b+1)*IT*256) of one workgroup of 256 threads.
 // Wave w owns the IT*64 entries from b*chunk + w*IT*64 and each lane keeps its IT ids in registers.
 // 64 ids at a time, lanes holding the same id find each other with one ballot per id bit; the rank
