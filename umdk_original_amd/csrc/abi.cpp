@@ -1403,6 +1403,7 @@ camStatus camMoeCombineShmemGetWorkspaceSize(
     CAM_TRY(check_aligned(expandX, "expandX", 16));
     CAM_TRY(check_aligned(out, "out", 16));
     Carver c;
+    c.take((uint64_t)T * K * 4);  // (a row per slot: not written any more, part of the size that callers provide)
     const uint64_t o_wire = wire ? c.take((uint64_t)A * (uint64_t)(H + H / 4)) : 0;
     cam::CombineArgs g{};
     g.y = (const uint16_t *)expandX->data;
