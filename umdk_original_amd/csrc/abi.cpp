@@ -328,7 +328,8 @@ hipError_t run_grouped_gemm(cam::GemmArgs g, const int64_t *group_list, int cumu
 
 // The GEMMs of a fused layer: per-expert counts from its plan, g.sched filled when the permute built schedules.  A token
 // names an expert once, so no expert has more than T rows.
-hipError_t layer_gemm(const cam::GemmArgs &g, const int64_t *counts, int E, int64_t A, int T, bool stream, hipStream_t s)
+hipError_t layer_gemm(const cam::GemmArgs &g, const int64_t *counts, int E, int64_t A, int T, bool stream, hipStream_t s,
+                      const float *products = nullptr)
 {
     if (!stream) {
         return cam::launch_gemm(g, s);
@@ -338,6 +339,7 @@ hipError_t layer_gemm(const cam::GemmArgs &g, const int64_t *counts, int E, int6
     sa.group_list = counts;
     sa.G = E;
     sa.max_rows = A;
+    sa.products = products;
     return cam::launch_stream_gemm(sa, T, s);
 }
 
@@ -1822,7 +1824,10 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     const uint64_t shared_bytes = std::max<uint64_t>((uint64_t)A * H * 2, x1_bytes + (uint64_t)A * I * 4);
     const uint64_t o_x1 = c.take(shared_bytes);
     const uint64_t o_prod = o_x1 + x1_bytes;
-    const uint64_t o_y = o_x1;
+    // Few rows: GMM2 quantises the products itself, and then writes its rows while they are still read.
+    const bool stream = cam::stream_gemm_applies(A, 2 * I);
+    const bool from_products = stream && cam::stream_gemm_takes_products(A, (int)Epr, (int)I, (int)H, T);
+    const uint64_t o_y = from_products ? c.take((uint64_t)A * H * 2) : o_x1;
     const uint64_t o_x1s = c.take((uint64_t)A * 4);
     const uint64_t o_x2 = c.take((uint64_t)A * I);
     const uint64_t o_x2s = c.take((uint64_t)A * 4);
@@ -1835,7 +1840,6 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     uint16_t *outp = (uint16_t *)output->data;
     int64_t *etn = (int64_t *)expertTokenNums->data;
     const int iT = (int)T, iK = (int)K, iH = (int)H, iI = (int)I, iE = (int)Epr;
-    const bool stream = cam::stream_gemm_applies(A, 2 * I);
 
     auto run = [=](void *wsp, hipStream_t s) -> hipError_t {
         char *w = (char *)wsp;
@@ -1907,8 +1911,10 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         g1.out = prod;
         e = layer_gemm(g1, etn, iE, A, iT, stream, s);
         if (e != hipSuccess) return e;
-        e = cam::launch_requant(prod, A, iI, stream ? meta : specs[0].sched, x2, x2s, s);  // [1] of both: rows that exist
-        if (e != hipSuccess) return e;
+        if (!from_products) {
+            e = cam::launch_requant(prod, A, iI, stream ? meta : specs[0].sched, x2, x2s, s);  // [1] of both: rows that exist
+            if (e != hipSuccess) return e;
+        }
 
         cam::GemmArgs g2{};
         g2.a = x2;
@@ -1924,7 +1930,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         g2.epilogue = cam::kEpiDequantBf16;
         g2.out = y;
         g2.out_fp16 = x_is_fp16;
-        e = layer_gemm(g2, etn, iE, A, iT, stream, s);
+        e = layer_gemm(g2, etn, iE, A, iT, stream, s, from_products ? prod : nullptr);
         if (e != hipSuccess) return e;
 
         cam::CombineArgs cb{};

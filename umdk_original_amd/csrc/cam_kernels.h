@@ -200,8 +200,12 @@ struct StreamGemmArgs {
     int cumulative, G;
     long long max_rows;         // rows of the tensors
     int32_t *rows_out;          // optional: [1] receives the total row count (where launch_requant looks for it)
+    const float *products;      // optional [max_rows,Kd], instead of g.a and g.a_scale: fp32 rows that the kernel quantises the
+                                // way launch_requant does, bit for bit (where stream_gemm_takes_products says so)
 };
 bool stream_gemm_applies(int64_t rows, int64_t N);  // whether it is the faster form
+// Whether a launch without a gate/up pair quantises its activations from fp32 rows faster than launch_requant before it.
+bool stream_gemm_takes_products(int64_t max_rows, int G, int Kd, int N, int64_t rows_per_expert);
 // rows_per_expert: the most rows one expert can have, as far as the host knows.
 hipError_t launch_stream_gemm(const StreamGemmArgs &a, int64_t rows_per_expert, hipStream_t stream);
 

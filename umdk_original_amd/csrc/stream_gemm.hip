@@ -27,6 +27,11 @@
 //   * No schedule: every workgroup derives the item list from the per-expert row counts by itself (a prefix sum over
 //     at most 512 experts) and takes items in a fixed order.  All items of a launch stream the same number of bytes,
 //     so nothing has to be balanced, and no builder runs before the GEMM.
+//   * In a layer whose tiles are a few thousand products each, the GMM2 launch quantises its activations itself (PRODUCTS):
+//     every workgroup reads the fp32 SwiGLU products of its tile, finds the row maxima and leaves the int8 rows in LDS while
+//     its first weights are on their way.  Column blocks repeat that work, but it is a microsecond or two of latency
+//     where a launch of requant_kernel takes 3.4 (layers: one token, H 4096, I 1536: 45.9 -> 44.1 us; 128 tokens on 8
+//     experts, H 1024, I 512: 26.3 -> 25.1).
 #include <algorithm>
 
 #include "cam_device.h"
@@ -42,6 +47,8 @@ namespace {
 constexpr int kSThreads = 512;
 constexpr int R = 2;                     // 64-byte K steps in flight per wave
 constexpr int kSMaxKb = 64;              // FP8: K blocks of 128 bytes (Kd <= 8192)
+constexpr int kSBuf32 = 32768;           // activation buffer of the 32-row tiles
+constexpr int kProductQuads = 16;        // PRODUCTS: quads of products a thread holds, i.e. 32 K products a workgroup
 
 __device__ __forceinline__ void lds_barrier()
 {
@@ -92,12 +99,12 @@ struct StreamItem {     // wave-uniform
     int wstep;          // bytes from one 64-byte K step to the next
 };
 
-template <int MF, bool FP8, int P>
+template <int MF, bool FP8, int P, bool PRODUCTS>
 __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel(StreamGemmArgs sa)
 {
     typedef typename SAcc<FP8>::v16 acc16;
     typedef typename SAcc<FP8>::v4 acc4;
-    constexpr int kABuf = MF == 1 ? 32768 : 65536;  // one of the two activation buffers
+    constexpr int kABuf = MF == 1 ? kSBuf32 : 65536;  // one of the two activation buffers
     constexpr int kSLds = 2 * kABuf;
     constexpr int NFR = MF == 1 ? 1 : 2;            // column fragments whose partial sums (32 KB each) fit a buffer
     const GemmArgs &a = sa.g;
@@ -111,7 +118,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     __shared__ __attribute__((aligned(16))) float row_scale_s[2][FP8 ? 4 : 32 * MF];
     __shared__ __attribute__((aligned(16))) uint8_t a_scale8_s[2][FP8 ? kSMaxKb * 32 * MF : 4];
     __shared__ uint8_t w_scale8_s[FP8 ? 16 * kSMaxKb : 4];
-    __shared__ float rowmax_s[FP8 ? 8 * 32 : 1];
+    __shared__ float rowmax_s[FP8 ? 8 * 32 : PRODUCTS ? 8 : 1];
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -128,6 +135,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     constexpr int quantum = S * R > 4 ? 64 * S * R : 256;  // K bytes of one turn of all S waves
     static_assert(NFR == 2 || S >= 4, "sums that pass one fragment at a time wait in registers for one block only");
     static_assert(32 * MF * quantum <= kABuf, "a turn of a full tile has to fit an activation buffer");
+    static_assert(!PRODUCTS || (MF == 1 && !FP8), "products are quantised by the 32-row tiles");
     const int kpad = (Kd + quantum - 1) / quantum * quantum;
 
     // ---- the item list: rows, first row and row tiles of every expert (thread e: expert e)
@@ -282,7 +290,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
                              : "memory", "m0");
             }
             const int r = tid - 128;        // the waves from the third on: a row each lane
-            if (r >= 0 && r < it.rows) {
+            if (!PRODUCTS && r >= 0 && r < it.rows) {
                 const unsigned dst = lds_addr(&row_scale_s[set][0]) + (unsigned)((wave - 2) * 256);
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                              :
@@ -339,6 +347,66 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
         }
     };
 
+    // ---- PRODUCTS: the tile's rows from fp32 products, all of K at once (the host has checked that it fits).  The threads
+    // share the rows evenly, 512 / (rows, rounded up to a power of two) to a row, so that one round trip brings
+    // everything; the arithmetic is requant_kernel's.
+    v4f prod[PRODUCTS ? kProductQuads : 1];
+    auto load_products = [&](const StreamItem &it) {
+        const int lg = 9 - (it.rows > 1 ? 32 - __clz(it.rows - 1) : 0);   // log2 of the threads per row
+        const int row = tid >> lg, l = tid & ((1 << lg) - 1);
+        const v4f *src = (const v4f *)(sa.products + (long long)(it.row0 + min(row, it.rows - 1)) * Kd);
+#pragma unroll
+        for (int j = 0; j < (PRODUCTS ? kProductQuads : 1); ++j) {
+            const int c = l + (j << lg);
+            prod[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            if (c < Kd >> 2) {
+                prod[j] = src[c];
+            }
+        }
+    };
+    auto quantise_products = [&](const StreamItem &it, int buf, int set) {
+        const int lg = 9 - (it.rows > 1 ? 32 - __clz(it.rows - 1) : 0);
+        const int row = tid >> lg, l = tid & ((1 << lg) - 1);
+        float m = 0.0f;
+#pragma unroll
+        for (int j = 0; j < (PRODUCTS ? kProductQuads : 1); ++j) {
+            m = fmaxf(m, fmaxf(fmaxf(fabsf(prod[j][0]), fabsf(prod[j][1])), fmaxf(fabsf(prod[j][2]), fabsf(prod[j][3]))));
+        }
+        for (int off = 1; off < min(1 << lg, kWave); off <<= 1) {
+            m = fmaxf(m, __shfl_xor(m, off, kWave));
+        }
+        if (lg > 6) {   // several waves to a row (all of them take this branch)
+            if (lane == 0) {
+                rowmax_s[wave] = m;
+            }
+            lds_barrier();
+            const int w0 = wave & ~((1 << (lg - 6)) - 1);
+            for (int i = 0; i < 1 << (lg - 6); ++i) {
+                m = fmaxf(m, rowmax_s[w0 + i]);
+            }
+        }
+        if (row < it.rows) {
+            const bool zero_row = m == 0.0f;
+            const float rcp = zero_row ? 0.0f : __fdiv_rn(1.0f, m);
+            if (l == 0) {
+                row_scale_s[set][row] = zero_row ? 0.0f : __fmul_rn(m, 1.0f / 127.0f);
+            }
+            int8_t *dst = lds + buf * kABuf + row * it.ckb;
+#pragma unroll
+            for (int j = 0; j < (PRODUCTS ? kProductQuads : 1); ++j) {
+                const int c = l + (j << lg);
+                if (c < Kd >> 2) {
+                    int b[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        b[e] = (int)rintf(__fmul_rn(__fmul_rn(prod[j][e], 127.0f), rcp));
+                    }
+                    *(uint32_t *)(dst + (((c >> 2) ^ (row & 15)) << 4) + (c & 3) * 4) = pack4(b[0], b[1], b[2], b[3]);
+                }
+            }
+        }
+    };
+
     // The youngest requests of a wave are its ring (4 pieces a step, younger than the activations): with no more than
     // those outstanding, its share of the activations has landed.
     auto a_landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * R) : "memory"); };
@@ -350,11 +418,18 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     if (cur.rows <= 0) {
         return;
     }
-    load_a(cur, 0, 0);
+    if constexpr (PRODUCTS) {
+        load_products(cur);
+    } else {
+        load_a(cur, 0, 0);
+    }
     load_scales(cur, 0);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         issue(r, cur, 0);
+    }
+    if constexpr (PRODUCTS) {
+        quantise_products(cur, 0, 0);
     }
     store_scales(cur, 0);
     a_landed();
@@ -393,7 +468,9 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
             if (!last_chunk) {
                 load_a(cur, c + 1, buf ^ 1);
             } else if (more) {
-                load_a(nxt, 0, buf ^ 1);
+                if constexpr (!PRODUCTS) {
+                    load_a(nxt, 0, buf ^ 1);
+                }
                 load_scales(nxt, set ^ 1);
             }
             const int8_t *abuf = lds + buf * kABuf;
@@ -621,13 +698,18 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
         buf ^= 1;
         set ^= 1;
         cur = nxt;
+        if constexpr (PRODUCTS) {
+            load_products(cur);
+            quantise_products(cur, buf, set);
+            lds_barrier();
+        }
     }
 }
 
-template <int MF, bool FP8, int P>
+template <int MF, bool FP8, int P, bool PRODUCTS = false>
 void launch_kernel(unsigned grid, hipStream_t stream, const StreamGemmArgs &sa)
 {
-    hipLaunchKernelGGL((stream_gemm_kernel<MF, FP8, P>), dim3(grid), dim3(kSThreads), 0, stream, sa);
+    hipLaunchKernelGGL((stream_gemm_kernel<MF, FP8, P, PRODUCTS>), dim3(grid), dim3(kSThreads), 0, stream, sa);
 }
 
 template <bool FP8>
@@ -642,6 +724,56 @@ void launch_variant(int mf, int P, unsigned grid, hipStream_t stream, const Stre
     }
 }
 
+struct StreamShape {
+    bool small;      // 32-row tiles
+    int P;           // column groups per item
+    long long items; // at most
+    unsigned grid;
+};
+
+StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool quad, int64_t rows_per_expert, int cus)
+{
+    StreamShape sh;
+    // live experts at most, and the column groups they stream
+    const long long live = std::min<long long>(G, max_rows);
+    const long long groups = live * (N / 64);
+    const bool many = groups >= 6ll * cus;
+    // 32-row tiles, two workgroups per CU, while the stream is short: few column groups and no expert with more rows, or
+    // all tiles resident at once.  Otherwise 128-row tiles, so that an expert's weights are read once.
+    sh.small = !quad && ((rows_per_expert <= 32 && !many) || groups + max_rows / 32 * (N / 64) <= 2ll * cus);
+    // Column groups per item: as few as it takes to give every CU work, then up to a megabyte of weights per item (an
+    // item's sums and stores interrupt its stream for about two microseconds).  kEpiSwigluFp8 needs the four groups
+    // of a 128-column block together, and the fp32 products of kEpiSwiglu are the same sums in the same order (quad).
+    sh.P = 2;
+    if (sh.small) {
+        sh.P = 2 * groups >= 3ll * cus ? 2 : 1;
+    } else if (many) {
+        sh.P = 512ll * Kd <= (1 << 20) ? 8 : 4;
+    } else if (quad) {
+        sh.P = 4;
+    }
+    const long long tiles = live + max_rows / (sh.small ? 32 : 128);
+    sh.items = tiles * ((N / 64 + sh.P - 1) / sh.P);
+    // a multiple of eight workgroups: every XCD takes an eighth of the items
+    sh.grid = (unsigned)((std::min<long long>(sh.items, (sh.small ? 2ll : 1ll) * cus) + kNumXcd - 1) / kNumXcd * kNumXcd);
+    return sh;
+}
+
+// Whether a tile's products fit the registers of a workgroup, and its int8 rows (padded to a turn of the eight waves) an
+// activation buffer.
+bool products_fit(const StreamShape &sh, long long max_rows, int Kd)
+{
+    if (!sh.small || Kd % 128 != 0) {
+        return false;
+    }
+    long long rows = 1;
+    while (rows < std::min<long long>(32, max_rows)) {
+        rows *= 2;
+    }
+    const long long turn = 64 * (8 / sh.P) * R;
+    return rows * Kd <= 4ll * kProductQuads * kSThreads && rows * ((Kd + turn - 1) / turn * turn) <= kSBuf32;
+}
+
 }  // namespace
 
 // Rows x columns up to which the stream is the faster form: 64 rows per expert where the tile kernel has half as many
@@ -651,6 +783,17 @@ bool stream_gemm_applies(int64_t rows, int64_t N)
 {
     constexpr int64_t kMostRowsTimesColumns = 32ll * 512 * 256;
     return rows > 0 && rows * N <= kMostRowsTimesColumns;
+}
+
+// Where every workgroup has one item at most: with more, the quantisation of an item would interrupt the stream.
+bool stream_gemm_takes_products(int64_t max_rows, int G, int Kd, int N, int64_t rows_per_expert)
+{
+    int cus = 0;
+    if (max_rows <= 0 || G <= 0 || gemm_workgroups(&cus) != hipSuccess) {
+        return false;
+    }
+    const StreamShape sh = stream_shape(G, max_rows, Kd, N, false, rows_per_expert, cus);
+    return sh.items <= (long long)sh.grid && products_fit(sh, max_rows, Kd);
 }
 
 hipError_t launch_stream_gemm(const StreamGemmArgs &sa, int64_t rows_per_expert, hipStream_t stream)
@@ -672,34 +815,16 @@ hipError_t launch_stream_gemm(const StreamGemmArgs &sa, int64_t rows_per_expert,
     if (e != hipSuccess) {
         return e;
     }
-    // live experts at most, and the column groups they stream
-    const long long live = std::min<long long>(sa.G, sa.max_rows);
-    const long long groups = live * (g.N / 64);
-    const bool many = groups >= 6ll * cus;
-    // 32-row tiles, two workgroups per CU, while the stream is short: few column groups and no expert with more rows, or
-    // all tiles resident at once.  Otherwise 128-row tiles, so that an expert's weights are read once.
-    const bool quad = g.fp8 && g.gate_up;
-    const bool small = !quad &&
-                       ((rows_per_expert <= 32 && !many) || groups + sa.max_rows / 32 * (g.N / 64) <= 2ll * cus);
-    // Column groups per item: as few as it takes to give every CU work, then up to a megabyte of weights per item (an
-    // item's sums and stores interrupt its stream for about two microseconds).  kEpiSwigluFp8 needs the four groups
-    // of a 128-column block together, and the fp32 products of kEpiSwiglu are the same sums in the same order (quad).
-    int P = 2;
-    if (small) {
-        P = 2 * groups >= 3ll * cus ? 2 : 1;
-    } else if (many) {
-        P = 512ll * g.Kd <= (1 << 20) ? 8 : 4;
-    } else if (quad) {
-        P = 4;
-    }
-    const long long tiles = live + sa.max_rows / (small ? 32 : 128);
-    const long long items = tiles * ((g.N / 64 + P - 1) / P);
-    // a multiple of eight workgroups: every XCD takes an eighth of the items
-    const unsigned grid = (unsigned)((std::min<long long>(items, (small ? 2ll : 1ll) * cus) + kNumXcd - 1) / kNumXcd * kNumXcd);
-    if (g.fp8) {
-        launch_variant<true>(small ? 1 : 4, P, grid, stream, sa);
+    const StreamShape sh = stream_shape(sa.G, sa.max_rows, g.Kd, g.N, g.fp8 && g.gate_up, rows_per_expert, cus);
+    if (sa.products != nullptr) {
+        if (g.fp8 || g.gate_up || !products_fit(sh, sa.max_rows, g.Kd)) {
+            return hipErrorInvalidValue;
+        }
+        sh.P == 1 ? launch_kernel<1, false, 1, true>(sh.grid, stream, sa) : launch_kernel<1, false, 2, true>(sh.grid, stream, sa);
+    } else if (g.fp8) {
+        launch_variant<true>(sh.small ? 1 : 4, sh.P, sh.grid, stream, sa);
     } else {
-        launch_variant<false>(small ? 1 : 4, P, grid, stream, sa);
+        launch_variant<false>(sh.small ? 1 : 4, sh.P, sh.grid, stream, sa);
     }
     return hipGetLastError();
 }
