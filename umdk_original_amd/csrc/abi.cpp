@@ -408,35 +408,21 @@ camStatus camDispatchLayoutGetWorkspaceSize(const camTensor *topkIdx, int64_t nu
         return fail(CAM_ERR_SHAPE, "DispatchLayout outputs must be [R], [E] and [T,R]");
     }
     Carver c;
-    const uint64_t o_pos = c.take((uint64_t)numTokens * numTopk * 4);
-    const uint64_t o_hist = c.take(cam::plan_workspace_bytes(numTokens, numTopk, (int)numExperts));
-    cam::PlanArgs p{};
-    p.idx = topkIdx->data;
-    p.idx_is64 = topkIdx->dtype == CAM_DT_INT64;
-    p.T = (int)numTokens;
-    p.K = (int)numTopk;
-    p.E = (int)numExperts;
-    p.R = (int)numRanks;
-    p.cnt = (int32_t *)numTokensPerExpert->data;
-    p.per_rank_zero = (int32_t *)numTokensPerRank->data;
-    cam::InRankArgs r{};
-    r.idx = p.idx;
-    r.idx_is64 = p.idx_is64;
-    r.T = p.T;
-    r.K = p.K;
-    r.E = p.E;
-    r.R = p.R;
-    r.in_rank = isTokenInRank->data;
-    r.in_rank_bytes = isTokenInRank->dtype == CAM_DT_INT32 ? 4 : 1;
-    r.per_rank = (int32_t *)numTokensPerRank->data;
-    auto run = [p, r, o_pos, o_hist](void *ws, hipStream_t s) mutable -> hipError_t {
-        p.pos = (int32_t *)((char *)ws + o_pos);
-        p.hist_ws = (int32_t *)((char *)ws + o_hist);
-        hipError_t e = cam::launch_plan(p, s);
-        if (e != hipSuccess) {
-            return e;
-        }
-        return cam::launch_in_rank(r, s);
+    const uint64_t o_partial = c.take(cam::layout_workspace_bytes(numTokens, (int)numExperts, (int)numRanks));
+    cam::LayoutArgs l{};
+    l.idx = topkIdx->data;
+    l.idx_is64 = topkIdx->dtype == CAM_DT_INT64;
+    l.T = (int)numTokens;
+    l.K = (int)numTopk;
+    l.E = (int)numExperts;
+    l.R = (int)numRanks;
+    l.in_rank = isTokenInRank->data;
+    l.in_rank_bytes = isTokenInRank->dtype == CAM_DT_INT32 ? 4 : 1;
+    l.per_expert = (int32_t *)numTokensPerExpert->data;
+    l.per_rank = (int32_t *)numTokensPerRank->data;
+    auto run = [l, o_partial](void *ws, hipStream_t s) mutable -> hipError_t {
+        l.partial = (int32_t *)((char *)ws + o_partial);
+        return cam::launch_layout(l, s);
     };
     return finish_phase1(kOpLayout, c.off, run, workspaceSize, executor);
 }
@@ -565,7 +551,6 @@ camStatus validate_plan(const camTensor *topkIdx, int64_t numExperts, int64_t nu
     p.T = (int)T;
     p.K = (int)K;
     p.E = (int)numExperts;
-    p.R = 1;
     p.pos = (int32_t *)sendTokenIdx->data;
     p.dst_row = slotRowOptional ? (int32_t *)slotRowOptional->data : nullptr;
     p.cnt = numTokensPerExpert ? (int32_t *)numTokensPerExpert->data : nullptr;
@@ -920,7 +905,6 @@ camStatus camMoeDispatchPrefillGetWorkspaceSize(const camTensor *x, const camTen
     p.T = (int)T;
     p.K = (int)K;
     p.E = (int)numExperts;
-    p.R = 1;
     p.pos = (int32_t *)sendTokenIdx->data;
     p.dst_row = slotRowOptional ? (int32_t *)slotRowOptional->data : nullptr;
     p.cnt = numTokensPerExpertOptional ? (int32_t *)numTokensPerExpertOptional->data : nullptr;
@@ -1281,7 +1265,6 @@ camStatus camMoeDispatchShmemGetWorkspaceSize(const camTensor *x, const camTenso
     p.T = (int)T;
     p.K = (int)K;
     p.E = (int)moeExpertNum;
-    p.R = 1;
     p.pos = (int32_t *)expandIdxOut->data;
     p.recv_count = (int32_t *)epRecvCountOut->data;
     if (expertTokenNumsType == 0) {
@@ -1860,7 +1843,6 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         p.T = iT;
         p.K = iK;
         p.E = iE;
-        p.R = 1;
         p.pos = pos;
         p.dst_row = row;
         p.tokens_per_expert = etn;
@@ -2218,7 +2200,6 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         p.T = iT;
         p.K = iK;
         p.E = iE;
-        p.R = 1;
         p.pos = pos;
         p.dst_row = row;
         p.tokens_per_expert = etn;

@@ -52,8 +52,6 @@ struct PlanArgs {
     int64_t *tokens_per_expert;  // [E] optional
     int64_t *group_list;      // [E]    optional cumulative rows, int64
     int64_t *total;           // [1]    optional
-    int32_t *per_rank_zero;   // [R]    optional: zeroed here so a later kernel can accumulate into it
-    int R;
     int32_t *meta;            // optional run metadata, kPlanMeta ints (see above)
     int32_t *hist_ws;         // required scratch of plan_workspace_bytes(T, K, E) bytes
 };
@@ -62,16 +60,19 @@ uint64_t plan_workspace_bytes(int64_t T, int64_t K, int E);
 void plan_geometry(long long n_all, int *it_out, int *nb_out);
 hipError_t launch_plan(const PlanArgs &a, hipStream_t stream);
 
-// isTokenInRank / numTokensPerRank (per_rank must have been zeroed on the same stream).
-struct InRankArgs {
-    const void *idx;
+// DispatchLayout: counts per expert and per rank, and which ranks a token goes to.
+struct LayoutArgs {
+    const void *idx;      // [T,K] int32 or int64
     int idx_is64;
     int T, K, E, R;
-    void *in_rank;     // [T,R] int32 or 1-byte
-    int in_rank_bytes; // 4 or 1
-    int32_t *per_rank; // [R]
+    void *in_rank;        // [T,R] int32 or 1-byte
+    int in_rank_bytes;    // 4 or 1
+    int32_t *per_expert;  // [E]
+    int32_t *per_rank;    // [R]
+    int32_t *partial;     // scratch of layout_workspace_bytes(T, E, R) bytes
 };
-hipError_t launch_in_rank(const InRankArgs &a, hipStream_t stream);
+uint64_t layout_workspace_bytes(int64_t T, int E, int R);
+hipError_t launch_layout(const LayoutArgs &a, hipStream_t stream);
 
 // NotifyDispatch on one rank: exclusive scan + triplets.
 hipError_t launch_notify_scan(const int32_t *cnt, int E, int num_tokens, int32_t *off, int32_t *send_data,

@@ -108,11 +108,6 @@ __device__ __forceinline__ void write_expert_outputs(const PlanArgs &a, int *cnt
     if (tid == 0 && a.total) {
         a.total[0] = total;
     }
-    if (a.per_rank_zero != nullptr) {
-        for (int r = tid; r < a.R; r += NT) {
-            a.per_rank_zero[r] = 0;
-        }
-    }
     if (tid == 0 && a.meta != nullptr) {
         a.meta[0] = 0;
         a.meta[1] = total;
