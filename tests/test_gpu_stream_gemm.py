@@ -48,6 +48,7 @@ def test_stream_gemm_operators_bit_exact(gpu, oracle, sizes, H, I, list_type):
     ([1, 33, 0, 128], 640, 768),     # five K blocks: a row's scales are no whole words
     ([9, 2], 4096, 512),             # 32 K blocks, two turns of a chunk
     ([130], 128, 256),               # one K block, two row tiles
+    ([0, 34, 62] * 10, 256, 8192),   # 32 rows per expert on average, beyond the limit of int8
 ])
 def test_stream_gemm_fp8_sums(gpu, oracle, sizes, K, N):
     announce("stream fp8 gemm sizes=%s K=%d N=%d" % (sizes, K, N))

@@ -307,7 +307,7 @@ hipError_t run_grouped_gemm(cam::GemmArgs g, const int64_t *group_list, int cumu
 {
     int32_t *ws = (int32_t *)sched_ws;
     *rows = ws;
-    if (g.epilogue != cam::kEpiInt32 && cam::stream_gemm_applies(A, g.N)) {
+    if (g.epilogue != cam::kEpiInt32 && cam::stream_gemm_applies(A, g.N, G, g.fp8 != 0)) {
         cam::StreamGemmArgs sa{};
         sa.g = g;
         sa.group_list = group_list;
@@ -1808,7 +1808,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     const uint64_t o_x1 = c.take(shared_bytes);
     const uint64_t o_prod = o_x1 + x1_bytes;
     // Few rows: GMM2 quantises the products itself, and then writes its rows while they are still read.
-    const bool stream = cam::stream_gemm_applies(A, 2 * I);
+    const bool stream = cam::stream_gemm_applies(A, 2 * I, Epr, false);
     const bool from_products = stream && cam::stream_gemm_takes_products(A, (int)Epr, (int)I, (int)H, T);
     const uint64_t o_y = from_products ? c.take((uint64_t)A * H * 2) : o_x1;
     const uint64_t o_x1s = c.take((uint64_t)A * 4);
@@ -2179,7 +2179,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
     uint16_t *outp = (uint16_t *)output->data;
     int64_t *etn = (int64_t *)expertTokenNums->data;
     const int iT = (int)T, iK = (int)K, iE = (int)E, iH = (int)H, iI = (int)I;
-    const bool stream = cam::stream_gemm_applies(A, 2 * I);
+    const bool stream = cam::stream_gemm_applies(A, 2 * I, E, true);
 
     auto run = [=](void *wsp, hipStream_t s) -> hipError_t {
         char *w = (char *)wsp;

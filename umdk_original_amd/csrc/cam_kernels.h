@@ -204,7 +204,7 @@ struct StreamGemmArgs {
     const float *products;      // optional [max_rows,Kd], instead of g.a and g.a_scale: fp32 rows that the kernel quantises the
                                 // way launch_requant does, bit for bit (where stream_gemm_takes_products says so)
 };
-bool stream_gemm_applies(int64_t rows, int64_t N);  // whether it is the faster form
+bool stream_gemm_applies(int64_t rows, int64_t N, int64_t G, bool fp8);  // whether it is the faster form
 // Whether a launch without a gate/up pair quantises its activations from fp32 rows faster than launch_requant before it.
 bool stream_gemm_takes_products(int64_t max_rows, int G, int Kd, int N, int64_t rows_per_expert);
 // rows_per_expert: the most rows one expert can have, as far as the host knows.

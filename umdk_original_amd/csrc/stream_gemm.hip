@@ -779,10 +779,15 @@ bool products_fit(const StreamShape &sh, long long max_rows, int Kd)
 // Rows x columns up to which the stream is the faster form: 64 rows per expert where the tile kernel has half as many
 // 512-column items as CUs, 32 where it has as many, 10 where it has three times as many (measured with the shapes of
 // DeepSeek-V3's, Qwen3's and smaller layers, 2 to 3072 rows; the two forms are within 5 % of each other along this line).
-bool stream_gemm_applies(int64_t rows, int64_t N)
+// FP8 goes on to three times as many while experts have no more than 32 rows on average, i.e. most of them one tile (layers,
+// tile form -> this: 150 tokens on 40 experts, top-8, H 7168, I 2048: 407 -> 342 us; 1500 on 64, top-1, H 3072, I 2560: 332 ->
+// 273; 512 on 128, top-8, H 4096, I 1536: 483 -> 464; with five times as many 1000 on 256, top-8, H 2048, I 1024 lost, 362 -> 367,
+// and with 37 rows on average 300 on 64, H 2048, I 1408, 160 -> 162).  The tiles of the other form fetch FP8 scales item by item;
+// int8 gains from 322 -> 296 to 391 -> 362 on some of these shapes and loses from 449 -> 465 to 480 -> 503 on others.
+bool stream_gemm_applies(int64_t rows, int64_t N, int64_t G, bool fp8)
 {
     constexpr int64_t kMostRowsTimesColumns = 32ll * 512 * 256;
-    return rows > 0 && rows * N <= kMostRowsTimesColumns;
+    return rows > 0 && (rows * N <= kMostRowsTimesColumns || (fp8 && rows <= 32 * G && rows * N <= 3 * kMostRowsTimesColumns));
 }
 
 // Where every workgroup has one item at most: with more, the quantisation of an item would interrupt the stream.
