@@ -48,11 +48,14 @@ __global__ void invert_src_info_kernel(const int32_t *src_info, long long A, con
     }
 }
 
-// The row of slot (t,k), or -1: from the map, or, with a.ids, the way the SHMEM combine finds it
+// The row of slot (t,k), or -1: from the map, or, with BY_COUNTS, the way the SHMEM combine finds it
 // (moe_combine_shmem.h:514-556,833-837): the rows of the experts before the slot's, plus its rank within the expert.
+// Chosen at compile time: asked per slot it stands between the row loads of a gather (dispatch + combine of 4096 tokens x 7168,
+// 151.0 us instead of 150.7).
+template <bool BY_COUNTS>
 __device__ __forceinline__ long long row_of_slot(const CombineArgs &a, long long slot)
 {
-    if (a.ids == nullptr) {
+    if (!BY_COUNTS) {
         return a.slot_row[slot];
     }
     // (no branch, so that the loads of a token's slots stay side by side)
@@ -111,7 +114,7 @@ __device__ __forceinline__ float comb_act_to_f32(uint32_t bits16)
     return ACT == 0 ? bf16_bits_to_f32(bits16) : fp16_bits_to_f32(bits16);
 }
 
-template <bool WIRE, int ACT>
+template <bool WIRE, int ACT, bool BY_COUNTS>
 __global__ __launch_bounds__(kCombThreads) void combine_kernel(CombineArgs a, int segs)
 {
     const int t = blockIdx.x / segs;
@@ -145,7 +148,7 @@ __global__ __launch_bounds__(kCombThreads) void combine_kernel(CombineArgs a, in
                 v[j] = v4u{0u, 0u, 0u, 0u};
                 if (k < a.K) {
                     const long long slot = (long long)t * a.K + k;
-                    const long long row = row_of_slot(a, slot);
+                    const long long row = row_of_slot<BY_COUNTS>(a, slot);
                     bool good = row >= 0 && row < rows;
                     if (good && a.src_info != nullptr) {
                         // The inverse map is not pre-cleared: accept a row only if it names this slot.
@@ -215,6 +218,7 @@ constexpr int kWireBatch = 4;
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
+template <bool BY_COUNTS>
 __global__ __launch_bounds__(kCombThreads) void combine_wire16_kernel(CombineArgs a, int segs)
 {
     const int t = blockIdx.x / segs;
@@ -246,7 +250,7 @@ __global__ __launch_bounds__(kCombThreads) void combine_wire16_kernel(CombineArg
                 sc2[j] = 0u;
                 if (k < a.K) {
                     const long long slot = (long long)t * a.K + k;
-                    const long long row = row_of_slot(a, slot);
+                    const long long row = row_of_slot<BY_COUNTS>(a, slot);
                     bool good = row >= 0 && row < rows;
                     if (good && a.src_info != nullptr) {
                         good = a.src_info[3 * row + 1] == t && a.src_info[3 * row + 2] == k;
@@ -336,7 +340,8 @@ hipError_t launch_comm_quant(const uint16_t *y, int act_fp16, int64_t A, int H, 
     return hipGetLastError();
 }
 
-hipError_t launch_combine(const CombineArgs &a, hipStream_t stream)
+template <bool BY_COUNTS>
+static hipError_t launch_combine_as(const CombineArgs &a, hipStream_t stream)
 {
     if (a.T <= 0) {
         return hipSuccess;
@@ -350,19 +355,24 @@ hipError_t launch_combine(const CombineArgs &a, hipStream_t stream)
         return hipErrorInvalidValue;
     }
     if (a.wire_rows && a.act_fp16) {
-        hipLaunchKernelGGL((combine_kernel<true, 1>), dim3((unsigned)blocks), dim3(kCombThreads), 0, stream, a, segs);
+        hipLaunchKernelGGL((combine_kernel<true, 1, BY_COUNTS>), dim3((unsigned)blocks), dim3(kCombThreads), 0, stream, a, segs);
     } else if (a.wire_rows && a.H % 64 == 0) {
         const int segs16 = (a.H / 16 + kCombThreads - 1) / kCombThreads;
-        hipLaunchKernelGGL(combine_wire16_kernel, dim3((unsigned)(a.T * segs16)), dim3(kCombThreads), 0, stream, a,
+        hipLaunchKernelGGL(combine_wire16_kernel<BY_COUNTS>, dim3((unsigned)(a.T * segs16)), dim3(kCombThreads), 0, stream, a,
                            segs16);
     } else if (a.wire_rows) {
-        hipLaunchKernelGGL((combine_kernel<true, 0>), dim3((unsigned)blocks), dim3(kCombThreads), 0, stream, a, segs);
+        hipLaunchKernelGGL((combine_kernel<true, 0, BY_COUNTS>), dim3((unsigned)blocks), dim3(kCombThreads), 0, stream, a, segs);
     } else if (a.act_fp16) {
-        hipLaunchKernelGGL((combine_kernel<false, 1>), dim3((unsigned)blocks), dim3(kCombThreads), 0, stream, a, segs);
+        hipLaunchKernelGGL((combine_kernel<false, 1, BY_COUNTS>), dim3((unsigned)blocks), dim3(kCombThreads), 0, stream, a, segs);
     } else {
-        hipLaunchKernelGGL((combine_kernel<false, 0>), dim3((unsigned)blocks), dim3(kCombThreads), 0, stream, a, segs);
+        hipLaunchKernelGGL((combine_kernel<false, 0, BY_COUNTS>), dim3((unsigned)blocks), dim3(kCombThreads), 0, stream, a, segs);
     }
     return hipGetLastError();
+}
+
+hipError_t launch_combine(const CombineArgs &a, hipStream_t stream)
+{
+    return a.ids != nullptr ? launch_combine_as<true>(a, stream) : launch_combine_as<false>(a, stream);
 }
 
 }  // namespace cam
