@@ -22,6 +22,7 @@
 // and fused_deep_moe accepts only weights that live in such a storage: views of a packed tensor pass, a copy
 // made by clone() or to() does not (its bytes would still be packed, but nothing says so) and is refused with a
 // message instead of being multiplied as if it were row-major.
+#include <ATen/FuncTorchTLS.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 
@@ -396,14 +397,27 @@ at::Tensor moe_combine_shmem_meta(const at::Tensor &expand_x, const at::Tensor &
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-// Whether a call takes part in a graph at all.  When it does not, which is every call of an inference program, the node and
-// its bookkeeping are skipped: the outputs are the same tensors without a grad_fn.
+// Whether a call has anything to do with derivatives.  When it has not, which is every call of an inference program, the
+// node and its bookkeeping are skipped: the outputs are the same tensors without a grad_fn.  Besides gradients that are
+// asked for, a tangent on an input (forward mode, which does not look at requires_grad or the grad mode) and a
+// functorch transform around the call, whose inputs need not be wrapped, go to Function::apply: it refuses both.
 bool wants_grad(const at::Tensor &t) { return t.defined() && t.requires_grad(); }
-bool wants_grad(const c10::optional<at::Tensor> &t) { return t.has_value() && wants_grad(*t); }
-bool wants_grad(at::TensorList ts)
+bool has_tangent(const at::Tensor &t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
+template <typename F>
+bool any_of(const F &f, const at::Tensor &t)
+{
+    return f(t);
+}
+template <typename F>
+bool any_of(const F &f, const c10::optional<at::Tensor> &t)
+{
+    return t.has_value() && f(*t);
+}
+template <typename F>
+bool any_of(const F &f, at::TensorList ts)
 {
     for (const at::Tensor &t : ts) {
-        if (wants_grad(t)) {
+        if (f(t)) {
             return true;
         }
     }
@@ -412,7 +426,8 @@ bool wants_grad(at::TensorList ts)
 template <typename... Ts>
 bool in_graph(const Ts &...ts)
 {
-    return at::GradMode::is_enabled() && (wants_grad(ts) || ...);
+    return (at::GradMode::is_enabled() && (any_of(wants_grad, ts) || ...)) || (any_of(has_tangent, ts) || ...) ||
+           at::functorch::functorchTLSAccessor() != nullptr;
 }
 
 template <int NumInputs>
