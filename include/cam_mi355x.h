@@ -221,8 +221,11 @@ CAM_API camStatus camMoeDispatchNormal(void *workspace, uint64_t workspaceSize, 
  * expandIdx int32 [3A] = (srcRank,
  * token, k) per row, sendTokenIdx int32 [T,K]; optional slotRow int32 [T,K], numTokensPerExpert int32 [E],
  * sendOffset int32 [E], recvCount int32 [E], numRecvTokensPerExpert int64 [E], totalRecvTokens int64 [1],
- * all exactly as MoeDispatchPlan / MoeDispatchNormal produce them.  Rows outside [0,A) are dropped, so A
- * may be a worst-case bound (T*K) and the true total read later from totalRecvTokens.
+ * all exactly as MoeDispatchPlan / MoeDispatchNormal produce them.  numRecvTokensPerExpert may be host memory that
+ * the device can store to (hipHostMalloc, coherent): every count is stored once, by one 8-byte store that the whole
+ * system sees, and none waits for the rows, so a host that has filled it with -1 can watch the counts arrive.
+ * Rows outside [0,A) are dropped, so A may be a worst-case bound (T*K) and the true total read later from
+ * totalRecvTokens.
  * The workspace may hold anything on first use.  Launches that share a workspace must not overlap. */
 CAM_API camStatus camMoeDispatchPrefillGetWorkspaceSize(
     const camTensor *x, const camTensor *topkIdx, int64_t numExperts, int64_t numRanks, int64_t rankId,

@@ -120,7 +120,8 @@ py::tuple moe_dispatch_prefill(const at::Tensor &x, const at::Tensor &ids, int64
     if (per_rank < 1 || per_rank > cam_torch::HostCounts::kMost) {
         fail(CAM_ERR_RANGE, ("numExperts " + std::to_string(experts) + " outside (0, 512]").c_str());
     }
-    ctpe.data = cam_torch::HostCounts::begin(per_rank);
+    cam_torch::HostCounts host(per_rank, x.get_device());
+    ctpe.data = host.data();
     ctpe.dtype = CAM_DT_INT64;
     ctpe.ndim = 1;
     ctpe.sizes[0] = per_rank;
@@ -129,11 +130,12 @@ py::tuple moe_dispatch_prefill(const at::Tensor &x, const at::Tensor &ids, int64
     camOpExecutor *ex = nullptr;
     check(camMoeDispatchPrefillGetWorkspaceSize(&cx, &ci, experts, ranks, rank, quant_mode, &crx, &crs, &cidx, &cpos, nullptr,
                                                 nullptr, nullptr, &crc, &ctpe, nullptr, &bytes, &ex));
+    at::Tensor counts = at::empty({per_rank}, at::TensorOptions().dtype(at::kLong));
+    host.queued();
     check(cam_torch::launch(camMoeDispatchPrefill, bytes, ex, x));
-    at::Tensor counts;
     {
         py::gil_scoped_release nogil;
-        counts = cam_torch::HostCounts::wait(per_rank, x);
+        host.wait(cam_torch::stream_of(x), counts.data_ptr<int64_t>());
     }
     return py::make_tuple(rx, rs, idx, rc, counts);
 }

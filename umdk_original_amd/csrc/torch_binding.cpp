@@ -188,7 +188,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> moe_dispatch_prefill(
     const int64_t per_rank = E / num_ranks;
     TORCH_CHECK(per_rank <= HostCounts::kMost, "numExperts ", E, " outside (0, ", HostCounts::kMost, "]");
     camTensor cpe{};   // the counts per expert, in host memory the plan kernel stores to
-    cpe.data = HostCounts::begin(per_rank);
+    HostCounts host(per_rank, x.get_device());
+    cpe.data = host.data();
     cpe.dtype = CAM_DT_INT64;
     cpe.ndim = 1;
     cpe.sizes[0] = per_rank;
@@ -198,9 +199,11 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> moe_dispatch_prefill(
     check(camMoeDispatchPrefillGetWorkspaceSize(&cx, &ci, E, num_ranks, rank, 0, &crx, nullptr, &cidx, &cpos, nullptr,
                                                 nullptr, nullptr, &crc, &cpe, nullptr, &bytes, &ex),
           "camMoeDispatchPrefill");
+    at::Tensor per_expert = at::empty({per_rank}, at::TensorOptions().dtype(at::kLong));
+    host.queued();
     run_phase2(camMoeDispatchPrefill, "camMoeDispatchPrefill", bytes, ex, x);
     // the one thing the host waits for: the shapes need the row total
-    at::Tensor per_expert = HostCounts::wait(per_rank, x);
+    host.wait(cam_torch::stream_of(x), per_expert.data_ptr<int64_t>());
     int64_t n = 0;
     for (int64_t e = 0; e < per_rank; ++e) {
         n += per_expert.data_ptr<int64_t>()[e];

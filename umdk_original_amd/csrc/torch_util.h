@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../../include/cam_mi355x.h"
+#include "host_counts.h"
 
 namespace cam_torch {
 
@@ -53,6 +54,12 @@ inline at::Tensor new_empty(at::IntArrayRef sizes, at::ScalarType dtype, const a
     return at::Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt));
 }
 
+// The current stream of the device `like` lives on.
+inline hipStream_t stream_of(const at::Tensor &like)
+{
+    return c10::hip::getCurrentHIPStream(like.device().index()).stream();
+}
+
 typedef camStatus (*Phase2)(void *, uint64_t, camOpExecutor *, camStream_t);
 
 // Phase 2 of an operator whose phase 1 has produced (bytes, executor): the workspace, the stream and the launches
@@ -64,76 +71,8 @@ inline camStatus launch(Phase2 fn, uint64_t bytes, camOpExecutor *executor, cons
     if (bytes > 0) {
         ws = new_empty({(int64_t)bytes}, at::kByte, like);
     }
-    return fn(bytes > 0 ? ws.data_ptr() : nullptr, bytes, executor,
-              (camStream_t)c10::hip::getCurrentHIPStream(like.device().index()).stream());
+    return fn(bytes > 0 ? ws.data_ptr() : nullptr, bytes, executor, (camStream_t)stream_of(like));
 }
-
-// The rows an operator's plan counts per expert, brought to the host without a copy and without waiting for anything
-// behind the plan: the kernel stores the counts into host memory and the host watches them arrive.  (Two blocking
-// copies after the permute took about 20 us of a call, and held the host until the rows had moved.)  One buffer per
-// thread, given back with it; a call is over when its counts are complete, so a thread needs no second one.
-class HostCounts {
-public:
-    static constexpr int64_t kMost = 512;  // experts an operator admits
-
-    // Memory for n counts, none of which has arrived.
-    static int64_t *begin(int64_t n)
-    {
-        HostCounts &b = of_thread();
-        if (b.p_ == nullptr) {
-            TORCH_CHECK(hipHostMalloc((void **)&b.p_, kMost * sizeof(int64_t), hipHostMallocCoherent) == hipSuccess,
-                        "out of pinned host memory");
-        }
-        TORCH_CHECK(n <= kMost, "too many experts");
-        for (int64_t i = 0; i < n; ++i) {
-            b.p_[i] = -1;
-        }
-        return b.p_;
-    }
-
-    // Waits for all of them.  The stream is asked now and then: once it has nothing left to run, or an error, the wait
-    // ends either way.
-    static at::Tensor wait(int64_t n, const at::Tensor &like)
-    {
-        volatile int64_t *p = of_thread().p_;
-        const hipStream_t stream = c10::hip::getCurrentHIPStream(like.device().index()).stream();
-        int64_t i = 0;
-        for (unsigned spin = 1; i < n; ++spin) {
-            while (i < n && p[i] >= 0) {
-                ++i;
-            }
-            if (i < n && (spin & 0xffff) == 0) {
-                const hipError_t e = hipStreamQuery(stream);
-                TORCH_CHECK(e == hipSuccess || e == hipErrorNotReady, "moe_dispatch_prefill: ", hipGetErrorString(e));
-                if (e == hipSuccess) {  // the kernels are done, so whatever they stored is there
-                    for (; i < n; ++i) {
-                        TORCH_CHECK(p[i] >= 0, "moe_dispatch_prefill: the counts did not arrive");
-                    }
-                }
-            }
-        }
-        at::Tensor out = at::empty({n}, at::TensorOptions().dtype(at::kLong));
-        int64_t *dst = out.data_ptr<int64_t>();
-        for (i = 0; i < n; ++i) {
-            dst[i] = p[i];
-        }
-        return out;
-    }
-
-private:
-    static HostCounts &of_thread()
-    {
-        static thread_local HostCounts b;
-        return b;
-    }
-    ~HostCounts()
-    {
-        if (p_ != nullptr) {
-            (void)hipHostFree(p_);
-        }
-    }
-    int64_t *p_ = nullptr;
-};
 
 }  // namespace cam_torch
 
