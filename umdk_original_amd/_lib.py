@@ -14,8 +14,8 @@ import os
 import torch
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
-# CAM_MI355X_LIB names another build of the same library (the clock-stamping profiling build); the default is the
-# product library beside this file.
+# CAM_MI355X_LIB names another build of the same library (the clock-stamping profiling build) for this module and for the
+# torch libraries on top of it; the default is the product library beside this file.
 LIB_PATH = os.environ.get("CAM_MI355X_LIB") or os.path.join(_PKG, "lib", "libcam_mi355x.so")
 
 CAM_MAX_DIMS = 8

@@ -52,7 +52,9 @@ def build(verbose=False, timeline=False):
         if verbose and out.strip():
             print(out)
     out_path = TIMELINE_LIB_PATH if timeline else LIB_PATH
-    cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out_path] + objs
+    # One soname for every build of the library: whichever is loaded first (CAM_MI355X_LIB) is the one that the torch
+    # libraries below find, too.
+    cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-soname," + os.path.basename(LIB_PATH), "-o", out_path] + objs
     subprocess.check_call(cmd)
     for o in objs:
         os.remove(o)

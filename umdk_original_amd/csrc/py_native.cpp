@@ -235,6 +235,8 @@ py::list fused_deep_moe(const at::Tensor &x, const at::Tensor &ids, const std::v
 
 PYBIND11_MODULE(_cam_native, m)
 {
+    // which build of the library this module calls: the address of one of its functions
+    m.def("library", [] { return (uintptr_t)&camGetVersion; });
     m.def("moe_dispatch_fused", &moe_dispatch_fused);
     m.def("moe_dispatch_prefill", &moe_dispatch_prefill);
     m.def("moe_combine_gather", &moe_combine_gather);

@@ -17,6 +17,7 @@ prepacked with `prepack_weight` (the reference needs `npu_format_cast(..., FRACT
 place); `moe_dispatch_prefill` takes an optional `quant_mode` keyword (the reference binding
 hard-codes 0 although its kernel supports dynamic quantisation).
 """
+import ctypes
 import importlib.util
 import os
 import weakref
@@ -51,9 +52,13 @@ def _native():
         if not os.path.exists(path):
             raise RuntimeError("%s is missing: build it with `python -m umdk_original_amd.build` "
                                "(there is no CPU fallback)" % path)
+        handle = _lib.lib()  # the kernel library first: the module takes the one that is loaded
         spec = importlib.util.spec_from_file_location("_cam_native", path)
-        _native_module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(_native_module)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        if module.library() != ctypes.cast(handle.camGetVersion, ctypes.c_void_p).value:
+            raise RuntimeError("%s is not the library the C++ module calls: build it again" % _lib.LIB_PATH)
+        _native_module = module
     return _native_module
 
 
