@@ -12,8 +12,6 @@ namespace py = pybind11;
 
 namespace {
 
-using cam_torch::new_empty;
-
 [[noreturn]] void fail(int status, const char *message)
 {
     const py::object cls = py::module_::import("umdk_original_amd._lib").attr("CamError");
@@ -27,6 +25,22 @@ void check(camStatus st)
     if (st != CAM_OK) {
         fail((int)st, camGetRecentErrMsg());
     }
+}
+
+// An output beside `like`.  Where that is in host memory nothing is launched, but phase 1 has its say first.
+at::Tensor new_empty(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor &like)
+{
+    return like.is_cuda() ? cam_torch::new_empty(sizes, dtype, like) : at::empty(sizes, at::TensorOptions().dtype(dtype));
+}
+
+// Phase 2 of an operator whose first input is `like`.
+void run(cam_torch::Phase2 fn, uint64_t bytes, camOpExecutor *executor, const at::Tensor &like)
+{
+    if (!like.is_cuda()) {
+        camDestroyExecutor(executor);
+        fail(CAM_ERR_WORKSPACE, "no device to allocate the workspace on");
+    }
+    check(cam_torch::launch(fn, bytes, executor, like));
 }
 
 camTensor to_cam(const at::Tensor &t, int32_t format = CAM_FORMAT_ND)
@@ -90,7 +104,7 @@ py::dict moe_dispatch_fused(const at::Tensor &x, const at::Tensor &ids, int64_t 
     camOpExecutor *ex = nullptr;
     check(camMoeDispatchPrefillGetWorkspaceSize(&cx, &ci, experts, ranks, rank, quant_mode, &crx, &crs, &cidx, &cpos, &cslot,
                                                 &ccnt, &coff, &crc, &ctpe, &ctotal, &bytes, &ex));
-    check(cam_torch::launch(camMoeDispatchPrefill, bytes, ex, x));
+    run(camMoeDispatchPrefill, bytes, ex, x);
     py::dict d;
     d["recv_x"] = rx;
     d["recv_x_scales"] = rs;
@@ -120,6 +134,7 @@ py::tuple moe_dispatch_prefill(const at::Tensor &x, const at::Tensor &ids, int64
     if (per_rank < 1 || per_rank > cam_torch::HostCounts::kMost) {
         fail(CAM_ERR_RANGE, ("numExperts " + std::to_string(experts) + " outside (0, 512]").c_str());
     }
+    at::Tensor counts = at::empty({per_rank}, at::TensorOptions().dtype(at::kLong));
     cam_torch::HostCounts host(per_rank, x.get_device());
     ctpe.data = host.data();
     ctpe.dtype = CAM_DT_INT64;
@@ -130,9 +145,8 @@ py::tuple moe_dispatch_prefill(const at::Tensor &x, const at::Tensor &ids, int64
     camOpExecutor *ex = nullptr;
     check(camMoeDispatchPrefillGetWorkspaceSize(&cx, &ci, experts, ranks, rank, quant_mode, &crx, &crs, &cidx, &cpos, nullptr,
                                                 nullptr, nullptr, &crc, &ctpe, nullptr, &bytes, &ex));
-    at::Tensor counts = at::empty({per_rank}, at::TensorOptions().dtype(at::kLong));
     host.queued();
-    check(cam_torch::launch(camMoeDispatchPrefill, bytes, ex, x));
+    run(camMoeDispatchPrefill, bytes, ex, x);
     {
         py::gil_scoped_release nogil;
         host.wait(cam_torch::stream_of(x), counts.data_ptr<int64_t>());
@@ -149,7 +163,7 @@ void moe_combine_gather(const at::Tensor &rows, const std::optional<at::Tensor> 
     uint64_t bytes = 0;
     camOpExecutor *ex = nullptr;
     check(camMoeCombineGatherGetWorkspaceSize(&cr, oi.p, &cs, oc.p, &cw, os.p, &co, &bytes, &ex));
-    check(cam_torch::launch(camMoeCombineGather, bytes, ex, rows));
+    run(camMoeCombineGather, bytes, ex, rows);
 }
 
 py::tuple grouped_matmul_swiglu_quant(const at::Tensor &x, const at::Tensor &x_scale, const std::vector<at::Tensor> &w,
@@ -162,7 +176,7 @@ py::tuple grouped_matmul_swiglu_quant(const at::Tensor &x, const at::Tensor &x_s
     uint64_t bytes = 0;
     camOpExecutor *ex = nullptr;
     check(camGroupedMatmulSwigluQuantGetWorkspaceSize(&cx, &cs, &lw.list, &ls.list, &cg, type, &cy, &cys, &bytes, &ex));
-    check(cam_torch::launch(camGroupedMatmulSwigluQuant, bytes, ex, x));
+    run(camGroupedMatmulSwigluQuant, bytes, ex, x);
     return py::make_tuple(y, ys);
 }
 
@@ -174,7 +188,7 @@ void grouped_matmul_dequant(const at::Tensor &x, const at::Tensor &x_scale, cons
     uint64_t bytes = 0;
     camOpExecutor *ex = nullptr;
     check(camGroupedMatmulDequantGetWorkspaceSize(&cx, &cs, &lw.list, &ls.list, &cg, type, &co, &bytes, &ex));
-    check(cam_torch::launch(camGroupedMatmulDequant, bytes, ex, x));
+    run(camGroupedMatmulDequant, bytes, ex, x);
 }
 
 void grouped_matmul_fp8(const at::Tensor &x, const at::Tensor &x_scale, const at::Tensor &w, const at::Tensor &ws, bool gate_up,
@@ -187,7 +201,7 @@ void grouped_matmul_fp8(const at::Tensor &x, const at::Tensor &x_scale, const at
     uint64_t bytes = 0;
     camOpExecutor *ex = nullptr;
     check(camGroupedMatmulFp8GetWorkspaceSize(&cx, &cs, &cw, &cws, gate_up ? 1 : 0, &cg, type, &co, oo.p, &bytes, &ex));
-    check(cam_torch::launch(camGroupedMatmulFp8, bytes, ex, x));
+    run(camGroupedMatmulFp8, bytes, ex, x);
 }
 
 py::list fused_deep_moe_fp8(const at::Tensor &x, const at::Tensor &ids, const at::Tensor &w1, const at::Tensor &w1s,
@@ -201,7 +215,7 @@ py::list fused_deep_moe_fp8(const at::Tensor &x, const at::Tensor &ids, const at
     uint64_t bytes = 0;
     camOpExecutor *ex = nullptr;
     check(camFusedDeepMoeFp8GetWorkspaceSize(&cx, &ci, &c1, &c1s, &c2, &c2s, &cg, om.p, experts, &co, &ce, &bytes, &ex));
-    check(cam_torch::launch(camFusedDeepMoeFp8, bytes, ex, x));
+    run(camFusedDeepMoeFp8, bytes, ex, x);
     py::list l;
     l.append(out);
     l.append(etn);
@@ -224,7 +238,7 @@ py::list fused_deep_moe(const at::Tensor &x, const at::Tensor &ids, const std::v
     check(camFusedDeepMoeGetWorkspaceSize(&cx, &ci, &l1.list, &l1s.list, &l2.list, &l2s.list, &cg, osm.p, om.p, group.data(),
                                           rank_size, rank_id, experts, shared_num, shared_rank_num, quant_mode, global_bs, &co,
                                           &ce, &bytes, &ex));
-    check(cam_torch::launch(camFusedDeepMoe, bytes, ex, x));
+    run(camFusedDeepMoe, bytes, ex, x);
     py::list l;
     l.append(out);
     l.append(etn);

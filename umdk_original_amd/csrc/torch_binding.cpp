@@ -188,6 +188,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> moe_dispatch_prefill(
     const int64_t per_rank = E / num_ranks;
     TORCH_CHECK(per_rank <= HostCounts::kMost, "numExperts ", E, " outside (0, ", HostCounts::kMost, "]");
     camTensor cpe{};   // the counts per expert, in host memory the plan kernel stores to
+    at::Tensor per_expert = at::empty({per_rank}, at::TensorOptions().dtype(at::kLong));
     HostCounts host(per_rank, x.get_device());
     cpe.data = host.data();
     cpe.dtype = CAM_DT_INT64;
@@ -199,7 +200,6 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> moe_dispatch_prefill(
     check(camMoeDispatchPrefillGetWorkspaceSize(&cx, &ci, E, num_ranks, rank, 0, &crx, nullptr, &cidx, &cpos, nullptr,
                                                 nullptr, nullptr, &crc, &cpe, nullptr, &bytes, &ex),
           "camMoeDispatchPrefill");
-    at::Tensor per_expert = at::empty({per_rank}, at::TensorOptions().dtype(at::kLong));
     host.queued();
     run_phase2(camMoeDispatchPrefill, "camMoeDispatchPrefill", bytes, ex, x);
     // the one thing the host waits for: the shapes need the row total

@@ -69,7 +69,12 @@ inline camStatus launch(Phase2 fn, uint64_t bytes, camOpExecutor *executor, cons
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(like.device());
     at::Tensor ws;
     if (bytes > 0) {
-        ws = new_empty({(int64_t)bytes}, at::kByte, like);
+        try {
+            ws = new_empty({(int64_t)bytes}, at::kByte, like);
+        } catch (...) {  // out of memory: phase 2, which frees the executor, will not run
+            camDestroyExecutor(executor);
+            throw;
+        }
     }
     return fn(bytes > 0 ? ws.data_ptr() : nullptr, bytes, executor, (camStream_t)stream_of(like));
 }
