@@ -55,35 +55,18 @@ camTensor to_cam(const at::Tensor &t, int32_t format = CAM_FORMAT_ND)
     return cam_torch::view_of(t, dtype, format);
 }
 
-// An optional argument: NULL when it is None.
-struct Optional {
-    camTensor c{};
-    const camTensor *p = nullptr;
-    explicit Optional(const std::optional<at::Tensor> &t)
+// This library's side of what torch_util.h shares (an operator's name is not part of a CamError).
+struct Host {
+    static camTensor view(const at::Tensor &t, int32_t format) { return to_cam(t, format); }
+    static at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor &like)
     {
-        if (t.has_value() && t->defined()) {
-            c = to_cam(*t);
-            p = &c;
-        }
+        return new_empty(sizes, dtype, like);
     }
+    static void check(camStatus st, const char *) { ::check(st); }
+    static void fail(int status, const std::string &message) { ::fail(status, message.c_str()); }
 };
-
-struct List {
-    std::vector<camTensor> items;
-    std::vector<const camTensor *> ptrs;
-    camTensorList list{};
-    List(const std::vector<at::Tensor> &ts, int32_t format)
-    {
-        items.reserve(ts.size());
-        ptrs.reserve(ts.size());
-        for (const at::Tensor &t : ts) {
-            items.push_back(to_cam(t, format));
-            ptrs.push_back(&items.back());
-        }
-        list.tensors = ptrs.data();
-        list.count = ptrs.size();
-    }
-};
+typedef cam_torch::ListView<Host> List;
+typedef cam_torch::OptionalView<Host> Optional;
 
 // Fresh outputs, by name, as the operators of ops.py return them.
 py::dict moe_dispatch_fused(const at::Tensor &x, const at::Tensor &ids, int64_t experts, int64_t quant_mode, int64_t rows,
@@ -123,35 +106,12 @@ py::dict moe_dispatch_fused(const at::Tensor &x, const at::Tensor &ids, int64_t 
 py::tuple moe_dispatch_prefill(const at::Tensor &x, const at::Tensor &ids, int64_t experts, int64_t quant_mode, int64_t rows,
                                int64_t rank, int64_t ranks)
 {
-    const int64_t T = x.size(0), H = x.size(1), K = ids.size(1), A = std::max<int64_t>(rows < 0 ? T * K : rows, 1);
-    camTensor cx = to_cam(x), ci = to_cam(ids);
-    const bool fp8 = quant_mode == 4;
-    at::Tensor rx = new_empty({A, H}, fp8 ? at::kFloat8_e4m3fn : quant_mode != 0 ? at::kChar : x.scalar_type(), x);
-    at::Tensor rs = fp8 ? new_empty({A, H / 128}, at::kByte, x) : new_empty({A}, at::kFloat, x);
-    at::Tensor idx = new_empty({3 * A}, at::kInt, x), pos = new_empty({T, K}, at::kInt, x), rc = new_empty({experts}, at::kInt, x);
-    camTensor crx = to_cam(rx), crs = to_cam(rs), cidx = to_cam(idx), cpos = to_cam(pos), crc = to_cam(rc), ctpe{};
-    const int64_t per_rank = experts / std::max<int64_t>(ranks, 1);
-    if (per_rank < 1 || per_rank > cam_torch::HostCounts::kMost) {
-        fail(CAM_ERR_RANGE, ("numExperts " + std::to_string(experts) + " outside (0, 512]").c_str());
-    }
-    at::Tensor counts = at::empty({per_rank}, at::TensorOptions().dtype(at::kLong));
-    cam_torch::HostCounts host(per_rank, x.get_device());
-    ctpe.data = host.data();
-    ctpe.dtype = CAM_DT_INT64;
-    ctpe.ndim = 1;
-    ctpe.sizes[0] = per_rank;
-    ctpe.strides[0] = 1;
-    uint64_t bytes = 0;
-    camOpExecutor *ex = nullptr;
-    check(camMoeDispatchPrefillGetWorkspaceSize(&cx, &ci, experts, ranks, rank, quant_mode, &crx, &crs, &cidx, &cpos, nullptr,
-                                                nullptr, nullptr, &crc, &ctpe, nullptr, &bytes, &ex));
-    host.queued();
-    run(camMoeDispatchPrefill, bytes, ex, x);
-    {
-        py::gil_scoped_release nogil;
-        host.wait(cam_torch::stream_of(x), counts.data_ptr<int64_t>());
-    }
-    return py::make_tuple(rx, rs, idx, rc, counts);
+    const cam_torch::PrefillRows r = cam_torch::dispatch_prefill<Host>(
+        x, ids, experts, quant_mode, rows < 0 ? x.size(0) * ids.size(1) : rows, rank, ranks, true, [](const auto &wait) {
+            py::gil_scoped_release nogil;
+            wait();
+        });
+    return py::make_tuple(r.rows, r.scales, r.info, r.recv_count, r.counts);
 }
 
 void moe_combine_gather(const at::Tensor &rows, const std::optional<at::Tensor> &info, const at::Tensor &slot_row,
@@ -226,22 +186,14 @@ py::list fused_deep_moe(const at::Tensor &x, const at::Tensor &ids, const std::v
                         const std::vector<at::Tensor> &w1s, const std::vector<at::Tensor> &w2,
                         const std::vector<at::Tensor> &w2s, const at::Tensor &gates, const std::optional<at::Tensor> &smooth,
                         const std::optional<at::Tensor> &mask, std::string group, int64_t rank_size, int64_t rank_id,
-                        int64_t experts, int64_t shared_num, int64_t shared_rank_num, int64_t quant_mode, int64_t global_bs,
-                        int64_t local_experts)
+                        int64_t experts, int64_t shared_num, int64_t shared_rank_num, int64_t quant_mode, int64_t global_bs)
 {
-    at::Tensor out = new_empty({x.size(0), x.size(1)}, x.scalar_type(), x), etn = new_empty({local_experts}, at::kLong, x);
-    camTensor cx = to_cam(x), ci = to_cam(ids), cg = to_cam(gates), co = to_cam(out), ce = to_cam(etn);
-    List l1(w1, CAM_FORMAT_MFMA_B), l1s(w1s, CAM_FORMAT_ND), l2(w2, CAM_FORMAT_MFMA_B), l2s(w2s, CAM_FORMAT_ND);
-    Optional osm(smooth), om(mask);
-    uint64_t bytes = 0;
-    camOpExecutor *ex = nullptr;
-    check(camFusedDeepMoeGetWorkspaceSize(&cx, &ci, &l1.list, &l1s.list, &l2.list, &l2s.list, &cg, osm.p, om.p, group.data(),
-                                          rank_size, rank_id, experts, shared_num, shared_rank_num, quant_mode, global_bs, &co,
-                                          &ce, &bytes, &ex));
-    run(camFusedDeepMoe, bytes, ex, x);
     py::list l;
-    l.append(out);
-    l.append(etn);
+    for (const at::Tensor &t : cam_torch::fused_deep_moe<Host>(x, ids, w1, w1s, w2, w2s, gates, smooth, mask, std::move(group),
+                                                               rank_size, rank_id, experts, shared_num, shared_rank_num,
+                                                               quant_mode, global_bs)) {
+        l.append(t);
+    }
     return l;
 }
 

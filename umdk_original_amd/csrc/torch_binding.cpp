@@ -35,7 +35,6 @@
 
 namespace {
 
-using cam_torch::HostCounts;
 using cam_torch::new_empty;
 using cam_torch::Phase2;
 
@@ -48,29 +47,21 @@ camTensor to_cam(const at::Tensor &t, int32_t format = CAM_FORMAT_ND)
     return cam_torch::view_of(t, dtype, format);
 }
 
-// Views of a TensorList for the C ABI; keeps the camTensor structs alive.
-struct CamList {
-    std::vector<camTensor> items;
-    std::vector<const camTensor *> ptrs;
-    camTensorList list{};
-    CamList(at::TensorList ts, int32_t format)
-    {
-        items.reserve(ts.size());
-        for (const at::Tensor &t : ts) {
-            items.push_back(to_cam(t, format));
-        }
-        for (const camTensor &c : items) {
-            ptrs.push_back(&c);
-        }
-        list.tensors = ptrs.data();
-        list.count = ptrs.size();
-    }
-};
-
 void check(camStatus st, const char *op)
 {
     TORCH_CHECK(st == CAM_OK, op, " failed with cam status ", (int)st, ": ", camGetRecentErrMsg());
 }
+
+// This library's side of what torch_util.h shares.
+struct Host {
+    static camTensor view(const at::Tensor &t, int32_t format) { return to_cam(t, format); }
+    static at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor &like)
+    {
+        return new_empty(sizes, dtype, like);
+    }
+    static void check(camStatus st, const char *op) { ::check(st, op); }
+    static void fail(int, const std::string &message) { TORCH_CHECK(false, message); }
+};
 
 void run_phase2(Phase2 fn, const char *op, uint64_t bytes, camOpExecutor *executor, const at::Tensor &like)
 {
@@ -177,43 +168,20 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> moe_dispatch_prefill(
     TORCH_CHECK(topk_weights.scalar_type() == at::kFloat, "Assertion failed: topkWeights.scalar_type() == at::kFloat");
 
     (void)num_worst_tokens;
-    const int64_t T = x.size(0), H = x.size(1), K = topk_idx.size(1);
-    const int64_t A = std::max<int64_t>(T * K, 1);
-    camTensor cx = to_cam(x), ci = to_cam(topk_idx);   // (checks that both are on the GPU)
-    at::Tensor recv_x = new_empty({A, H}, x.scalar_type(), x);
-    at::Tensor expand_idx = new_empty({3 * A}, at::kInt, x);
-    at::Tensor pos = new_empty({T, K}, at::kInt, x);
-    at::Tensor recv_count = new_empty({E}, at::kInt, x);
-    camTensor crx = to_cam(recv_x), cidx = to_cam(expand_idx), cpos = to_cam(pos), crc = to_cam(recv_count);
-    const int64_t per_rank = E / num_ranks;
-    TORCH_CHECK(per_rank <= HostCounts::kMost, "numExperts ", E, " outside (0, ", HostCounts::kMost, "]");
-    camTensor cpe{};   // the counts per expert, in host memory the plan kernel stores to
-    at::Tensor per_expert = at::empty({per_rank}, at::TensorOptions().dtype(at::kLong));
-    HostCounts host(per_rank, x.get_device());
-    cpe.data = host.data();
-    cpe.dtype = CAM_DT_INT64;
-    cpe.ndim = 1;
-    cpe.sizes[0] = per_rank;
-    cpe.strides[0] = 1;
-    uint64_t bytes = 0;
-    camOpExecutor *ex = nullptr;
-    check(camMoeDispatchPrefillGetWorkspaceSize(&cx, &ci, E, num_ranks, rank, 0, &crx, nullptr, &cidx, &cpos, nullptr,
-                                                nullptr, nullptr, &crc, &cpe, nullptr, &bytes, &ex),
-          "camMoeDispatchPrefill");
-    host.queued();
-    run_phase2(camMoeDispatchPrefill, "camMoeDispatchPrefill", bytes, ex, x);
-    // the one thing the host waits for: the shapes need the row total
-    host.wait(cam_torch::stream_of(x), per_expert.data_ptr<int64_t>());
+    // the host waits for the counts alone: the shapes need the row total
+    const int64_t A = std::max<int64_t>(x.size(0) * topk_idx.size(1), 1);
+    cam_torch::PrefillRows r = cam_torch::dispatch_prefill<Host>(x, topk_idx, E, 0, A, rank, num_ranks, false,
+                                                                 [](const auto &wait) { wait(); });
     int64_t n = 0;
-    for (int64_t e = 0; e < per_rank; ++e) {
-        n += per_expert.data_ptr<int64_t>()[e];
+    for (int64_t e = 0; e < r.counts.size(0); ++e) {
+        n += r.counts.data_ptr<int64_t>()[e];
     }
     n = std::max<int64_t>(n, 1);
     if (n != A) {
-        recv_x = recv_x.narrow(0, 0, n);
-        expand_idx = expand_idx.narrow(0, 0, 3 * n);
+        r.rows = r.rows.narrow(0, 0, n);
+        r.info = r.info.narrow(0, 0, 3 * n);
     }
-    return {recv_x, expand_idx, recv_count, per_expert};
+    return {r.rows, r.info, r.recv_count, r.counts};
 }
 
 at::Tensor moe_combine_prefill(const at::Tensor &x, const at::Tensor &topk_idx, const at::Tensor &topk_weights,
@@ -247,32 +215,9 @@ std::vector<at::Tensor> fused_deep_moe(const at::Tensor &x, const at::Tensor &ex
     require_packed(w1, true, "gmm1PermutedWeight");
     require_packed(w2, false, "gmm2Weight");
     TORCH_CHECK(x.is_cuda(), "umdk_cam_op_lib: tensors must live on a ROCm device (the CAM kernels have no CPU path)");
-    at::Tensor output = new_empty({x.size(0), x.size(1)}, x.scalar_type(), x);
-    const bool shared = ep_rank_id < shared_expert_rank_num;
-    const int64_t local = shared ? 1 : moe_expert_num / std::max<int64_t>(ep_rank_size - shared_expert_rank_num, 1);
-    at::Tensor expert_token_nums = new_empty({local}, at::kLong, x);
-    camTensor cx = to_cam(x), ci = to_cam(expert_ids), cs = to_cam(expert_scales), co = to_cam(output),
-              cn = to_cam(expert_token_nums);
-    CamList l1(w1, CAM_FORMAT_MFMA_B), l1s(w1s, CAM_FORMAT_ND), l2(w2, CAM_FORMAT_MFMA_B), l2s(w2s, CAM_FORMAT_ND);
-    camTensor csm{}, cm{};
-    const camTensor *psm = nullptr, *pm = nullptr;
-    if (smooth.has_value() && smooth->defined()) {
-        csm = to_cam(*smooth);
-        psm = &csm;
-    }
-    if (mask.has_value() && mask->defined()) {
-        cm = to_cam(*mask);
-        pm = &cm;
-    }
-    const std::string group(group_ep);
-    uint64_t bytes = 0;
-    camOpExecutor *ex = nullptr;
-    check(camFusedDeepMoeGetWorkspaceSize(&cx, &ci, &l1.list, &l1s.list, &l2.list, &l2s.list, &cs, psm, pm, const_cast<char *>(group.c_str()),
-                                          ep_rank_size, ep_rank_id, moe_expert_num, shared_expert_num,
-                                          shared_expert_rank_num, quant_mode, global_bs, &co, &cn, &bytes, &ex),
-          "camFusedDeepMoe");
-    run_phase2(camFusedDeepMoe, "camFusedDeepMoe", bytes, ex, x);
-    return {output, expert_token_nums};
+    return cam_torch::fused_deep_moe<Host>(x, expert_ids, w1, w1s, w2, w2s, expert_scales, smooth, mask, std::string(group_ep),
+                                           ep_rank_size, ep_rank_id, moe_expert_num, shared_expert_num,
+                                           shared_expert_rank_num, quant_mode, global_bs);
 }
 
 std::vector<at::Tensor> fused_deep_moe_meta(const at::Tensor &x, const at::Tensor &expert_ids, at::TensorList,

@@ -393,12 +393,10 @@ def fused_deep_moe(x, expertIds, gmm1PermutedWeight, gmm1PermutedWeightScale, gm
                    moeExpertNum=0, sharedExpertNum=1, sharedExpertRankNum=0, quantMode=0, globalBs=0):
     """-> [output bf16 [bs,H], expertTokenNums int64 [local experts]]."""
     _require_gpu(x, "x")
-    is_shared = epRankId < sharedExpertRankNum
-    local_experts = 1 if is_shared else moeExpertNum // max(epRankSize - sharedExpertRankNum, 1)
     return _native().fused_deep_moe(x, expertIds, _tag_list(gmm1PermutedWeight), list(gmm1PermutedWeightScale),
                                     _tag_list(gmm2Weight), list(gmm2WeightScale), expertScales, expertSmoothScales,
                                     xActiveMask, groupEp or "", epRankSize, epRankId, moeExpertNum, sharedExpertNum,
-                                    sharedExpertRankNum, quantMode, globalBs, local_experts)
+                                    sharedExpertRankNum, quantMode, globalBs)
 
 
 # --------------------------------------------------------------------------------------------------
