@@ -437,7 +437,10 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
 
     for (;;) {
         item += item_step;
-        StreamItem nxt = find_item(item);
+        StreamItem nxt{};   // PRODUCTS: a workgroup has one item
+        if constexpr (!PRODUCTS) {
+            nxt = find_item(item);
+        }
         const bool more = nxt.rows > 0;
 
         acc16 acc[MF][2];
@@ -468,9 +471,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
             if (!last_chunk) {
                 load_a(cur, c + 1, buf ^ 1);
             } else if (more) {
-                if constexpr (!PRODUCTS) {
-                    load_a(nxt, 0, buf ^ 1);
-                }
+                load_a(nxt, 0, buf ^ 1);
                 load_scales(nxt, set ^ 1);
             }
             const int8_t *abuf = lds + buf * kABuf;
@@ -698,11 +699,6 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
         buf ^= 1;
         set ^= 1;
         cur = nxt;
-        if constexpr (PRODUCTS) {
-            load_products(cur);
-            quantise_products(cur, buf, set);
-            lds_barrier();
-        }
     }
 }
 
@@ -825,7 +821,9 @@ hipError_t launch_stream_gemm(const StreamGemmArgs &sa, int64_t rows_per_expert,
         if (g.fp8 || g.gate_up || !products_fit(sh, sa.max_rows, g.Kd)) {
             return hipErrorInvalidValue;
         }
-        sh.P == 1 ? launch_kernel<1, false, 1, true>(sh.grid, stream, sa) : launch_kernel<1, false, 2, true>(sh.grid, stream, sa);
+        // an item to a workgroup, which is what the kernel is written for
+        const unsigned grid = (unsigned)((sh.items + kNumXcd - 1) / kNumXcd * kNumXcd);
+        sh.P == 1 ? launch_kernel<1, false, 1, true>(grid, stream, sa) : launch_kernel<1, false, 2, true>(grid, stream, sa);
     } else if (g.fp8) {
         launch_variant<true>(sh.small ? 1 : 4, sh.P, sh.grid, stream, sa);
     } else {
