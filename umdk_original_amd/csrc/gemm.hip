@@ -302,9 +302,13 @@ __device__ __forceinline__ void run_item(const GemmArgs &a, const ItemCtx &t, in
     // and the wait is for what remains: with `rem` stages after the current one, stage s+1 has landed once at most
     // rem - 1 stages are outstanding.
     //   barrier A(s): every load of stage s+1 has landed; team 1 is done reading stage s
-    //   barrier B(s): team 0 is done reading stage s+1
-    // Stage s is free once both teams have its fragments in registers, i.e. after barrier A(s): team 0 refills
-    // it in the phase that follows, team 1 at the end of its own reading phase.
+    //   barrier B(s): team 0 is done reading stage s+1; B(-1) stands in front of the loop
+    // Stage s is free once both teams have its fragments in registers: team 1 reads it behind B(s-1), when team 0 has it,
+    // and refills its part at the end of that reading phase; team 0 refills its own in the phase behind A(s).
+    // B(-1) is needed as much as the others: without it a wave of team 0 that is late with its first fragments (behind an
+    // instruction cache miss, say) may read weights of sub-step NS in their place.  It costs nothing that shows (8192 tokens x
+    // 4096, 128 experts, top-8, I 1536: 1717 -> 1721 us, runs of one side 0.2 % apart; 8192 skewed rows on 32 experts, H 7168,
+    // I 2048: 496.4 -> 496.0): the teams share the LDS, and now team 0, which multiplies first, is served first.
     auto wait_stages = [&](int n) {  // at most n stages of this wave's loads outstanding (n wave-uniform)
         if (n <= 0) {
             wait_loads_outstanding<0>();
@@ -346,6 +350,7 @@ __device__ __forceinline__ void run_item(const GemmArgs &a, const ItemCtx &t, in
     if (TEAM == 0) {
         read_frags(0, 0);
         wait_lds_reads();
+        barrier_no_fence();                               // B(-1)
         for (int s = 0; s < KT; ++s) {
             const int next = slot + 1 == NS ? 0 : slot + 1;
             multiply();                                   // phase 1: stage s, from registers
@@ -364,6 +369,7 @@ __device__ __forceinline__ void run_item(const GemmArgs &a, const ItemCtx &t, in
             slot = next;
         }
     } else {
+        barrier_no_fence();                               // B(-1)
         for (int s = 0; s < KT; ++s) {
             const int next = slot + 1 == NS ? 0 : slot + 1;
             read_frags(slot, s);                          // phase 1: fragments of stage s ...
