@@ -300,6 +300,19 @@ cam::SchedSpec sched_spec(int64_t rows, int64_t G, int64_t N, int64_t Kd, bool s
     return sp;
 }
 
+// Whether one grouped GEMM of an operator goes to the streaming form: not the raw sums, which it has no epilogue for.
+bool gemm_streams(int64_t A, int64_t N, int64_t G, int epilogue, bool fp8)
+{
+    return epilogue != cam::kEpiInt32 && cam::stream_gemm_applies(A, N, G, fp8);
+}
+
+// Bytes of the workspace in front of such a GEMM's other buffers: its schedule, or the two words of which the kernels
+// behind a streaming one read the row total.
+uint64_t gemm_sched_bytes(int64_t A, int64_t N, int64_t G, int epilogue, bool fp8)
+{
+    return gemm_streams(A, N, G, epilogue, fp8) ? 2 * sizeof(int32_t) : cam::sched_bytes(A, (int)G, (int)N);
+}
+
 // One grouped GEMM behind its schedule (tiles) or its row counts (few rows per expert: no schedule is needed).
 // `rows` receives where the kernels after it find the row total.
 hipError_t run_grouped_gemm(cam::GemmArgs g, const int64_t *group_list, int cumulative, int64_t G, int64_t A,
@@ -307,7 +320,7 @@ hipError_t run_grouped_gemm(cam::GemmArgs g, const int64_t *group_list, int cumu
 {
     int32_t *ws = (int32_t *)sched_ws;
     *rows = ws;
-    if (g.epilogue != cam::kEpiInt32 && cam::stream_gemm_applies(A, g.N, G, g.fp8 != 0)) {
+    if (gemm_streams(A, g.N, G, g.epilogue, g.fp8 != 0)) {
         cam::StreamGemmArgs sa{};
         sa.g = g;
         sa.group_list = group_list;
@@ -1537,7 +1550,7 @@ camStatus camGroupedMatmulSwigluQuantGetWorkspaceSize(const camTensor *x, const 
     CAM_TRY(check_aligned(y, "y", 16));
     cam::SchedSpec sp = sched_spec(gc.A, gc.G, 2 * I, gc.Kd, true);
     Carver c;
-    const uint64_t o_sched = c.take(cam::sched_bytes(gc.A, (int)gc.G, (int)(2 * I)));
+    const uint64_t o_sched = c.take(gemm_sched_bytes(gc.A, 2 * I, gc.G, cam::kEpiSwiglu, false));
     const uint64_t o_prod = c.take((uint64_t)gc.A * I * 4);
     cam::GemmArgs g{};
     g.a = (const int8_t *)x->data;
@@ -1597,7 +1610,7 @@ camStatus camGroupedMatmulDequantGetWorkspaceSize(const camTensor *x, const camT
     CAM_TRY(resolve_weights(weight, weightScale, "weight", gc.G, gc.Kd, N, true, &ws));
     cam::SchedSpec sp = sched_spec(gc.A, gc.G, N, gc.Kd, false);
     Carver c;
-    const uint64_t o_sched = c.take(cam::sched_bytes(gc.A, (int)gc.G, (int)N));
+    const uint64_t o_sched = c.take(gemm_sched_bytes(gc.A, N, gc.G, cam::kEpiDequantBf16, false));
     const uint64_t o_rows = wire ? c.take((uint64_t)gc.A * N * 2) : 0;  // the bf16 rows before quantisation
     cam::GemmArgs g{};
     g.a = (const int8_t *)x->data;
@@ -1793,12 +1806,16 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     const int64_t A = T * K;  // maxTokenNum of AK/fused_deep_moe/op_kernel/fused_deep_moe.h:336 for one rank
     cam::SchedSpec sp1 = sched_spec(A, Epr, 2 * I, H, true);
     cam::SchedSpec sp2 = sched_spec(A, Epr, H, I, false);
+    // Few rows: the GEMMs need no schedule.  Fewer still: GMM2 quantises the products itself, and then writes its rows while
+    // they are still read.
+    const bool stream = cam::stream_gemm_applies(A, 2 * I, Epr, false);
+    const bool from_products = stream && cam::stream_gemm_takes_products(A, (int)Epr, (int)I, (int)H, T);
     Carver c;
     const uint64_t o_pos = c.take((uint64_t)A * 4);
     const uint64_t o_row = c.take((uint64_t)A * 4);
     const uint64_t o_meta = c.take(cam::kPlanMeta * 4);
-    const uint64_t o_sched1 = c.take(cam::sched_bytes(A, (int)Epr, (int)(2 * I)));
-    const uint64_t o_sched2 = c.take(cam::sched_bytes(A, (int)Epr, (int)H));
+    const uint64_t o_sched1 = stream ? 0 : c.take(cam::sched_bytes(A, (int)Epr, (int)(2 * I)));
+    const uint64_t o_sched2 = stream ? 0 : c.take(cam::sched_bytes(A, (int)Epr, (int)H));
     const uint64_t o_hist = c.take(cam::plan_workspace_bytes(T, K, (int)Epr));
     // The bf16 rows GMM2 writes (2*A*H bytes) live where the quantised rows (A*H) and the fp32 SwiGLU products
     // (4*A*I) lived: both are dead once the re-quantisation has run (the reference overlays its stages the same
@@ -1807,13 +1824,10 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     const uint64_t shared_bytes = std::max<uint64_t>((uint64_t)A * H * 2, x1_bytes + (uint64_t)A * I * 4);
     const uint64_t o_x1 = c.take(shared_bytes);
     const uint64_t o_prod = o_x1 + x1_bytes;
-    // Few rows: GMM2 quantises the products itself, and then writes its rows while they are still read.
-    const bool stream = cam::stream_gemm_applies(A, 2 * I, Epr, false);
-    const bool from_products = stream && cam::stream_gemm_takes_products(A, (int)Epr, (int)I, (int)H, T);
     const uint64_t o_y = from_products ? c.take((uint64_t)A * H * 2) : o_x1;
     const uint64_t o_x1s = c.take((uint64_t)A * 4);
-    const uint64_t o_x2 = c.take((uint64_t)A * I);
-    const uint64_t o_x2s = c.take((uint64_t)A * 4);
+    const uint64_t o_x2 = from_products ? 0 : c.take((uint64_t)A * I);
+    const uint64_t o_x2s = from_products ? 0 : c.take((uint64_t)A * 4);
 
     const uint16_t *xp = (const uint16_t *)x->data;
     const int x_is_fp16 = x->dtype == CAM_DT_FLOAT16;
@@ -2037,8 +2051,6 @@ camStatus camGroupedMatmulFp8GetWorkspaceSize(const camTensor *x, const camTenso
     Fp8Weight fw{};
     CAM_TRY(check_fp8_weight(weight, weightScale, "weight", G, Kd, N, &fw));
     cam::SchedSpec sp = sched_spec(A, G, N, Kd, gate_up);
-    Carver c;
-    const uint64_t o_sched = c.take(cam::sched_bytes(A, (int)G, (int)N));
     cam::GemmArgs g{};
     g.a = (const int8_t *)x->data;
     g.w = fw.w;
@@ -2053,6 +2065,8 @@ camStatus camGroupedMatmulFp8GetWorkspaceSize(const camTensor *x, const camTenso
                                       : (out->dtype == CAM_DT_BF16 ? cam::kEpiDequantBf16 : cam::kEpiInt32));
     g.out = out->data;
     g.out_scale8 = quant_out ? (uint8_t *)outScaleOptional->data : nullptr;
+    Carver c;
+    const uint64_t o_sched = c.take(gemm_sched_bytes(A, N, G, g.epilogue, true));
     const int64_t *gl = (const int64_t *)groupList->data;
     const int cumulative = groupListType == 0;
     auto run = [=](void *wsp, hipStream_t s) mutable -> hipError_t {
@@ -2154,12 +2168,13 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
     const int64_t A = T * K;
     cam::SchedSpec sp1 = sched_spec(A, E, 2 * I, H, true);
     cam::SchedSpec sp2 = sched_spec(A, E, H, I, false);
+    const bool stream = cam::stream_gemm_applies(A, 2 * I, E, true);   // few rows: no schedules
     Carver c;
     const uint64_t o_pos = c.take((uint64_t)A * 4);
     const uint64_t o_row = c.take((uint64_t)A * 4);
     const uint64_t o_meta = c.take(cam::kPlanMeta * 4);
-    const uint64_t o_sched1 = c.take(cam::sched_bytes(A, (int)E, (int)(2 * I)));
-    const uint64_t o_sched2 = c.take(cam::sched_bytes(A, (int)E, (int)H));
+    const uint64_t o_sched1 = stream ? 0 : c.take(cam::sched_bytes(A, (int)E, (int)(2 * I)));
+    const uint64_t o_sched2 = stream ? 0 : c.take(cam::sched_bytes(A, (int)E, (int)H));
     const uint64_t o_hist = c.take(cam::plan_workspace_bytes(T, K, (int)E));
     // as in the int8 layer, the bf16 rows of GMM2 overlay the quantised input rows and the fp32 products
     const uint64_t x1_bytes = align_up((uint64_t)A * H);
@@ -2179,7 +2194,6 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
     uint16_t *outp = (uint16_t *)output->data;
     int64_t *etn = (int64_t *)expertTokenNums->data;
     const int iT = (int)T, iK = (int)K, iE = (int)E, iH = (int)H, iI = (int)I;
-    const bool stream = cam::stream_gemm_applies(A, 2 * I, E, true);
 
     auto run = [=](void *wsp, hipStream_t s) -> hipError_t {
         char *w = (char *)wsp;
