@@ -4,6 +4,9 @@ The FP8 layer is this library's own definition (include/cam_fp8_spec.h); the ref
 (src/cam/README.md:20-21), so nothing here is pinned against reference outputs.  Quantised values and scales
 are compared bit for bit; the matrix products accumulate in fp32 in hardware order and are compared with the
 tolerances written in each test.
+
+SwiGLU products, quantised products and bf16 rows of these small shapes take the streaming form of the GEMM, fp32 sums and the
+8192-token layer the tile form, whose other epilogues are in test_gpu_tile_epilogues.py.
 """
 import numpy as np
 import pytest
@@ -120,7 +123,7 @@ def test_grouped_matmul_fp8_bf16_output(gpu, oracle):
 @pytest.mark.parametrize("sizes,K,N", [
     ([33, 257, 0, 5], 1024, 512),      # flat and tall experts, an empty one, two product blocks
     ([129, 3, 64], 4096, 768),         # three product blocks, K of the C5 layer
-    ([700, 130, 1], 256, 1280),        # 1280 = 2.5 flat column blocks: the last flat item has one live team
+    ([700, 130, 1], 256, 1280),        # 1280 columns are five blocks of 128 products
     ([520], 512, 3072),                # three row tiles, N of the C5 layer
 ])
 def test_grouped_matmul_fp8_quantised_product_bit_exact(gpu, oracle, sizes, K, N):

@@ -1,4 +1,7 @@
-"""GPU parity: grouped w8a8 GEMM (int32 accumulators bit-exact) and its two epilogues against the oracle."""
+"""GPU parity: grouped w8a8 GEMM (int32 accumulators bit-exact) and its two epilogues against the oracle.
+
+Raw sums always take the tile form.  With an epilogue, launches of few rows x columns, i.e. all here but the full-size
+ones, take the streaming form; the tile form's epilogues are in test_gpu_tile_epilogues.py."""
 import numpy as np
 import pytest
 import torch

@@ -779,7 +779,9 @@ bool products_fit(const StreamShape &sh, long long max_rows, int Kd)
 // tile form -> this: 150 tokens on 40 experts, top-8, H 7168, I 2048: 407 -> 342 us; 1500 on 64, top-1, H 3072, I 2560: 332 ->
 // 273; 512 on 128, top-8, H 4096, I 1536: 483 -> 464; with five times as many 1000 on 256, top-8, H 2048, I 1024 lost, 362 -> 367,
 // and with 37 rows on average 300 on 64, H 2048, I 1408, 160 -> 162).  The tiles of the other form fetch FP8 scales item by item;
-// int8 gains from 322 -> 296 to 391 -> 362 on some of these shapes and loses from 449 -> 465 to 480 -> 503 on others.
+// int8 gains from 322 -> 296 to 391 -> 362 on some of these shapes and loses from 449 -> 465 to 480 -> 503 on others: rows x columns
+// alone does not tell them apart, so int8 stops where it never loses.  A layer asks once, with the columns of its GMM1, and
+// its GMM2 takes the same form.
 bool stream_gemm_applies(int64_t rows, int64_t N, int64_t G, bool fp8)
 {
     constexpr int64_t kMostRowsTimesColumns = 32ll * 512 * 256;
