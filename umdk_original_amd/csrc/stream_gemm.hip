@@ -73,6 +73,26 @@ __device__ __forceinline__ unsigned long long scalar_address(const void *p)
     return ((unsigned long long)hi << 32) | lo;
 }
 
+// Direct-to-LDS loads: lane i of the wave fetches 16 (4) bytes at base + off(i), which land at LDS byte dst + 16 i (4 i).  A
+// scalar register that the vector ALU has just written (both arguments may come out of a v_readfirstlane) must not be read
+// by a vector memory instruction within five wait states.  The compiler sees to that for its own instructions, not for these:
+// s_mov and s_nop are the five.
+__device__ __forceinline__ void load_lds16(const void *base, unsigned off, unsigned dst)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(scalar_address(base))
+                 : "memory", "m0");
+}
+
+__device__ __forceinline__ void load_lds4(const void *base, unsigned off, unsigned dst)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dword %1, %2"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(scalar_address(base))
+                 : "memory", "m0");
+}
+
 // The same value, computed anew as far as the compiler can tell: keeps loop-invariant address arithmetic out of registers.
 __device__ __forceinline__ int opaque(int v)
 {
@@ -259,10 +279,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
             const unsigned off = (unsigned)(row * Kd + min(c * it.ckb + ls * 16, Kd - 16));
             const unsigned dst = lds_addr(lds) + (unsigned)(buf * kABuf + (q * 8 + wave) * 1024);
             if (row < it.rows) {
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                             :
-                             : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(scalar_address(base))
-                             : "memory", "m0");
+                load_lds16(base, off, dst);
             }
         }
     };
@@ -284,18 +301,12 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
                 const int c4 = (tid & 15) * 4;
                 const int col = a.gate_up ? grp * 32 + (c4 < 32 ? c4 : c4 - 32 + (N >> 1)) : grp * 64 + c4;
                 const unsigned dst = lds_addr(&col_scale_s[set][0]) + (unsigned)(wave * 1024);
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                             :
-                             : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"((unsigned)(col * 4)), "s"(scalar_address(sg))
-                             : "memory", "m0");
+                load_lds16(sg, (unsigned)(col * 4), dst);
             }
             const int r = tid - 128;        // the waves from the third on: a row each lane
             if (!PRODUCTS && r >= 0 && r < it.rows) {
                 const unsigned dst = lds_addr(&row_scale_s[set][0]) + (unsigned)((wave - 2) * 256);
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-                             :
-                             : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"((unsigned)(r * 4)), "s"(scalar_address(a.a_scale + it.row0))
-                             : "memory", "m0");
+                load_lds4(a.a_scale + it.row0, (unsigned)(r * 4), dst);
             }
             return;
         }
@@ -305,10 +316,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
                 const int idx = tid + q * kSThreads;
                 if (idx < n) {
                     const unsigned dst = lds_addr(&a_scale8_s[set][0]) + (unsigned)((q * 8 + wave) * 256);
-                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-                                 :
-                                 : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"((unsigned)(idx * 4)), "s"(scalar_address(a.a_scale8 + (long long)it.row0 * KB))
-                                 : "memory", "m0");
+                    load_lds4(a.a_scale8 + (long long)it.row0 * KB, (unsigned)(idx * 4), dst);
                 }
             }
         }
