@@ -51,7 +51,7 @@ __global__ void invert_src_info_kernel(const int32_t *src_info, long long A, con
 // The row of slot (t,k), or -1: from the map, or, with BY_COUNTS, the way the SHMEM combine finds it
 // (moe_combine_shmem.h:514-556,833-837): the rows of the experts before the slot's, plus its rank within the expert.
 // Chosen at compile time, so that nothing is asked between the row loads of a gather.  (No difference in time that shows: dispatch
-// + combine of 4096 tokens x 7168 take 150.5 to 151.2 us either way.)
+// + combine of 4096 tokens x 7168 take 150.7 to 151.2 us either way.)
 template <bool BY_COUNTS>
 __device__ __forceinline__ long long row_of_slot(const CombineArgs &a, long long slot)
 {
