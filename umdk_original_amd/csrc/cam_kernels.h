@@ -27,9 +27,8 @@ constexpr int kSchedQueueStart = 4;
 constexpr int kSchedQueueCount = 544;
 constexpr int kSchedQueueStride = 32;
 constexpr int kSchedHeader = kSchedQueueCount + kMaxQueues * kSchedQueueStride;
-// One work item: rows [m0, m0 + rows) of expert g times column block nb.  flat != 0: at most 128 rows x 512
-// packed columns, the two wave teams split the columns; flat == 0: at most 256 rows x 256 packed columns, team
-// 0 takes tile rows [0, split), team 1 the rest.
+// One work item: rows [m0, m0 + rows) of expert g times column block nb.  flat != 0: at most 128 rows x 512 packed
+// columns; flat == 0: at most 256 rows x 256 packed columns.  split: half of a tall tile's rows, a multiple of 32.
 struct SchedItem {
     int32_t g, m0, rows, split, nb, flat, pad0, pad1;
 };

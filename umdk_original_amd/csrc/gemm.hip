@@ -9,35 +9,35 @@
 //   GMM2 epilogue   FDM/epilogue/block/block_epilogue_per_token_dequant.hpp:665-684
 //
 // Design (not a translation of the cube/vector split above).
-//   * Persistent kernel, one workgroup of 8 waves per CU.  Work items (one row tile of ONE expert x one
-//     block of packed weight columns) come from a device-built schedule (sched_device.h).  Short schedules
-//     give every workgroup a queue of its own, dealt so that the queues last equally long and that the
-//     workgroups of an XCD work on tiles which share operands; a workgroup whose queue runs out takes from
-//     the fullest one.  Long schedules use one queue per XCD, shared by its workgroups, in which the row
-//     tiles of an expert that read the same weight columns sit next to each other and big experts come
-//     first, which leaves the small items for the end, where they even out the finishing times.
-//   * Two tile shapes.  Tall tiles (129..256 rows) x 256 columns: the two teams of four waves split the
-//     rows, every wave owns 64 columns.  Flat tiles (<= 128 rows) x 512 columns: the teams split the
-//     columns, so that the weights, which is all such an expert streams from HBM, feed every wave and
-//     twice as many weight bytes are in flight per CU.  A wave always owns up to 128 rows x 64 columns
-//     (up to 128 int32 accumulators per lane), in 32-row fragments; the fragment count is a template
-//     parameter, so the main loop has no control flow.
-//   * Both operands travel global -> LDS with direct-to-LDS loads (16 bytes per lane, no registers),
-//     four (tall) or three (flat) stages of 64 K-bytes each, up to a whole ring ahead of the MFMAs: the
-//     fragments of a stage are read into registers one phase before they are multiplied, which frees the
-//     stage for the next load at once.  Weights were laid out once by the prepack kernel in the lane
-//     order the MFMA wants; activation rows are placed with an XOR swizzle of their 16-byte chunks
-//     (chosen on the global side, since a direct-to-LDS load writes lane i at base + 16*i), which makes
-//     the ds_read_b128 fragment reads bank-conflict free.
-//   * Ping-pong.  Every sub-step has two phases separated by workgroup barriers.  In the first, team 0
-//     issues nothing but its 16 MFMAs while team 1 reads its fragments and issues its loads; in the
-//     second they swap.  A SIMD holds one wave of each team, so its matrix pipe always has a wave that
-//     does nothing else.  Loads are addressed by a scalar base plus a per-lane 32-bit offset computed
-//     once per item: vector ALU work in the load path would queue behind the other wave's MFMAs (64-bit
-//     vector address arithmetic per load made the issue of eight loads take 2.3x as long).
-//   * The loads are issued from inline assembly and the waits are written out by hand: left to itself
-//     the compiler drains every outstanding load at each barrier and before LDS reads it cannot prove
-//     independent, which serialises the pipeline.
+//   * Persistent kernel, one workgroup of four waves per CU, one wave per SIMD with all 512 of its registers.  Work items
+//     (one row tile of ONE expert x one block of packed weight columns) come from a device-built schedule
+//     (sched_device.h).  Short schedules give every workgroup a queue of its own, dealt so that the queues last equally
+//     long and that the workgroups of an XCD work on tiles which share operands; a workgroup whose queue runs out takes
+//     from the fullest one.  Long schedules use one queue per XCD, shared by its workgroups, in which the row tiles of
+//     an expert that read the same weight columns sit next to each other and big experts come first, which leaves the
+//     small items for the end, where they even out the finishing times.
+//   * Two tile shapes.  Tall tiles (up to 256 rows) x 256 columns: a wave owns ALL rows of the tile and 64 of its columns.
+//     Flat tiles (<= 128 rows) x 512 columns, for experts that only stream weights: all rows and 128 columns.  Either
+//     way a wave holds up to sixteen 32 x 32 sums (256 registers, all of the accumulation file).  The numbers of row and
+//     column fragments are template parameters, so the main loop has no control flow.
+//   * A weight byte is needed by one wave only.  It goes from memory straight to that wave's registers (prepack_kernel laid
+//     the weights out in the lane order the MFMA wants), a ring of four 64-byte K steps.  Only the activations go
+//     through LDS: direct-to-LDS loads (16 bytes per lane, no registers) into a ring of four stages of 128 K bytes, a
+//     whole line of every row, their 16-byte chunks placed with an XOR swizzle (chosen on the global side, since such a
+//     load writes lane i at base + 16*i) that makes the ds_read_b128 fragment reads bank-conflict free.
+//     What bounds the loop is what crosses the LDS and the clock the power limit leaves.  Per 64 bytes of K and 256 rows the
+//     CU moves 16 KB of activations into LDS and 64 KB out of it, 640 of the 1024 cycles in which the matrix cores
+//     multiply them.  With two teams of four waves of 128 rows, both operands in LDS and two barriers per 64 bytes of K, it
+//     was 32 KB in and 96 KB out, 1024 of 1024 cycles: 1237 cycles for a step of 256 rows and 1027 for one of
+//     160, now 1079 and 729 (w8a8 gate/up GEMM, 65536 rows on 128 experts, K 4096, I 1536; stamps of a --timeline build).
+//     The clock falls as the matrix cores get busier (1.41 -> 1.35 GHz there), so time falls less than cycles.
+//   * Between two multiplications stands at most what the wave can issue while the first is in the matrix pipe: a
+//     request, or a fragment read, and a few scalar instructions.  The fragments are read six multiplications' pairs
+//     ahead, across the one barrier per 128 bytes of K.  Requests past the end of K go out with an empty buffer
+//     descriptor: they fetch nothing, and the counts that the waits rely on stay what they are.
+//   * The loads are issued from inline assembly and the waits are written out by hand: left to itself the compiler
+//     drains every outstanding load at each barrier and before LDS reads it cannot prove independent, which
+//     serialises the pipeline.  The sums are named registers for a similar reason (below).
 //   * The int32 accumulators stay in registers through the epilogue: dequantisation, SiLU and the
 //     gate*up product are applied in place; the int32 tile never goes to memory.  The MFMAs take the
 //     weights as their first operand, so a lane ends up with ONE activation row and runs of four
@@ -46,13 +46,14 @@
 //     stored.  For GMM1 the prepack pairs gate column c with up column I+c inside one wave.
 //   * The K order inside a 32-deep MFMA step is whatever the two operands agree on (an integer dot
 //     product does not care), which is what lets both be loaded as plain 16-byte pieces.
-//   * Flat items are bound by the memory, and three things in this file exist for them alone: their weight
-//     panels are fetched with non-temporal loads (nobody else reads them); they stop requesting stages in
-//     their last sub-steps, where tall items keep a branch-free loop body and fetch the last sub-step again;
-//     and between the K loop and the epilogue of a flat item the workgroup takes its next item and, if that
-//     is flat too, touches the lines of its first stages so that they travel to L2 under the epilogue.
+//   * Flat items are bound by the memory, and two things in this file exist for them alone: their weight panels are
+//     fetched with non-temporal loads (nobody else reads them), and between the K loop and the epilogue of a flat item
+//     the workgroup takes its next item and, if that is flat too, touches the lines of its first stages so that they
+//     travel to L2 under the epilogue.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
+#include <utility>
 
 #include "cam_device.h"
 #include "cam_kernels.h"
@@ -66,42 +67,78 @@ namespace cam {
 namespace {
 
 constexpr int kBK = 64;                         // K bytes per sub-step
-constexpr int kThreads = 512;                   // two teams of four waves
-constexpr int kMaxStages = 4;
-constexpr int kStageTall = 256 * kBK + 256 * kBK;   // 16 KB of activations + 16 KB of weights
-constexpr int kStageFlat = 128 * kBK + 512 * kBK;   //  8 KB of activations + 32 KB of weights
-constexpr int kLdsBytes = kMaxStages * kStageTall;  // 128 KB (flat: 3 x 40 KB = 120 KB)
+constexpr int kThreads = 256;                   // four waves, one per SIMD
+constexpr int kStageK = 128;                    // K bytes per stage of activations
+constexpr int kStages = 4;
+constexpr int kStage = 256 * kStageK;           // 32 KB
+constexpr int kLdsBytes = kStages * kStage;     // 128 KB
+constexpr int kRing = 4;                        // sub-steps of weights a wave has registers for
 constexpr int kScaleKb = 64;                    // FP8: K-blocks of 128 bytes an item may span (Kd <= 8192)
 constexpr int kEpiRowBytes = 144;               // epilogue staging: 128 data bytes + 16 of padding per row
 constexpr int kEpiSlice = 32 * kEpiRowBytes;    // one 32-row fragment per wave
 
-// LDS offset (bytes) inside a stage of the 16-byte chunk `c` (0..3) of activation row `r`.
-__device__ __forceinline__ int a_lds_offset(int r, int c)
+// Buffer descriptor words of `bytes` bytes at p.
+__device__ __forceinline__ v4i buffer_words(const void *p, unsigned bytes)
 {
-    return r * kBK + ((c ^ ((r >> 2) & 3)) << 4);
+    const unsigned long long v = (unsigned long long)p;
+    return v4i{(int)(unsigned)v, (int)((unsigned)(v >> 32) & 0xffffu), (int)bytes, 0x00020000};
 }
 
-// One direct-to-LDS load: lane i of the wave fetches 16 bytes at base + voff(i) and the data lands at LDS byte
-// address lds_addr + 16*i.  The base is a scalar register pair, so issuing the load needs no vector ALU work.
-// That pair comes from the scalar ALU, which needs no wait; one that the vector ALU had just written would need five wait
-// states in front of the load, which the compiler does not provide for inline assembly.  A test looks the built code
-// over for it (three more states here cost 0.2 to 0.3 % of the prefill layers).
+// Loads.  A vector memory instruction must not read a scalar register that the vector ALU wrote within five wait states, and the
+// compiler does not see to that for inline assembly.  Where a scalar operand may come out of a register the compiler had
+// parked in a vector lane (in front of the K loop; anywhere in the FP8 kernel, whose multiplications leave room for it),
+// WAITS provides the five.  A test looks the built code over.
+
+// One direct-to-LDS load: lane i of the wave fetches 16 bytes at its offset from the base, and the data lands at LDS byte
+// address lds_addr + LDS_OFFSET + 16*i.  Base and offsets are scalar but for one vector register, so that issuing the load
+// takes no vector ALU work.
+template <int LDS_OFFSET, bool WAITS>
+__device__ __forceinline__ void dma16(v4i words, unsigned voff, unsigned soff, unsigned lds_addr)
+{
+    if (WAITS) {
+        asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                     :
+                     : "s"(lds_addr), "v"(voff), "s"(words), "s"(soff), "n"(LDS_OFFSET)
+                     : "memory", "m0", "scc");
+    } else {
+        asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                     :
+                     : "s"(lds_addr), "v"(voff), "s"(words), "s"(soff), "n"(LDS_OFFSET)
+                     : "memory", "m0", "scc");
+    }
+}
+
+template <int LDS_OFFSET>
 __device__ __forceinline__ void dma16(const void *base, unsigned voff, unsigned lds_addr)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
                  :
-                 : "s"(lds_addr), "v"(voff), "s"((unsigned long long)base)
-                 : "memory", "m0");
+                 : "s"(lds_addr), "v"(voff), "s"((unsigned long long)base), "n"(LDS_OFFSET)
+                 : "memory", "m0", "scc");
 }
 
-// The same load marked non-temporal, for bytes that are read once: a stream of them moves at 6.6-7.1 TB/s from
-// HBM where the plain form stays at 5.8-6.0 (measured with a bare ring of these loads, 256 workgroups).
-__device__ __forceinline__ void dma16_stream(const void *base, unsigned voff, unsigned lds_addr)
+// 16 bytes per lane to registers.  STREAM: marked non-temporal, for bytes that are read once: a stream of them moves at
+// 6.6-7.1 TB/s from HBM where the plain form stays at 5.8-6.0 (measured with a bare ring of such loads, 256 workgroups).
+template <int OFFSET, bool STREAM, bool WAITS>
+__device__ __forceinline__ void request16(v4i &dst, v4i words, unsigned voff, unsigned soff)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
-                 :
-                 : "s"(lds_addr), "v"(voff), "s"((unsigned long long)base)
-                 : "memory", "m0");
+    if (WAITS) {
+        asm volatile("s_nop 4");
+    }
+    if (STREAM) {
+        asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:%4 nt"
+                     : "=v"(dst) : "v"(voff), "s"(words), "s"(soff), "n"(OFFSET) : "memory");
+    } else {
+        asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:%4"
+                     : "=v"(dst) : "v"(voff), "s"(words), "s"(soff), "n"(OFFSET) : "memory");
+    }
+}
+
+// The same value, computed anew as far as the compiler can tell: keeps loop-invariant address arithmetic out of registers.
+__device__ __forceinline__ int opaque(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
 }
 
 template <int N>
@@ -129,493 +166,592 @@ struct ItemCtx {
     const int8_t *wg;       // the expert's packed weights
     const float *sg;        // the expert's per-channel scales
     int m0, rows;           // first row and rows of the tile
-    int a_row0, my_rows;    // first tile row of this wave's fragments, rows of them that exist
-    int bslot;              // this wave's 64-column group inside the stage
-    int nw;                 // this wave's packed 64-column group of the weight (clamped to a valid one)
-    bool wave_live;         // the group exists (ragged last column block)
-    int stage_a, stage_bytes;
+    int group;              // this wave's first 64-column group of the weight
     int Kd, N;
 #ifdef CAM_GEMM_TIMELINE
     int *phase_s;           // LDS: wall clock at the first multiply and after the K loop (written by thread 0)
 #endif
 };
 
-// One wave's part of one item.  TEAM 0 multiplies in the first phase of every sub-step, TEAM 1 in the second.
-// FLAT selects the tile shape (it fixes the loads per wave and sub-step); MF is the wave's fragment count.
-__device__ __forceinline__ int acc_bits(int v) { return v; }
-__device__ __forceinline__ int acc_bits(float v) { return __float_as_int(v); }
+// f(std::integral_constant<int, I>) for I in [B, E), unrolled.
+template <int B, int E, typename F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>());
+        static_for<B + 1, E>(f);
+    }
+}
+
+// Accumulators.  All 256 accumulation registers of a wave hold sixteen 32 x 32 tiles, tile T in a[16 T : 16 T + 15], named here
+// and not by the compiler: with that file full it spills and copies around the loop, and cannot know that no other value
+// wants a place there.
+#define CAM_ACC_0 "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15"
+#define CAM_ACC_1 "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31"
+#define CAM_ACC_2 "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47"
+#define CAM_ACC_3 "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63"
+#define CAM_ACC_4 "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79"
+#define CAM_ACC_5 "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95"
+#define CAM_ACC_6 "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111"
+#define CAM_ACC_7 "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127"
+#define CAM_ACC_8 "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143"
+#define CAM_ACC_9 "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159"
+#define CAM_ACC_10 "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175"
+#define CAM_ACC_11 "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191"
+#define CAM_ACC_12 "a192", "a193", "a194", "a195", "a196", "a197", "a198", "a199", "a200", "a201", "a202", "a203", "a204", "a205", "a206", "a207"
+#define CAM_ACC_13 "a208", "a209", "a210", "a211", "a212", "a213", "a214", "a215", "a216", "a217", "a218", "a219", "a220", "a221", "a222", "a223"
+#define CAM_ACC_14 "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239"
+#define CAM_ACC_15 "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
+#define CAM_ACC_TILES(X) \
+    X(0, 0, 15, CAM_ACC_0) X(1, 16, 31, CAM_ACC_1) X(2, 32, 47, CAM_ACC_2) X(3, 48, 63, CAM_ACC_3) \
+    X(4, 64, 79, CAM_ACC_4) X(5, 80, 95, CAM_ACC_5) X(6, 96, 111, CAM_ACC_6) X(7, 112, 127, CAM_ACC_7) \
+    X(8, 128, 143, CAM_ACC_8) X(9, 144, 159, CAM_ACC_9) X(10, 160, 175, CAM_ACC_10) X(11, 176, 191, CAM_ACC_11) \
+    X(12, 192, 207, CAM_ACC_12) X(13, 208, 223, CAM_ACC_13) X(14, 224, 239, CAM_ACC_14) X(15, 240, 255, CAM_ACC_15)
+
+template <int TILE>
+__device__ __forceinline__ void acc_multiply(v4i w, v4i x)
+{
+#define CAM_X(T, LO, HI, ...) \
+    if constexpr (TILE == T) { \
+        asm volatile("v_mfma_i32_32x32x32_i8 a[" #LO ":" #HI "], %0, %1, a[" #LO ":" #HI "]" ::"v"(w), "v"(x) : __VA_ARGS__); \
+    }
+    CAM_ACC_TILES(CAM_X)
+#undef CAM_X
+}
+
+template <int TILE>
+__device__ __forceinline__ void acc_multiply(v8i w, v8i x, int sw, int sx)
+{
+#define CAM_X(T, LO, HI, ...) \
+    if constexpr (TILE == T) { \
+        asm volatile("v_mfma_scale_f32_32x32x64_f8f6f4 a[" #LO ":" #HI "], %0, %1, a[" #LO ":" #HI "], %2, %3 op_sel_hi:[0,0,0]" \
+                     ::"v"(w), "v"(x), "v"(sw), "v"(sx) : __VA_ARGS__); \
+    }
+    CAM_ACC_TILES(CAM_X)
+#undef CAM_X
+}
+
+template <int TILE>
+__device__ __forceinline__ void acc_clear()
+{
+#define CAM_X(T, LO, HI, ...) \
+    if constexpr (TILE == T) { \
+        asm volatile(".irp r, 0,1,2,3,4,5,6,7,8,9,10,11,12,13,14,15\n\tv_accvgpr_write_b32 a[" #LO "+\\r], 0\n\t.endr" ::: __VA_ARGS__); \
+    }
+    CAM_ACC_TILES(CAM_X)
+#undef CAM_X
+}
+
+template <int REG>
+__device__ __forceinline__ int acc_bits()
+{
+    int v;
+    asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(v) : "n"(REG));
+    return v;
+}
+
+template <int REG, bool FP8>
+__device__ __forceinline__ float acc_value()
+{
+    return FP8 ? __int_as_float(acc_bits<REG>()) : (float)acc_bits<REG>();
+}
 
 template <bool FP8>
-struct AccType {
-    typedef v16i type;
+struct FragType {
+    typedef v4i type;
 };
 template <>
-struct AccType<true> {
-    typedef v16f type;
+struct FragType<true> {
+    typedef v8i type;
 };
 
-// FP8 items (FP8 = true) run the same pipeline with v_mfma_scale_f32_32x32x64_f8f6f4: one instruction covers
-// the 64 K bytes of a sub-step (the two 16-byte pieces a lane holds), takes the E8M0 scale of the lane's weight
-// column block and of its activation row for the current 128-byte K block, and accumulates in fp32.  The
-// scales of the item wait in LDS (a_scale8_s[kb * 256 + tile row], w_scale8_s[column group * kScaleKb + kb]) and
-// are read with the fragments.
-template <int MF, int TEAM, bool FLAT, bool FP8, typename Hook, typename Stage>
-__device__ __forceinline__ void run_item(const GemmArgs &a, const ItemCtx &t, int nb, int8_t *lds,
-                                         const float *row_scale_s, const uint8_t *a_scale8_s,
-                                         const uint8_t *w_scale8_s, Hook &between, Stage &stage_scales)
+// The K loop, for one wave: MF row fragments x NF column fragments, sums in tiles mf * NF + nf.
+//   stage s:     requests stage s + 3 of the activations (into the slot of stage s - 1, which the barrier before has set free)
+//   sub-step k:  (two per stage) multiplies the weights of k with the fragments of its half of the stage, and requests the
+//                weights of k + 3 into the registers that k - 1 has been multiplied from
+//   slot:        (2 MF per sub-step, FP8: MF) NF multiplications with one activation fragment; reads the fragment of PD
+//                slots later and sends the slot's share of the requests between the multiplications
+// A stage ends with a wait and a barrier.  Fragments are read across it, i.e. stage s + 1 is read in stage s, and so has to be
+// in LDS one stage early.  Loads retire in order, and the order of the requests is the same in every sub-step (activations,
+// then weights), so "at most WAIT outstanding" in front of sub-step k says that its weights have come, which were the last
+// requests of sub-step k - 3: since then two sub-steps have sent NB weight loads each and a stage's MF activation
+// loads.  In front of a stage's first sub-step that covers the activations of stage s + 1, which are older.
+// Requests past the end are for nothing (empty descriptors).
+//
+// FP8: v_mfma_scale_f32_32x32x64_f8f6f4 covers the 64 K bytes of a sub-step (the two 16-byte pieces a lane holds), takes the E8M0
+// scale of the lane's weight column block and of its activation row for the current 128-byte K block, and accumulates in fp32.
+// The scales of the item wait in LDS (a_scale8_s[kb * 256 + tile row], w_scale8_s[column fragment of the item * kScaleKb +
+// kb]).
+template <int MF, int NF, bool FP8, typename Stage>
+__device__ __forceinline__ void k_loop(const ItemCtx &t, int8_t *lds, const uint8_t *a_scale8_s,
+                                       const uint8_t *w_scale8_s, Stage &stage_scales)
 {
-    constexpr int NS = FLAT ? 3 : 4;                       // ring of stages
-    constexpr int LPS = FLAT ? (TEAM == 0 ? 6 : 4) : 4;    // loads per wave and sub-step
-    constexpr int MFR = MF > 0 ? MF : 1;
+    constexpr bool STREAM = NF == 4;                // a flat item is the only reader of its weight panel
+    constexpr int SLOTS = FP8 ? MF : 2 * MF;
+    constexpr int AR = FP8 ? 4 : 8;                 // fragments in registers
+    constexpr int PD = FP8 ? (MF == 1 ? 2 : 3) : (MF == 1 ? 4 : 6);  // (at most a stage)
+    constexpr int NB = 2 * NF;                      // weight loads per sub-step
+    constexpr int kHalf = (MF + 1) / 2;             // activation loads in a stage's first sub-step
+    constexpr int WAIT = 2 * NB + MF;
     const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wn = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
-    const int KT = t.Kd / kBK;
-    const int last = KT - 1;
+    const int lane = opaque(tid) & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ST = t.Kd / kStageK;
+    const int KT = 2 * ST;
     const unsigned lds0 = (unsigned)(unsigned long long)(__attribute__((address_space(3))) int8_t *)lds;
 
-    typename AccType<FP8>::type acc[MFR][2];
-#pragma unroll
-    for (int mf = 0; mf < MFR; ++mf) {
-#pragma unroll
-        for (int nf = 0; nf < 2; ++nf) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                acc[mf][nf][i] = 0;
-            }
-        }
-    }
+    // ---- activations: wave w brings tile rows 8 MF w .. 8 MF (w + 1) - 1, eight rows a load.  Lane i of a load brings row i / 8
+    // of its eight and the 16-byte chunk whose swizzled slot is i % 8: chunk c of row r lies at slot c ^ (r / 2 % 8) of the
+    // row's 128 bytes, so that sixteen neighbouring rows cover all 64 banks.  Rows beyond the tile are out of the
+    // descriptor's range, which the vector offset is checked against, and come as zeros; the first two stages, which are
+    // requested by address, repeat the last row there, and the last chunk of a row where K ends.
+    const v4i a_words = buffer_words(t.a_tile, (unsigned)t.rows * (unsigned)t.Kd);
+    const unsigned a_dst = lds0 + (unsigned)(wave * (MF * 1024));
+    unsigned a_voff[MF];
+    static_for<0, MF>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const int r = 8 * (wave * MF + j) + (lane >> 3);
+        const int c16 = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+        a_voff[j] = (unsigned)(r * t.Kd + c16);
+    });
+    auto bring_first = [&](int s) {
+        static_for<0, MF>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            const int r = 8 * (wave * MF + j) + (lane >> 3);
+            const int c16 = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+            const unsigned voff = (unsigned)(min(r, t.rows - 1) * t.Kd + min(s * kStageK + c16, t.Kd - 16));
+            dma16<j * 1024>(t.a_tile, voff, a_dst + (unsigned)(s * kStage));
+        });
+    };
+    auto bring = [&](int s, auto jc, auto wc) {  // load j of stage s
+        constexpr int j = decltype(jc)::value;
+        v4i words = a_words;
+        words[2] = s < ST ? words[2] : 0;
+        dma16<j * 1024, decltype(wc)::value>(words, a_voff[j], (unsigned)(s * kStageK),
+                                                  a_dst + (unsigned)((s & (kStages - 1)) * kStage));
+    };
 
-    // ---- loads.  Tall: team 0 brings the activations (wave wn: tile rows 64wn .. 64wn+63, four loads of 16
-    // rows), team 1 the weights (wave wn: the 4 KB of column group wn).  Flat: team 0 brings the activations
-    // (wave wn: rows 32wn .. 32wn+31) and column groups 0..3, team 1 column groups 4..7.  Lane i of an
-    // activation load brings row (i / 4) of its 16 and the chunk whose swizzled slot is i % 4; rows beyond the
-    // tile repeat its last row (their results are dropped in the epilogue).
-    constexpr int NA = FLAT ? (TEAM == 0 ? 2 : 0) : (TEAM == 0 ? 4 : 0);
-    constexpr int NB = LPS - NA;
-    unsigned a_voff[NA > 0 ? NA : 1];
-    unsigned a_dst[NA > 0 ? NA : 1];
-#pragma unroll
-    for (int j = 0; j < NA; ++j) {
-        const int r0 = (FLAT ? 32 : 64) * wn + 16 * j;
-        const int r = r0 + (lane >> 2);
-        const int c = (lane & 3) ^ ((r >> 2) & 3);
-        a_voff[j] = (unsigned)(min(r, t.rows - 1) * t.Kd + c * 16);
-        a_dst[j] = (unsigned)(r0 * kBK);
-    }
+    // ---- weights.  Column groups lie in blocks of eight; inside a block the 4 KB of a K step of its groups lie side by
+    // side, so the loads of one step of a workgroup cover one contiguous stretch of memory.
+    v4i ring[kRing][NB];
     const int ngroups = t.N / 64;
-    const int bgroup = FLAT ? TEAM * 4 + wn : wn;  // the column group of the stage this wave loads
-    const int nw_load = min(nb * (FLAT ? 8 : 4) + bgroup, ngroups - 1);
-    // Packed weights: column groups in blocks of eight; inside a block the 4 KB of a K step of its groups lie
-    // side by side, so the loads of one step of a workgroup cover one contiguous stretch of memory.
-    const int b_block = nw_load >> 3;
+    const int nw0 = min(t.group, ngroups - 1);
+    const int nw1 = min(t.group + 1, ngroups - 1);
+    const int b_block = nw0 >> 3;
     const int b_step = min(8, ngroups - 8 * b_block) * 4096;
-    const int8_t *b_base = t.wg + (long long)b_block * 8 * t.Kd * 64 + (nw_load & 7) * 4096;
-    const unsigned b_voff = (unsigned)(lane * 16);
-    const unsigned b_dst = (unsigned)(t.stage_a + bgroup * 4096);
-
-    auto issue = [&](int s_idx, int slot) {
-        const int s = min(s_idx, last);
-        const unsigned sbase = lds0 + (unsigned)(slot * t.stage_bytes);
-        if (NA > 0) {
-            const int8_t *ab = t.a_tile + (long long)s * kBK;
-#pragma unroll
-            for (int j = 0; j < NA; ++j) {
-                dma16(ab, a_voff[j], sbase + a_dst[j]);
-            }
-        }
-        if (NB > 0) {
-            const int8_t *bb = b_base + (long long)s * b_step;
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                if (FLAT) {  // a flat item is the only reader of its weight panel
-                    dma16_stream(bb + j * 1024, b_voff, sbase + b_dst + j * 1024);
-                } else {
-                    dma16(bb + j * 1024, b_voff, sbase + b_dst + j * 1024);
-                }
-            }
+    const v4i b_words = buffer_words(t.wg + (long long)b_block * 8 * t.Kd * 64 + (nw0 & 7) * 4096, 0x7fffffffu);
+    const unsigned b_voff0 = (unsigned)(lane * 16);
+    const unsigned b_voff1 = b_voff0 + (unsigned)((nw1 - nw0) * 4096);
+    auto request = [&](v4i (&dst)[NB], int k, auto jc, auto wc) {
+        constexpr int j = decltype(jc)::value;     // K half j / NF, column fragment j % NF
+        constexpr int nf = j % NF, kk = j / NF;
+        constexpr int off = kk * 2048 + (nf & 1) * 1024;
+        v4i words = b_words;
+        words[2] = k < KT ? words[2] : 0;
+        request16<off, STREAM, decltype(wc)::value>(dst[j], words, nf < 2 ? b_voff0 : b_voff1, (unsigned)(k * b_step));
+    };
+    // The registers of a sub-step are passed through the wait for them: nothing that reads them is moved in front of it.
+    // (Between the request and here nothing may read or move them at all; a test looks the built code over.)
+    auto landed = [&](v4i (&r)[NB]) {
+        if constexpr (NB == 4) {
+            asm volatile("s_waitcnt vmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(WAIT) : "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(%8)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]),
+                         "+v"(r[6]), "+v"(r[7]) : "n"(WAIT) : "memory");
         }
     };
 
-    // ---- fragments: read from LDS one phase before they are multiplied.
-    v8i af[MFR];  // .lo: the K bytes of the first 32-byte half of the sub-step, .hi: of the second
-    v8i bf[2];
-    int sa[MFR];  // FP8: E8M0 scales of this lane's activation rows, and of its two weight column fragments
-    int sw[2] = {0, 0};
-    const int a_row = lane & 31;
-    const int a_half = lane >> 5;
-    auto read_frags = [&](int slot, int s_idx) {
-        const int8_t *st = lds + slot * t.stage_bytes;
-        const int8_t *sb = st + t.stage_a + t.bslot * 4096 + lane * 16;
-#pragma unroll
-        for (int nf = 0; nf < 2; ++nf) {
-            bf[nf].lo = *(const v4i *)(sb + nf * 1024);
-            bf[nf].hi = *(const v4i *)(sb + (2 + nf) * 1024);
-        }
-#pragma unroll
-        for (int mf = 0; mf < MF; ++mf) {
-            af[mf].lo = *(const v4i *)(st + a_lds_offset(t.a_row0 + mf * 32 + a_row, a_half));
-            af[mf].hi = *(const v4i *)(st + a_lds_offset(t.a_row0 + mf * 32 + a_row, 2 + a_half));
-        }
-        if (FP8) {
-            const int kb = min(s_idx, last) >> 1;
-            sw[0] = w_scale8_s[(t.bslot * 2 + 0) * kScaleKb + kb];
-            sw[1] = w_scale8_s[(t.bslot * 2 + 1) * kScaleKb + kb];
-#pragma unroll
-            for (int mf = 0; mf < MF; ++mf) {
-                sa[mf] = a_scale8_s[kb * 256 + t.a_row0 + mf * 32 + a_row];
-            }
-        }
-    };
-    auto multiply = [&]() {
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_setprio(2);
-        // Weights as the first operand: the result tile comes out transposed, i.e. a lane holds ONE
-        // activation row and 4 consecutive weight columns per register quad.
+    // ---- fragments
+    typename FragType<FP8>::type af[AR];
+    int sa[2][MF];
+    int sw[2][NF];
+    const int frow = lane & 31;
+    const int fbase = frow * kStageK + (((lane >> 5) ^ ((frow >> 1) & 7)) << 4);
+    auto read_frag = [&](typename FragType<FP8>::type &dst, int slot, auto qc) {
+        constexpr int q = decltype(qc)::value;  // slot inside the stage
+        constexpr int u = q / SLOTS, i = q % SLOTS;
         if constexpr (FP8) {
+            dst.lo = *(const v4i *)(lds + slot * kStage + (fbase ^ (u * 64)) + i * 4096);
+            dst.hi = *(const v4i *)(lds + slot * kStage + (fbase ^ (u * 64 + 32)) + i * 4096);
+        } else {
+            dst = *(const v4i *)(lds + slot * kStage + (fbase ^ (u * 64 + (i / MF) * 32)) + (i % MF) * 4096);
+        }
+    };
+    auto read_scales = [&](int b, int s) {
+        if constexpr (FP8) {
+            const int kb = min(s, ST - 1);
+#pragma unroll
+            for (int nf = 0; nf < NF; ++nf) {
+                sw[b][nf] = w_scale8_s[(wave * NF + nf) * kScaleKb + kb];
+            }
 #pragma unroll
             for (int mf = 0; mf < MF; ++mf) {
-#pragma unroll
-                for (int nf = 0; nf < 2; ++nf) {
-                    acc[mf][nf] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[nf], af[mf], acc[mf][nf], 0, 0, 0,
-                                                                                 sw[nf], 0, sa[mf]);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-                for (int mf = 0; mf < MF; ++mf) {
-#pragma unroll
-                    for (int nf = 0; nf < 2; ++nf) {
-                        acc[mf][nf] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kk == 0 ? bf[nf].lo : bf[nf].hi,
-                                                                            kk == 0 ? af[mf].lo : af[mf].hi,
-                                                                            acc[mf][nf], 0, 0, 0);
-                    }
-                }
+                sa[b][mf] = a_scale8_s[kb * 256 + mf * 32 + (lane & 31)];
             }
         }
-        __builtin_amdgcn_s_setprio(0);
-        __builtin_amdgcn_sched_barrier(0);
     };
 
-    // ---- pipeline.  Loads retire in order and every sub-step that requests a stage issues exactly LPS loads per
-    // wave, so "at most n * LPS outstanding" says which sub-steps of this wave's loads have landed; the barrier
-    // after the wait makes that true for the whole workgroup.  In the last NS sub-steps nothing is left to request
-    // and the wait is for what remains: with `rem` stages after the current one, stage s+1 has landed once at most
-    // rem - 1 stages are outstanding.
-    //   barrier A(s): every load of stage s+1 has landed; team 1 is done reading stage s
-    //   barrier B(s): team 0 is done reading stage s+1; B(-1) stands in front of the loop
-    // Stage s is free once both teams have its fragments in registers: team 1 reads it behind B(s-1), when team 0 has it,
-    // and refills its part at the end of that reading phase; team 0 refills its own in the phase behind A(s).
-    // B(-1) is needed as much as the others: without it a wave of team 0 that is late with its first fragments (behind an
-    // instruction cache miss, say) may read weights of sub-step NS in their place.  It costs nothing that shows (8192 tokens x
-    // 4096, 128 experts, top-8, I 1536: 1717 -> 1721 us, runs of one side 0.2 % apart; 8192 skewed rows on 32 experts, H 7168,
-    // I 2048: 496.4 -> 496.0): the teams share the LDS, and now team 0, which multiplies first, is served first.
-    auto wait_stages = [&](int n) {  // at most n stages of this wave's loads outstanding (n wave-uniform)
-        if (n <= 0) {
-            wait_loads_outstanding<0>();
-        } else if (n == 1) {
-            wait_loads_outstanding<LPS>();
-        } else if (n == 2) {
-            wait_loads_outstanding<2 * LPS>();
-        } else {
-            wait_loads_outstanding<3 * LPS>();
-        }
-    };
-    // Tall tiles keep a loop body without control flow instead (their long bodies schedule worse with it: +2-4 %):
-    // sub-step indices past the end are clamped, i.e. the last sub-step is fetched again into a stage nobody
-    // reads, and every sub-step requests a stage.
-#pragma unroll
-    for (int p = 0; p < NS; ++p) {
-        if (!FLAT || p <= last) {
-            issue(p, p);
-        }
-    }
+    // ---- pipeline.  The first requests go out in the order the loop would have sent them in.
+    const std::true_type waits;
+    bring_first(0);
+    bring_first(1);
+    static_for<0, NB>([&](auto j) { request(ring[0], 0, j, waits); });
+    static_for<0, kHalf>([&](auto j) { bring(2, j, waits); });
+    static_for<0, NB>([&](auto j) { request(ring[1], 1, j, waits); });
+    static_for<kHalf, MF>([&](auto j) { bring(2, j, waits); });
+    static_for<0, NB>([&](auto j) { request(ring[2], 2, j, waits); });
     // The item's scales go to LDS now, behind the requests for the first stages, so that their round trip to
-    // memory runs beside that of the weights instead of ahead of it.  (Their loads are younger than the stage
-    // loads and complete after them: the wait below is then met at once.)
+    // memory runs beside that of the weights instead of ahead of it.
     stage_scales();
+    static_for<0, MF * NF>([&](auto tc) { acc_clear<decltype(tc)::value>(); });
     wait_lds_reads();
-    if (FLAT) {
-        wait_stages(min(NS - 1, last));
-    } else {
-        wait_loads_outstanding<(NS - 1) * LPS>();
-    }
-    barrier_no_fence();  // stage 0 has landed and every wave's share of the scales is in LDS
+    landed(ring[0]);
+    barrier_no_fence();
 #ifdef CAM_GEMM_TIMELINE
     if (tid == 0) {
         t.phase_s[0] = (int)wall_clock64();
     }
 #endif
-    int slot = 0;        // slot of stage s
-    const int steady = FLAT ? KT - NS : KT;  // sub-steps that request the stage NS ahead
-    if (TEAM == 0) {
-        read_frags(0, 0);
-        wait_lds_reads();
-        barrier_no_fence();                               // B(-1)
-        for (int s = 0; s < KT; ++s) {
-            const int next = slot + 1 == NS ? 0 : slot + 1;
-            multiply();                                   // phase 1: stage s, from registers
-            if (!FLAT || s < steady) {
-                wait_loads_outstanding<(NS - 2) * LPS>(); // my part of stage s+1 has landed
-            } else if (s < last) {
-                wait_stages(last - s - 1);
+    read_scales(0, 0);
+    static_for<0, PD>([&](auto f) { read_frag(af[decltype(f)::value % AR], 0, f); });
+
+    // Stage s0 + b, s0 even.  TAIL: the stage behind the last pair of an odd number of them, which requests nothing.
+    auto stage = [&](int s0, auto bc, auto tc) {
+        constexpr int b = decltype(bc)::value;
+        constexpr bool TAIL = decltype(tc)::value;
+        const int s = s0 + b;
+        const int base = s0 & 2;   // slot of stage s0
+        static_for<0, 2>([&](auto uc) {
+            constexpr int u = decltype(uc)::value;
+            constexpr int r = (2 * b + u) % kRing;
+            constexpr int NA = u == 0 ? kHalf : MF / 2;
+            constexpr int OPS = NA + NB;
+            const std::integral_constant<bool, FP8> waits_fp8;
+            if (u == 1) {
+                if (TAIL) {
+                    wait_loads_outstanding<0>();
+                }
+                landed(ring[r]);
+                read_scales(b ^ 1, s + 1);
             }
-            barrier_no_fence();                           // A(s)
-            if (!FLAT || s < steady) {
-                issue(s + NS, slot);                      // phase 2: refill stage s's slot ...
-            }
-            read_frags(next, s + 1);                      // ... and fetch the fragments of stage s+1
-            wait_lds_reads();
-            barrier_no_fence();                           // B(s)
-            slot = next;
+            static_for<0, SLOTS>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                constexpr int f = (2 * b + u) * SLOTS + i;    // slot of the loop body
+                constexpr int fn = f + PD, sn = fn / (2 * SLOTS);
+                read_frag(af[fn % AR], sn == 2 ? base ^ 2 : base + sn, std::integral_constant<int, fn % (2 * SLOTS)>());
+                __builtin_amdgcn_sched_barrier(0);
+                // this slot's share of the sub-step's requests, spread over the gaps between its multiplications
+                constexpr int o0 = i * OPS / SLOTS, on = (i + 1) * OPS / SLOTS - o0;
+                static_for<0, NF>([&](auto nc) {
+                    constexpr int n = decltype(nc)::value;
+                    constexpr int nf = (i & 1) ? NF - 1 - n : n;  // (one operand stays from one multiplication to the next)
+                    if constexpr (FP8) {
+                        const v8i w = __builtin_shufflevector(ring[r][nf], ring[r][NF + nf], 0, 1, 2, 3, 4, 5, 6, 7);
+                        acc_multiply<i * NF + nf>(w, af[f % AR], sw[b][nf], sa[b][i]);
+                    } else {
+                        acc_multiply<(i % MF) * NF + nf>(ring[r][(i / MF) * NF + nf], af[f % AR]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (n < NF - 1 && !TAIL) {
+                        static_for<o0 + n * on / (NF - 1), o0 + (n + 1) * on / (NF - 1)>([&](auto oc) {
+                            constexpr int o = decltype(oc)::value;
+                            if constexpr (o < NA) {
+                                bring(s + 3, std::integral_constant<int, u * kHalf + o>(), waits_fp8);
+                            } else {
+                                request(ring[(r + 3) % kRing], 2 * s + u + 3, std::integral_constant<int, o - NA>(), waits_fp8);
+                            }
+                        });
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                });
+            });
+        });
+        if constexpr (!TAIL) {
+            landed(ring[(2 * b + 2) % kRing]);
+            barrier_no_fence();
         }
-    } else {
-        barrier_no_fence();                               // B(-1)
-        for (int s = 0; s < KT; ++s) {
-            const int next = slot + 1 == NS ? 0 : slot + 1;
-            read_frags(slot, s);                          // phase 1: fragments of stage s ...
-            wait_lds_reads();
-            if (!FLAT || s < steady) {
-                issue(s + NS, slot);                      // ... then refill its slot
-                wait_loads_outstanding<(NS - 1) * LPS>(); // my part of stage s+1 has landed
-            } else if (s < last) {
-                wait_stages(last - s - 1);
-            }
-            barrier_no_fence();                           // A(s)
-            multiply();                                   // phase 2: stage s
-            barrier_no_fence();                           // B(s)
-            slot = next;
-        }
+    };
+    int s0 = 0;
+    for (; s0 + 1 < ST; s0 += 2) {
+        stage(s0, std::integral_constant<int, 0>(), std::false_type());
+        stage(s0, std::integral_constant<int, 1>(), std::false_type());
     }
-    if (!FLAT) {
-        wait_loads_outstanding<0>();
+    if (s0 < ST) {
+        stage(s0, std::integral_constant<int, 0>(), std::true_type());
     }
+    wait_loads_outstanding<0>();
+#pragma unroll
+    for (int j = 0; j < kRing * NB; ++j) {  // the registers of the last requests are taken until here
+        asm volatile("" ::"v"(ring[j / NB][j % NB]));
+    }
+    wait_lds_reads();
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products are in their registers
     barrier_no_fence();  // nobody reads or fills the stages any more: the epilogue may stage through them
 #ifdef CAM_GEMM_TIMELINE
     if (tid == 0) {
         t.phase_s[1] = (int)wall_clock64();
     }
 #endif
+}
+
+// The epilogue of an item, for one wave: n row fragments x NF column fragments, sums in tiles mf * NF + nf.  One function for all
+// numbers of row fragments: it is long straight-line code (the sums are named registers), and a copy for each of them would
+// not stay in the instruction cache, which a CU shares with its neighbour.
+template <int NF, bool FP8, typename Hook>
+__device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &t, int n, int8_t *lds, const float *row_scale_s,
+                                              Hook &between)
+{
+    constexpr bool FLAT = NF == 4;
+    constexpr int MF = FLAT ? 4 : 8;
+    constexpr int NG = NF / 2;       // 64-column groups of this wave
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = opaque(tid) & (kWave - 1);
+    const int row_in = lane & 31;
+    const int col_half = (lane >> 5) * 4;
+    const int N = t.N;
+    const int ngroups = N / 64;
 
     // ---- epilogue, accumulators in registers.
     // Lane l holds activation row (l & 31) of each 32x32 fragment; registers 4j .. 4j+3 hold the four
     // consecutive weight columns 8j + 4*(l/32) + 0..3.  Dequantisation runs on that layout with one row scale
     // per lane and fragment and the column scales fetched as 16-byte vectors.  To store whole 128-byte lines,
-    // every wave passes one fragment at a time through its own slice of LDS: 128 staged bytes per row, then
-    // 16 bytes per lane and 8 rows per store instruction.
+    // every wave passes one 32-row block of 128 bytes at a time through its own slice of LDS: it writes the block, requests
+    // it back as 16 bytes per lane and 8 rows per register, and stores it when the next block is computed, so that the
+    // round trip through LDS runs under arithmetic (the wave has its SIMD to itself).  Stores past the tile's rows are out of
+    // the range of their descriptor.
     // `between` is the workgroup's business between two items (taking the next one and asking for its first
     // bytes, see gemm_kernel).  It runs after this wave has requested its column scales and before it uses them,
     // so that its memory traffic travels under the arithmetic of the epilogue; it returns a value that depends on
     // what it loaded, consumed at the very end so that nothing waits for those loads earlier.
     int between_sink = 0;
+    int8_t *slice = lds + wave * kEpiSlice;
+    const int sub = lane >> 3;    // row inside a group of 8
+    const int piece = lane & 7;   // 16-byte piece of the 128-byte row
+
+    // compute(mf) for the n row fragments, each of which leaves a block in the slice; store(mf, v) gets it back as v[4].
+    auto blocks = [&](auto &&compute, auto &&store) {
+        v4u held[4];
+        static_for<0, MF>([&](auto mc) {
+            constexpr int mf = decltype(mc)::value;
+            if (mf < n) {
+                compute(mc);
+                if constexpr (mf > 0) {
+                    store(mf - 1, held);
+                }
+#pragma unroll
+                for (int it = 0; it < 4; ++it) {
+                    held[it] = *(const v4u *)(slice + (it * 8 + sub) * kEpiRowBytes + piece * 16);
+                }
+            }
+        });
+        store(n - 1, held);
+    };
+    // 128 bytes of columns from `col` on, in rows of `pitch` bytes: a descriptor for them and the offset of this lane's piece.
+    // The next kernel reads these rows once; stored non-temporally (2) they do not push weight panels and activation tiles out
+    // of the L2 (C3 both operators 519 -> 506 us, decode layer 427 -> 420 us).
+    auto columns = [&](int col, int pitch) {
+        return __builtin_amdgcn_make_buffer_rsrc((int8_t *)a.out + (long long)t.m0 * pitch + col, 0,
+                                                 (unsigned)((t.rows - 1) * pitch + 128), 0x00020000);
+    };
+    auto store_rows = [&](__amdgpu_buffer_rsrc_t out, int pitch, int mf, const v4u (&v)[4]) {
+        const unsigned at = (unsigned)((mf * 32 + sub) * pitch + piece * 16);
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+            __builtin_amdgcn_raw_buffer_store_b128(v[it], out, at + (unsigned)(it * 8 * pitch), 0, 2);
+        }
+    };
+
     auto epilogue = [&]() {
-    const bool work = MF > 0 && t.wave_live;
-    v4f csc[2][4];  // column scales: [0] gate / [1] up of a paired group, or the two fragments of a plain one
-    if (FLAT && !FP8 && work && a.epilogue != kEpiInt32) {
-        const int col_half = (lane >> 5) * 4;
+        v4f csc[NG][2][4];  // column scales: [0] gate / [1] up of a paired group, or the two fragments of a plain one
+        if (!FP8 && a.epilogue != kEpiInt32) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (a.epilogue == kEpiSwiglu) {
-                csc[0][j] = *(const v4f *)(t.sg + t.nw * 32 + 8 * j + col_half);
-                csc[1][j] = *(const v4f *)(t.sg + t.N / 2 + t.nw * 32 + 8 * j + col_half);
-            } else {
-                csc[0][j] = *(const v4f *)(t.sg + t.nw * 64 + 8 * j + col_half);
-                csc[1][j] = *(const v4f *)(t.sg + t.nw * 64 + 32 + 8 * j + col_half);
-            }
-        }
-    }
-    if (FLAT) {
-        between_sink = between();
-    }
-    if (work) {
-        const int wave = tid >> 6;
-        const int row_in = lane & 31;
-        const int col_half = (lane >> 5) * 4;
-        int8_t *slice = lds + wave * kEpiSlice;
-        const int N = t.N;
-        const int nw = t.nw;
-
-        // Copies rows [0, 32) of the slice (128 bytes each) to dst + (first + row) * row_pitch_bytes.
-        auto flush_fragment = [&](int8_t *dst, long long row_pitch_bytes, int mf) {
-            const int sub = lane >> 3;    // row inside a group of 8
-            const int piece = lane & 7;   // 16-byte piece of the 128-byte row
-#pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                const int row = it * 8 + sub;
-                const v4u v = *(const v4u *)(slice + row * kEpiRowBytes + piece * 16);
-                const int trow = mf * 32 + row;
-                if (trow < t.my_rows) {
-                    // the next kernel reads these rows once; stored non-temporally they do not push weight panels
-                    // and activation tiles out of the L2 (C3 both operators 519 -> 506 us, decode layer 427 -> 420 us)
-                    __builtin_nontemporal_store(v, (v4u *)(dst + (long long)(t.m0 + t.a_row0 + trow) * row_pitch_bytes + piece * 16));
-                }
-            }
-        };
-
-        if (a.epilogue == kEpiInt32) {
-#pragma unroll
-            for (int nf = 0; nf < 2; ++nf) {
-                const int col0 = a.gate_up ? (nf * (N / 2) + nw * 32) : (nw * 64 + nf * 32);
-#pragma unroll
-                for (int mf = 0; mf < MF; ++mf) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        // int32 sums, or the bits of the fp32 sums of an FP8 item
-                        const v4i v = {acc_bits(acc[mf][nf][4 * j]), acc_bits(acc[mf][nf][4 * j + 1]),
-                                       acc_bits(acc[mf][nf][4 * j + 2]), acc_bits(acc[mf][nf][4 * j + 3])};
-                        *(v4i *)(slice + row_in * kEpiRowBytes + (8 * j + col_half) * 4) = v;
-                    }
-                    flush_fragment((int8_t *)a.out + (long long)col0 * 4, (long long)N * 4, mf);
-                }
-            }
-        } else if (a.epilogue == kEpiSwiglu) {
-            // t = (float(C) * w_scale[n]) * x_scale[m]; y = silu(t_gate) * t_up
-            const int I = N / 2;
-            v4f sg_gate[4], sg_up[4];
-            if (!FP8) {
+            for (int gi = 0; gi < NG; ++gi) {
+                const int nw = min(t.group + gi, ngroups - 1);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    if (FLAT) {
-                        sg_gate[j] = csc[0][j];
-                        sg_up[j] = csc[1][j];
+                    if (a.epilogue == kEpiSwiglu) {
+                        csc[gi][0][j] = *(const v4f *)(t.sg + nw * 32 + 8 * j + col_half);
+                        csc[gi][1][j] = *(const v4f *)(t.sg + N / 2 + nw * 32 + 8 * j + col_half);
                     } else {
-                        sg_gate[j] = *(const v4f *)(t.sg + nw * 32 + 8 * j + col_half);
-                        sg_up[j] = *(const v4f *)(t.sg + I + nw * 32 + 8 * j + col_half);
+                        csc[gi][0][j] = *(const v4f *)(t.sg + nw * 64 + 8 * j + col_half);
+                        csc[gi][1][j] = *(const v4f *)(t.sg + nw * 64 + 32 + 8 * j + col_half);
                     }
                 }
-            }
-#pragma unroll
-            for (int mf = 0; mf < MF; ++mf) {
-                const float xs = FP8 ? 1.0f : row_scale_s[t.a_row0 + mf * 32 + row_in];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    v4f y;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float tg, tu;
-                        if constexpr (FP8) {  // the sums carry their scales already
-                            tg = acc[mf][0][4 * j + e];
-                            tu = acc[mf][1][4 * j + e];
-                        } else {
-                            tg = __fmul_rn(__fmul_rn((float)acc[mf][0][4 * j + e], sg_gate[j][e]), xs);
-                            tu = __fmul_rn(__fmul_rn((float)acc[mf][1][4 * j + e], sg_up[j][e]), xs);
-                        }
-                        y[e] = __fmul_rn(cam_silu_spec(tg), tu);
-                    }
-                    *(v4f *)(slice + row_in * kEpiRowBytes + (8 * j + col_half) * 4) = y;
-                }
-                flush_fragment((int8_t *)a.out + (long long)(nw * 32) * 4, (long long)I * 4, mf);
-            }
-        } else {
-            v4f ws[2][4];
-            if (!FP8) {
-#pragma unroll
-                for (int nf = 0; nf < 2; ++nf) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        ws[nf][j] = FLAT ? csc[nf][j] : *(const v4f *)(t.sg + nw * 64 + nf * 32 + 8 * j + col_half);
-                    }
-                }
-            }
-#pragma unroll
-            for (int mf = 0; mf < MF; ++mf) {
-                const float xs = FP8 ? 1.0f : row_scale_s[t.a_row0 + mf * 32 + row_in];
-#pragma unroll
-                for (int nf = 0; nf < 2; ++nf) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        float f[4];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            if constexpr (FP8) {
-                                f[e] = acc[mf][nf][4 * j + e];
-                            } else {
-                                f[e] = __fmul_rn(__fmul_rn((float)acc[mf][nf][4 * j + e], ws[nf][j][e]), xs);
-                            }
-                        }
-                        // two values per conversion instruction: with the rounding spelled out in integer
-                        // arithmetic this epilogue took a quarter of a short-K tile's time in the vector ALU
-                        v2u v;
-                        if (a.out_fp16) {
-                            v = v2u{f32_to_fp16_bits(f[0]) | (f32_to_fp16_bits(f[1]) << 16),
-                                    f32_to_fp16_bits(f[2]) | (f32_to_fp16_bits(f[3]) << 16)};
-                        } else {
-                            v = v2u{f32x2_to_bf16x2_bits(f[0], f[1]), f32x2_to_bf16x2_bits(f[2], f[3])};
-                        }
-                        *(v2u *)(slice + row_in * kEpiRowBytes + (nf * 32 + 8 * j + col_half) * 2) = v;
-                    }
-                }
-                flush_fragment((int8_t *)a.out + (long long)(nw * 64) * 2, (long long)N * 2, mf);
             }
         }
-    }
+        if (FLAT) {
+            between_sink = between();
+        }
+        static_for<0, NG>([&](auto gc) {
+            constexpr int gi = decltype(gc)::value;
+            const int nw = t.group + gi;
+            if (nw >= ngroups) {
+                return;
+            }
+            if (a.epilogue == kEpiInt32) {
+                static_for<0, 2>([&](auto nc) {
+                    constexpr int nf = decltype(nc)::value;
+                    const int col0 = a.gate_up ? (nf * (N / 2) + nw * 32) : (nw * 64 + nf * 32);
+                    const __amdgpu_buffer_rsrc_t out = columns(col0 * 4, N * 4);
+                    blocks([&](auto qc) {
+                        static_for<0, 4>([&](auto jc) {
+                            constexpr int j = decltype(jc)::value;
+                            constexpr int r = (decltype(qc)::value * NF + 2 * gi + nf) * 16 + 4 * j;
+                            // int32 sums, or the bits of the fp32 sums of an FP8 item
+                            const v4i v = {acc_bits<r>(), acc_bits<r + 1>(), acc_bits<r + 2>(), acc_bits<r + 3>()};
+                            *(v4i *)(slice + row_in * kEpiRowBytes + (8 * j + col_half) * 4) = v;
+                        });
+                    }, [&](int mf, const v4u (&v)[4]) { store_rows(out, N * 4, mf, v); });
+                });
+            } else if (a.epilogue == kEpiSwiglu) {
+                // t = (float(C) * w_scale[n]) * x_scale[m]; y = silu(t_gate) * t_up
+                const __amdgpu_buffer_rsrc_t out = columns(nw * 32 * 4, N * 2);
+                blocks([&](auto qc) {
+                    constexpr int mf = decltype(qc)::value;
+                    const float xs = FP8 ? 1.0f : row_scale_s[mf * 32 + row_in];
+                    static_for<0, 4>([&](auto jc) {
+                        constexpr int j = decltype(jc)::value;
+                        v4f y;
+                        static_for<0, 4>([&](auto ec) {
+                            constexpr int e = decltype(ec)::value;
+                            constexpr int r = (mf * NF + 2 * gi) * 16 + 4 * j + e;
+                            float tg = acc_value<r, FP8>(), tu = acc_value<r + 16, FP8>();
+                            if constexpr (!FP8) {  // (FP8: the sums carry their scales already)
+                                tg = __fmul_rn(__fmul_rn(tg, csc[gi][0][j][e]), xs);
+                                tu = __fmul_rn(__fmul_rn(tu, csc[gi][1][j][e]), xs);
+                            }
+                            y[e] = __fmul_rn(cam_silu_spec(tg), tu);
+                        });
+                        *(v4f *)(slice + row_in * kEpiRowBytes + (8 * j + col_half) * 4) = y;
+                    });
+                }, [&](int mf, const v4u (&v)[4]) { store_rows(out, N * 2, mf, v); });
+            } else {
+                const __amdgpu_buffer_rsrc_t out = columns(nw * 64 * 2, N * 2);
+                auto dequant = [&](auto fp16) {
+                    blocks([&](auto qc) {
+                        constexpr int mf = decltype(qc)::value;
+                        const float xs = FP8 ? 1.0f : row_scale_s[mf * 32 + row_in];
+                        static_for<0, 8>([&](auto jc) {
+                            constexpr int nf = decltype(jc)::value / 4, j = decltype(jc)::value % 4;
+                            float f[4];
+                            static_for<0, 4>([&](auto ec) {
+                                constexpr int e = decltype(ec)::value;
+                                f[e] = acc_value<(mf * NF + 2 * gi + nf) * 16 + 4 * j + e, FP8>();
+                                if constexpr (!FP8) {
+                                    f[e] = __fmul_rn(__fmul_rn(f[e], csc[gi][nf][j][e]), xs);
+                                }
+                            });
+                            // two values per conversion instruction: with the rounding spelled out in integer
+                            // arithmetic this epilogue took a quarter of a short-K tile's time in the vector ALU
+                            v2u v;
+                            if constexpr (decltype(fp16)::value) {
+                                // each product rounded to fp32 first: the compiler would make one instruction of the
+                                // multiplication and the conversion, with one rounding
+                                asm("" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]));
+                                v = v2u{f32_to_fp16_bits(f[0]) | (f32_to_fp16_bits(f[1]) << 16),
+                                        f32_to_fp16_bits(f[2]) | (f32_to_fp16_bits(f[3]) << 16)};
+                            } else {
+                                v = v2u{f32x2_to_bf16x2_bits(f[0], f[1]), f32x2_to_bf16x2_bits(f[2], f[3])};
+                            }
+                            *(v2u *)(slice + row_in * kEpiRowBytes + (nf * 32 + 8 * j + col_half) * 2) = v;
+                        });
+                    }, [&](int mf, const v4u (&v)[4]) { store_rows(out, N * 2, mf, v); });
+                };
+                if (a.out_fp16) {
+                    dequant(std::true_type());
+                } else {
+                    dequant(std::false_type());
+                }
+            }
+        });
     };
 
     // ---- FP8 gate/up GEMM whose output feeds the next FP8 GEMM: quantise the SwiGLU product here.  A block of
-    // 128 product columns is exactly what the four waves of a team hold for their rows (32 columns each), so the
-    // block maximum needs one exchange through LDS; every wave of the workgroup takes part in its barrier.
+    // 128 product columns is what four neighbouring column groups hold (the four waves of a tall item, two waves of a
+    // flat one), so the block maximum needs one exchange through LDS; every wave of the workgroup takes part in its barrier.
     auto epilogue_quant = [&]() {
         if (FLAT) {
             between_sink = between();
         }
-        const bool work = MF > 0 && t.wave_live;
-        const int wave = tid >> 6;
-        const int row_in = lane & 31;
-        const int col_half = (lane >> 5) * 4;
-        float *rowmax = (float *)(lds + 8 * kEpiSlice);  // [wave][tile row of the wave's fragments]
         if constexpr (FP8) {
-            if (work) {
-#pragma unroll
-                for (int mf = 0; mf < MF; ++mf) {
-                    float m = 0.0f;
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const float y = __fmul_rn(cam_silu_spec(acc[mf][0][i]), acc[mf][1][i]);
-                        acc[mf][0][i] = y;
-                        m = fmaxf(m, fabsf(y));
-                    }
-                    m = fmaxf(m, __shfl_xor(m, 32, kWave));
-                    if (lane < 32) {
-                        rowmax[wave * 128 + mf * 32 + lane] = m;
-                    }
+            float *rowmax = (float *)(lds + 4 * kEpiSlice);  // [wave][tile row]
+            float y[MF][NG][16];
+            static_for<0, MF>([&](auto mc) {
+                constexpr int mf = decltype(mc)::value;
+                if (mf >= n) {
+                    return;
                 }
-            }
+                float m = 0.0f;
+                static_for<0, NG * 16>([&](auto ic) {
+                    constexpr int gi = decltype(ic)::value / 16, i = decltype(ic)::value % 16;
+                    constexpr int r = (mf * NF + 2 * gi) * 16 + i;
+                    y[mf][gi][i] = __fmul_rn(cam_silu_spec(acc_value<r, true>()), acc_value<r + 16, true>());
+                    m = fmaxf(m, fabsf(y[mf][gi][i]));
+                });
+                m = fmaxf(m, __shfl_xor(m, 32, kWave));
+                if (lane < 32) {
+                    rowmax[wave * 256 + mf * 32 + lane] = m;
+                }
+            });
             wait_lds_reads();
             barrier_no_fence();
-            if (work) {
-                const int I = t.N / 2;
-                int8_t *slice = lds + wave * kEpiSlice;
-                uint8_t *q = (uint8_t *)a.out;
+            if (t.group >= ngroups) {
+                return;
+            }
+            const int I = N / 2;
+            // 32 rows x 32 bytes per column group (48-byte pitch in the slice): two lanes per row store its two 16-byte halves
+            const int qrow = lane >> 1, qpiece = lane & 1;
+            const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
+                (int8_t *)a.out + (long long)t.m0 * I + t.group * 32, 0, (unsigned)((t.rows - 1) * I + NG * 32), 0x00020000);
+            v4u held[NG];
+            auto store = [&](int mf) {
 #pragma unroll
-                for (int mf = 0; mf < MF; ++mf) {
-                    const float *pm = rowmax + (wave & 4) * 128 + mf * 32 + row_in;  // the team's four waves
-                    const float m = fmaxf(fmaxf(pm[0], pm[128]), fmaxf(pm[256], pm[384]));
-                    const int ex = fp8_block_scale_exp(m);
-                    const float f1 = exp2_int(-(ex / 2)), f2 = exp2_int(-(ex - ex / 2));
+                for (int gi = 0; gi < NG; ++gi) {
+                    __builtin_amdgcn_raw_buffer_store_b128(held[gi], out, (unsigned)((mf * 32 + qrow) * I + gi * 32 + qpiece * 16),
+                                                           0, 0);
+                }
+            };
+#pragma unroll
+            for (int mf = 0; mf < MF; ++mf) {
+                if (mf >= n) {
+                    break;
+                }
+                const float *pm = rowmax + (FLAT ? (wave & 2) * 256 : 0) + mf * 32 + row_in;
+                const float m = FLAT ? fmaxf(pm[0], pm[256]) : fmaxf(fmaxf(pm[0], pm[256]), fmaxf(pm[512], pm[768]));
+                const int ex = fp8_block_scale_exp(m);
+                const float f1 = exp2_int(-(ex / 2)), f2 = exp2_int(-(ex - ex / 2));
+                int w[NG][4];
+#pragma unroll
+                for (int gi = 0; gi < NG; ++gi) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        int w = 0;
-                        w = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(__fmul_rn(acc[mf][0][4 * j], f1), f2),
-                                                            __fmul_rn(__fmul_rn(acc[mf][0][4 * j + 1], f1), f2), w, false);
-                        w = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(__fmul_rn(acc[mf][0][4 * j + 2], f1), f2),
-                                                            __fmul_rn(__fmul_rn(acc[mf][0][4 * j + 3], f1), f2), w, true);
-                        *(int *)(slice + row_in * 48 + 8 * j + col_half) = w;
-                    }
-                    // 32 rows x 32 bytes staged (48-byte pitch): two lanes per row write its two 16-byte halves
-                    const int row = lane >> 1, piece = lane & 1;
-                    const v4u v = *(const v4u *)(slice + row * 48 + piece * 16);
-                    if (mf * 32 + row < t.my_rows) {
-                        const long long grow = t.m0 + t.a_row0 + mf * 32 + row;
-                        *(v4u *)(q + grow * I + t.nw * 32 + piece * 16) = v;
-                    }
-                    if ((wave & 3) == 0 && lane < 32 && mf * 32 + lane < t.my_rows) {
-                        const long long grow = t.m0 + t.a_row0 + mf * 32 + lane;
-                        a.out_scale8[grow * (I >> 7) + (t.nw >> 2)] = (uint8_t)(ex + 127);
+                        const float *c = y[mf][gi] + 4 * j;
+                        w[gi][j] = 0;
+                        w[gi][j] = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(__fmul_rn(c[0], f1), f2),
+                                                                   __fmul_rn(__fmul_rn(c[1], f1), f2), w[gi][j], false);
+                        w[gi][j] = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(__fmul_rn(c[2], f1), f2),
+                                                                   __fmul_rn(__fmul_rn(c[3], f1), f2), w[gi][j], true);
                     }
                 }
+                if (mf > 0) {
+                    store(mf - 1);
+                }
+#pragma unroll
+                for (int gi = 0; gi < NG; ++gi) {
+                    int8_t *part = slice + gi * (kEpiSlice / 2);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        *(int *)(part + row_in * 48 + 8 * j + col_half) = w[gi][j];
+                    }
+                    held[gi] = *(const v4u *)(part + qrow * 48 + qpiece * 16);
+                }
+                if ((FLAT ? (wave & 1) : wave) == 0 && lane < 32 && mf * 32 + lane < t.rows) {
+                    const long long grow = t.m0 + mf * 32 + lane;
+                    a.out_scale8[grow * (I >> 7) + (t.group >> 2)] = (uint8_t)(ex + 127);
+                }
             }
+            store(n - 1);
         }
     };
 
@@ -626,20 +762,6 @@ __device__ __forceinline__ void run_item(const GemmArgs &a, const ItemCtx &t, in
     }
     barrier_no_fence();  // the staging slices are free again before the next item's loads land
     asm volatile("" ::"v"(between_sink));
-}
-
-template <int TEAM, bool FLAT, bool FP8, typename Hook, typename Stage>
-__device__ __forceinline__ void run_item_mf(int mf, const GemmArgs &a, const ItemCtx &t, int nb, int8_t *lds,
-                                            const float *row_scale_s, const uint8_t *a_scale8_s,
-                                            const uint8_t *w_scale8_s, Hook &between, Stage &stage_scales)
-{
-    switch (mf) {
-        case 0: run_item<0, TEAM, FLAT, FP8>(a, t, nb, lds, row_scale_s, a_scale8_s, w_scale8_s, between, stage_scales); break;
-        case 1: run_item<1, TEAM, FLAT, FP8>(a, t, nb, lds, row_scale_s, a_scale8_s, w_scale8_s, between, stage_scales); break;
-        case 2: run_item<2, TEAM, FLAT, FP8>(a, t, nb, lds, row_scale_s, a_scale8_s, w_scale8_s, between, stage_scales); break;
-        case 3: run_item<3, TEAM, FLAT, FP8>(a, t, nb, lds, row_scale_s, a_scale8_s, w_scale8_s, between, stage_scales); break;
-        default: run_item<4, TEAM, FLAT, FP8>(a, t, nb, lds, row_scale_s, a_scale8_s, w_scale8_s, between, stage_scales); break;
-    }
 }
 
 template <bool FP8>
@@ -656,8 +778,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
 #endif
 
     const int tid = threadIdx.x;
-    const int team = __builtin_amdgcn_readfirstlane(tid >> 8);
-    const int wn = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int32_t *sched = a.sched;
     const int32_t *qstart = sched + kSchedQueueStart;
     int32_t *qcount = sched + kSchedQueueCount;
@@ -764,7 +885,6 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
         const int g = __builtin_amdgcn_readfirstlane(it.g);
         const int m0 = __builtin_amdgcn_readfirstlane(it.m0);
         const int rows = __builtin_amdgcn_readfirstlane(it.rows);
-        const int split = __builtin_amdgcn_readfirstlane(it.split);
         const int nb = __builtin_amdgcn_readfirstlane(it.nb);
         const bool flat = __builtin_amdgcn_readfirstlane(it.flat) != 0;
 
@@ -779,22 +899,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
         t.a_tile = a.a + (long long)m0 * a.Kd;
         t.wg = a.per_expert ? a.list.w[g] : a.w + (long long)g * a.Kd * a.N;
         t.sg = a.per_expert ? a.list.s[g] : a.w_scale + (long long)g * a.N;
-        if (flat) {
-            t.a_row0 = 0;
-            t.my_rows = rows;
-            t.bslot = team * 4 + wn;
-            t.stage_a = 128 * kBK;
-            t.stage_bytes = kStageFlat;
-        } else {
-            t.a_row0 = team == 0 ? 0 : split;
-            t.my_rows = team == 0 ? min(split, rows) : rows - split;
-            t.bslot = wn;
-            t.stage_a = 256 * kBK;
-            t.stage_bytes = kStageTall;
-        }
-        const int group = nb * (flat ? 8 : 4) + t.bslot;
-        t.wave_live = group < a.N / 64;
-        t.nw = min(group, a.N / 64 - 1);
+        t.group = flat ? nb * 8 + 2 * wave : nb * 4 + wave;
         auto stage_scales = [&]() {
             if (FP8) {
                 // the item's scales: activation rows x K blocks (transposed, so that the lanes of a fragment read
@@ -864,47 +969,53 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
                 const int nm0 = __builtin_amdgcn_readfirstlane(nx.m0);
                 const int nrows = __builtin_amdgcn_readfirstlane(nx.rows);
                 const int nnb = __builtin_amdgcn_readfirstlane(nx.nb);
-                const bool nflat = __builtin_amdgcn_readfirstlane(nx.flat) != 0;
-                const int stages = nflat ? 3 : 4;
                 const int lane = tid & (kWave - 1);
-                if (nflat || team == 1) {  // the waves that load weights: 4 KB per stage and wave
-                    const int8_t *wgn = a.per_expert ? a.list.w[ng] : a.w + (long long)ng * a.Kd * a.N;
-                    const int ngroups = a.N / 64;
-                    const int grp = min(nnb * (nflat ? 8 : 4) + (nflat ? team * 4 + wn : wn), ngroups - 1);
+                const int8_t *wgn = a.per_expert ? a.list.w[ng] : a.w + (long long)ng * a.Kd * a.N;
+                const int ngroups = a.N / 64;
+                const int steps = min(3, a.Kd / kBK);
+#pragma unroll
+                for (int gi = 0; gi < 2; ++gi) {
+                    const int grp = min(nnb * 8 + 2 * wave + gi, ngroups - 1);
                     const int blk = grp >> 3;
                     const long long step = (long long)min(8, ngroups - 8 * blk) * 4096;
                     const int8_t *base = wgn + (long long)blk * 8 * a.Kd * 64 + (grp & 7) * 4096;
-                    const int steps = min(stages, a.Kd / kBK);
                     for (int i = lane; i < steps * 32; i += kWave) {  // 32 lines per stage
                         sink ^= *(const int *)(base + (long long)(i >> 5) * step + (i & 31) * 128);
                     }
                 }
-                if (team == 0) {  // the waves that load activations: rows of 64 bytes per stage
-                    const int per_wave = nflat ? 32 : 64;
-                    const int span = min(stages * kBK, a.Kd);          // bytes of a row the first stages cover
-                    const int lines = (span + 127) / 128;
-                    for (int i = lane; i < per_wave * lines; i += kWave) {
-                        const int r = min(per_wave * wn + i / lines, nrows - 1);
-                        sink ^= *(const int *)(a.a + (long long)(nm0 + r) * a.Kd + (i % lines) * 128);
-                    }
+                const int span = min(3 * kBK, a.Kd);          // bytes of a row the first stages cover
+                const int lines = (span + 127) / 128;
+                for (int i = lane; i < 32 * lines; i += kWave) {
+                    const int r = min(32 * wave + i / lines, nrows - 1);
+                    sink ^= *(const int *)(a.a + (long long)(nm0 + r) * a.Kd + (i % lines) * 128);
                 }
             }
             return sink;
         };
 
-        const int mf = t.my_rows <= 0 ? 0 : (t.my_rows + 31) >> 5;
+        const int mf = (rows + 31) >> 5;
+        auto run = [&](auto mc, auto nc) {
+            k_loop<decltype(mc)::value, decltype(nc)::value, FP8>(t, lds, a_scale8_s, w_scale8_s, stage_scales);
+        };
         if (flat) {
-            if (team == 0) {
-                run_item_mf<0, true, FP8>(mf, a, t, nb, lds, row_scale_s, a_scale8_s, w_scale8_s, between, stage_scales);
-            } else {
-                run_item_mf<1, true, FP8>(mf, a, t, nb, lds, row_scale_s, a_scale8_s, w_scale8_s, between, stage_scales);
+            const std::integral_constant<int, 4> nf;
+            switch (mf) {
+                case 1: run(std::integral_constant<int, 1>(), nf); break;
+                case 2: run(std::integral_constant<int, 2>(), nf); break;
+                case 3: run(std::integral_constant<int, 3>(), nf); break;
+                default: run(std::integral_constant<int, 4>(), nf); break;
             }
+            epilogue_item<4, FP8>(a, t, mf, lds, row_scale_s, between);
         } else {
-            if (team == 0) {
-                run_item_mf<0, false, FP8>(mf, a, t, nb, lds, row_scale_s, a_scale8_s, w_scale8_s, between, stage_scales);
-            } else {
-                run_item_mf<1, false, FP8>(mf, a, t, nb, lds, row_scale_s, a_scale8_s, w_scale8_s, between, stage_scales);
+            const std::integral_constant<int, 2> nf;
+            switch (mf) {
+                case 5: run(std::integral_constant<int, 5>(), nf); break;
+                case 6: run(std::integral_constant<int, 6>(), nf); break;
+                case 7: run(std::integral_constant<int, 7>(), nf); break;
+                case 8: run(std::integral_constant<int, 8>(), nf); break;
+                default: run(std::integral_constant<int, 4>(), nf); break;
             }
+            epilogue_item<2, FP8>(a, t, mf, lds, row_scale_s, between);
         }
 #ifdef CAM_GEMM_TIMELINE
         if (tid == 0) {
@@ -1167,7 +1278,7 @@ hipError_t launch_gemm(const GemmArgs &a, hipStream_t stream)
     if (a.sched == nullptr) {
         return hipErrorInvalidValue;
     }
-    if (a.Kd % kBK != 0 || a.Kd < kBK || a.N % 64 != 0 || (a.gate_up && a.N % 128 != 0)) {
+    if (a.Kd % kStageK != 0 || a.Kd < kStageK || a.N % 64 != 0 || (a.gate_up && a.N % 128 != 0)) {
         return hipErrorInvalidValue;
     }
     int num_cus = 0;
