@@ -1,5 +1,5 @@
-"""The machine code of the tile GEMM, as built here from its source.  Its K loop requests weights into registers from inline assembly
-and waits for them by hand, and it names its accumulation registers itself; both rest on what the compiler makes of the code
+"""The machine code of the tile GEMM, as built here from its source.  Its K loop requests weights (FP8: and their scales) into
+registers from inline assembly and waits for them by hand, and it names its accumulation registers itself; both rest on what the compiler makes of the code
 around them:
   * from a request to the wait that covers it, no instruction on any path reads or writes the registers it loads into;
   * nothing but the multiplications, their clearing and the epilogue's reads touches an accumulation register, and nothing is
@@ -25,12 +25,12 @@ def _registers(text):
 
 
 def _in_flight(code, targets):
-    """Instructions that touch the registers of a 16-byte load of weights (registers, not LDS) which may still be under way."""
+    """Instructions that touch the registers of a load (to registers, not to LDS) which may still be under way."""
     touched = [_registers(text) for text in code]
     waits = [int(m[1]) if (m := re.search(r"vmcnt\((\d+)\)", t)) and t.startswith("s_waitcnt") else None for t in code]
     found = []
     for start, text in enumerate(code):
-        if not re.match(r"buffer_load_dwordx4 v\[", text) or text.endswith("lds"):
+        if not re.match(r"(buffer|global)_load_\w+ v", text) or "_lds_" in text or text.endswith("lds"):
             continue
         dst = _registers(text.split(",")[0])
         todo, seen = [(start + 1, 0)], set()

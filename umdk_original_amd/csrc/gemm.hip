@@ -46,10 +46,12 @@
 //     stored.  For GMM1 the prepack pairs gate column c with up column I+c inside one wave.
 //   * The K order inside a 32-deep MFMA step is whatever the two operands agree on (an integer dot
 //     product does not care), which is what lets both be loaded as plain 16-byte pieces.
-//   * Flat items are bound by the memory, and two things in this file exist for them alone: their weight panels are
-//     fetched with non-temporal loads (nobody else reads them), and between the K loop and the epilogue of a flat item
-//     the workgroup takes its next item and, if that is flat too, touches the lines of its first stages so that they
-//     travel to L2 under the epilogue.
+//   * Flat items are bound by the memory; their weight panels are fetched with non-temporal loads (nobody else reads them).
+//   * Between two items.  What a workgroup has to know and to fetch before it can multiply is asked for during the item before
+//     (ask_ahead, publish): from an item's start to its first multiplication it is 2 us instead of 4, of which the
+//     requests for the weights take most.  Layers of 8192 / 1021 tokens 1567 -> 1535 / 181 -> 176 us, FP8 layer of 4093
+//     tokens 850 -> 828.  Loading a word of every line of a flat item's first sub-steps under the epilogue as well, to have
+//     them in L2, cost the layer of 1021 tokens 1 % with one sub-step, 3 % with three and 8 % with ten.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -108,13 +110,32 @@ __device__ __forceinline__ void dma16(v4i words, unsigned voff, unsigned soff, u
     }
 }
 
-template <int LDS_OFFSET>
-__device__ __forceinline__ void dma16(const void *base, unsigned voff, unsigned lds_addr)
+// A wave-uniform address the compiler does not know to be one, as a scalar register pair.
+__device__ __forceinline__ unsigned long long scalar_address(const void *p)
 {
-    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds_addr), "v"(voff), "s"((unsigned long long)base), "n"(LDS_OFFSET)
-                 : "memory", "m0", "scc");
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// (base and lds_addr: scalar registers already, see scalar_address)
+__device__ __forceinline__ void dma16(unsigned long long base, unsigned voff, unsigned lds_addr)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(base)
+                 : "memory", "m0");
+}
+
+__device__ __forceinline__ unsigned lds_address(const void *p)
+{
+    return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void *)p;
+}
+
+// The same for 4 bytes per lane.
+__device__ __forceinline__ void dma4(unsigned long long base, unsigned voff, unsigned lds_addr)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_addr), "v"(voff), "s"(base)
+                 : "memory", "m0");
 }
 
 // 16 bytes per lane to registers.  STREAM: marked non-temporal, for bytes that are read once: a stream of them moves at
@@ -165,8 +186,11 @@ struct ItemCtx {
     const int8_t *a_tile;   // first activation row of the tile
     const int8_t *wg;       // the expert's packed weights
     const float *sg;        // the expert's per-channel scales
-    int m0, rows;           // first row and rows of the tile
+    int g, m0, rows;        // expert, first row and rows of the tile
     int group;              // this wave's first 64-column group of the weight
+    int mf;                 // row fragments the K loop runs on
+    bool flat;
+    int buf;                // which of the two scale buffers
     int Kd, N;
 #ifdef CAM_GEMM_TIMELINE
     int *phase_s;           // LDS: wall clock at the first multiply and after the K loop (written by thread 0)
@@ -280,11 +304,14 @@ struct FragType<true> {
 //
 // FP8: v_mfma_scale_f32_32x32x64_f8f6f4 covers the 64 K bytes of a sub-step (the two 16-byte pieces a lane holds), takes the E8M0
 // scale of the lane's weight column block and of its activation row for the current 128-byte K block, and accumulates in fp32.
-// The scales of the item wait in LDS (a_scale8_s[kb * 256 + tile row], w_scale8_s[column fragment of the item * kScaleKb +
-// kb]).
-template <int MF, int NF, bool FP8, typename Stage>
-__device__ __forceinline__ void k_loop(const ItemCtx &t, int8_t *lds, const uint8_t *a_scale8_s,
-                                       const uint8_t *w_scale8_s, Stage &stage_scales)
+// The scales of the rows wait in LDS (a_scale8_s), those of the wave's column fragments, one byte per fragment and K block, in a
+// register each (lane kb holds K block kb).
+//
+// The item's first two stages and its row scales have been requested (ask_ahead in gemm_kernel).  `publish` runs between the
+// requests and the wait for them.
+template <int MF, int NF, bool FP8, typename Publish>
+__device__ __forceinline__ void k_loop(const GemmArgs &a, const ItemCtx &t, int8_t *lds, const uint8_t *a_scale8_s,
+                                       Publish &publish)
 {
     constexpr bool STREAM = NF == 4;                // a flat item is the only reader of its weight panel
     constexpr int SLOTS = FP8 ? MF : 2 * MF;
@@ -298,13 +325,12 @@ __device__ __forceinline__ void k_loop(const ItemCtx &t, int8_t *lds, const uint
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ST = t.Kd / kStageK;
     const int KT = 2 * ST;
-    const unsigned lds0 = (unsigned)(unsigned long long)(__attribute__((address_space(3))) int8_t *)lds;
+    const unsigned lds0 = lds_address(lds);
 
     // ---- activations: wave w brings tile rows 8 MF w .. 8 MF (w + 1) - 1, eight rows a load.  Lane i of a load brings row i / 8
     // of its eight and the 16-byte chunk whose swizzled slot is i % 8: chunk c of row r lies at slot c ^ (r / 2 % 8) of the
     // row's 128 bytes, so that sixteen neighbouring rows cover all 64 banks.  Rows beyond the tile are out of the
-    // descriptor's range, which the vector offset is checked against, and come as zeros; the first two stages, which are
-    // requested by address, repeat the last row there, and the last chunk of a row where K ends.
+    // descriptor's range, which the vector offset is checked against, and come as zeros.
     const v4i a_words = buffer_words(t.a_tile, (unsigned)t.rows * (unsigned)t.Kd);
     const unsigned a_dst = lds0 + (unsigned)(wave * (MF * 1024));
     unsigned a_voff[MF];
@@ -314,15 +340,6 @@ __device__ __forceinline__ void k_loop(const ItemCtx &t, int8_t *lds, const uint
         const int c16 = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
         a_voff[j] = (unsigned)(r * t.Kd + c16);
     });
-    auto bring_first = [&](int s) {
-        static_for<0, MF>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
-            const int r = 8 * (wave * MF + j) + (lane >> 3);
-            const int c16 = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
-            const unsigned voff = (unsigned)(min(r, t.rows - 1) * t.Kd + min(s * kStageK + c16, t.Kd - 16));
-            dma16<j * 1024>(t.a_tile, voff, a_dst + (unsigned)(s * kStage));
-        });
-    };
     auto bring = [&](int s, auto jc, auto wc) {  // load j of stage s
         constexpr int j = decltype(jc)::value;
         v4i words = a_words;
@@ -377,35 +394,52 @@ __device__ __forceinline__ void k_loop(const ItemCtx &t, int8_t *lds, const uint
             dst = *(const v4i *)(lds + slot * kStage + (fbase ^ (u * 64 + (i / MF) * 32)) + (i % MF) * 4096);
         }
     };
+    int w_scale[FP8 ? NF : 1];
     auto read_scales = [&](int b, int s) {
         if constexpr (FP8) {
             const int kb = min(s, ST - 1);
 #pragma unroll
             for (int nf = 0; nf < NF; ++nf) {
-                sw[b][nf] = w_scale8_s[(wave * NF + nf) * kScaleKb + kb];
+                // moved here, well before the multiplication that reads it
+                asm volatile("v_mov_b32 %0, %1" : "=v"(sw[b][nf]) : "s"(__builtin_amdgcn_readlane(w_scale[nf], kb)));
             }
 #pragma unroll
             for (int mf = 0; mf < MF; ++mf) {
-                sa[b][mf] = a_scale8_s[kb * 256 + mf * 32 + (lane & 31)];
+                sa[b][mf] = a_scale8_s[((kb >> 2) * 256 + mf * 32 + (lane & 31)) * 4 + (kb & 3)];
             }
         }
     };
 
     // ---- pipeline.  The first requests go out in the order the loop would have sent them in.
+    if constexpr (FP8) {
+        const int KB = t.Kd >> 7, nblk = t.N >> 7;
+        const unsigned voff = (unsigned)(min(lane, KB - 1) * nblk);
+#pragma unroll
+        for (int nf = 0; nf < NF; ++nf) {
+            const int grp = nf < 2 ? nw0 : nw1, f = nf & 1;
+            // first logical column of the fragment (a paired group holds 32 gate and 32 up columns)
+            const int col = a.gate_up ? f * (t.N / 2) + grp * 32 : grp * 64 + f * 32;
+            const uint8_t *base = a.w_scale8 + (long long)t.g * KB * nblk + (col >> 7);
+            asm volatile("s_nop 4\n\tglobal_load_ubyte %0, %1, %2"
+                         : "=v"(w_scale[nf]) : "v"(voff), "s"((unsigned long long)base) : "memory");
+        }
+    }
     const std::true_type waits;
-    bring_first(0);
-    bring_first(1);
     static_for<0, NB>([&](auto j) { request(ring[0], 0, j, waits); });
     static_for<0, kHalf>([&](auto j) { bring(2, j, waits); });
     static_for<0, NB>([&](auto j) { request(ring[1], 1, j, waits); });
     static_for<kHalf, MF>([&](auto j) { bring(2, j, waits); });
     static_for<0, NB>([&](auto j) { request(ring[2], 2, j, waits); });
-    // The item's scales go to LDS now, behind the requests for the first stages, so that their round trip to
-    // memory runs beside that of the weights instead of ahead of it.
-    stage_scales();
     static_for<0, MF * NF>([&](auto tc) { acc_clear<decltype(tc)::value>(); });
+    publish();
     wait_lds_reads();
     landed(ring[0]);
+    if constexpr (FP8) {
+#pragma unroll
+        for (int nf = 0; nf < NF; ++nf) {
+            asm volatile("" : "+v"(w_scale[nf]));
+        }
+    }
     barrier_no_fence();
 #ifdef CAM_GEMM_TIMELINE
     if (tid == 0) {
@@ -486,7 +520,7 @@ __device__ __forceinline__ void k_loop(const ItemCtx &t, int8_t *lds, const uint
     }
     wait_lds_reads();
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products are in their registers
-    barrier_no_fence();  // nobody reads or fills the stages any more: the epilogue may stage through them
+    barrier_no_fence();  // nobody reads or fills the stages any more
 #ifdef CAM_GEMM_TIMELINE
     if (tid == 0) {
         t.phase_s[1] = (int)wall_clock64();
@@ -497,9 +531,12 @@ __device__ __forceinline__ void k_loop(const ItemCtx &t, int8_t *lds, const uint
 // The epilogue of an item, for one wave: n row fragments x NF column fragments, sums in tiles mf * NF + nf.  One function for all
 // numbers of row fragments: it is long straight-line code (the sums are named registers), and a copy for each of them would
 // not stay in the instruction cache, which a CU shares with its neighbour.
-template <int NF, bool FP8, typename Hook>
-__device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &t, int n, int8_t *lds, const float *row_scale_s,
-                                              Hook &between)
+//
+// row_scale and col_scale: the item's scales in LDS, the columns by group of the item.  The stages 0 and 1 of the ring belong to the
+// next item by now; what is staged here goes through the other two.
+template <int NF, bool FP8>
+__device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &t, int8_t *lds, const float *row_scale,
+                                              const float *col_scale)
 {
     constexpr bool FLAT = NF == 4;
     constexpr int MF = FLAT ? 4 : 8;
@@ -511,6 +548,7 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
     const int col_half = (lane >> 5) * 4;
     const int N = t.N;
     const int ngroups = N / 64;
+    const int n = (t.rows + 31) >> 5;
 
     // ---- epilogue, accumulators in registers.
     // Lane l holds activation row (l & 31) of each 32x32 fragment; registers 4j .. 4j+3 hold the four
@@ -520,12 +558,8 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
     // it back as 16 bytes per lane and 8 rows per register, and stores it when the next block is computed, so that the
     // round trip through LDS runs under arithmetic (the wave has its SIMD to itself).  Stores past the tile's rows are out of
     // the range of their descriptor.
-    // `between` is the workgroup's business between two items (taking the next one and asking for its first
-    // bytes, see gemm_kernel).  It runs after this wave has requested its column scales and before it uses them,
-    // so that its memory traffic travels under the arithmetic of the epilogue; it returns a value that depends on
-    // what it loaded, consumed at the very end so that nothing waits for those loads earlier.
-    int between_sink = 0;
-    int8_t *slice = lds + wave * kEpiSlice;
+    int8_t *stage = lds + 2 * kStage;
+    int8_t *slice = stage + wave * kEpiSlice;
     const int sub = lane >> 3;    // row inside a group of 8
     const int piece = lane & 7;   // 16-byte piece of the 128-byte row
 
@@ -566,22 +600,9 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
         v4f csc[NG][2][4];  // column scales: [0] gate / [1] up of a paired group, or the two fragments of a plain one
         if (!FP8 && a.epilogue != kEpiInt32) {
 #pragma unroll
-            for (int gi = 0; gi < NG; ++gi) {
-                const int nw = min(t.group + gi, ngroups - 1);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (a.epilogue == kEpiSwiglu) {
-                        csc[gi][0][j] = *(const v4f *)(t.sg + nw * 32 + 8 * j + col_half);
-                        csc[gi][1][j] = *(const v4f *)(t.sg + N / 2 + nw * 32 + 8 * j + col_half);
-                    } else {
-                        csc[gi][0][j] = *(const v4f *)(t.sg + nw * 64 + 8 * j + col_half);
-                        csc[gi][1][j] = *(const v4f *)(t.sg + nw * 64 + 32 + 8 * j + col_half);
-                    }
-                }
+            for (int i = 0; i < NG * 8; ++i) {
+                csc[i >> 3][(i >> 2) & 1][i & 3] = *(const v4f *)(col_scale + (wave * NG + (i >> 3)) * 64 + (i & 7) * 8 + col_half);
             }
-        }
-        if (FLAT) {
-            between_sink = between();
         }
         static_for<0, NG>([&](auto gc) {
             constexpr int gi = decltype(gc)::value;
@@ -609,7 +630,7 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
                 const __amdgpu_buffer_rsrc_t out = columns(nw * 32 * 4, N * 2);
                 blocks([&](auto qc) {
                     constexpr int mf = decltype(qc)::value;
-                    const float xs = FP8 ? 1.0f : row_scale_s[mf * 32 + row_in];
+                    const float xs = FP8 ? 1.0f : row_scale[mf * 32 + row_in];
                     static_for<0, 4>([&](auto jc) {
                         constexpr int j = decltype(jc)::value;
                         v4f y;
@@ -631,7 +652,7 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
                 auto dequant = [&](auto fp16) {
                     blocks([&](auto qc) {
                         constexpr int mf = decltype(qc)::value;
-                        const float xs = FP8 ? 1.0f : row_scale_s[mf * 32 + row_in];
+                        const float xs = FP8 ? 1.0f : row_scale[mf * 32 + row_in];
                         static_for<0, 8>([&](auto jc) {
                             constexpr int nf = decltype(jc)::value / 4, j = decltype(jc)::value % 4;
                             float f[4];
@@ -671,11 +692,8 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
     // 128 product columns is what four neighbouring column groups hold (the four waves of a tall item, two waves of a
     // flat one), so the block maximum needs one exchange through LDS; every wave of the workgroup takes part in its barrier.
     auto epilogue_quant = [&]() {
-        if (FLAT) {
-            between_sink = between();
-        }
         if constexpr (FP8) {
-            float *rowmax = (float *)(lds + 4 * kEpiSlice);  // [wave][tile row]
+            float *rowmax = (float *)(stage + 4 * kEpiSlice);  // [wave][tile row]
             float y[MF][NG][16];
             static_for<0, MF>([&](auto mc) {
                 constexpr int mf = decltype(mc)::value;
@@ -761,20 +779,21 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
         epilogue();
     }
     barrier_no_fence();  // the staging slices are free again before the next item's loads land
-    asm volatile("" ::"v"(between_sink));
 }
 
 template <bool FP8>
 __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
 {
     __shared__ __attribute__((aligned(1024))) int8_t lds[kLdsBytes];
-    __shared__ float row_scale_s[256];
+    // int8: row scales, then column scales (64 per group), of the item at work and of the next one.  FP8: row scales of the item at
+    // work, a word of four K blocks per row: [K block / 4][row].
+    __shared__ __attribute__((aligned(16))) float scale_s[FP8 ? 1 : 2][FP8 ? 4 : 256 + 8 * 64];
     __shared__ __attribute__((aligned(16))) uint8_t a_scale8_s[FP8 ? kScaleKb * 256 : 4];
-    __shared__ uint8_t w_scale8_s[FP8 ? 16 * kScaleKb : 4];
+    __shared__ __attribute__((aligned(16))) SchedItem next_s;
     __shared__ int item_s;
-    __shared__ int next_s;
 #ifdef CAM_GEMM_TIMELINE
     __shared__ int phase_s[2];
+    __shared__ int next_idx_s;
 #endif
 
     const int tid = threadIdx.x;
@@ -791,15 +810,29 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
 
     // Work items.  Short schedules: every workgroup has a queue of its own, built to last as long as the others
     // (sched_device.h).  Its first item is its own without asking; for the following ones it advances its queue's
-    // counter with a device-scope atomic, a round trip to the memory side that is issued at the START of an item
-    // and looked at only when the item is done (take_begin / take_end).  Long schedules: the workgroups of an XCD
-    // share one queue and ask for every item, the first included.  Every counter has a cache line of its own.  A
-    // workgroup whose queue has run out helps the queue with the most items left (its own XCD's first, so that
+    // counter with a device-scope atomic, a round trip to the memory side.  Long schedules: the workgroups of an XCD share one
+    // queue and ask for every item, the first included.  Every counter has a cache line of its own.
+    // The item after the current one is asked for in front of the epilogue before it, its number looked at and its
+    // descriptor requested (to LDS) while the first loads of the current item are on their way, and its own first loads go
+    // out between the K loop and the epilogue of the current item: no item but a workgroup's first starts with a chain of
+    // round trips.
+    // A workgroup whose queue has run out helps the queue with the most items left (its own XCD's first, so that
     // what it fetches is likely to be in its L2): wave 0 looks at every counter at once, one round trip, and its
     // first lane then advances the chosen one.  A counter only ever grows and every queue is finite, so every
     // workgroup leaves.
-    auto take_begin = [&]() -> int {  // thread 0
-        return own_empty ? 0 : atomicAdd(&qcount[me * kSchedQueueStride], 1);
+    int taken = 0;  // thread 0
+    auto take_begin = [&]() {
+        if (tid == 0 && !own_empty) {
+            taken = atomicAdd(&qcount[me * kSchedQueueStride], 1);
+        }
+    };
+    auto take_end = [&]() -> int {  // all threads of wave 0
+        const int i = __builtin_amdgcn_readfirstlane(taken);
+        if (own_empty || i >= qlen) {
+            own_empty = true;
+            return -1;
+        }
+        return q0 + i;
     };
     auto steal = [&]() -> int {  // all lanes of wave 0; the result is valid in every lane
         const int lane = tid & (kWave - 1);
@@ -839,187 +872,170 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
         }
         return -1;
     };
-    // The item after the one whose take was `taken`; called by all threads of wave 0 (the answer is for thread 0).
-    auto take_end = [&](int taken) -> int {
-        taken = __shfl(taken, 0, kWave);
-        if (!own_empty) {
-            if (taken < qlen) {
-                return q0 + taken;
-            }
-            own_empty = true;
-        }
-        return steal();
+
+    auto decode = [&](const SchedItem &it, int buf) {
+        ItemCtx t;
+        t.g = __builtin_amdgcn_readfirstlane(it.g);
+        t.m0 = __builtin_amdgcn_readfirstlane(it.m0);
+        t.rows = __builtin_amdgcn_readfirstlane(it.rows);
+        const int nb = __builtin_amdgcn_readfirstlane(it.nb);
+        t.flat = __builtin_amdgcn_readfirstlane(it.flat) != 0;
+        t.mf = (t.rows + 31) >> 5;
+        t.mf = t.flat ? min(t.mf, 4) : min(max(t.mf, 4), 8);
+        t.group = t.flat ? nb * 8 + 2 * wave : nb * 4 + wave;
+        t.buf = buf;
+        t.Kd = a.Kd;
+        t.N = a.N;
+        t.a_tile = a.a + (long long)t.m0 * a.Kd;
+        t.wg = a.per_expert ? a.list.w[t.g] : a.w + (long long)t.g * a.Kd * a.N;
+        t.sg = a.per_expert ? a.list.s[t.g] : a.w_scale + (long long)t.g * a.N;
+#ifdef CAM_GEMM_TIMELINE
+        t.phase_s = phase_s;
+#endif
+        return t;
     };
 
-    int next = -1;
-    if (tid < kWave) {
-        if (shared) {
-            int taken = 0;
-            if (tid == 0) {
-                taken = take_begin();
+    // The first loads of an item: stages 0 and 1 of its rows and its scales, to LDS.  Rows beyond the tile repeat its last one, what
+    // lies beyond the end of K the last chunk of the row.
+    auto ask_ahead = [&](const ItemCtx &t) {
+        const int lane = opaque(tid) & (kWave - 1);
+        const unsigned long long tile = scalar_address(t.a_tile);
+        const unsigned dst = __builtin_amdgcn_readfirstlane(lds_address(lds) + (unsigned)(wave * t.mf * 1024));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (j < t.mf) {
+                const int r = 8 * (wave * t.mf + j) + (lane >> 3);
+                const int c16 = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+                const int at = min(r, t.rows - 1) * t.Kd;
+                dma16(tile, (unsigned)(at + c16), dst + (unsigned)(j * 1024));
+                dma16(tile, (unsigned)(at + min(kStageK + c16, t.Kd - 16)), dst + (unsigned)(kStage + j * 1024));
             }
-            next = take_end(taken);
-        } else {
-            next = qlen > 0 ? q0 : steal();
         }
-    }
-    for (;;) {
-        if (tid == 0) {
-            item_s = next;
+        const int row = min(wave * kWave + lane, t.rows - 1);
+        const int ngroups = t.N / 64;
+        if constexpr (FP8) {
+            const int KB = t.Kd >> 7;
+            const uint8_t *base = a.a_scale8 + (long long)t.m0 * KB;
+            if ((KB & 3) == 0) {
+                const unsigned long long words = scalar_address(base);
+                const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(a_scale8_s) + (unsigned)(wave * kWave * 4));
+                for (int q = 0; q < KB >> 2; ++q) {
+                    dma4(words, (unsigned)(row * KB + 4 * q), to + (unsigned)(q * 1024));
+                }
+            } else {  // (rows that are no whole words)
+                for (int kb = 0; kb < KB; ++kb) {
+                    a_scale8_s[((kb >> 2) * 256 + wave * kWave + lane) * 4 + (kb & 3)] = base[(long long)row * KB + kb];
+                }
+            }
+        } else if (a.epilogue != kEpiInt32) {
+            const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(scale_s[t.buf]));
+            dma4(scalar_address(a.a_scale + t.m0), (unsigned)(row * 4), to + (unsigned)(wave * kWave * 4));
+            const unsigned long long columns = scalar_address(t.sg);
+            const int per_wave = t.flat ? 2 : 1;
+            for (int gi = 0; gi < per_wave; ++gi) {
+                const int nw = min(t.group + gi, ngroups - 1);
+                const int col = a.gate_up ? (lane >> 5) * (t.N / 2) + nw * 32 + (lane & 31) : nw * 64 + lane;
+                dma4(columns, (unsigned)(col * 4), to + (unsigned)((256 + (wave * per_wave + gi) * 64) * 4));
+            }
+        }
+    };
+
+#ifdef CAM_GEMM_TIMELINE
+    int cur_idx = -1;
+#endif
+    auto first_item = [&](int buf, bool steal_only) -> ItemCtx {  // rows 0: there is none
+        if (tid < kWave) {
+            int idx = -1;
+            if (!steal_only) {
+                if (shared) {
+                    take_begin();
+                    idx = take_end();
+                } else {
+                    idx = qlen > 0 ? q0 : -1;
+                }
+            }
+            idx = idx >= 0 ? idx : steal();
+            if (tid == 0) {
+                item_s = idx;
+            }
         }
         __syncthreads();
-        const int idx = item_s;
-        if (idx < 0) {
-            return;
+        const int idx = __builtin_amdgcn_readfirstlane(item_s);
+        ItemCtx t;
+        t.rows = 0;
+        if (idx >= 0) {
+            t = decode(items[idx], buf);
+            ask_ahead(t);
+#ifdef CAM_GEMM_TIMELINE
+            cur_idx = idx;
+#endif
         }
-        int taken = 0;
-        if (tid == 0) {
-            taken = take_begin();  // in flight while this item runs
-        }
-        SchedItem it = items[idx];
+        return t;
+    };
+    ItemCtx t = first_item(0, false);
+    take_begin();
+    while (t.rows > 0) {
 #ifdef CAM_GEMM_TIMELINE
         // Build option for profiling only: thread 0 leaves the item's start and end times (wall_clock64, 100 MHz)
         // and the workgroup that ran it in the item's two spare words.
         const long long timeline_t0 = wall_clock64();
 #endif
-        const int g = __builtin_amdgcn_readfirstlane(it.g);
-        const int m0 = __builtin_amdgcn_readfirstlane(it.m0);
-        const int rows = __builtin_amdgcn_readfirstlane(it.rows);
-        const int nb = __builtin_amdgcn_readfirstlane(it.nb);
-        const bool flat = __builtin_amdgcn_readfirstlane(it.flat) != 0;
-
-        ItemCtx t;
-#ifdef CAM_GEMM_TIMELINE
-        t.phase_s = phase_s;
-#endif
-        t.Kd = a.Kd;
-        t.N = a.N;
-        t.m0 = m0;
-        t.rows = rows;
-        t.a_tile = a.a + (long long)m0 * a.Kd;
-        t.wg = a.per_expert ? a.list.w[g] : a.w + (long long)g * a.Kd * a.N;
-        t.sg = a.per_expert ? a.list.s[g] : a.w_scale + (long long)g * a.N;
-        t.group = flat ? nb * 8 + 2 * wave : nb * 4 + wave;
-        auto stage_scales = [&]() {
-            if (FP8) {
-                // the item's scales: activation rows x K blocks (transposed, so that the lanes of a fragment read
-                // neighbouring bytes), and one row of K blocks per 64-column group of the item
-                // Only the rows the fragments read (the tile's rows, to the next multiple of 32), and, where a row's
-                // scales are whole words, four K blocks per load and four loads in flight per thread: fetched a byte
-                // at a time for all 256 rows, with a wait per byte, this took 3-4 us of every item.
-                const int KB = a.Kd >> 7;
-                const int rpad = min(256, (rows + 31) & ~31);
-                if ((KB & 3) == 0) {
-                    // a thread takes four K blocks of four consecutive rows: four word loads, a 4x4 byte transpose,
-                    // four word stores (neighbouring lanes write neighbouring words)
-                    const int wpr = KB >> 2;    // words per row
-                    const int rgs = rpad >> 2;  // groups of four rows
-                    for (int i = tid; i < rgs * wpr; i += kThreads) {
-                        const int q = i / rgs, rg = i - q * rgs;
-                        uint32_t v[4];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            v[u] = *(const uint32_t *)(a.a_scale8 + (long long)(m0 + min(4 * rg + u, rows - 1)) * KB + 4 * q);
-                        }
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const uint32_t w = ((v[0] >> (8 * j)) & 0xffu) | (((v[1] >> (8 * j)) & 0xffu) << 8) |
-                                               (((v[2] >> (8 * j)) & 0xffu) << 16) | (((v[3] >> (8 * j)) & 0xffu) << 24);
-                            *(uint32_t *)(a_scale8_s + (4 * q + j) * 256 + 4 * rg) = w;
-                        }
-                    }
-                } else {
-                    for (int i = tid; i < rpad * KB; i += kThreads) {
-                        const int r = i / KB, kb = i - r * KB;
-                        a_scale8_s[kb * 256 + r] = a.a_scale8[(long long)(m0 + min(r, rows - 1)) * KB + kb];
-                    }
-                }
-                const int ngr = flat ? 8 : 4;
-                const int nblk = a.N >> 7;
-                for (int i = tid; i < ngr * 2 * KB; i += kThreads) {
-                    const int gf = i / KB, kb = i - gf * KB;  // gf = column group of the item * 2 + fragment
-                    const int grp = min(nb * ngr + (gf >> 1), a.N / 64 - 1);  // packed 64-column group of the weight
-                    const int nf = gf & 1;
-                    // first logical column of the fragment (a paired group holds 32 gate and 32 up columns)
-                    const int col = a.gate_up ? nf * (a.N / 2) + grp * 32 : grp * 64 + nf * 32;
-                    w_scale8_s[gf * kScaleKb + kb] = a.w_scale8[((long long)g * KB + kb) * nblk + (col >> 7)];
-                }
-            } else if (a.epilogue != kEpiInt32 && tid < 256) {
-                row_scale_s[tid] = a.a_scale[m0 + min(tid, rows - 1)];
-            }
-        };
-
-        // Between the K loop and the epilogue of this item: thread 0 learns which item comes next (its take has
-        // been in flight since this item began), and every wave asks for the first bytes that item will load --
-        // one word of every 128-byte line of its first stages -- so that they are on their way to this XCD's L2
-        // while the epilogue computes, and the next item's first direct-to-LDS loads find them there.
-        auto between = [&]() -> int {
+        auto publish = [&]() {
             if (tid < kWave) {
-                next = take_end(taken);
-                if (tid == 0) {
-                    next_s = next;
-                }
-            }
-            __syncthreads();
-            const int nidx = next_s;
-            int sink = 0;
-            if (nidx >= 0 && items[nidx].flat != 0) {  // tall items find their panels in L2 (sibling tiles)
-                const SchedItem nx = items[nidx];
-                const int ng = __builtin_amdgcn_readfirstlane(nx.g);
-                const int nm0 = __builtin_amdgcn_readfirstlane(nx.m0);
-                const int nrows = __builtin_amdgcn_readfirstlane(nx.rows);
-                const int nnb = __builtin_amdgcn_readfirstlane(nx.nb);
-                const int lane = tid & (kWave - 1);
-                const int8_t *wgn = a.per_expert ? a.list.w[ng] : a.w + (long long)ng * a.Kd * a.N;
-                const int ngroups = a.N / 64;
-                const int steps = min(3, a.Kd / kBK);
-#pragma unroll
-                for (int gi = 0; gi < 2; ++gi) {
-                    const int grp = min(nnb * 8 + 2 * wave + gi, ngroups - 1);
-                    const int blk = grp >> 3;
-                    const long long step = (long long)min(8, ngroups - 8 * blk) * 4096;
-                    const int8_t *base = wgn + (long long)blk * 8 * a.Kd * 64 + (grp & 7) * 4096;
-                    for (int i = lane; i < steps * 32; i += kWave) {  // 32 lines per stage
-                        sink ^= *(const int *)(base + (long long)(i >> 5) * step + (i & 31) * 128);
+                const int n = take_end();
+                if (n < 0) {
+                    if (tid == 0) {
+                        next_s.rows = 0;
                     }
+                } else if (tid < 2) {
+                    dma16(scalar_address(items + n), (unsigned)(tid * 16), __builtin_amdgcn_readfirstlane(lds_address(&next_s)));
                 }
-                const int span = min(3 * kBK, a.Kd);          // bytes of a row the first stages cover
-                const int lines = (span + 127) / 128;
-                for (int i = lane; i < 32 * lines; i += kWave) {
-                    const int r = min(32 * wave + i / lines, nrows - 1);
-                    sink ^= *(const int *)(a.a + (long long)(nm0 + r) * a.Kd + (i % lines) * 128);
+#ifdef CAM_GEMM_TIMELINE
+                if (tid == 0) {
+                    next_idx_s = n;
                 }
+#endif
             }
-            return sink;
         };
-
-        const int mf = (rows + 31) >> 5;
         auto run = [&](auto mc, auto nc) {
-            k_loop<decltype(mc)::value, decltype(nc)::value, FP8>(t, lds, a_scale8_s, w_scale8_s, stage_scales);
+            k_loop<decltype(mc)::value, decltype(nc)::value, FP8>(a, t, lds, a_scale8_s, publish);
         };
-        if (flat) {
+        if (t.flat) {
             const std::integral_constant<int, 4> nf;
-            switch (mf) {
+            switch (t.mf) {
                 case 1: run(std::integral_constant<int, 1>(), nf); break;
                 case 2: run(std::integral_constant<int, 2>(), nf); break;
                 case 3: run(std::integral_constant<int, 3>(), nf); break;
                 default: run(std::integral_constant<int, 4>(), nf); break;
             }
-            epilogue_item<4, FP8>(a, t, mf, lds, row_scale_s, between);
         } else {
             const std::integral_constant<int, 2> nf;
-            switch (mf) {
+            switch (t.mf) {
                 case 5: run(std::integral_constant<int, 5>(), nf); break;
                 case 6: run(std::integral_constant<int, 6>(), nf); break;
                 case 7: run(std::integral_constant<int, 7>(), nf); break;
                 case 8: run(std::integral_constant<int, 8>(), nf); break;
                 default: run(std::integral_constant<int, 4>(), nf); break;
             }
-            epilogue_item<2, FP8>(a, t, mf, lds, row_scale_s, between);
+        }
+        // next_s is there: wave 0 has waited for younger loads, and a barrier ends the K loop
+        const SchedItem nx = next_s;
+        ItemCtx next;
+        next.rows = __builtin_amdgcn_readfirstlane(nx.rows);
+        if (next.rows > 0) {
+            next = decode(nx, t.buf ^ 1);
+            ask_ahead(next);
+            take_begin();
+        }
+        const float *scales = scale_s[FP8 ? 0 : t.buf];
+        if (t.flat) {
+            epilogue_item<4, FP8>(a, t, lds, scales, scales + 256);
+        } else {
+            epilogue_item<2, FP8>(a, t, lds, scales, scales + 256);
         }
 #ifdef CAM_GEMM_TIMELINE
         if (tid == 0) {
-            int32_t *stamp = (int32_t *)&items[idx];
+            int32_t *stamp = (int32_t *)&items[cur_idx];
             stamp[6] = (int32_t)timeline_t0;
             stamp[7] = (int32_t)wall_clock64();
             stamp[3] = (stamp[3] & 0xffff) | ((int)blockIdx.x << 16);  // split is read at the start of the item only
@@ -1030,10 +1046,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
             stamp[4] = (stamp[4] & 0xffff) | (d1 << 16);
             stamp[5] = (stamp[5] & 0xffff) | (d2 << 16);
         }
+        cur_idx = next_idx_s;
 #endif
-        if (!flat && tid < kWave) {  // a flat item has taken its successor between its K loop and its epilogue
-            next = take_end(taken);
+        if (next.rows == 0) {
+            next = first_item(t.buf ^ 1, true);
         }
+        t = next;
     }
 }
 
