@@ -60,36 +60,75 @@ __device__ __forceinline__ int lane_id()
     return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
 }
 
-__device__ __forceinline__ float wave_max(float v)
+// Reductions and scans across the lanes of a wave go through the data-parallel primitives of the vector ALU: a lane reads a
+// neighbour's register in the instruction that combines the two, a few cycles a step, where a shuffle through the LDS
+// crossbar takes about a hundred.  Every lane of the wave has to be active.
+constexpr int kDppRowShr = 0x110;      // + n: lane i reads lane i - n of its row of sixteen
+constexpr int kDppRowRor = 0x120;      // + n: rotation by n inside the row
+constexpr int kDppRowBcast15 = 0x142;  // lane 15 of every row to the whole next row
+constexpr int kDppRowBcast31 = 0x143;  // lane 31 to rows 2 and 3
+constexpr int kDppSwapPairs = 0xb1;    // lane i reads lane i ^ 1
+constexpr int kDppSwapQuads = 0x4e;    // i ^ 2
+constexpr int kDppHalfMirror = 0x141;  // 7 - i of each eight
+constexpr int kDppMirror = 0x140;      // 15 - i of each sixteen
+
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ int dpp(int none, int v)  // `none` where there is no lane to read, or the row is not in ROWS
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
+    return __builtin_amdgcn_update_dpp(none, v, CTRL, ROWS, 0xf, false);
+}
+
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ float dpp_max(float v)
+{
+    return fmaxf(v, __int_as_float(dpp<CTRL, ROWS>(__float_as_int(v), __float_as_int(v))));
+}
+
+// Maximum over the sixteen lanes of a row, in all of them.
+__device__ __forceinline__ float row_max(float v)
+{
+    v = dpp_max<kDppRowRor + 8>(v);
+    v = dpp_max<kDppRowRor + 4>(v);
+    v = dpp_max<kDppRowRor + 2>(v);
+    return dpp_max<kDppRowRor + 1>(v);
+}
+
+// Maximum over aligned groups of n lanes (a power of two, wave-uniform), in all of them.
+__device__ __forceinline__ float group_max(float v, int n)
+{
+    v = n > 1 ? dpp_max<kDppSwapPairs>(v) : v;
+    v = n > 2 ? dpp_max<kDppSwapQuads>(v) : v;
+    v = n > 4 ? dpp_max<kDppHalfMirror>(v) : v;
+    v = n > 8 ? dpp_max<kDppMirror>(v) : v;
+    for (int off = 16; off < n; off <<= 1) {
         v = fmaxf(v, __shfl_xor(v, off, kWave));
     }
     return v;
 }
 
-__device__ __forceinline__ int wave_sum(int v)
+__device__ __forceinline__ float wave_max(float v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        v += __shfl_xor(v, off, kWave);
-    }
-    return v;
+    v = row_max(v);
+    v = dpp_max<kDppRowBcast15, 0xa>(v);
+    v = dpp_max<kDppRowBcast31, 0xc>(v);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), kWave - 1));
 }
 
 // Inclusive scan across the 64 lanes of a wave.
-__device__ __forceinline__ int wave_inclusive_scan(int v, int lane)
+__device__ __forceinline__ int wave_inclusive_scan(int v)
 {
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        int n = __shfl_up(v, off, kWave);
-        if (lane >= off) {
-            v += n;
-        }
-    }
-    return v;
+    v += dpp<kDppRowShr + 1>(0, v);
+    v += dpp<kDppRowShr + 2>(0, v);
+    v += dpp<kDppRowShr + 4>(0, v);
+    v += dpp<kDppRowShr + 8>(0, v);
+    v += dpp<kDppRowBcast15, 0xa>(0, v);
+    return v + dpp<kDppRowBcast31, 0xc>(0, v);
 }
+
+// The last lane's value of such a scan, in all of them.
+__device__ __forceinline__ int wave_last(int v) { return __builtin_amdgcn_readlane(v, kWave - 1); }
+
+__device__ __forceinline__ int wave_sum(int v) { return wave_last(wave_inclusive_scan(v)); }
 
 }  // namespace cam
 

@@ -1150,10 +1150,7 @@ __global__ __launch_bounds__(256) void requant_fp8_kernel(const float *__restric
                 x[e] = 0.0f;
             }
         }
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-            m = fmaxf(m, __shfl_xor(m, off, kWave));
-        }
+        m = row_max(m);
         const int ex = fp8_block_scale_exp(m);
         const float f1 = exp2_int(-(ex / 2)), f2 = exp2_int(-(ex - ex / 2));
         int lo = 0, hi = 0;

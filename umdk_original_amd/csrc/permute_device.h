@@ -132,10 +132,7 @@ __device__ __forceinline__ void quant_token_row_fp8(Row &r)
             x[2 * i + 1] = act_bits_to_f32<ACT>(r.raw[j][i] >> 16);
             m = fmaxf(m, fmaxf(fabsf(x[2 * i]), fabsf(x[2 * i + 1])));
         }
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-            m = fmaxf(m, __shfl_xor(m, off, kWave));
-        }
+        m = row_max(m);
         const int e = fp8_block_scale_exp(m);
         r.scale8[j] = (uint32_t)(e + 127);
         const float f1 = exp2_int(-(e / 2)), f2 = exp2_int(-(e - e / 2));

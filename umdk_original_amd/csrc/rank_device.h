@@ -28,14 +28,14 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int tid, int *scratch
 {
     int lane = tid & (kWave - 1);
     int w = tid >> 6;
-    int inc = wave_inclusive_scan(v, lane);
+    int inc = wave_inclusive_scan(v);
     if (lane == kWave - 1) {
         scratch[w] = inc;
     }
     __syncthreads();
     if (w == 0) {
         int t = lane < NWAVES ? scratch[lane] : 0;
-        int ti = wave_inclusive_scan(t, lane);
+        int ti = wave_inclusive_scan(t);
         if (lane < NWAVES) {
             scratch[lane] = ti - t;
         }

@@ -186,14 +186,14 @@ __device__ __forceinline__ void build_shared_queues(SchedShared &sh, const Sched
             const int rank = base + lane;
             const ExpertShape e = expert_shape(rank < G ? sh.rows[sh.order[rank]] : 0);
             const int vw = e.tall ? nb_tall * e.units : 0, vf = e.flat ? 1 : 0;
-            const int iw = wave_inclusive_scan(vw, lane);
-            const int jf = wave_inclusive_scan(vf, lane);
+            const int iw = wave_inclusive_scan(vw);
+            const int jf = wave_inclusive_scan(vf);
             if (rank < G) {
                 t.work_before[rank] = work_run + iw - vw;
                 t.flat_rank[rank] = flat_run + jf - vf;
             }
-            work_run += __shfl(iw, kWave - 1, kWave);
-            flat_run += __shfl(jf, kWave - 1, kWave);
+            work_run += wave_last(iw);
+            flat_run += wave_last(jf);
         }
         if (lane == 0) {
             t.wtotal = max(work_run, 1);
@@ -223,11 +223,11 @@ __device__ __forceinline__ void build_shared_queues(SchedShared &sh, const Sched
                 t.ngroups[x][rank] = (short)mine;
                 v = mine * e.tiles;
             }
-            const int inc = wave_inclusive_scan(v, lane);
+            const int inc = wave_inclusive_scan(v);
             if (rank < G && (flat_wave ? e.flat : e.tall)) {
                 t.qbase[x][rank] = run + inc - v;
             }
-            run += __shfl(inc, kWave - 1, kWave);
+            run += wave_last(inc);
         }
         if (lane == 0) {
             (flat_wave ? t.qflat : t.qtall)[x] = run;
@@ -335,10 +335,10 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
                 }
             } else {
                 const int c = g < G ? sh.order[g] : 0;
-                const int inc = wave_inclusive_scan(c, lane);
+                const int inc = wave_inclusive_scan(c);
                 m0 = (int)min(max((long long)run + inc - c, 0ll), sb.max_rows);
                 m1 = (int)min(max((long long)m0 + c, (long long)m0), sb.max_rows);
-                run = (int)min(max((long long)run + __shfl(inc, kWave - 1, kWave), 0ll), sb.max_rows);
+                run = (int)min(max((long long)run + wave_last(inc), 0ll), sb.max_rows);
             }
             if (g < G) {
                 sh.rows[g] = m1 - m0;
@@ -377,7 +377,7 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
             const ExpertShape e = expert_shape(rank < G ? sh.rows[sh.order[rank]] : 0);
             const int blocks = e.tall ? nb_tall : (e.flat ? nb_flat : 0);
             const int v = (c == kClasses ? e.tiles : class_count(e, c)) * blocks;
-            const int inc = wave_inclusive_scan(v, lane);
+            const int inc = wave_inclusive_scan(v);
             if (rank < G) {
                 if (c == kClasses) {
                     sh.first_item[rank] = run + inc - v;
@@ -385,7 +385,7 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
                     sh.own.class_before[c][rank] = run + inc - v;
                 }
             }
-            run += __shfl(inc, kWave - 1, kWave);
+            run += wave_last(inc);
         }
         if (lane == 0) {
             if (c == kClasses) {
@@ -433,7 +433,7 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
             v[i] = w < m ? R + (column_of_workgroup(w, m) >= m - b ? 1 : 0) : 0;
             run += v[i];
         }
-        const int inc = wave_inclusive_scan(run, lane);
+        const int inc = wave_inclusive_scan(run);
         int before = inc - run;
 #pragma unroll
         for (int i = 0; i < PER; ++i) {

@@ -380,9 +380,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
         for (int j = 0; j < (PRODUCTS ? kProductQuads : 1); ++j) {
             m = fmaxf(m, fmaxf(fmaxf(fabsf(prod[j][0]), fabsf(prod[j][1])), fmaxf(fabsf(prod[j][2]), fabsf(prod[j][3]))));
         }
-        for (int off = 1; off < min(1 << lg, kWave); off <<= 1) {
-            m = fmaxf(m, __shfl_xor(m, off, kWave));
-        }
+        m = group_max(m, min(1 << lg, kWave));
         if (lg > 6) {   // several waves to a row (all of them take this branch)
             if (lane == 0) {
                 rowmax_s[wave] = m;
@@ -638,9 +636,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
                             if constexpr (FP8 && P >= 4) {
                                 if (a.epilogue == kEpiSwigluFp8) {
                                     keep[b] = y;
-                                    m = fmaxf(m, __shfl_xor(m, 1, kWave));
-                                    m = fmaxf(m, __shfl_xor(m, 2, kWave));
-                                    m = fmaxf(m, __shfl_xor(m, 4, kWave));
+                                    m = group_max(m, 8);
                                     if (piece == 0 && s < 4) {
                                         rowmax_s[p * 32 + row] = m;
                                     }
