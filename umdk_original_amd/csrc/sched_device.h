@@ -100,7 +100,8 @@ struct SchedSharedTables {
     int wtotal;
 };
 struct SchedShared {
-    int rows[kMaxExperts], off[kMaxExperts], order[kMaxExperts];
+    __attribute__((aligned(16))) int rows[kMaxExperts];
+    int off[kMaxExperts], order[kMaxExperts];
     int first_item[kMaxExperts + 1];       // by rank: items of the experts ranked before
     union {
         SchedOwnTables own;
@@ -123,7 +124,7 @@ __device__ __forceinline__ int queue_of_group(long long before, int units, long 
     return x;
 }
 
-// Workgroup of column j when the columns are numbered XCD by XCD, and the inverse.
+// Workgroup of column j when the columns are numbered XCD by XCD.
 __device__ __forceinline__ int workgroup_of_column(int j, int m)
 {
     int x = 0;
@@ -135,16 +136,6 @@ __device__ __forceinline__ int workgroup_of_column(int j, int m)
         j -= here;
     }
     return x + kNumXcd * j;
-}
-
-__device__ __forceinline__ int column_of_workgroup(int w, int m)
-{
-    const int x = w % kNumXcd;
-    int before = 0;
-    for (int xx = 0; xx < x; ++xx) {
-        before += (m - xx + kNumXcd - 1) / kNumXcd;
-    }
-    return before + w / kNumXcd;
 }
 
 // One item of a schedule from its expert's shape: column block c, row tile j.
@@ -343,6 +334,8 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
             if (g < G) {
                 sh.rows[g] = m1 - m0;
                 sh.off[g] = m0;
+            } else {
+                sh.rows[g] = -1;  // (the ranking reads a few behind the last; smaller than any)
             }
             const int chunk_rows = wave_sum(g < G ? m1 - m0 : 0);
             if (lane == 0) {
@@ -351,13 +344,21 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
         }
     }
     __syncthreads();
-    // rank by rows, largest first (ties: lower index first)
+    // rank by rows, largest first (ties: lower index first); sixteen experts a turn, so that the reads overlap
     for (int g = tid; g < G; g += NT) {
         const int cnt = sh.rows[g];
         int rank = 0;
-        for (int j = 0; j < G; ++j) {
-            const int rj = sh.rows[j];
-            rank += (rj > cnt || (rj == cnt && j < g)) ? 1 : 0;
+        for (int j = 0; j < G; j += 16) {
+            v4i r[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                r[q] = *(const v4i *)(sh.rows + j + 4 * q);
+            }
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int rj = r[q >> 2][q & 3];
+                rank += (rj > cnt || (rj == cnt && j + q < g)) ? 1 : 0;
+            }
         }
         sh.order[rank] = g;
     }
@@ -424,25 +425,16 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
     // the matrix: R items in each of the first m - b columns, R + 1 in the last b
     const int R = n_items / m, b = n_items - R * m;
     const int n_big = (m - b) * R;
-    if (wave == 0) {  // first item of every workgroup's queue: prefix sum of the column heights in workgroup order
-        constexpr int PER = kMaxQueues / kWave;
-        int v[PER], run = 0;
+    for (int w = tid; w <= m; w += NT) {  // first item of every workgroup's queue: R items for each workgroup before, ...
+        int before = w * R, columns = 0;
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int w = lane * PER + i;
-            v[i] = w < m ? R + (column_of_workgroup(w, m) >= m - b ? 1 : 0) : 0;
-            run += v[i];
+        for (int x = 0; x < kNumXcd; ++x) {  // ... one more for each of them whose column is one of the last b
+            const int here = (m - x + kNumXcd - 1) / kNumXcd;      // workgroups of XCD x, x + 8 k for k < here
+            const int first = max(m - b - columns, 0);             // those from k = first on
+            before += max(min(max((w - x + kNumXcd - 1) / kNumXcd, 0), here) - first, 0);
+            columns += here;
         }
-        const int inc = wave_inclusive_scan(run);
-        int before = inc - run;
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            sh.qstart[lane * PER + i] = before;
-            before += v[i];
-        }
-        if (lane == kWave - 1) {
-            sh.qstart[kMaxQueues] = inc;
-        }
+        sh.qstart[w] = before;
     }
     __syncthreads();
     if (tid == 0 && part == 0) {
