@@ -92,22 +92,27 @@ __global__ __launch_bounds__(kGlobalThreads) void plan_global_kernel(PlanArgs a,
                 base += (bb + j) < b ? v[j] : 0;
             }
         }
-        for (; bb + 8 <= nb; bb += 8) {
-            int v[8];
+        if (bb < nb) {  // what is left, in one round trip as well: eight at a time as far as there are rows, the last one repeated
+            int v[64];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                v[j] = col[(long long)(bb + j) * E];
+            for (int q = 0; q < 64; q += 8) {
+                if (bb + q < nb) {
+#pragma unroll
+                    for (int j = q; j < q + 8; ++j) {
+                        v[j] = col[min(bb + j, nb - 1) * E];
+                    }
+                }
             }
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                cnt += v[j];
-                base += (bb + j) < b ? v[j] : 0;
+            for (int q = 0; q < 64; q += 8) {
+                if (bb + q < nb) {
+#pragma unroll
+                    for (int j = q; j < q + 8; ++j) {
+                        cnt += bb + j < nb ? v[j] : 0;
+                        base += bb + j < b ? v[j] : 0;
+                    }
+                }
             }
-        }
-        for (; bb < nb; ++bb) {
-            const int v = col[(long long)bb * E];
-            cnt += v;
-            base += bb < b ? v : 0;
         }
     }
     const int off = block_exclusive_scan<NW>(cnt, tid, scan_s, &total_s);
