@@ -69,3 +69,21 @@ def test_stream_gemm_fp8_sums(gpu, oracle, sizes, K, N):
         r += n
     assert (got - want).abs().max() <= 2e-2 * want.abs().max()
     assert ((got - want).norm() / want.norm()).item() <= 5e-3
+
+
+@pytest.mark.parametrize("experts", [1, 63, 64, 65, 128, 511, 512])
+@pytest.mark.parametrize("list_type", [0, 1])
+def test_stream_gemm_item_list_at_wave_edges(gpu, oracle, experts, list_type):
+    """A wave lists 64 experts at a turn: rows in the first and the last expert of every turn, none in most others."""
+    announce("stream item list experts=%d list_type=%d" % (experts, list_type))
+    sizes = [(1 + e % 3 if e % 64 in (0, 1, 63) else 0) for e in range(experts)]
+    sizes[-1] = 33   # two 32-row tiles at the end of the list
+    K, N, A = 128, 64, sum(sizes)
+    cnt = torch.tensor(sizes, dtype=torch.int64)
+    gl = torch.cumsum(cnt, 0)
+    x, xs = synth.uniform_int8((A, K), experts), synth.channel_scales((A,), experts + 1, lo=0.005, hi=0.05)
+    w, ws = synth.uniform_int8((experts, K, N), experts + 2, -16, 16), synth.channel_scales((experts, N), experts + 3)
+    out = cam.grouped_matmul_dequant(x.to(gpu), xs.to(gpu), cam.prepack_weight(w.to(gpu), False), ws.to(gpu),
+                                     (gl if list_type == 0 else cnt).to(gpu), list_type)
+    c = oracle.gmm_int32(x.numpy(), w.numpy(), gl.numpy())
+    assert_bits_equal(to_np(out), oracle.gmm2_epilogue(c, ws.numpy(), xs.numpy(), gl.numpy()), "rows")

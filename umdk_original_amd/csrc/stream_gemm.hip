@@ -131,8 +131,6 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     __shared__ __attribute__((aligned(1024))) int8_t lds[kSLds];
     __shared__ int tile_start[kMaxExperts + 1];  // row tiles of the experts before
     __shared__ int first_row[kMaxExperts + 1];
-    __shared__ int scan_s[kSThreads / kWave];
-    __shared__ int total_s;
     // scales of the current and of the next item: int8 column (per group: 64, or 32 gate + 32 up) and row scales
     __shared__ __attribute__((aligned(16))) float col_scale_s[2][FP8 ? 4 : P * 64];
     __shared__ __attribute__((aligned(16))) float row_scale_s[2][FP8 ? 4 : 32 * MF];
@@ -158,43 +156,55 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     static_assert(!PRODUCTS || (MF == 1 && !FP8), "products are quantised by the 32-row tiles");
     const int kpad = (Kd + quantum - 1) / quantum * quantum;
 
-    // ---- the item list: rows, first row and row tiles of every expert (thread e: expert e)
+    // ---- the item list: every expert's first row and the row tiles before it.  Every wave works it out for itself, a lane an
+    // expert, and stores it: the same values into the same places, so that no wave waits for another before it knows its first
+    // weights (two block scans and five workgroup barriers until then: the layer of 128 tokens x 1024, top-2 of 8 experts,
+    // 26.5 -> 25.8 us of back-to-back calls; nothing where the weights take longer).
     {
-        int m0 = 0, rows = 0;
-        if (tid < G) {
-            const long long v = min(max(sa.group_list[tid], (int64_t)0), (int64_t)sa.max_rows);
-            if (sa.cumulative) {
-                m0 = tid == 0 ? 0 : (int)min(max(sa.group_list[tid - 1], (int64_t)0), (int64_t)sa.max_rows);
-                rows = max((int)v - m0, 0);
-            } else {
-                rows = (int)v;
+        constexpr int kChunks = kMaxExperts / kWave;
+        auto listed = [&](int e) { return (int)min(max(sa.group_list[e], (int64_t)0), (int64_t)sa.max_rows); };
+        int entry[kChunks], before[kChunks];
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const int e = c * kWave + lane;
+            entry[c] = 0;
+            before[c] = 0;
+            if (c * kWave < G) {
+                entry[c] = e < G ? listed(e) : 0;
+                before[c] = sa.cumulative && e > 0 && e < G ? listed(e - 1) : 0;
             }
         }
-        if (!sa.cumulative) {
-            m0 = block_exclusive_scan<kSThreads / kWave>(rows, tid, scan_s, &total_s);
-            m0 = min(max(m0, 0), (int)sa.max_rows);
-            rows = min(rows, (int)sa.max_rows - m0);
-        }
-        const int tiles = (rows + 32 * MF - 1) / (32 * MF);
-        const int ts = block_exclusive_scan<kSThreads / kWave>(tiles, tid, scan_s, &total_s);
-        if (tid <= G) {
-            tile_start[tid] = ts;
-            first_row[tid] = m0;
-        }
-        if (tid == 0) {
-            tile_start[G] = total_s;   // (for G == 512, which no thread has)
-        }
-        __syncthreads();
-        if (sa.rows_out != nullptr && blockIdx.x == 0 && tid == G - 1) {
-            sa.rows_out[1] = m0 + rows;  // the rows the next kernel finds (the lists are ascending)
-        }
-        if (tid < G) {
-            // where the expert's rows end: kept in the slot after its first row's (experts are contiguous)
-            if (tid == G - 1) {
-                first_row[G] = m0 + rows;
+        int row = 0, tile = 0;   // of the experts before this chunk
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const int e = c * kWave + lane;
+            if (c * kWave < G) {
+                int m0 = before[c], rows = max(entry[c] - m0, 0);
+                if (!sa.cumulative) {
+                    const int inc = wave_inclusive_scan(entry[c]);
+                    m0 = min(max(row + inc - entry[c], 0), (int)sa.max_rows);
+                    rows = min(entry[c], (int)sa.max_rows - m0);
+                    row += wave_last(inc);
+                }
+                rows = e < G ? rows : 0;
+                const int tiles = (rows + 32 * MF - 1) / (32 * MF);
+                const int inc = wave_inclusive_scan(tiles);
+                if (e < G) {
+                    tile_start[e] = tile + inc - tiles;
+                    first_row[e] = m0;
+                }
+                tile += wave_last(inc);
+                if (e == G - 1) {
+                    tile_start[G] = tile;
+                    first_row[G] = m0 + rows;   // where the last expert's rows end
+                    if (sa.rows_out != nullptr && blockIdx.x == 0 && wave == 0) {
+                        sa.rows_out[1] = m0 + rows;  // the rows the next kernel finds (the lists are ascending)
+                    }
+                }
             }
         }
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // lanes read what other lanes of their wave stored
+        __builtin_amdgcn_wave_barrier();
     }
     const int n_items = tile_start[G] * blocks;
 
