@@ -290,12 +290,10 @@ camStatus check_gemm_dims(const char *op, int64_t Kd, int64_t N, bool gate_up)
 }
 
 // One schedule for a GEMM of N packed columns over `rows` rows of G experts, carved out of a workspace.
-cam::SchedSpec sched_spec(int64_t rows, int64_t G, int64_t N, int64_t Kd, bool swiglu)
+cam::SchedSpec sched_spec(int64_t rows, int64_t G, int64_t N)
 {
     cam::SchedSpec sp{};
     sp.N = (int)N;
-    sp.Kd = (int)Kd;
-    sp.swiglu = swiglu ? 1 : 0;
     sp.max_items = cam::sched_max_items(rows, (int)G, (int)N);
     return sp;
 }
@@ -1548,7 +1546,7 @@ camStatus camGroupedMatmulSwigluQuantGetWorkspaceSize(const camTensor *x, const 
     WeightSet ws{};
     CAM_TRY(resolve_weights(weight, weightScale, "weight", gc.G, gc.Kd, 2 * I, true, &ws));
     CAM_TRY(check_aligned(y, "y", 16));
-    cam::SchedSpec sp = sched_spec(gc.A, gc.G, 2 * I, gc.Kd, true);
+    cam::SchedSpec sp = sched_spec(gc.A, gc.G, 2 * I);
     Carver c;
     const uint64_t o_sched = c.take(gemm_sched_bytes(gc.A, 2 * I, gc.G, cam::kEpiSwiglu, false));
     const uint64_t o_prod = c.take((uint64_t)gc.A * I * 4);
@@ -1608,7 +1606,7 @@ camStatus camGroupedMatmulDequantGetWorkspaceSize(const camTensor *x, const camT
     CAM_TRY(check_aligned(out, "out", 16));
     WeightSet ws{};
     CAM_TRY(resolve_weights(weight, weightScale, "weight", gc.G, gc.Kd, N, true, &ws));
-    cam::SchedSpec sp = sched_spec(gc.A, gc.G, N, gc.Kd, false);
+    cam::SchedSpec sp = sched_spec(gc.A, gc.G, N);
     Carver c;
     const uint64_t o_sched = c.take(gemm_sched_bytes(gc.A, N, gc.G, cam::kEpiDequantBf16, false));
     const uint64_t o_rows = wire ? c.take((uint64_t)gc.A * N * 2) : 0;  // the bf16 rows before quantisation
@@ -1664,7 +1662,7 @@ camStatus camGroupedMatmulInt32GetWorkspaceSize(const camTensor *x, const camTen
     CAM_TRY(check_aligned(out, "out", 16));
     WeightSet ws{};
     CAM_TRY(resolve_weights(weight, nullptr, "weight", gc.G, gc.Kd, N, false, &ws));
-    cam::SchedSpec sp = sched_spec(gc.A, gc.G, N, gc.Kd, false);
+    cam::SchedSpec sp = sched_spec(gc.A, gc.G, N);
     Carver c;
     const uint64_t o_sched = c.take(cam::sched_bytes(gc.A, (int)gc.G, (int)N));
     cam::GemmArgs g{};
@@ -1804,8 +1802,8 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     CAM_TRY(check_aligned(output, "output", 16));
 
     const int64_t A = T * K;  // maxTokenNum of AK/fused_deep_moe/op_kernel/fused_deep_moe.h:336 for one rank
-    cam::SchedSpec sp1 = sched_spec(A, Epr, 2 * I, H, true);
-    cam::SchedSpec sp2 = sched_spec(A, Epr, H, I, false);
+    cam::SchedSpec sp1 = sched_spec(A, Epr, 2 * I);
+    cam::SchedSpec sp2 = sched_spec(A, Epr, H);
     // Few rows: the GEMMs need no schedule.  Fewer still: GMM2 quantises the products itself, and then writes its rows while
     // they are still read.
     const bool stream = cam::stream_gemm_applies(A, 2 * I, Epr, false);
@@ -2050,7 +2048,7 @@ camStatus camGroupedMatmulFp8GetWorkspaceSize(const camTensor *x, const camTenso
     CAM_TRY(check_aligned(xScale, "xScale", 4));  // a row's block scales are fetched as words
     Fp8Weight fw{};
     CAM_TRY(check_fp8_weight(weight, weightScale, "weight", G, Kd, N, &fw));
-    cam::SchedSpec sp = sched_spec(A, G, N, Kd, gate_up);
+    cam::SchedSpec sp = sched_spec(A, G, N);
     cam::GemmArgs g{};
     g.a = (const int8_t *)x->data;
     g.w = fw.w;
@@ -2166,8 +2164,8 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
     CAM_TRY(check_aligned(output, "output", 16));
 
     const int64_t A = T * K;
-    cam::SchedSpec sp1 = sched_spec(A, E, 2 * I, H, true);
-    cam::SchedSpec sp2 = sched_spec(A, E, H, I, false);
+    cam::SchedSpec sp1 = sched_spec(A, E, 2 * I);
+    cam::SchedSpec sp2 = sched_spec(A, E, H);
     const bool stream = cam::stream_gemm_applies(A, 2 * I, E, true);   // few rows: no schedules
     Carver c;
     const uint64_t o_pos = c.take((uint64_t)A * 4);

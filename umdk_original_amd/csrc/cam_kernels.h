@@ -81,8 +81,6 @@ hipError_t launch_notify_scan(const int32_t *cnt, int E, int num_tokens, int32_t
 // one or two GEMMs over the same rows (they differ in the number of weight columns).
 struct SchedSpec {
     int N;             // packed weight columns of the GEMM
-    int Kd;            // its reduction length (the cost model of the builder needs it)
-    int swiglu;        // its epilogue forms SiLU(gate) * up (costlier per row than a plain dequantisation)
     int max_items;     // capacity of the item table (sched_max_items)
     int32_t *sched;    // sched_bytes() of device memory
 };

@@ -12,13 +12,13 @@ namespace cam {
 // Work items.  Expert g with r rows: r == 0 owns nothing; r <= 128 is "flat": one row tile and ceil(N/512) column
 // blocks, each an item that streams its weight panel at the pace one CU pulls bytes from memory; otherwise "tall":
 // ceil(r/256) row tiles of (nearly) equal height, a multiple of 32 rows (tiles of one expert differ by at most 32),
-// times ceil(N/256) column blocks.  Shorter tall tiles are no cheaper per row: below 256 rows the K loop is bound
-// by the loads of its 256-column weight panel, not by the matrix cores.
+// times ceil(N/256) column blocks.
 //
 // The schedule gives every workgroup of the persistent GEMM (one per CU) a queue of its own.  The items are put in
-// one line, costliest first by the model below and otherwise in the order in which they share operands (experts
-// largest first; per expert column block by column block; the row tiles of a column block side by side), and the
-// line is dealt row by row into a matrix with one column per workgroup:
+// one line, costliest first (a flat item, then the taller tiles: GMM1 items of K = 2048 / 4096 / 7168 take, in us, flat 37 / 72 /
+// 117, eight row units 30 / 69 / 99, four 18 / 42 / 69; the order is the same in GMM2) and otherwise in the order in which
+// they share operands (experts largest first; per expert column block by column block; the row tiles of a column block side
+// by side), and the line is dealt row by row into a matrix with one column per workgroup:
 //   * with n items and m workgroups, R = n / m: the first m - b columns take R items each from the costly end of
 //     the line, the last b = n - R m columns take R + 1 from the cheap end, so that no column holds one item more
 //     than another of the same kind and the columns with more items hold the cheaper ones;
@@ -29,7 +29,7 @@ namespace cam {
 //     weight panel through that XCD's L2, the column blocks of one expert its activation rows.  Measured on the
 //     Zipf-skewed shape this matters more than balance: the same items dealt for balance alone run a third slower.
 // A queue is run front to back by its workgroup; one that runs out takes the next item of the queue with the most
-// items left (gemm.hip), which covers what the cost model gets wrong.
+// items left (gemm.hip), which covers what the order gets wrong.
 //
 // Long schedules (kSharedFrom items per workgroup or more) get eight shared queues instead, one per XCD, from which
 // the workgroups of that XCD take item by item: with many short items per workgroup the sums of fixed queues
@@ -42,15 +42,6 @@ namespace cam {
 //   * Flat experts are dealt to the queues whole, in rank order, and a queue spreads its flat items evenly among
 //     its tall ones except for the last kTallTail places: a flat item streams its weights and needs the memory,
 //     a tall one the matrix cores, so they run well side by side, and the queues end with items of even length.
-//
-// Cost model, nanoseconds; it only ranks the item kinds.  A tall tile of u row units (32 rows) over KT sub-steps
-// of 64 K bytes: fixed + KT * max(load-bound step, u * matrix step); a flat item: fixed + KT * streaming step.
-constexpr float kTallFixedSwiglu = 15000.0f;
-constexpr float kTallFixedPlain = 10000.0f;
-constexpr float kTallLoadStep = 550.0f;
-constexpr float kTallUnitStep = 92.0f;
-constexpr float kFlatFixed = 22400.0f;
-constexpr float kFlatStep = 862.0f;
 constexpr int kClasses = 9;  // item kinds: 0 = flat, h = 1..8 = tall tile of h row units
 constexpr int kSharedFrom = 12;                       // items per workgroup from which the queues are shared
 constexpr int kTallTail = 24;                        // tall items a shared queue ends with
@@ -405,19 +396,11 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
         return;
     }
 
-    // the classes in the order of the line: costliest first (ties: flat, then the taller tile)
+    // the classes in the order of the line: flat, then the taller tiles first
     if (tid < kClasses) {
-        const float KT = (float)(spec.Kd / 64);
-        auto cost = [&](int c) {
-            return c == 0 ? kFlatFixed + KT * kFlatStep
-                          : (spec.swiglu ? kTallFixedSwiglu : kTallFixedPlain) +
-                                KT * fmaxf(kTallLoadStep, (float)c * kTallUnitStep);
-        };
-        const float mine = cost(tid);
         int start = 0;
         for (int c = 0; c < kClasses; ++c) {
-            const float other = cost(c);
-            const bool ahead = other > mine || (other == mine && c != tid && (c == 0 || (tid != 0 && c > tid)));
+            const bool ahead = c != tid && tid != 0 && (c == 0 || c > tid);
             start += ahead ? sh.own.class_total[c] : 0;
         }
         sh.own.class_start[tid] = start;
