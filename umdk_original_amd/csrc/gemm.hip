@@ -266,18 +266,32 @@ __device__ __forceinline__ void acc_clear()
 #undef CAM_X
 }
 
+// Four accumulator registers from REG on.  Together, because a value that comes out of inline assembly costs a wait state if
+// the next instruction uses it: read one by one as they were needed, an FP8 product cost up to two of them beside its 24
+// instructions (with the one that quiet() saves: FP8 layer of 8000 tokens x 2048, top-6 of 64 experts, I 1408: 572 -> 566 us; of
+// 4093 x 4096, top-8 of 128, I 1536: 832.5 -> 831; int8, where the products need no such read, within 0.3 %).
 template <int REG>
-__device__ __forceinline__ int acc_bits()
+__device__ __forceinline__ v4i acc_bits4()
 {
-    int v;
-    asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(v) : "n"(REG));
-    return v;
+    int v[4];
+    asm volatile("v_accvgpr_read_b32 %0, a[%4]\n\tv_accvgpr_read_b32 %1, a[%4+1]\n\t"
+                 "v_accvgpr_read_b32 %2, a[%4+2]\n\tv_accvgpr_read_b32 %3, a[%4+3]"
+                 : "=v"(v[0]), "=v"(v[1]), "=v"(v[2]), "=v"(v[3]) : "n"(REG));
+    return v4i{v[0], v[1], v[2], v[3]};
 }
 
 template <int REG, bool FP8>
-__device__ __forceinline__ float acc_value()
+__device__ __forceinline__ v4f acc_values()
 {
-    return FP8 ? __int_as_float(acc_bits<REG>()) : (float)acc_bits<REG>();
+    const v4i v = acc_bits4<REG>();
+    return FP8 ? __builtin_bit_cast(v4f, v) : v4f{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+}
+
+// A gate sum of an FP8 item: cam_silu_spec takes its minimum and its maximum, and the compiler, which does not know that the
+// matrix cores make no signalling NaN, would quiet it for each of them.
+__device__ __forceinline__ float quiet(float t)
+{
+    return __builtin_canonicalizef(t);
 }
 
 template <bool FP8>
@@ -620,8 +634,7 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
                             constexpr int j = decltype(jc)::value;
                             constexpr int r = (decltype(qc)::value * NF + 2 * gi + nf) * 16 + 4 * j;
                             // int32 sums, or the bits of the fp32 sums of an FP8 item
-                            const v4i v = {acc_bits<r>(), acc_bits<r + 1>(), acc_bits<r + 2>(), acc_bits<r + 3>()};
-                            *(v4i *)(slice + row_in * kEpiRowBytes + (8 * j + col_half) * 4) = v;
+                            *(v4i *)(slice + row_in * kEpiRowBytes + (8 * j + col_half) * 4) = acc_bits4<r>();
                         });
                     }, [&](int mf, const v4u (&v)[4]) { store_rows(out, N * 4, mf, v); });
                 });
@@ -633,17 +646,19 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
                     const float xs = FP8 ? 1.0f : row_scale[mf * 32 + row_in];
                     static_for<0, 4>([&](auto jc) {
                         constexpr int j = decltype(jc)::value;
+                        constexpr int r = (mf * NF + 2 * gi) * 16 + 4 * j;
+                        const v4f gate = acc_values<r, FP8>(), up = acc_values<r + 16, FP8>();
                         v4f y;
-                        static_for<0, 4>([&](auto ec) {
-                            constexpr int e = decltype(ec)::value;
-                            constexpr int r = (mf * NF + 2 * gi) * 16 + 4 * j + e;
-                            float tg = acc_value<r, FP8>(), tu = acc_value<r + 16, FP8>();
-                            if constexpr (!FP8) {  // (FP8: the sums carry their scales already)
-                                tg = __fmul_rn(__fmul_rn(tg, csc[gi][0][j][e]), xs);
-                                tu = __fmul_rn(__fmul_rn(tu, csc[gi][1][j][e]), xs);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            if constexpr (FP8) {  // the sums carry their scales already
+                                y[e] = __fmul_rn(cam_silu_spec(quiet(gate[e])), up[e]);
+                            } else {
+                                const float tg = __fmul_rn(__fmul_rn(gate[e], csc[gi][0][j][e]), xs);
+                                const float tu = __fmul_rn(__fmul_rn(up[e], csc[gi][1][j][e]), xs);
+                                y[e] = __fmul_rn(cam_silu_spec(tg), tu);
                             }
-                            y[e] = __fmul_rn(cam_silu_spec(tg), tu);
-                        });
+                        }
                         *(v4f *)(slice + row_in * kEpiRowBytes + (8 * j + col_half) * 4) = y;
                     });
                 }, [&](int mf, const v4u (&v)[4]) { store_rows(out, N * 2, mf, v); });
@@ -655,14 +670,12 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
                         const float xs = FP8 ? 1.0f : row_scale[mf * 32 + row_in];
                         static_for<0, 8>([&](auto jc) {
                             constexpr int nf = decltype(jc)::value / 4, j = decltype(jc)::value % 4;
+                            const v4f sum = acc_values<(mf * NF + 2 * gi + nf) * 16 + 4 * j, FP8>();
                             float f[4];
-                            static_for<0, 4>([&](auto ec) {
-                                constexpr int e = decltype(ec)::value;
-                                f[e] = acc_value<(mf * NF + 2 * gi + nf) * 16 + 4 * j + e, FP8>();
-                                if constexpr (!FP8) {
-                                    f[e] = __fmul_rn(__fmul_rn(f[e], csc[gi][nf][j][e]), xs);
-                                }
-                            });
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                f[e] = FP8 ? sum[e] : __fmul_rn(__fmul_rn(sum[e], csc[gi][nf][j][e]), xs);
+                            }
                             // two values per conversion instruction: with the rounding spelled out in integer
                             // arithmetic this epilogue took a quarter of a short-K tile's time in the vector ALU
                             v2u v;
@@ -701,11 +714,15 @@ __device__ __forceinline__ void epilogue_item(const GemmArgs &a, const ItemCtx &
                     return;
                 }
                 float m = 0.0f;
-                static_for<0, NG * 16>([&](auto ic) {
-                    constexpr int gi = decltype(ic)::value / 16, i = decltype(ic)::value % 16;
+                static_for<0, NG * 4>([&](auto ic) {
+                    constexpr int gi = decltype(ic)::value / 4, i = decltype(ic)::value % 4 * 4;
                     constexpr int r = (mf * NF + 2 * gi) * 16 + i;
-                    y[mf][gi][i] = __fmul_rn(cam_silu_spec(acc_value<r, true>()), acc_value<r + 16, true>());
-                    m = fmaxf(m, fabsf(y[mf][gi][i]));
+                    const v4f gate = acc_values<r, true>(), up = acc_values<r + 16, true>();
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        y[mf][gi][i + e] = __fmul_rn(cam_silu_spec(quiet(gate[e])), up[e]);
+                        m = fmaxf(m, fabsf(y[mf][gi][i + e]));
+                    }
                 });
                 m = fmaxf(m, __shfl_xor(m, 32, kWave));
                 if (lane < 32) {
