@@ -17,8 +17,8 @@
 //     an expert that read the same weight columns sit next to each other and big experts come first, which leaves the
 //     small items for the end, where they even out the finishing times.
 //   * Two tile shapes.  Tall tiles (up to 256 rows) x 256 columns: a wave owns ALL rows of the tile and 64 of its columns.
-//     Flat tiles (<= 128 rows) x 512 columns, for experts that only stream weights: all rows and 128 columns.  Either
-//     way a wave holds up to sixteen 32 x 32 sums (256 registers, all of the accumulation file).  The numbers of row and
+//     Flat tiles (<= 128 rows) x 512 columns, for experts that only stream weights: all rows and 128 columns (in a narrow
+//     schedule, sched_device.h, x 256 like tall ones).  Either way a wave holds up to sixteen 32 x 32 sums (256 registers, all of the accumulation file).  The numbers of row and
 //     column fragments are template parameters, so the main loop has no control flow.
 //   * A weight byte is needed by one wave only.  It goes from memory straight to that wave's registers (prepack_kernel laid
 //     the weights out in the lane order the MFMA wants), a ring of four 64-byte K steps.  Only the activations go
@@ -327,7 +327,7 @@ template <int MF, int NF, bool FP8, typename Publish>
 __device__ __forceinline__ void k_loop(const GemmArgs &a, const ItemCtx &t, int8_t *lds, const uint8_t *a_scale8_s,
                                        Publish &publish)
 {
-    constexpr bool STREAM = NF == 4;                // a flat item is the only reader of its weight panel
+    constexpr bool STREAM = NF == 4 || MF < 4;      // a flat or a narrow item is the only reader of its weight panel
     constexpr int SLOTS = FP8 ? MF : 2 * MF;
     constexpr int AR = FP8 ? 4 : 8;                 // fragments in registers
     constexpr int PD = FP8 ? (MF == 1 ? 2 : 3) : (MF == 1 ? 4 : 6);  // (at most a stage)
@@ -898,7 +898,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
         const int nb = __builtin_amdgcn_readfirstlane(it.nb);
         t.flat = __builtin_amdgcn_readfirstlane(it.flat) != 0;
         t.mf = (t.rows + 31) >> 5;
-        t.mf = t.flat ? min(t.mf, 4) : min(max(t.mf, 4), 8);
+        t.mf = min(t.mf, t.flat ? 4 : 8);
         t.group = t.flat ? nb * 8 + 2 * wave : nb * 4 + wave;
         t.buf = buf;
         t.Kd = a.Kd;
@@ -1028,6 +1028,9 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
         } else {
             const std::integral_constant<int, 2> nf;
             switch (t.mf) {
+                case 1: run(std::integral_constant<int, 1>(), nf); break;
+                case 2: run(std::integral_constant<int, 2>(), nf); break;
+                case 3: run(std::integral_constant<int, 3>(), nf); break;
                 case 5: run(std::integral_constant<int, 5>(), nf); break;
                 case 6: run(std::integral_constant<int, 6>(), nf); break;
                 case 7: run(std::integral_constant<int, 7>(), nf); break;

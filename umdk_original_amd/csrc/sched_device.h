@@ -14,6 +14,15 @@ namespace cam {
 // ceil(r/256) row tiles of (nearly) equal height, a multiple of 32 rows (tiles of one expert differ by at most 32),
 // times ceil(N/256) column blocks.
 //
+// Narrow schedules: a flat item is the longest there is, and a launch whose items are more than the m workgroups but no more
+// than two for each takes two of them, the second beside workgroups that have run dry.  If the items fit three per workgroup
+// with the flat ones cut in two (a tile of up to 128 rows x 256 columns, 0.55 of the time), they are: three short rounds
+// instead of two long ones.  us per layer, int8: 1021 fp16 tokens x 2048, top-6 of 64 experts, I 1408 169.5 -> 164.0, 700
+// tokens 159.4 -> 154.5; 400 x 4096, top-4 of 32, I 2048 191.4 -> 187.1; 512 x 7168, top-4 of 24, I 2048 250.8 -> 252.0.  FP8:
+// 900 x 4096, top-4 of 48, I 1536 224.1 -> 214.2; 600 x 1536, top-6 of 64, I 1024 104.0 -> 95.9; 1021 x 2048 154.0 -> 154.7.  (Two
+// runs of one side differ by 0.3-0.6 %.)  With four or more narrow items per workgroup their rounds would take longer than the
+// two wide ones, and a single wide round needs no cut.
+//
 // The schedule gives every workgroup of the persistent GEMM (one per CU) a queue of its own.  The items are put in
 // one line, costliest first (a flat item, then the taller tiles: GMM1 items of K = 2048 / 4096 / 7168 take, in us, flat 37 / 72 /
 // 117, eight row units 30 / 69 / 99, four 18 / 42 / 69; the order is the same in GMM2) and otherwise in the order in which
@@ -43,19 +52,22 @@ namespace cam {
 //     its tall ones except for the last kTallTail places: a flat item streams its weights and needs the memory,
 //     a tall one the matrix cores, so they run well side by side, and the queues end with items of even length.
 constexpr int kClasses = 9;  // item kinds: 0 = flat, h = 1..8 = tall tile of h row units
-constexpr int kSharedFrom = 12;                       // items per workgroup from which the queues are shared
+// Items per workgroup from which the queues are shared.  Layer of 8192 tokens x 4096, top-8 of 128 experts, I 1536 (14 and 18
+// items): 1543 us shared, 1651 with own queues; the FP8 layer of 4093 tokens (7 and 9): 822 shared, 816 with own queues.
+constexpr int kSharedFrom = 12;
 constexpr int kTallTail = 24;                        // tall items a shared queue ends with
 
+// How the items of an expert of `rows` rows lie.  narrow: those of <= 128 rows are cut like tall ones.
 struct ExpertShape {
     int rows, units, tiles, base, extra;  // tall: `extra` tiles of base + 1 units, then tiles - extra of base units
     bool tall, flat;
 };
 
-__device__ __forceinline__ ExpertShape expert_shape(int rows)
+__device__ __forceinline__ ExpertShape expert_shape(int rows, bool narrow = false)
 {
     ExpertShape e;
     e.rows = rows;
-    e.tall = rows > 128;
+    e.tall = rows > (narrow ? 0 : 128);
     e.flat = rows > 0 && !e.tall;
     e.units = (rows + 31) / 32;
     e.tiles = e.tall ? (rows + 255) / 256 : (e.flat ? 1 : 0);
@@ -100,6 +112,7 @@ struct SchedShared {
     };
     int qstart[kMaxQueues + 1];
     int total_rows;
+    int narrow;
 };
 
 // Shared queues: the queue of the tall group whose work (in row units) starts at `before` and is `units` long is
@@ -304,9 +317,14 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
         sh.order[g] = (int)min(max(sb.group_list[g], (int64_t)0), (int64_t)sb.max_rows);
     }
     __syncthreads();
-    // rows and first row of every expert (wave 0)
+    const SchedSpec spec = sb.spec[which];
+    const int nb_tall = (spec.N + 255) / 256;
+    const int nb_flat = (spec.N + 511) / 512;
+
+    // rows and first row of every expert, and the column blocks of its items (wave 0)
     if (wave == 0) {
         int run = 0;  // rows before this chunk (counts)
+        int n_wide = 0, n_narrow = 0;
         for (int base = 0; base < G; base += kWave) {
             const int g = base + lane;
             int m0 = 0, m1 = 0;
@@ -329,12 +347,19 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
                 sh.rows[g] = -1;  // (the ranking reads a few behind the last; smaller than any)
             }
             const int chunk_rows = wave_sum(g < G ? m1 - m0 : 0);
+            const ExpertShape e = expert_shape(g < G ? m1 - m0 : 0);
+            n_wide += wave_sum(e.tiles * (e.flat ? nb_flat : nb_tall));
+            n_narrow += wave_sum(e.tiles * nb_tall);
             if (lane == 0) {
                 sh.total_rows = (base == 0 ? 0 : sh.total_rows) + chunk_rows;
             }
         }
+        if (lane == 0) {
+            sh.narrow = n_wide > m && n_wide <= 2 * m && n_narrow <= 3 * m ? 1 : 0;
+        }
     }
     __syncthreads();
+    const bool narrow = sh.narrow != 0;
     // rank by rows, largest first (ties: lower index first); sixteen experts a turn, so that the reads overlap
     for (int g = tid; g < G; g += NT) {
         const int cnt = sh.rows[g];
@@ -355,18 +380,15 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
     }
     __syncthreads();
 
-    const SchedSpec spec = sb.spec[which];
     int32_t *sched = spec.sched;
     SchedItem *items = (SchedItem *)(sched + kSchedHeader);
-    const int nb_tall = (spec.N + 255) / 256;
-    const int nb_flat = (spec.N + 511) / 512;
 
     // by rank: items before, in all and per class.  One wave per prefix sum (class c, or the total for c == kClasses).
     for (int c = wave; c <= kClasses; c += NT / kWave) {
         int run = 0;
         for (int base = 0; base < G; base += kWave) {
             const int rank = base + lane;
-            const ExpertShape e = expert_shape(rank < G ? sh.rows[sh.order[rank]] : 0);
+            const ExpertShape e = expert_shape(rank < G ? sh.rows[sh.order[rank]] : 0, narrow);
             const int blocks = e.tall ? nb_tall : (e.flat ? nb_flat : 0);
             const int v = (c == kClasses ? e.tiles : class_count(e, c)) * blocks;
             const int inc = wave_inclusive_scan(v);
@@ -447,7 +469,7 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
         }
         const int rank = lo;
         const int eg = sh.order[rank];
-        const ExpertShape e = expert_shape(sh.rows[eg]);
+        const ExpertShape e = expert_shape(sh.rows[eg], narrow);
         const int local = i - sh.first_item[rank];
         int c, j, cls, pos;  // column block, row tile, class, place among the expert's items of that class
         if (e.flat) {
