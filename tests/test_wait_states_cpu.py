@@ -2,74 +2,10 @@
 the vector ALU has written within the five instructions before it (the CDNA ISA documents list that as a wait the program has
 to provide).  The compiler provides it for its own instructions, but not for the ones in inline assembly: the direct-to-LDS
 loads with a scalar base."""
-import os
-import re
-import struct
 import subprocess
 
-import pytest
-
 from umdk_original_amd import build
-
-OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
-MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
-WAIT_STATES = 5
-
-
-def _code_objects(path):
-    """The gfx950 code objects in a library's offload bundles."""
-    data = open(path, "rb").read()
-    at = data.find(MAGIC)
-    while at >= 0:
-        count, = struct.unpack_from("<Q", data, at + len(MAGIC))
-        pos = at + len(MAGIC) + 8
-        for _ in range(count):
-            offset, size, name = struct.unpack_from("<QQQ", data, pos)
-            target = data[pos + 24:pos + 24 + name].decode()
-            pos += 24 + name
-            if "gfx950" in target:
-                yield data[at + offset:at + offset + size]
-        at = data.find(MAGIC, at + len(MAGIC))
-
-
-def _scalars(operand):
-    m = re.match(r"s\[(\d+):(\d+)\]$", operand)
-    if m:
-        return set(range(int(m[1]), int(m[2]) + 1))
-    m = re.match(r"s(\d+)$", operand)
-    return {int(m[1])} if m else set()
-
-
-def _operands(text):
-    return [w for part in text.split(None, 1)[1:] for t in part.split(",") for w in t.split()]
-
-
-WRITES_SCALAR = re.compile(r"v_(readfirstlane|readlane|cmpx?_|add_co|sub_co|addc_co|subb_co|div_scale)")
-NO_RESULT = re.compile(r"s_(waitcnt|nop|cbranch|branch|barrier|cmp|bitcmp|setprio|sleep|endpgm|sethalt)")
-
-
-def _too_close(code):
-    """Vector memory instructions that read a scalar register the vector ALU wrote fewer than WAIT_STATES before."""
-    found = []
-    for k, text in enumerate(code):
-        if not re.match(r"(global|buffer|flat|scratch)_", text):
-            continue
-        want = set().union(*(_scalars(o) for o in _operands(text)), set())
-        states, j = 0, k - 1
-        while want and j >= 0 and states < WAIT_STATES:
-            before = code[j]
-            operands = _operands(before)
-            if WRITES_SCALAR.match(before):
-                # the result is the first operand, or the second of those that have a carry or a condition beside it
-                if any(_scalars(o) & want for o in operands[:2] if not before.startswith("v_read") or o is operands[0]):
-                    found.append(" ; ".join(code[j:k + 1]))
-                    break
-            elif before.startswith("s_") and not NO_RESULT.match(before) and operands:
-                want -= _scalars(operands[0])   # what is read is the scalar ALU's, which needs no wait
-            m = re.match(r"s_nop (\d+)", before)
-            states += int(m[1]) + 1 if m else 1
-            j -= 1
-    return found
+from umdk_original_amd.machine_code import OBJDUMP, code_objects as _code_objects, too_close as _too_close
 
 
 def test_the_check_sees_what_it_is_for():
@@ -82,7 +18,6 @@ def test_the_check_sees_what_it_is_for():
     assert not _too_close(["v_readlane_b32 s7, v255, s4", "global_store_dword v0, v1, s[4:5]"])
 
 
-@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
 def test_no_load_reads_a_scalar_too_soon(tmp_path):
     objects = list(_code_objects(build.LIB_PATH))
     assert len(objects) >= 5    # plan, dispatch, combine, and the two GEMMs

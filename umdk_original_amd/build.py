@@ -5,10 +5,15 @@ the host compiler, all in-tree.
 `python -m umdk_original_amd.build --timeline` builds a second library beside them, libcam_mi355x_timeline.so:
 the same sources with -DCAM_GEMM_TIMELINE, whose grouped-GEMM kernel stamps every tile of its schedule with
 the device clock.  It is a profiling aid and is only loaded when CAM_MI355X_LIB names it.  libcam_calib.so holds the
-calibration micro-benchmarks behind `bench.py --only calib` and nothing of the product."""
+calibration micro-benchmarks behind `bench.py --only calib` and nothing of the product.
+
+The machine code of either kernel library is looked over before the build is done (machine_code.py): its inline assembly rests
+on what the compiler makes of the code around it, and a library for which that does not hold is removed again."""
 import os
 import subprocess
 import sys
+
+from . import machine_code
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 _CSRC = os.path.join(_PKG, "csrc")
@@ -31,7 +36,7 @@ HIPCC_FLAGS = [
 
 
 def build(verbose=False, timeline=False):
-    """Compile every source and link the shared library. Always recompiles."""
+    """Compile every source, link the shared library and look its machine code over. Always recompiles."""
     os.makedirs(LIB_DIR, exist_ok=True)
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     objs = []
@@ -58,6 +63,11 @@ def build(verbose=False, timeline=False):
     subprocess.check_call(cmd)
     for o in objs:
         os.remove(o)
+    try:
+        machine_code.check(out_path)
+    except Exception:
+        os.remove(out_path)  # nothing is to load it
+        raise
     if not timeline:
         build_calib(verbose)
         build_abi_consumer(verbose)

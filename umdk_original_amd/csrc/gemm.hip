@@ -89,7 +89,7 @@ __device__ __forceinline__ v4i buffer_words(const void *p, unsigned bytes)
 // Loads.  A vector memory instruction must not read a scalar register that the vector ALU wrote within five wait states, and the
 // compiler does not see to that for inline assembly.  Where a scalar operand may come out of a register the compiler had
 // parked in a vector lane (in front of the K loop; anywhere in the FP8 kernel, whose multiplications leave room for it),
-// WAITS provides the five.  A test looks the built code over.
+// WAITS provides the five.  The build looks the code over that the compiler made of this (machine_code.py).
 
 // One direct-to-LDS load: lane i of the wave fetches 16 bytes at its offset from the base, and the data lands at LDS byte
 // address lds_addr + LDS_OFFSET + 16*i.  Base and offsets are scalar but for one vector register, so that issuing the load
@@ -382,7 +382,7 @@ __device__ __forceinline__ void k_loop(const GemmArgs &a, const ItemCtx &t, int8
         request16<off, STREAM, decltype(wc)::value>(dst[j], words, nf < 2 ? b_voff0 : b_voff1, (unsigned)(k * b_step));
     };
     // The registers of a sub-step are passed through the wait for them: nothing that reads them is moved in front of it.
-    // (Between the request and here nothing may read or move them at all; a test looks the built code over.)
+    // (Between the request and here nothing may read or move them at all; the build looks the code over, machine_code.py.)
     auto landed = [&](v4i (&r)[NB]) {
         if constexpr (NB == 4) {
             asm volatile("s_waitcnt vmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(WAIT) : "memory");
