@@ -28,7 +28,8 @@ constexpr int kSchedQueueCount = 544;
 constexpr int kSchedQueueStride = 32;
 constexpr int kSchedHeader = kSchedQueueCount + kMaxQueues * kSchedQueueStride;
 // One work item: rows [m0, m0 + rows) of expert g times column block nb.  flat != 0: at most 128 rows x 512 packed
-// columns; flat == 0: at most 256 rows x 256 packed columns.  split: half of a tall tile's rows, a multiple of 32.
+// columns; flat == 0: at most 256 rows x 256 packed columns.  split: half of a tall tile's rows, a multiple of 32; a
+// record for whoever reads the schedule back, no kernel looks at it.
 struct SchedItem {
     int32_t g, m0, rows, split, nb, flat, pad0, pad1;
 };

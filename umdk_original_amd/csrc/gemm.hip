@@ -18,8 +18,9 @@
 //     small items for the end, where they even out the finishing times.
 //   * Two tile shapes.  Tall tiles (up to 256 rows) x 256 columns: a wave owns ALL rows of the tile and 64 of its columns.
 //     Flat tiles (<= 128 rows) x 512 columns, for experts that only stream weights: all rows and 128 columns (in a narrow
-//     schedule, sched_device.h, x 256 like tall ones).  Either way a wave holds up to sixteen 32 x 32 sums (256 registers, all of the accumulation file).  The numbers of row and
-//     column fragments are template parameters, so the main loop has no control flow.
+//     schedule, sched_device.h, x 256 like tall ones).  Either way a wave holds up to sixteen 32 x 32 sums (256 registers, all
+//     of the accumulation file; a narrow item eight of them at most).  The numbers of row and column fragments are template
+//     parameters, so the main loop has no control flow.
 //   * A weight byte is needed by one wave only.  It goes from memory straight to that wave's registers (prepack_kernel laid
 //     the weights out in the lane order the MFMA wants), a ring of four 64-byte K steps.  Only the activations go
 //     through LDS: direct-to-LDS loads (16 bytes per lane, no registers) into a ring of four stages of 128 K bytes, a
@@ -46,7 +47,8 @@
 //     stored.  For GMM1 the prepack pairs gate column c with up column I+c inside one wave.
 //   * The K order inside a 32-deep MFMA step is whatever the two operands agree on (an integer dot
 //     product does not care), which is what lets both be loaded as plain 16-byte pieces.
-//   * Flat items are bound by the memory; their weight panels are fetched with non-temporal loads (nobody else reads them).
+//   * Flat items are bound by the memory; their weight panels are fetched with non-temporal loads (nobody else reads them), and so
+//     are those of narrow items of up to 96 rows.
 //   * Between two items.  What a workgroup has to know and to fetch before it can multiply is asked for during the item before
 //     (ask_ahead, publish): from an item's start to its first multiplication it is 2 us instead of 4, of which the
 //     requests for the weights take most.  Layers of 8192 / 1021 tokens 1567 -> 1535 / 181 -> 176 us, FP8 layer of 4093
@@ -327,7 +329,14 @@ template <int MF, int NF, bool FP8, typename Publish>
 __device__ __forceinline__ void k_loop(const GemmArgs &a, const ItemCtx &t, int8_t *lds, const uint8_t *a_scale8_s,
                                        Publish &publish)
 {
-    constexpr bool STREAM = NF == 4 || MF < 4;      // a flat or a narrow item is the only reader of its weight panel
+    // A flat item is the only reader of its weight panel, and so is one of 256 columns and up to three row units, which only narrow
+    // schedules hold.  Four units are either a narrow item of 97-128 rows, the only reader too, or the lower of the two tiles of
+    // an expert of 257-288 rows, whose panel the other one shares; they run the same code and load plainly.  us, streaming items of
+    // 256 columns never / up to three / up to four units: layer of 1021 fp16 tokens x 2048, top-6 of 64 experts, I 1408 166.3 /
+    // 161.2 / 161.1, of 1150 tokens 176.1 / 168.7 / 167.4, FP8 layer of 1900 x 4096, top-2 of 40, I 2048 246.3 / 236.6 / 233.2; both GEMMs
+    // over 272 rows on each of 128 experts, H 4096, I 1536 (three / four units) 855 / 929, on each of 32, H 7168, I 2048 604 / 564, over 288
+    // on each of 8, H 4096, I 2048 112 / 123.
+    constexpr bool STREAM = NF == 4 || MF < 4;
     constexpr int SLOTS = FP8 ? MF : 2 * MF;
     constexpr int AR = FP8 ? 4 : 8;                 // fragments in registers
     constexpr int PD = FP8 ? (MF == 1 ? 2 : 3) : (MF == 1 ? 4 : 6);  // (at most a stage)
@@ -939,7 +948,10 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
                 for (int q = 0; q < KB >> 2; ++q) {
                     dma4(words, (unsigned)(row * KB + 4 * q), to + (unsigned)(q * 1024));
                 }
-            } else {  // (rows that are no whole words)
+            } else {
+                // Rows that are no whole words go through registers byte by byte, in front of the epilogue: up to 5 us of a tile.
+                // FP8 GEMM of two tiles of 256 rows a workgroup, N 4096, K / 128 = 12 13 15 16: 68.5 72.4 84.0 80.0 us; 40 41 43 44: 164.9
+                // 163.9 182.9 175.9.
                 for (int kb = 0; kb < KB; ++kb) {
                     a_scale8_s[((kb >> 2) * 256 + wave * kWave + lane) * 4 + (kb & 3)] = base[(long long)row * KB + kb];
                 }
@@ -1058,7 +1070,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
             int32_t *stamp = (int32_t *)&items[cur_idx];
             stamp[6] = (int32_t)timeline_t0;
             stamp[7] = (int32_t)wall_clock64();
-            stamp[3] = (stamp[3] & 0xffff) | ((int)blockIdx.x << 16);  // split is read at the start of the item only
+            stamp[3] = (stamp[3] & 0xffff) | ((int)blockIdx.x << 16);  // (no kernel reads split)
             // ticks from the start of the item to its first multiply and to the end of its K loop, in the upper
             // halves of the column-block and shape words (both below 2^16 and read before an item starts)
             const int d1 = min(max(phase_s[0] - (int32_t)timeline_t0, 0), 0xffff);
