@@ -226,8 +226,8 @@ def _check_fused(oracle, d, x, idx_np, E, quant_mode, fp16=False):
 @pytest.mark.parametrize("T,K,E,H,dtype,neg", [
     (1, 1, 2, 1024, torch.int64, 0.0),
     (37, 3, 8, 1024, torch.int32, 0.2),
-    (300, 8, 256, 7168, torch.int64, 0.0),     # two chunks of 2048 ids
-    (1500, 16, 512, 1032, torch.int64, 0.05),  # twelve chunks, odd row length
+    (300, 8, 256, 7168, torch.int64, 0.0),     # ten chunks of 256 ids
+    (1500, 16, 512, 1032, torch.int64, 0.05),  # 47 chunks of 512 ids, odd row length
 ])
 def test_dispatch_prefill_operator(gpu, oracle, T, K, E, H, dtype, neg, quant_mode):
     announce("dispatch prefill T=%d K=%d E=%d H=%d quant=%d" % (T, K, E, H, quant_mode))

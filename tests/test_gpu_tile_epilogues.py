@@ -154,7 +154,7 @@ def test_fp8_sums(gpu, oracle, sizes, K, N, gate_up):
 
 
 @pytest.mark.parametrize("sizes,K,N", [
-    (MIXED, 256, 2304),              # 9 tall and 4.5 flat column blocks: the last flat item has one live team
+    (MIXED, 256, 2304),              # 9 tall and 4.5 flat column blocks: the last two waves of the last flat item have no columns
     (MIXED, 640, 2816),              # 5.5 flat blocks; scales that are no whole words
     ([700, 130, 1, 1000], 4096, 2560),
     (FP8_FLAT, 256, 13568),          # flat tiles alone, 26.5 blocks
@@ -260,3 +260,75 @@ def test_random_shapes_bit_exact(gpu, oracle, seed):
     out = cam.grouped_matmul_dequant(y, ys, cam.prepack_weight(w2.to(gpu), False), w2s.to(gpu), given, list_type)
     c = oracle.gmm_int32(want, w2.numpy(), gl.numpy())
     assert_bits_equal(to_np(out), oracle.gmm2_epilogue(c, w2s.numpy(), want_s, gl.numpy()), "rows")
+
+
+# Rows per expert at the edges of every number of row fragments a narrow tile has, and column counts for which the items of a
+# launch are more than the CUs (256) and at most two for each, and at most three with the flat ones cut in two.
+NARROW = [1, 31, 32, 33, 64, 65, 96, 97, 127, 128] * 4 + [0]
+
+
+def _narrow_tiles(sizes, N, gpu):
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    cut = sum((s + 255) // 256 for s in sizes) * ((N + 255) // 256)
+    wide = _tiles(sizes, N)
+    if cus == 256:
+        assert cus < wide <= 2 * cus and cut <= 3 * cus
+    return cut if cus < wide <= 2 * cus and cut <= 3 * cus else wide
+
+
+@pytest.mark.parametrize("list_type", [0, 1])
+def test_narrow_int8_bit_exact(gpu, oracle, list_type):
+    H, I, N2 = 256, 1984, 4032   # 31 groups of 128 columns gate and up, 63 of 64: the last column block is ragged
+    announce("tile form, narrow tiles, int8: H=%d I=%d N2=%d list_type=%d" % (H, I, N2, list_type))
+    gl, x, xs, w, ws, wp, wsp = _int8_case(NARROW, H, 2 * I, 31, False, gpu, True)
+    given = gl.to(gpu) if list_type == 0 else torch.tensor(NARROW, dtype=torch.int64, device=gpu)
+    y, ys = cam.grouped_matmul_swiglu_quant(x.to(gpu), xs.to(gpu), wp, wsp, given, list_type)
+    c = oracle.gmm_int32(x.numpy(), w.numpy(), gl.numpy())
+    want, want_s = oracle.swiglu_quant(oracle.gmm1_epilogue(c, ws.numpy(), xs.numpy(), gl.numpy()), rows=x.size(0))
+    assert_bits_equal(to_np(ys).view(np.uint32), want_s.view(np.uint32), "y_scale")
+    assert_bits_equal(to_np(y), want, "y")
+    assert _scheduled("GroupedMatmulSwigluQuant", [x.to(gpu), xs.to(gpu), wp, wsp, given, list_type, y, ys],
+                      gpu) == _narrow_tiles(NARROW, 2 * I, gpu)
+    gl, x, xs, w, ws, wp, wsp = _int8_case(NARROW, 384, N2, 37, False, gpu)
+    c = oracle.gmm_int32(x.numpy(), w.numpy(), gl.numpy())
+    for fp16 in (False, True):
+        out = cam.grouped_matmul_dequant(x.to(gpu), xs.to(gpu), wp, wsp, given, list_type,
+                                         out_dtype=torch.float16 if fp16 else torch.bfloat16)
+        want = oracle.gmm2_epilogue_act(c, ws.numpy(), xs.numpy(), gl.numpy(), fp16)
+        assert_bits_equal(out.cpu().view(torch.int16).numpy().view(np.uint16), want, "rows")
+        assert _scheduled("GroupedMatmulDequant", [x.to(gpu), xs.to(gpu), wp, wsp, given, list_type, out],
+                          gpu) == _narrow_tiles(NARROW, N2, gpu)
+
+
+@pytest.mark.parametrize("K", [128, 384, 512])   # scales that are no whole words, and words
+def test_narrow_fp8(gpu, oracle, K):
+    """Tolerances of test_fp8_sums; the quantised product bit for bit, as above."""
+    announce("tile form, narrow tiles, fp8: K=%d" % K)
+    for N, gate_up in ((3840, True), (3968, False)):
+        gl, a, sa, w, sw, wp = _fp8_case(NARROW, K, N, gpu, gate_up)
+        c = oracle.fp8_gemm(_u8(a), sa.numpy(), _u8(w), sw.numpy(), gl.numpy())
+        want = oracle.fp8_swiglu(c) if gate_up else c
+        biggest = np.abs(want).max()
+        args = (a.to(gpu), sa.to(gpu), wp, sw.to(gpu), gl.to(gpu))
+        got = cam.grouped_matmul_fp8(*args)
+        assert (np.abs(got.cpu().numpy() - want) <= 1e-3 * np.abs(want) + 2e-4 * biggest).all()
+        s = None
+        if gate_up:
+            want_q, want_s = cam.quant_rows_fp8(got)
+            got, s = cam.grouped_matmul_fp8(*args, out_dtype=torch.float8_e4m3fn)
+            assert torch.equal(s, want_s) and np.array_equal(_u8(got), _u8(want_q))
+        else:
+            got = cam.grouped_matmul_fp8(*args, out_dtype=torch.bfloat16)
+            assert (np.abs(got.float().cpu().numpy() - want) <= (2.0 ** -8 + 1e-3) * np.abs(want) + 2e-4 * biggest).all()
+        assert _scheduled("GroupedMatmulFp8", [args[0], args[1], wp, args[3], 1 if gate_up else 0, args[4], 0, got, s],
+                          gpu) == _narrow_tiles(NARROW, N, gpu)
+
+
+def test_narrow_layer_bit_exact(gpu, oracle):
+    """The narrow schedule as the permute launch builds it."""
+    T, H, E, K, I = 1021, 512, 64, 6, 1152
+    announce("tile form, narrow tiles, layer T=%d H=%d E=%d K=%d I=%d" % (T, H, E, K, I))
+    d = _layer(T, H, E, K, I, 5)
+    out, etn = _run(gpu, d)
+    assert _check(oracle, d, out, etn) == 0
+    _narrow_tiles(etn.tolist(), 2 * I, gpu)
