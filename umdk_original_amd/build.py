@@ -8,7 +8,7 @@ the device clock.  It is a profiling aid and is only loaded when CAM_MI355X_LIB 
 calibration micro-benchmarks behind `bench.py --only calib` and nothing of the product.
 
 The machine code of either kernel library is looked over before the build is done (machine_code.py): its inline assembly rests
-on what the compiler makes of the code around it, and a library for which that does not hold is removed again."""
+on what the compiler makes of the code around it, and a library for which that does not hold is not kept."""
 import os
 import subprocess
 import sys
@@ -57,17 +57,21 @@ def build(verbose=False, timeline=False):
         if verbose and out.strip():
             print(out)
     out_path = TIMELINE_LIB_PATH if timeline else LIB_PATH
+    if os.path.exists(out_path):
+        os.remove(out_path)  # what is there to load is what this build has looked over, or nothing
+    unchecked = out_path + ".unchecked"
     # One soname for every build of the library: whichever is loaded first (CAM_MI355X_LIB) is the one that the torch
     # libraries below find, too.
-    cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-soname," + os.path.basename(LIB_PATH), "-o", out_path] + objs
+    cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-soname," + os.path.basename(LIB_PATH), "-o", unchecked] + objs
     subprocess.check_call(cmd)
     for o in objs:
         os.remove(o)
     try:
-        machine_code.check(out_path)
-    except Exception:
-        os.remove(out_path)  # nothing is to load it
-        raise
+        machine_code.check(unchecked)
+        os.replace(unchecked, out_path)
+    finally:
+        if os.path.exists(unchecked):
+            os.remove(unchecked)
     if not timeline:
         build_calib(verbose)
         build_abi_consumer(verbose)
