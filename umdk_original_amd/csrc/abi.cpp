@@ -337,6 +337,21 @@ hipError_t run_grouped_gemm(cam::GemmArgs g, const int64_t *group_list, int cumu
     return cam::launch_gemm(g, s);
 }
 
+// What is in front of a layer's GEMMs: plan, quantised rows and, unless they stream, their schedules.  With row_token the rows
+// stay one per token and GMM1 gathers them.
+hipError_t layer_plan(const cam::PlanArgs &p, const cam::DispatchArgs &d, const cam::SchedSpec *specs, int32_t *row_token,
+                      bool stream, hipStream_t s)
+{
+    if (row_token != nullptr) {
+        return cam::launch_plan_quant(p, d, row_token, specs, s);
+    }
+    const hipError_t e = cam::launch_plan_dispatch(p, d, s);
+    if (e != hipSuccess || stream) {
+        return e;
+    }
+    return cam::launch_build_sched(p.tokens_per_expert, 0, p.E, d.A, 2, specs, s);
+}
+
 // The GEMMs of a fused layer: per-expert counts from its plan, g.sched filled when the permute built schedules.  A token
 // names an expert once, so no expert has more than T rows.
 hipError_t layer_gemm(const cam::GemmArgs &g, const int64_t *counts, int E, int64_t A, int T, bool stream, hipStream_t s,
@@ -1807,10 +1822,13 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     // Few rows: the GEMMs need no schedule.  Fewer still: GMM2 quantises the products itself, and then writes its rows while
     // they are still read.
     const bool stream = cam::stream_gemm_applies(A, 2 * I, Epr, false);
+    // Where there is a schedule, GMM1 gathers its rows from the quantised tokens: a row per token and not one per copy.
+    const bool gather = !stream && cam::gemm_gathers(T, H);
     const bool from_products = stream && cam::stream_gemm_takes_products(A, (int)Epr, (int)I, (int)H, T);
     Carver c;
     const uint64_t o_pos = c.take((uint64_t)A * 4);
     const uint64_t o_row = c.take((uint64_t)A * 4);
+    const uint64_t o_token = gather ? c.take((uint64_t)A * 4) : 0;
     const uint64_t o_meta = c.take(cam::kPlanMeta * 4);
     const uint64_t o_sched1 = stream ? 0 : c.take(cam::sched_bytes(A, (int)Epr, (int)(2 * I)));
     const uint64_t o_sched2 = stream ? 0 : c.take(cam::sched_bytes(A, (int)Epr, (int)H));
@@ -1818,7 +1836,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     // The bf16 rows GMM2 writes (2*A*H bytes) live where the quantised rows (A*H) and the fp32 SwiGLU products
     // (4*A*I) lived: both are dead once the re-quantisation has run (the reference overlays its stages the same
     // way, AK/fused_deep_moe/op_kernel/fused_deep_moe.h:362-391).  GMM2's own input stays apart.
-    const uint64_t x1_bytes = align_up((uint64_t)A * H);
+    const uint64_t x1_bytes = align_up((uint64_t)(gather ? T : A) * H);
     const uint64_t shared_bytes = std::max<uint64_t>((uint64_t)A * H * 2, x1_bytes + (uint64_t)A * I * 4);
     const uint64_t o_x1 = c.take(shared_bytes);
     const uint64_t o_prod = o_x1 + x1_bytes;
@@ -1877,22 +1895,15 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         d.quant = 2;
         d.out = x1;
         d.scales = x1s;
-        if (!stream) {
-            // the plan has written the per-expert counts: spare workgroups of the permute build both schedules
-            d.sched.group_list = etn;
-            d.sched.cumulative = 0;
-            d.sched.G = iE;
-            d.sched.nspec = 2;
-            d.sched.max_rows = A;
-            d.sched.spec[0] = specs[0];
-            d.sched.spec[1] = specs[1];
-        }
-        e = cam::launch_plan_dispatch(p, d, s);
+        int32_t *token = (int32_t *)(w + o_token);
+        e = layer_plan(p, d, specs, gather ? token : nullptr, stream, s);
         if (e != hipSuccess) return e;
 
         cam::GemmArgs g1{};
         g1.a = x1;
         g1.a_scale = x1s;
+        g1.a_rows = gather ? token : nullptr;
+        g1.a_count = iT;
         g1.w = w1.w;
         g1.w_scale = w1.s;
         g1.per_expert = w1.per_expert;
@@ -2167,15 +2178,17 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
     cam::SchedSpec sp1 = sched_spec(A, E, 2 * I);
     cam::SchedSpec sp2 = sched_spec(A, E, H);
     const bool stream = cam::stream_gemm_applies(A, 2 * I, E, true);   // few rows: no schedules
+    const bool gather = !stream && cam::gemm_gathers(T, H);  // GMM1 gathers its rows from the quantised tokens
     Carver c;
     const uint64_t o_pos = c.take((uint64_t)A * 4);
     const uint64_t o_row = c.take((uint64_t)A * 4);
+    const uint64_t o_token = gather ? c.take((uint64_t)A * 4) : 0;
     const uint64_t o_meta = c.take(cam::kPlanMeta * 4);
     const uint64_t o_sched1 = stream ? 0 : c.take(cam::sched_bytes(A, (int)E, (int)(2 * I)));
     const uint64_t o_sched2 = stream ? 0 : c.take(cam::sched_bytes(A, (int)E, (int)H));
     const uint64_t o_hist = c.take(cam::plan_workspace_bytes(T, K, (int)E));
     // as in the int8 layer, the bf16 rows of GMM2 overlay the quantised input rows and the fp32 products
-    const uint64_t x1_bytes = align_up((uint64_t)A * H);
+    const uint64_t x1_bytes = align_up((uint64_t)(gather ? T : A) * H);
     const uint64_t shared_bytes = std::max<uint64_t>((uint64_t)A * H * 2, x1_bytes + (uint64_t)A * I * 4);
     const uint64_t o_x1 = c.take(shared_bytes);
     const uint64_t o_prod = o_x1 + x1_bytes;
@@ -2234,16 +2247,8 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         d.quant = 3;
         d.out = x1;
         d.scales = (float *)x1s;
-        if (!stream) {
-            d.sched.group_list = etn;  // spare workgroups of the permute build both schedules
-            d.sched.cumulative = 0;
-            d.sched.G = iE;
-            d.sched.nspec = 2;
-            d.sched.max_rows = A;
-            d.sched.spec[0] = specs[0];
-            d.sched.spec[1] = specs[1];
-        }
-        e = cam::launch_plan_dispatch(p, d, s);
+        int32_t *token = (int32_t *)(w + o_token);
+        e = layer_plan(p, d, specs, gather ? token : nullptr, stream, s);
         if (e != hipSuccess) return e;
 
         cam::GemmArgs g1{};
@@ -2251,6 +2256,8 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         g1.w = w1.w;
         g1.fp8 = 1;
         g1.a_scale8 = x1s;
+        g1.a_rows = gather ? token : nullptr;
+        g1.a_count = iT;
         g1.w_scale8 = w1.s;
         g1.sched = specs[0].sched;
         g1.Kd = iH;

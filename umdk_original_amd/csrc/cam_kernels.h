@@ -120,14 +120,15 @@ struct DispatchArgs {
     // quant == 2 only: optional per-expert smooth scales fp32 [E,H].  Copy (t,k) is then quantised on its own,
     // from float(x[t]) * smooth[idx[t,k]] (moe_dispatch_shmem.h:693-733); idx must be set.
     const float *smooth;
-    // GEMM schedules to build in the same launch (sched.nspec > 0): sched.nspec extra workgroups do what
-    // launch_build_sched would, beside the ones that move rows.  The group list must be complete before the
-    // launch (it is when it comes from launch_plan on the same stream).  sched.queues is set by the launcher.
-    SchedBuild sched;
 };
 hipError_t launch_dispatch(const DispatchArgs &a, hipStream_t stream);
 // launch_plan, then launch_dispatch with a.dst_row == p.dst_row; for few ids both as one launch.
 hipError_t launch_plan_dispatch(const PlanArgs &p, const DispatchArgs &a, hipStream_t stream);
+// The first part of a layer whose gate/up GEMM gathers its rows, in two launches: the plan (int32 ids), every token quantised into
+// row t of a.out ([T,H]; a.quant 2 or 3) with its scales in row t of a.scales, row_token[row] the token of a row in the order of
+// the experts (GemmArgs::a_rows), and the schedules of both GEMMs (specs), what launch_build_sched makes of the plan's counts.
+hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &a, int32_t *row_token, const SchedSpec *specs,
+                             hipStream_t stream);
 
 // ---------------------------------------------------------------------------------------------
 // Combine.
@@ -168,6 +169,8 @@ enum GemmEpilogue { kEpiInt32 = 0, kEpiSwiglu = 1, kEpiDequantBf16 = 2, kEpiSwig
 struct GemmArgs {
     const int8_t *a;       // [A,Kd] int8
     const float *a_scale;  // [A]
+    const int32_t *a_rows; // optional [A]: row r of the GEMM is row a_rows[r] of a and of its scales, which then have a_count rows
+    int64_t a_count;       // (launch_gemm, where gemm_gathers says so)
     const int8_t *w;       // stacked packed weights [G,Kd,N] (per_expert == 0)
     const float *w_scale;  // stacked [G,N]
     int per_expert;        // weights given per expert through `list`
@@ -190,6 +193,7 @@ struct GemmArgs {
     uint8_t *out_scale8;   // kEpiSwigluFp8: [A, N/256]
 };
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t stream);
+bool gemm_gathers(int64_t a_count, int64_t Kd);  // whether launch_gemm takes a_rows for a matrix of this size
 
 // The same GEMM for few rows per expert (stream_gemm.hip): takes the row counts instead of a schedule (g.sched is
 // not used) and leaves kEpiInt32 to launch_gemm.

@@ -18,7 +18,6 @@
 #include "cam_kernels.h"
 #include "permute_device.h"
 #include "rank_device.h"
-#include "sched_device.h"
 
 namespace cam {
 
@@ -45,16 +44,7 @@ __device__ __forceinline__ long long dispatch_row(const DispatchArgs &a, int t, 
 template <int QUANT, int ACT>
 __global__ __launch_bounds__(kDispWaves * kWave, QUANT == 3 ? 3 : 4) void dispatch_kernel(DispatchArgs a)
 {
-    // The first workgroups of the launch build the GEMM schedules (they start first and finish under the row
-    // traffic of the others); they depend on nothing this launch writes.
-    __shared__ SchedShared sched_s;
-    const int builders = a.sched.nspec * a.sched.parts;
-    if ((int)blockIdx.x < builders) {
-        build_sched_part<kDispWaves * kWave>(sched_s, a.sched, (int)blockIdx.x / a.sched.parts,
-                                             (int)blockIdx.x % a.sched.parts, a.sched.parts);
-        return;
-    }
-    const int t = ((int)blockIdx.x - builders) * kDispWaves + (threadIdx.x >> 6);
+    const int t = (int)blockIdx.x * kDispWaves + (threadIdx.x >> 6);
     const int lane = threadIdx.x & (kWave - 1);
     if (t >= a.T) {
         return;
@@ -259,8 +249,7 @@ hipError_t launch_small(const PlanArgs &p, const DispatchArgs &a, hipStream_t st
 hipError_t launch_plan_dispatch(const PlanArgs &p, const DispatchArgs &a, hipStream_t stream)
 {
     const long long n = (long long)p.T * p.K;
-    // One launch up to 2048 ids, where the permute builds no schedules (their builders need the plan's counts first)
-    if (n > 0 && n <= kSmallIds && a.sched.nspec == 0) {
+    if (n > 0 && n <= kSmallIds) {  // one launch
         if (a.H % 8 != 0 || a.H / 8 > kDispMaxChunks * kWave || (a.quant == 3 && a.H % 128 != 0) ||
             (a.smooth != nullptr && a.quant != 2) || p.K > kMaxTopk || p.E > kMaxExperts) {
             return hipErrorInvalidValue;
@@ -274,38 +263,17 @@ hipError_t launch_plan_dispatch(const PlanArgs &p, const DispatchArgs &a, hipStr
     return launch_dispatch(a, stream);
 }
 
-hipError_t launch_dispatch(const DispatchArgs &a_in, hipStream_t stream)
+hipError_t launch_dispatch(const DispatchArgs &a, hipStream_t stream)
 {
-    if (a_in.T <= 0) {
-        if (a_in.sched.nspec > 0) {  // no rows to move, but the schedules are still owed
-            return launch_build_sched(a_in.sched.group_list, a_in.sched.cumulative, a_in.sched.G, a_in.sched.max_rows,
-                                      a_in.sched.nspec, a_in.sched.spec, stream);
-        }
+    if (a.T <= 0) {
         return hipSuccess;
     }
-    const DispatchArgs &a0 = a_in;
-    if (a0.H % 8 != 0 || a0.H / 8 > kDispMaxChunks * kWave || (a0.quant == 3 && a0.H % 128 != 0)) {
+    if (a.H % 8 != 0 || a.H / 8 > kDispMaxChunks * kWave || (a.quant == 3 && a.H % 128 != 0)) {
         return hipErrorInvalidValue;
     }
-    DispatchArgs a = a_in;
-    if (a.sched.nspec != 0) {
-        if (a.sched.nspec < 0 || a.sched.nspec > 2 || a.sched.G <= 0 || a.sched.G > kMaxExperts ||
-            a.sched.group_list == nullptr) {
-            return hipErrorInvalidValue;
-        }
-        const hipError_t qe = gemm_workgroups(&a.sched.queues);
-        if (qe != hipSuccess) {
-            return qe;
-        }
-        // a turn of items per builder workgroup where the item tables could be full
-        const int cap = max(a.sched.spec[0].max_items, a.sched.spec[a.sched.nspec - 1].max_items);
-        a.sched.parts = min(max((cap + kDispWaves * kWave - 1) / (kDispWaves * kWave), 1), 8);
-    } else {
-        a.sched.parts = 1;
-    }
-    dim3 grid((a.T + kDispWaves - 1) / kDispWaves + a.sched.nspec * a.sched.parts), block(kDispWaves * kWave);
+    dim3 grid((a.T + kDispWaves - 1) / kDispWaves), block(kDispWaves * kWave);
     if (a.smooth != nullptr) {
-        if (a.quant != 2 || a.idx == nullptr || a.sched.nspec != 0) {
+        if (a.quant != 2 || a.idx == nullptr) {
             return hipErrorInvalidValue;
         }
         if (a.x_is_fp16) {

@@ -185,7 +185,7 @@ __device__ __forceinline__ void barrier_no_fence()
 
 // What a wave needs to know about the item it works on (all wave-uniform).
 struct ItemCtx {
-    const int8_t *a_tile;   // first activation row of the tile
+    const int8_t *a_tile;   // first activation row of the tile; with a_rows, of the whole matrix
     const int8_t *wg;       // the expert's packed weights
     const float *sg;        // the expert's per-channel scales
     int g, m0, rows;        // expert, first row and rows of the tile
@@ -325,9 +325,9 @@ struct FragType<true> {
 //
 // The item's first two stages and its row scales have been requested (ask_ahead in gemm_kernel).  `publish` runs between the
 // requests and the wait for them.
-template <int MF, int NF, bool FP8, typename Publish>
+template <int MF, int NF, bool FP8, typename Publish, typename AskRows>
 __device__ __forceinline__ void k_loop(const GemmArgs &a, const ItemCtx &t, int8_t *lds, const uint8_t *a_scale8_s,
-                                       Publish &publish)
+                                       const int32_t *rows_s, Publish &publish, AskRows &ask_rows)
 {
     // A flat item is the only reader of its weight panel, and so is one of 256 columns and up to three row units, which only narrow
     // schedules hold.  Four units are either a narrow item of 97-128 rows, the only reader too, or the lower of the two tiles of
@@ -353,15 +353,20 @@ __device__ __forceinline__ void k_loop(const GemmArgs &a, const ItemCtx &t, int8
     // ---- activations: wave w brings tile rows 8 MF w .. 8 MF (w + 1) - 1, eight rows a load.  Lane i of a load brings row i / 8
     // of its eight and the 16-byte chunk whose swizzled slot is i % 8: chunk c of row r lies at slot c ^ (r / 2 % 8) of the
     // row's 128 bytes, so that sixteen neighbouring rows cover all 64 banks.  Rows beyond the tile are out of the
-    // descriptor's range, which the vector offset is checked against, and come as zeros.
-    const v4i a_words = buffer_words(t.a_tile, (unsigned)t.rows * (unsigned)t.Kd);
+    // descriptor's range, which the vector offset is checked against, and come as zeros.  Gathered rows (a_rows) lie anywhere in a
+    // matrix of less than 2^31 bytes.
+    const bool gather = a.a_rows != nullptr;
+    const v4i a_words = buffer_words(t.a_tile, (gather ? (unsigned)a.a_count : (unsigned)t.rows) * (unsigned)t.Kd);
     const unsigned a_dst = lds0 + (unsigned)(wave * (MF * 1024));
     unsigned a_voff[MF];
     static_for<0, MF>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         const int r = 8 * (wave * MF + j) + (lane >> 3);
         const int c16 = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
-        a_voff[j] = (unsigned)(r * t.Kd + c16);
+        a_voff[j] = (unsigned)((gather ? rows_s[r] : r) * t.Kd + c16);
+        if (gather && r >= t.rows) {
+            a_voff[j] = 0x80000000u;
+        }
     });
     auto bring = [&](int s, auto jc, auto wc) {  // load j of stage s
         constexpr int j = decltype(jc)::value;
@@ -530,6 +535,9 @@ __device__ __forceinline__ void k_loop(const GemmArgs &a, const ItemCtx &t, int8
     };
     int s0 = 0;
     for (; s0 + 1 < ST; s0 += 2) {
+        if (s0 == 2 && gather) {
+            ask_rows();
+        }
         stage(s0, std::integral_constant<int, 0>(), std::false_type());
         stage(s0, std::integral_constant<int, 1>(), std::false_type());
     }
@@ -816,6 +824,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
     __shared__ __attribute__((aligned(16))) float scale_s[FP8 ? 1 : 2][FP8 ? 4 : 256 + 8 * 64];
     __shared__ __attribute__((aligned(16))) uint8_t a_scale8_s[FP8 ? kScaleKb * 256 : 4];
     __shared__ __attribute__((aligned(16))) SchedItem next_s;
+    __shared__ __attribute__((aligned(16))) int32_t rows_s[256];  // with a_rows: where the rows of the item lie
     __shared__ int item_s;
 #ifdef CAM_GEMM_TIMELINE
     __shared__ int phase_s[2];
@@ -912,7 +921,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
         t.buf = buf;
         t.Kd = a.Kd;
         t.N = a.N;
-        t.a_tile = a.a + (long long)t.m0 * a.Kd;
+        t.a_tile = a.a_rows != nullptr ? a.a : a.a + (long long)t.m0 * a.Kd;
         t.wg = a.per_expert ? a.list.w[t.g] : a.w + (long long)t.g * a.Kd * a.N;
         t.sg = a.per_expert ? a.list.s[t.g] : a.w_scale + (long long)t.g * a.N;
 #ifdef CAM_GEMM_TIMELINE
@@ -932,16 +941,20 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
             if (j < t.mf) {
                 const int r = 8 * (wave * t.mf + j) + (lane >> 3);
                 const int c16 = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
-                const int at = min(r, t.rows - 1) * t.Kd;
+                const int rr = min(r, t.rows - 1);
+                const int at = (a.a_rows != nullptr ? rows_s[rr] : rr) * t.Kd;
                 dma16(tile, (unsigned)(at + c16), dst + (unsigned)(j * 1024));
                 dma16(tile, (unsigned)(at + min(kStageK + c16, t.Kd - 16)), dst + (unsigned)(kStage + j * 1024));
             }
         }
-        const int row = min(wave * kWave + lane, t.rows - 1);
+        const bool gather = a.a_rows != nullptr;
+        int row = min(wave * kWave + lane, t.rows - 1);
+        row = gather ? rows_s[row] : row;
+        const long long row0 = gather ? 0 : t.m0;
         const int ngroups = t.N / 64;
         if constexpr (FP8) {
             const int KB = t.Kd >> 7;
-            const uint8_t *base = a.a_scale8 + (long long)t.m0 * KB;
+            const uint8_t *base = a.a_scale8 + row0 * KB;
             if ((KB & 3) == 0) {
                 const unsigned long long words = scalar_address(base);
                 const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(a_scale8_s) + (unsigned)(wave * kWave * 4));
@@ -958,7 +971,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
             }
         } else if (a.epilogue != kEpiInt32) {
             const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(scale_s[t.buf]));
-            dma4(scalar_address(a.a_scale + t.m0), (unsigned)(row * 4), to + (unsigned)(wave * kWave * 4));
+            dma4(scalar_address(a.a_scale + row0), (unsigned)(row * 4), to + (unsigned)(wave * kWave * 4));
             const unsigned long long columns = scalar_address(t.sg);
             const int per_wave = t.flat ? 2 : 1;
             for (int gi = 0; gi < per_wave; ++gi) {
@@ -994,6 +1007,10 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
         t.rows = 0;
         if (idx >= 0) {
             t = decode(items[idx], buf);
+            if (a.a_rows != nullptr) {
+                rows_s[tid] = a.a_rows[t.m0 + min(tid, t.rows - 1)];
+                __syncthreads();
+            }
             ask_ahead(t);
 #ifdef CAM_GEMM_TIMELINE
             cur_idx = idx;
@@ -1026,8 +1043,20 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
 #endif
             }
         };
+        // With a_rows: where the rows of the next item lie, asked for in the third stage of the K loop.  Its descriptor has come (wave 0
+        // has waited for younger loads, and a barrier has followed), and every wave has its own item's rows in registers.  One
+        // more load in flight makes the waits that count them stricter, not laxer.
+        auto ask_rows = [&]() {
+            const int rows = __builtin_amdgcn_readfirstlane(next_s.rows);
+            if (rows > 0) {
+                const int m0 = __builtin_amdgcn_readfirstlane(next_s.m0);
+                const int lane = opaque(tid) & (kWave - 1);
+                dma4(scalar_address(a.a_rows + m0), (unsigned)(min(wave * kWave + lane, rows - 1) * 4),
+                     __builtin_amdgcn_readfirstlane(lds_address(rows_s) + (unsigned)(wave * kWave * 4)));
+            }
+        };
         auto run = [&](auto mc, auto nc) {
-            k_loop<decltype(mc)::value, decltype(nc)::value, FP8>(a, t, lds, a_scale8_s, publish);
+            k_loop<decltype(mc)::value, decltype(nc)::value, FP8>(a, t, lds, a_scale8_s, rows_s, publish, ask_rows);
         };
         if (t.flat) {
             const std::integral_constant<int, 4> nf;
@@ -1090,6 +1119,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
 __global__ __launch_bounds__(1024) void build_sched_kernel(SchedBuild sb)
 {
     __shared__ SchedShared sh;
+    load_group_list<1024>(sh, sb);
     build_sched_part<1024>(sh, sb, (int)blockIdx.y, (int)blockIdx.x, (int)gridDim.x);
 }
 
@@ -1320,9 +1350,16 @@ hipError_t launch_build_sched(const int64_t *group_list, int cumulative, int G, 
     return hipGetLastError();
 }
 
+// Offsets of gathered rows are 32 bits wide, half of which mean "none", and the next item's rows are asked for in the third stage of
+// the K loop.
+bool gemm_gathers(int64_t a_count, int64_t Kd)
+{
+    return a_count > 0 && Kd >= 4 * kStageK && a_count <= 0x7fffffff / Kd;
+}
+
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t stream)
 {
-    if (a.sched == nullptr) {
+    if (a.sched == nullptr || (a.a_rows != nullptr && !gemm_gathers(a.a_count, a.Kd))) {
         return hipErrorInvalidValue;
     }
     if (a.Kd % kStageK != 0 || a.Kd < kStageK || a.N % 64 != 0 || (a.gate_up && a.N % 128 != 0)) {

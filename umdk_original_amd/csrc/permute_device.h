@@ -243,6 +243,23 @@ __device__ __forceinline__ void quant_token_row_smooth(Row &r, const float *__re
     }
 }
 
+// QUANT 3: one E8M0 byte per 128 columns, written by the first of its sixteen threads.
+template <typename Row>
+__device__ __forceinline__ void store_row_scales8(const Row &r, uint8_t *scales, long long row, int H, int lane)
+{
+    const int nch = H >> 3;
+    uint8_t *sc = scales + row * (H >> 7);
+    if ((lane & 15) == 0) {
+#pragma unroll
+        for (int j = 0; j < Row::kChunks; ++j) {
+            const int c = j * Row::kLanes + lane;
+            if (c < nch) {
+                sc[c >> 4] = (uint8_t)r.scale8[j];
+            }
+        }
+    }
+}
+
 // Stores the row (quantised or raw) to output row `row`, with its scale and triple.
 template <int QUANT, typename Row>
 __device__ __forceinline__ void store_token_row(const Row &r, void *out, float *scales, int32_t *src_info,
@@ -269,17 +286,7 @@ __device__ __forceinline__ void store_token_row(const Row &r, void *out, float *
         }
     }
     if (QUANT == 3) {
-        // one E8M0 byte per 128 columns, written by the first of its sixteen threads
-        uint8_t *sc = (uint8_t *)scales + row * (H >> 7);
-        if ((lane & 15) == 0) {
-#pragma unroll
-            for (int j = 0; j < Row::kChunks; ++j) {
-                const int c = j * Row::kLanes + lane;
-                if (c < nch) {
-                    sc[c >> 4] = (uint8_t)r.scale8[j];
-                }
-            }
-        }
+        store_row_scales8(r, (uint8_t *)scales, row, H, lane);
     }
     if (lane == 0) {
         if (QUANT == 1 || QUANT == 2) {

@@ -1,6 +1,5 @@
-// Device code that builds the work-item schedule of the grouped GEMM: used by the stand-alone builder kernel and
-// by the permute kernel of the dispatch, one of whose spare workgroups builds each schedule of the GEMMs that
-// follow while the others move rows.
+// Device code that builds the work-item schedule of the grouped GEMM: used by the stand-alone builder kernel and, in a layer,
+// by workgroups of the plan's second launch.
 #ifndef CAM_SCHED_DEVICE_H_
 #define CAM_SCHED_DEVICE_H_
 
@@ -298,7 +297,18 @@ __device__ __forceinline__ void build_shared_queues(SchedShared &sh, const Sched
     }
 }
 
-// Schedule sb.spec[which]; called by all NT threads of a workgroup (NT a multiple of 64, at least 256).  `parts`
+// The group list of a schedule that build_sched_part starts from: in LDS (sh.order), clamped to the rows that exist so that a
+// corrupt list cannot index past the tensors.  (sh.order is free until the experts are ranked.)
+template <int NT>
+__device__ __forceinline__ void load_group_list(SchedShared &sh, const SchedBuild &sb)
+{
+    for (int g = threadIdx.x; g < sb.G; g += NT) {
+        sh.order[g] = (int)min(max(sb.group_list[g], (int64_t)0), (int64_t)sb.max_rows);
+    }
+    __syncthreads();
+}
+
+// Schedule sb.spec[which]; the group list lies in sh.order.  Called by all NT threads of a workgroup (NT a multiple of 64, at least 256).  `parts`
 // workgroups share a schedule: each works out the same tables in its own LDS, part 0 writes the header and the queue
 // tables, and the items go round the parts in turns of NT (placing an item costs about a microsecond of dependent
 // lookups and divisions, and a long schedule has several thousand).
@@ -311,12 +321,6 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
     const int wave = tid >> 6;
     const int m = min(max(sb.queues, 1), kMaxQueues);
 
-    // the group list, clamped to the rows that exist so that a corrupt list cannot index past the tensors
-    // (sh.order is free until the ranking below)
-    for (int g = tid; g < G; g += NT) {
-        sh.order[g] = (int)min(max(sb.group_list[g], (int64_t)0), (int64_t)sb.max_rows);
-    }
-    __syncthreads();
     const SchedSpec spec = sb.spec[which];
     const int nb_tall = (spec.N + 255) / 256;
     const int nb_flat = (spec.N + 511) / 512;
