@@ -16,6 +16,7 @@
 //      totals into offsets, and finishes its chunk.  The reference does this part on the CPU after a
 //      device-to-host copy.
 #include <algorithm>
+#include <type_traits>
 
 #include "cam_device.h"
 #include "cam_kernels.h"
@@ -50,11 +51,14 @@ __global__ __launch_bounds__(kLocalThreads) void plan_local_kernel(PlanArgs a, i
 // Phase 1 of a layer whose gate/up GEMM gathers its rows: the workgroups behind the nb that rank quantise the tokens, a wave each,
 // which depends on nothing that the plan finds out.  A token's row is stored once, not once per copy, and plainly: the GEMM
 // is to find it in a cache.  HBM bound where there are many tokens.  us, ranks + their second half + permute with schedules ->
-// this + phase 2 with schedules: 8192 tokens x 4096, top-8, int8 7.6 + 6.3 + 70.9 -> 21.5 + 22.1 (layer 1558 -> 1521); 4093 in
-// FP8 5.5 + 5.8 + 45.0 -> 19.2 + 16.5 (841 -> 828); 1021 x 2048, top-6, 4.8 + 4.8 + 9.1 -> 5.1 + 8.6 (165.8 -> 162.2).
-template <int IT, int QUANT, int ACT>
-__global__ __launch_bounds__(kLocalThreads, QUANT == 3 ? 3 : 4) void plan_quant_kernel(PlanArgs a, DispatchArgs d, int nb)
+// this + phase 2 with schedules: 8192 tokens x 4096, top-8, int8 7.6 + 6.3 + 70.9 -> 20.9 + 15.5 (layer 1512 -> 1474); 4093 in
+// FP8 5.5 + 5.8 + 45.0 -> 15.5 + 13.5 (823 -> 787); 1021 x 2048, top-6, 4.8 + 4.8 + 9.1 -> 5.0 + 7.5 (160.9 -> 158.9).  With
+// rows of 4096 columns in the registers for 7168, at 3 (FP8) and 4 waves a SIMD, FP8 took 19.2.
+template <int CHUNKS, int QUANT, int ACT>
+__global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 5) void plan_quant_kernel(PlanArgs a, DispatchArgs d,
+                                                                                                         int it, int nb)
 {
+    typedef TokenRow<CHUNKS, kWave> Row;
     static_assert(kLocalThreads == kDispWaves * kWave, "both kinds of workgroups are as large");
     __shared__ int hist[kLocalWaves * kMaxExperts];
     __shared__ int active_s;
@@ -62,8 +66,16 @@ __global__ __launch_bounds__(kLocalThreads, QUANT == 3 ? 3 : 4) void plan_quant_
     const int b = blockIdx.x;
     if (b < nb) {
         const int t_active = count_active(a.mask, a.T, tid, kLocalThreads, &active_s);
-        rank_chunk<int32_t, IT>((const int32_t *)a.idx, b, (long long)t_active * a.K, (long long)a.T * a.K, a.E, hist, a.pos,
-                                a.hist_ws + (long long)b * a.E);
+        auto rank = [&](auto ic) {
+            rank_chunk<int32_t, decltype(ic)::value>((const int32_t *)a.idx, b, (long long)t_active * a.K, (long long)a.T * a.K,
+                                                     a.E, hist, a.pos, a.hist_ws + (long long)b * a.E);
+        };
+        switch (it) {
+            case 1: rank(std::integral_constant<int, 1>()); break;
+            case 2: rank(std::integral_constant<int, 2>()); break;
+            case 4: rank(std::integral_constant<int, 4>()); break;
+            default: rank(std::integral_constant<int, 8>()); break;
+        }
         if (b == 0 && tid == 0) {
             a.hist_ws[(long long)nb * a.E] = t_active;
         }
@@ -74,13 +86,13 @@ __global__ __launch_bounds__(kLocalThreads, QUANT == 3 ? 3 : 4) void plan_quant_
     if (t >= d.T) {
         return;
     }
-    WaveRow r;
+    Row r;
     load_token_row(d.x, t, d.H, lane, r);
     quant_token_row<QUANT, ACT>(r, WaveMax());
     const int nch = d.H >> 3;
     v2u *dst = (v2u *)((int8_t *)d.out + (long long)t * d.H);
 #pragma unroll
-    for (int j = 0; j < WaveRow::kChunks; ++j) {
+    for (int j = 0; j < Row::kChunks; ++j) {
         const int c = j * kWave + lane;
         if (c < nch) {
             dst[c] = r.q[j];
@@ -415,11 +427,11 @@ template <int QUANT, int ACT>
 hipError_t launch_plan_quant_as(const PlanArgs &p, const DispatchArgs &d, int it, int nb, hipStream_t stream)
 {
     const dim3 grid((unsigned)nb + (unsigned)((d.T + kDispWaves - 1) / kDispWaves)), block(kLocalThreads);
-    switch (it) {
-        case 1: hipLaunchKernelGGL((plan_quant_kernel<1, QUANT, ACT>), grid, block, 0, stream, p, d, nb); break;
-        case 2: hipLaunchKernelGGL((plan_quant_kernel<2, QUANT, ACT>), grid, block, 0, stream, p, d, nb); break;
-        case 4: hipLaunchKernelGGL((plan_quant_kernel<4, QUANT, ACT>), grid, block, 0, stream, p, d, nb); break;
-        default: hipLaunchKernelGGL((plan_quant_kernel<8, QUANT, ACT>), grid, block, 0, stream, p, d, nb); break;
+    // rows of up to 4096 columns in registers for 4096: more waves to a SIMD
+    if (d.H <= 8 * kWave * 8) {
+        hipLaunchKernelGGL((plan_quant_kernel<8, QUANT, ACT>), grid, block, 0, stream, p, d, it, nb);
+    } else {
+        hipLaunchKernelGGL((plan_quant_kernel<kDispMaxChunks, QUANT, ACT>), grid, block, 0, stream, p, d, it, nb);
     }
     return hipGetLastError();
 }
@@ -486,9 +498,10 @@ hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &d, int32_t *
     if (e != hipSuccess) {
         return e;
     }
-    // a turn of items per builder workgroup where the item tables could be full
+    // a turn of items per builder workgroup where the item tables could be full: nothing else waits for the CUs, and with at
+    // most 8 builders and 64-bit divisions in their turns phase 2 took 22.1 us at 8192 tokens
     const int cap = std::max(specs[0].max_items, specs[1].max_items);
-    l.sched.parts = std::min(std::max((cap + kGlobalThreads - 1) / kGlobalThreads, 1), 8);
+    l.sched.parts = std::min(std::max((cap + kGlobalThreads - 1) / kGlobalThreads, 1), 32);
     if (d.quant == 3) {
         e = launch_plan_quant_as<3, 0>(p, d, it, nb, stream);
     } else {

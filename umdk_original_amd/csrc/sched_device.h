@@ -70,8 +70,11 @@ __device__ __forceinline__ ExpertShape expert_shape(int rows, bool narrow = fals
     e.flat = rows > 0 && !e.tall;
     e.units = (rows + 31) / 32;
     e.tiles = e.tall ? (rows + 255) / 256 : (e.flat ? 1 : 0);
-    e.base = e.tall ? e.units / e.tiles : 0;
-    e.extra = e.tall ? e.units % e.tiles : 0;
+    // units / tiles without a division: units = 8 tiles - d with d < 8, so it is 8 - d / tiles, rounded up
+    const int d = 8 * e.tiles - e.units;
+    const int low = e.tiles == 1 ? d : (d > 0) + (d > e.tiles) + (d > 2 * e.tiles) + (d > 3 * e.tiles);
+    e.base = e.tall ? 8 - low : 0;
+    e.extra = e.tall ? e.units - e.base * e.tiles : 0;
     return e;
 }
 
@@ -96,7 +99,7 @@ struct SchedOwnTables {
 struct SchedSharedTables {
     int work_before[kMaxExperts];         // by rank: work of the tall experts ranked before
     int flat_rank[kMaxExperts];           // by rank: flat experts ranked before
-    short ngroups[kNumXcd][kMaxExperts];  // by rank: the expert's groups in queue x (tall)
+    short cfirst[kNumXcd + 1][kMaxExperts];  // by rank: the expert's groups in queues before x (tall)
     int qbase[kNumXcd][kMaxExperts];      // by rank: items of earlier experts of its kind in queue x
     int qtall[kNumXcd], qflat[kNumXcd];
     int wtotal;
@@ -114,17 +117,23 @@ struct SchedShared {
     int narrow;
 };
 
-// Shared queues: the queue of the tall group whose work (in row units) starts at `before` and is `units` long is
-// the one its middle falls into when the total work is cut into eight equal runs.
-__device__ __forceinline__ int queue_of_group(long long before, int units, long long wtotal)
+// Shared queues: a tall group (units of work, in row units) belongs to the queue its middle falls into when the total work is cut
+// into eight equal runs.  The groups of an expert follow one another from `before` on, so those in queues before x are the
+// first ones: as many as have 8 (2 (before + c units) + units) < 2 x wtotal.
+__device__ __forceinline__ int groups_before_queue(int x, long long before, int units, int groups, long long wtotal)
 {
-    const long long mid16 = (2 * before + units) * kNumXcd;  // 2 * middle * 8
-    int x = 0;
-#pragma unroll
-    for (int k = 1; k < kNumXcd; ++k) {
-        x += mid16 >= 2 * wtotal * k ? 1 : 0;
+    const long long lead = 2 * x * wtotal - kNumXcd * (2 * before + units);
+    if (lead <= 0) {
+        return 0;
     }
-    return x;
+    const long long step = 2 * kNumXcd * (long long)units;
+    if (lead > step * (groups - 1)) {
+        return groups;
+    }
+    if (lead + step <= 0x7fffffff) {  // (64-bit divisions are several times as long)
+        return (int)(((unsigned)lead + (unsigned)step - 1) / (unsigned)step);
+    }
+    return (int)((lead + step - 1) / step);
 }
 
 // Workgroup of column j when the columns are numbered XCD by XCD.
@@ -209,13 +218,11 @@ __device__ __forceinline__ void build_shared_queues(SchedShared &sh, const Sched
             if (flat_wave) {
                 v = (e.flat && t.flat_rank[rank] % kNumXcd == x) ? nb_flat : 0;
             } else if (e.tall) {
-                int mine = 0;
-                const long long before = t.work_before[rank];
-                for (int c = 0; c < nb_tall; ++c) {
-                    mine += queue_of_group(before + (long long)c * e.units, e.units, wtotal) == x ? 1 : 0;
-                }
-                t.ngroups[x][rank] = (short)mine;
-                v = mine * e.tiles;
+                const int c0 = x == 0 ? 0 : groups_before_queue(x, t.work_before[rank], e.units, nb_tall, wtotal);
+                const int c1 = x == kNumXcd - 1 ? nb_tall
+                                                : groups_before_queue(x + 1, t.work_before[rank], e.units, nb_tall, wtotal);
+                t.cfirst[x][rank] = (short)c0;
+                v = (c1 - c0) * e.tiles;
             }
             const int inc = wave_inclusive_scan(v);
             if (rank < G && (flat_wave ? e.flat : e.tall)) {
@@ -256,34 +263,35 @@ __device__ __forceinline__ void build_shared_queues(SchedShared &sh, const Sched
         const int eg = sh.order[rank];
         const ExpertShape e = expert_shape(sh.rows[eg]);
         const int local = i - sh.first_item[rank];
-        const int c = local / e.tiles;
+        const int c = (int)((unsigned)local / (unsigned)e.tiles);
         const int j = local - c * e.tiles;
         int x, qpos;
         if (e.flat) {
             x = t.flat_rank[rank] % kNumXcd;
             qpos = t.qbase[x][rank] + c;
         } else {
-            x = queue_of_group(t.work_before[rank] + (long long)c * e.units, e.units, wtotal);
-            int cfirst = 0;  // the expert's groups in earlier queues
-            for (int xx = 0; xx < x; ++xx) {
-                cfirst += t.ngroups[xx][rank];
+            x = 0;
+#pragma unroll
+            for (int k = 1; k < kNumXcd; ++k) {
+                x += c >= t.cfirst[k][rank] ? 1 : 0;
             }
-            qpos = t.qbase[x][rank] + (c - cfirst) * e.tiles + j;
+            qpos = t.qbase[x][rank] + (c - t.cfirst[x][rank]) * e.tiles + j;
         }
         {
             // Queue order: the flat items spread evenly among the tall ones (flat item j has key (2j+1)/(2F), tall
             // item i key (2i+1)/(2T), smaller keys first, a tall item first on a tie), except that the last
             // kTallTail tall items follow the last flat one.
-            const long long F = t.qflat[x];
-            const long long T = max(t.qtall[x] - kTallTail, 0);
-            if (e.flat) {
-                const long long num = (2ll * qpos + 1) * T - F;
-                qpos += (int)(num < 0 ? 0 : min(T, num / (2 * F) + 1));
-            } else if (qpos < T) {
-                const long long num = (2ll * qpos + 1) * F - T;
-                qpos += (int)(num <= 0 ? 0 : min(F, (num + 2 * T - 1) / (2 * T)));
+            const int F = t.qflat[x];
+            const int T = max(t.qtall[x] - kTallTail, 0);
+            const int other = e.flat ? T : F, own = e.flat ? F : T;
+            if (!e.flat && qpos >= T) {
+                qpos += F;
             } else {
-                qpos += (int)F;
+                const long long num = (2ll * qpos + 1) * other - own + (e.flat ? 2 * own : 2 * own - 1);
+                if (num >= 2 * own) {  // (a flat item's place is one further where both would have the same)
+                    const long long q = num <= 0x7fffffff ? (long long)((unsigned)num / (2 * (unsigned)own)) : num / (2 * own);
+                    qpos += (int)min((long long)other, q);
+                }
             }
         }
         int pos = qpos;
@@ -364,11 +372,14 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
     }
     __syncthreads();
     const bool narrow = sh.narrow != 0;
-    // rank by rows, largest first (ties: lower index first); sixteen experts a turn, so that the reads overlap
-    for (int g = tid; g < G; g += NT) {
+    // rank by rows, largest first (ties: lower index first); four, two or one threads per expert, each looking at sixteen others a
+    // turn, so that the reads overlap
+    const int share = 4 * G <= NT ? 2 : (2 * G <= NT ? 1 : 0);  // (log2)
+    for (int i = tid; i < G << share; i += NT) {
+        const int g = i >> share;
         const int cnt = sh.rows[g];
         int rank = 0;
-        for (int j = 0; j < G; j += 16) {
+        for (int j = (i & ((1 << share) - 1)) * 16; j < G; j += 16 << share) {
             v4i r[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -380,6 +391,8 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
                 rank += (rj > cnt || (rj == cnt && j + q < g)) ? 1 : 0;
             }
         }
+        rank += share > 0 ? __shfl_xor(rank, 1, kWave) : 0;
+        rank += share > 1 ? __shfl_xor(rank, 2, kWave) : 0;
         sh.order[rank] = g;
     }
     __syncthreads();
@@ -482,7 +495,7 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
             cls = 0;
             pos = local;
         } else {
-            c = local / e.tiles;
+            c = (int)((unsigned)local / (unsigned)e.tiles);
             j = local - c * e.tiles;
             const bool taller = j < e.extra;
             cls = taller ? e.base + 1 : e.base;
@@ -493,7 +506,7 @@ __device__ __forceinline__ void build_sched_part(SchedShared &sh, const SchedBui
         {
             const bool small = s >= n_big;
             const int cols = small ? b : m - b, t = small ? s - n_big : s;
-            row = t / cols;
+            row = (int)((unsigned)t / (unsigned)cols);
             const int k = t - row * cols;
             col = (small ? m - b : 0) + ((row & 1) ? cols - 1 - k : k);
         }
