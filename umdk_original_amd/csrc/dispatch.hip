@@ -39,9 +39,24 @@ __device__ __forceinline__ long long dispatch_row(const DispatchArgs &a, int t, 
     return pre + (window_row - a.recv_offset[e]);
 }
 
+// How the rows are stored.  Plain stores leave the L2 (32 MB) in a better order than the waves wrote the pieces of far apart rows in,
+// and their reader finds more of them in the memory-side cache.  But what still lies in the L2 at the end of the launch has to be
+// written back before the next one, which costs more than it gains while that is most of the output; and 8-bit rows, whose
+// pieces are half as long, lose again where there are many more of them than the caches hold.  us, non-temporal / plain:
+// dispatch of 16-bit rows alone, 16 MB 9.3 / 9.5, 33 MB 14.8 / 16.3, 49 MB 16.8 / 19.0; with a gather of other rows behind it
+// 72 MB 37.8 / 38.3, 79 MB 40.9 / 40.1, 196 MB 89.0 / 89.3, 803 MB 346 / 341; with layout and a gather of these rows, 79 MB 53.4 / 49.7,
+// 98 MB 59.8 / 55.5, 128 MB 73.3 / 65.4, 197 MB 103.6 / 89.3, 393 MB 187 / 169.  8-bit rows with a gather of other rows, 72 MB 54.7 /
+// 54.7, 86 MB 62.5 / 61.1, 131 MB 97.3 / 94.5, 143 MB 95.9 / 92.5 (FP8 98.3 / 95.7), 172 MB 113.0 / 115.1 (115.0 / 118.2), 235 MB
+// 150.0 / 151.2 (153.3 / 157.0).
+bool stores_plainly(const DispatchArgs &a)
+{
+    const long long values = (long long)a.T * a.K * a.H;
+    return a.quant == 0 ? values * 2 >= 72ll << 20 : values >= 72ll << 20 && values < 152ll << 20;
+}
+
 // Four workgroups per CU (128 registers a lane) keep all 1024 workgroups of a 4096-token batch resident at once;
 // the FP8 variant would spill at that size and stays at three.
-template <int QUANT, int ACT>
+template <int QUANT, int ACT, bool PLAIN>
 __global__ __launch_bounds__(kDispWaves * kWave, QUANT == 3 ? 3 : 4) void dispatch_kernel(DispatchArgs a)
 {
     const int t = (int)blockIdx.x * kDispWaves + (threadIdx.x >> 6);
@@ -59,14 +74,14 @@ __global__ __launch_bounds__(kDispWaves * kWave, QUANT == 3 ? 3 : 4) void dispat
         if (row < 0 || row >= a.A) {
             continue;
         }
-        store_token_row<QUANT>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, lane);
+        store_token_row<QUANT, PLAIN>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, lane);
     }
 }
 
 // The quantising permute with per-expert smooth scales: every copy of a token is quantised on its own, under the
 // scale row of its destination expert (moe_dispatch_shmem.h:492-549,693-733).  One wave per token; the token row
 // is loaded once and stays in registers across its copies.
-template <int ACT>
+template <int ACT, bool PLAIN>
 __global__ __launch_bounds__(kDispWaves * kWave) void dispatch_smooth_kernel(DispatchArgs a)
 {
     const int t = (int)blockIdx.x * kDispWaves + (threadIdx.x >> 6);
@@ -83,7 +98,7 @@ __global__ __launch_bounds__(kDispWaves * kWave) void dispatch_smooth_kernel(Dis
             continue;
         }
         quant_token_row_smooth<ACT>(r, a.smooth + (long long)e * a.H, a.H, lane, WaveMax());
-        store_token_row<2>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, lane);
+        store_token_row<2, PLAIN>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, lane);
     }
 }
 
@@ -95,7 +110,7 @@ __global__ __launch_bounds__(kDispWaves * kWave) void dispatch_smooth_kernel(Dis
 // row is what the launch takes, so it is spread over sixteen waves (four from 257 tokens on) instead of one.
 // Launches: one token x 4096 to 128 experts, top-8: 3.5 + 7.4 us -> 5.9; 64 x 4096 FP8: 6.2 + 15.6 -> 7.4; 128 x 7168 to 256
 // experts: 6.1 + 9.8 -> 7.8.
-constexpr int kSmallIds = 2048;   // ids per launch
+constexpr int kSmallIds = 2048;   // ids per launch (rows of at most 29 MB)
 template <typename IdT, int QUANT, int ACT, bool SMOOTH, int NT>
 __global__ __launch_bounds__(NT) void dispatch_small_kernel(PlanArgs p, DispatchArgs a)
 {
@@ -206,7 +221,7 @@ __global__ __launch_bounds__(NT) void dispatch_small_kernel(PlanArgs p, Dispatch
             const int e = __builtin_amdgcn_readlane(own_ids, k);
             quant_token_row_smooth<ACT>(r, a.smooth + (long long)e * a.H, a.H, tid, GroupMax<NT>{max_s});
         }
-        store_token_row<QUANT>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, tid);
+        store_token_row<QUANT, false>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, tid);
     }
 }
 
@@ -244,6 +259,40 @@ hipError_t launch_small(const PlanArgs &p, const DispatchArgs &a, hipStream_t st
     }
 }
 
+template <bool PLAIN>
+void launch_dispatch_as(const DispatchArgs &a, hipStream_t stream)
+{
+    const dim3 grid((a.T + kDispWaves - 1) / kDispWaves), block(kDispWaves * kWave);
+    const bool fp16 = a.x_is_fp16 != 0;
+    if (a.smooth != nullptr) {
+        if (fp16) {
+            hipLaunchKernelGGL((dispatch_smooth_kernel<1, PLAIN>), grid, block, 0, stream, a);
+        } else {
+            hipLaunchKernelGGL((dispatch_smooth_kernel<0, PLAIN>), grid, block, 0, stream, a);
+        }
+    } else if (a.quant == 0) {
+        hipLaunchKernelGGL((dispatch_kernel<0, 0, PLAIN>), grid, block, 0, stream, a);  // a copy does not look at the format
+    } else if (a.quant == 1) {
+        if (fp16) {
+            hipLaunchKernelGGL((dispatch_kernel<1, 1, PLAIN>), grid, block, 0, stream, a);
+        } else {
+            hipLaunchKernelGGL((dispatch_kernel<1, 0, PLAIN>), grid, block, 0, stream, a);
+        }
+    } else if (a.quant == 3) {
+        if (fp16) {
+            hipLaunchKernelGGL((dispatch_kernel<3, 1, PLAIN>), grid, block, 0, stream, a);
+        } else {
+            hipLaunchKernelGGL((dispatch_kernel<3, 0, PLAIN>), grid, block, 0, stream, a);
+        }
+    } else {
+        if (fp16) {
+            hipLaunchKernelGGL((dispatch_kernel<2, 1, PLAIN>), grid, block, 0, stream, a);
+        } else {
+            hipLaunchKernelGGL((dispatch_kernel<2, 0, PLAIN>), grid, block, 0, stream, a);
+        }
+    }
+}
+
 }  // namespace
 
 hipError_t launch_plan_dispatch(const PlanArgs &p, const DispatchArgs &a, hipStream_t stream)
@@ -271,38 +320,13 @@ hipError_t launch_dispatch(const DispatchArgs &a, hipStream_t stream)
     if (a.H % 8 != 0 || a.H / 8 > kDispMaxChunks * kWave || (a.quant == 3 && a.H % 128 != 0)) {
         return hipErrorInvalidValue;
     }
-    dim3 grid((a.T + kDispWaves - 1) / kDispWaves), block(kDispWaves * kWave);
-    if (a.smooth != nullptr) {
-        if (a.quant != 2 || a.idx == nullptr) {
-            return hipErrorInvalidValue;
-        }
-        if (a.x_is_fp16) {
-            hipLaunchKernelGGL((dispatch_smooth_kernel<1>), grid, block, 0, stream, a);
-        } else {
-            hipLaunchKernelGGL((dispatch_smooth_kernel<0>), grid, block, 0, stream, a);
-        }
-        return hipGetLastError();
+    if (a.smooth != nullptr && (a.quant != 2 || a.idx == nullptr)) {
+        return hipErrorInvalidValue;
     }
-    if (a.quant == 0) {
-        hipLaunchKernelGGL((dispatch_kernel<0, 0>), grid, block, 0, stream, a);  // a copy does not look at the format
-    } else if (a.quant == 1) {
-        if (a.x_is_fp16) {
-            hipLaunchKernelGGL((dispatch_kernel<1, 1>), grid, block, 0, stream, a);
-        } else {
-            hipLaunchKernelGGL((dispatch_kernel<1, 0>), grid, block, 0, stream, a);
-        }
-    } else if (a.quant == 3) {
-        if (a.x_is_fp16) {
-            hipLaunchKernelGGL((dispatch_kernel<3, 1>), grid, block, 0, stream, a);
-        } else {
-            hipLaunchKernelGGL((dispatch_kernel<3, 0>), grid, block, 0, stream, a);
-        }
+    if (stores_plainly(a)) {
+        launch_dispatch_as<true>(a, stream);
     } else {
-        if (a.x_is_fp16) {
-            hipLaunchKernelGGL((dispatch_kernel<2, 1>), grid, block, 0, stream, a);
-        } else {
-            hipLaunchKernelGGL((dispatch_kernel<2, 0>), grid, block, 0, stream, a);
-        }
+        launch_dispatch_as<false>(a, stream);
     }
     return hipGetLastError();
 }

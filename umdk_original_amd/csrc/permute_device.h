@@ -260,8 +260,19 @@ __device__ __forceinline__ void store_row_scales8(const Row &r, uint8_t *scales,
     }
 }
 
+// 16 or 8 bytes of a row; PLAIN: through the L2 like any store, else non-temporal.
+template <bool PLAIN, typename T>
+__device__ __forceinline__ void store_piece(T v, T *dst)
+{
+    if constexpr (PLAIN) {
+        *dst = v;
+    } else {
+        __builtin_nontemporal_store(v, dst);
+    }
+}
+
 // Stores the row (quantised or raw) to output row `row`, with its scale and triple.
-template <int QUANT, typename Row>
+template <int QUANT, bool PLAIN, typename Row>
 __device__ __forceinline__ void store_token_row(const Row &r, void *out, float *scales, int32_t *src_info,
                                                 int src_rank, long long row, int t, int k, int H, int lane)
 {
@@ -272,7 +283,7 @@ __device__ __forceinline__ void store_token_row(const Row &r, void *out, float *
         for (int j = 0; j < Row::kChunks; ++j) {
             const int c = j * Row::kLanes + lane;
             if (c < nch) {
-                __builtin_nontemporal_store(r.q[j], dst + c);
+                store_piece<PLAIN>(r.q[j], dst + c);
             }
         }
     } else {
@@ -281,7 +292,7 @@ __device__ __forceinline__ void store_token_row(const Row &r, void *out, float *
         for (int j = 0; j < Row::kChunks; ++j) {
             const int c = j * Row::kLanes + lane;
             if (c < nch) {
-                __builtin_nontemporal_store(r.raw[j], dst + c);
+                store_piece<PLAIN>(r.raw[j], dst + c);
             }
         }
     }
