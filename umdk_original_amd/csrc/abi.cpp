@@ -1039,6 +1039,7 @@ camStatus camMoeCombineNormalGetWorkspaceSize(const camTensor *recvX, const camT
     CAM_TRY(check_aligned(recvX, "recvX", 16));
     CAM_TRY(check_aligned(out, "out", 16));
     Carver c;
+    const bool scan = cam::combine_scans(T, K, A);
     const uint64_t o_slot = c.take((uint64_t)T * K * 4);
     cam::CombineArgs g{};
     g.y = (const uint16_t *)recvX->data;
@@ -1052,7 +1053,10 @@ camStatus camMoeCombineNormalGetWorkspaceSize(const camTensor *recvX, const camT
     // Rows at or past the receive total were never written (moe_combine_normal.h:206-207 bounds its loop the same way).
     g.row_limit = (const int32_t *)epRecvCounts->data + (moeExpertNum - 1);
     g.out = (uint16_t *)out->data;
-    auto run = [g, o_slot](void *ws, hipStream_t s) mutable -> hipError_t {
+    auto run = [g, o_slot, scan](void *ws, hipStream_t s) mutable -> hipError_t {
+        if (scan) {
+            return cam::launch_combine(g, s);
+        }
         int32_t *slot = (int32_t *)((char *)ws + o_slot);
         hipError_t e = cam::launch_invert_src_info(g.src_info, g.A, g.row_limit, g.T, g.K, slot, s);
         if (e != hipSuccess) {

@@ -139,7 +139,8 @@ struct CombineArgs {
     const uint16_t *y;        // [A,H] bf16 bits, or wire rows [A, H + H/4] bytes (wire_rows != 0)
     int wire_rows;            // rows are H int8 values + H/8 block scales of the activation type (launch_comm_quant's output)
     int act_fp16;             // rows and output are IEEE fp16 instead of bf16 (not with wire_rows)
-    const int32_t *slot_row;  // [T,K] row of slot (t,k) (<0: skip)
+    const int32_t *slot_row;  // [T,K] row of slot (t,k) (<0: skip); null without ids where combine_scans says so: src_info, which
+                              // has to be set then, is looked through instead
     // instead of slot_row, when ids is set: the row of slot i is (e ? ep_send_counts[e-1] : 0) + expand_idx[i] for
     // e = ids[i] in [0,E), none otherwise
     const int32_t *ids, *expand_idx, *ep_send_counts;
@@ -154,6 +155,8 @@ struct CombineArgs {
     uint16_t *out;            // [T,H]
 };
 hipError_t launch_combine(const CombineArgs &a, hipStream_t stream);
+// Whether a combine of rows of the activation type needs no map (launch_invert_src_info) beside the triples of its A rows.
+bool combine_scans(int64_t T, int64_t K, int64_t A);
 // bf16 rows [A,H] -> wire rows [A, H + H/4] bytes: per block of 8 columns int8 values and one bf16 scale.
 // row_limit: optional device scalar; rows >= *row_limit are left untouched.
 hipError_t launch_comm_quant(const uint16_t *y, int act_fp16, int64_t A, int H, const int32_t *row_limit, uint8_t *out,

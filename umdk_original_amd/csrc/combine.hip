@@ -28,6 +28,7 @@ namespace {
 
 constexpr int kCombThreads = 128;
 constexpr int kCombBatch = 8;
+constexpr int kScanRows = 1024;  // triples a workgroup looks through at most, 8 a thread
 
 // Rows at or beyond *row_limit (the receive total, epRecvCounts[E-1] of moe_combine_normal.h:206-207) were
 // never written by the dispatch that filled the buffers; whatever triple they hold is ignored.
@@ -114,12 +115,39 @@ __device__ __forceinline__ float comb_act_to_f32(uint32_t bits16)
     return ACT == 0 ? bf16_bits_to_f32(bits16) : fp16_bits_to_f32(bits16);
 }
 
-template <bool WIRE, int ACT, bool BY_COUNTS>
+// SCAN: no map has been made; a workgroup looks through the triples for its token's rows by itself (the last of several that name the
+// same slot).  It takes the place of invert_src_info_kernel where there are few of them (combine_scans).
+template <bool WIRE, int ACT, bool BY_COUNTS, bool SCAN = false>
 __global__ __launch_bounds__(kCombThreads) void combine_kernel(CombineArgs a, int segs)
 {
     const int t = blockIdx.x / segs;
     const int seg = blockIdx.x - t * segs;
     const int col = (seg * kCombThreads + threadIdx.x) * 8;
+    __shared__ int row_s[SCAN ? kMaxTopk : 1];
+    if constexpr (SCAN) {
+        int token[kScanRows / kCombThreads];
+#pragma unroll
+        for (int i = 0; i < kScanRows / kCombThreads; ++i) {  // all in one round trip
+            const int r = i * kCombThreads + (int)threadIdx.x;
+            token[i] = r < a.A ? a.src_info[3 * r + 1] : -1;
+        }
+        if (threadIdx.x < kMaxTopk) {
+            row_s[threadIdx.x] = -1;
+        }
+        __syncthreads();
+        const int limit = a.row_limit == nullptr ? (int)a.A : min((int)a.A, *a.row_limit);
+#pragma unroll
+        for (int i = 0; i < kScanRows / kCombThreads; ++i) {
+            const int r = i * kCombThreads + (int)threadIdx.x;
+            if (r < limit && token[i] == t) {
+                const int k = a.src_info[3 * r + 2];
+                if (k >= 0 && k < a.K) {
+                    atomicMax(&row_s[k], r);
+                }
+            }
+        }
+        __syncthreads();
+    }
     if (col >= a.H) {
         return;
     }
@@ -148,9 +176,9 @@ __global__ __launch_bounds__(kCombThreads) void combine_kernel(CombineArgs a, in
                 v[j] = v4u{0u, 0u, 0u, 0u};
                 if (k < a.K) {
                     const long long slot = (long long)t * a.K + k;
-                    const long long row = row_of_slot<BY_COUNTS>(a, slot);
+                    const long long row = SCAN ? row_s[k] : row_of_slot<BY_COUNTS>(a, slot);
                     bool good = row >= 0 && row < rows;
-                    if (good && a.src_info != nullptr) {
+                    if (!SCAN && good && a.src_info != nullptr) {
                         // The inverse map is not pre-cleared: accept a row only if it names this slot.
                         good = a.src_info[3 * row + 1] == t && a.src_info[3 * row + 2] == k;
                     }
@@ -370,8 +398,33 @@ static hipError_t launch_combine_as(const CombineArgs &a, hipStream_t stream)
     return hipGetLastError();
 }
 
+// A combine of few rows is as long as its launches.  us, layout + dispatch + combine, with the map / without: one token x 4096, top-8 34.6 /
+// 30.7, 64 x 2048, top-4 31.5 / 27.8, 100 x 4096, top-6 35.1 / 31.2, 128 x 7168, top-8 50.5 / 46.8 (1024 rows), 1000 x 1024, top-1
+// 32.4 / 28.9.  A thread's triples are one round trip to the L2; with more of them, each workgroup reading all, the launch that is
+// saved costs less.
+bool combine_scans(int64_t T, int64_t K, int64_t A)
+{
+    return A > 0 && A <= kScanRows && K <= kMaxTopk && T * K <= kScanRows;
+}
+
 hipError_t launch_combine(const CombineArgs &a, hipStream_t stream)
 {
+    if (a.ids == nullptr && a.slot_row == nullptr) {
+        if (a.src_info == nullptr || a.wire_rows || !combine_scans(a.T, a.K, a.A) || a.H % 8 != 0) {
+            return hipErrorInvalidValue;
+        }
+        if (a.T <= 0) {
+            return hipSuccess;
+        }
+        const int segs = (a.H / 8 + kCombThreads - 1) / kCombThreads;
+        const dim3 grid((unsigned)(a.T * segs)), block(kCombThreads);
+        if (a.act_fp16) {
+            hipLaunchKernelGGL((combine_kernel<false, 1, false, true>), grid, block, 0, stream, a, segs);
+        } else {
+            hipLaunchKernelGGL((combine_kernel<false, 0, false, true>), grid, block, 0, stream, a, segs);
+        }
+        return hipGetLastError();
+    }
     return a.ids != nullptr ? launch_combine_as<true>(a, stream) : launch_combine_as<false>(a, stream);
 }
 
