@@ -282,8 +282,9 @@ __global__ __launch_bounds__(kLocalThreads) void plan_single_kernel(PlanArgs a)
 // workgroup alone writes the results itself.  Latency bound: 1999 tokens x 6 ids to 64 experts, with layout, dispatch and
 // combine of 4096 columns 69.9 us when the layout was the two launches of the plan and one for the flags, 63.5 now.
 constexpr int kLayoutThreads = 256;
-template <typename IdT, typename OutT>
-__global__ __launch_bounds__(kLayoutThreads) void layout_kernel(LayoutArgs a, int span)
+constexpr int kLayoutOne = 1024;  // threads of a workgroup alone
+template <typename IdT, typename OutT, int NT>
+__global__ __launch_bounds__(NT) void layout_kernel(LayoutArgs a, int span)
 {
     __shared__ int count_s[kMaxExperts + kMaxRanks];
     const int tid = threadIdx.x;
@@ -292,14 +293,14 @@ __global__ __launch_bounds__(kLayoutThreads) void layout_kernel(LayoutArgs a, in
     const int E = a.E, R = a.R, K = a.K;
     const int epr = E / R;
     OutT *out = (OutT *)a.in_rank;
-    for (int c = tid; c < E + R; c += kLayoutThreads) {
+    for (int c = tid; c < E + R; c += NT) {
         count_s[c] = 0;
     }
-    for (long long i = (long long)t0 * R + tid; i < (long long)t1 * R; i += kLayoutThreads) {
+    for (long long i = (long long)t0 * R + tid; i < (long long)t1 * R; i += NT) {
         out[i] = (OutT)0;
     }
     __syncthreads();
-    for (int t = t0 + tid; t < t1; t += kLayoutThreads) {
+    for (int t = t0 + tid; t < t1; t += NT) {
         const IdT *ids = (const IdT *)a.idx + (long long)t * K;
         int e[kMaxTopk];
 #pragma unroll
@@ -325,7 +326,7 @@ __global__ __launch_bounds__(kLayoutThreads) void layout_kernel(LayoutArgs a, in
         }
     }
     __syncthreads();
-    for (int c = tid; c < E + R; c += kLayoutThreads) {
+    for (int c = tid; c < E + R; c += NT) {
         if (gridDim.x > 1) {
             a.partial[(long long)blockIdx.x * (E + R) + c] = count_s[c];
         } else if (c < E) {
@@ -363,10 +364,17 @@ __global__ __launch_bounds__(kWave) void layout_sum_kernel(LayoutArgs a, int row
     }
 }
 
-// Workgroups of a layout and tokens of each: one round of tokens per workgroup up to 64 of them, whose counts are two
-// round trips to add up.
-int layout_workgroups(long long T, int *span)
+// Workgroups of a layout and tokens of each: one of kLayoutOne threads alone for a round of tokens and few flags, which saves the
+// launch that adds the counts up; else one round of tokens per workgroup up to 64 of them, whose counts are two round trips to
+// add up.  us, layout + dispatch + combine, added up / alone: 300 tokens x 4096, top-3 34.4 / 30.2, 500 x 2048, top-8 37.5 / 33.5, 1000 x
+// 4096, top-6 38.0 / 36.9, 1024 x 1024, top-8 41.1 / 38.0; with two rounds 1999 x 4096, top-6 58.7 / 64.2 (the counts of one
+// workgroup's LDS collide).
+int layout_workgroups(long long T, int R, int *span)
 {
+    if (T <= kLayoutOne && T * R <= 8 * kLayoutOne) {
+        *span = kLayoutOne;
+        return 1;
+    }
     const long long rounds = std::max<long long>((T + 64 * kLayoutThreads - 1) / (64 * kLayoutThreads), 1);
     *span = (int)(rounds * kLayoutThreads);
     return (int)std::max<long long>((T + *span - 1) / *span, 1);
@@ -518,7 +526,18 @@ hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &d, int32_t *
 uint64_t layout_workspace_bytes(int64_t T, int E, int R)
 {
     int span;
-    return (uint64_t)layout_workgroups(T, &span) * (uint64_t)(E + R) * sizeof(int32_t);
+    return (uint64_t)layout_workgroups(T, R, &span) * (uint64_t)(E + R) * sizeof(int32_t);
+}
+
+template <typename IdT, int NT>
+void launch_layout_as(const LayoutArgs &a, int workgroups, int span, hipStream_t stream)
+{
+    const dim3 grid(workgroups), block(NT);
+    if (a.in_rank_bytes == 4) {
+        hipLaunchKernelGGL((layout_kernel<IdT, int32_t, NT>), grid, block, 0, stream, a, span);
+    } else {
+        hipLaunchKernelGGL((layout_kernel<IdT, uint8_t, NT>), grid, block, 0, stream, a, span);
+    }
 }
 
 hipError_t launch_layout(const LayoutArgs &a, hipStream_t stream)
@@ -527,20 +546,12 @@ hipError_t launch_layout(const LayoutArgs &a, hipStream_t stream)
         return hipErrorInvalidValue;
     }
     int span;
-    const int n = layout_workgroups(a.T, &span);
-    const dim3 grid(n), block(kLayoutThreads);
-    if (a.idx_is64) {
-        if (a.in_rank_bytes == 4) {
-            hipLaunchKernelGGL((layout_kernel<int64_t, int32_t>), grid, block, 0, stream, a, span);
-        } else {
-            hipLaunchKernelGGL((layout_kernel<int64_t, uint8_t>), grid, block, 0, stream, a, span);
-        }
+    const int n = layout_workgroups(a.T, a.R, &span);
+    if (n == 1 && a.T > kLayoutThreads) {
+        a.idx_is64 ? launch_layout_as<int64_t, kLayoutOne>(a, n, span, stream) : launch_layout_as<int32_t, kLayoutOne>(a, n, span, stream);
     } else {
-        if (a.in_rank_bytes == 4) {
-            hipLaunchKernelGGL((layout_kernel<int32_t, int32_t>), grid, block, 0, stream, a, span);
-        } else {
-            hipLaunchKernelGGL((layout_kernel<int32_t, uint8_t>), grid, block, 0, stream, a, span);
-        }
+        a.idx_is64 ? launch_layout_as<int64_t, kLayoutThreads>(a, n, span, stream)
+                   : launch_layout_as<int32_t, kLayoutThreads>(a, n, span, stream);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || n == 1) {
