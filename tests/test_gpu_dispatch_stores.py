@@ -1,5 +1,5 @@
-"""The permute on both sides of the output sizes between which its rows are stored plainly (72 and, 8-bit rows, 152 MiB): 16-bit,
-int8 and FP8 rows, rows under smooth scales, ids that name no expert.  Bit for bit, as everywhere in the dispatch."""
+"""The permute on both sides of the output sizes between which its rows are stored plainly (72 and, 8-bit rows, 152 MiB; rows that
+are no whole lines 48): 16-bit, int8 and FP8 rows, rows under smooth scales, ids that name no expert.  Bit for bit, as everywhere in the dispatch."""
 import numpy as np
 import pytest
 import torch
@@ -14,9 +14,10 @@ pytestmark = pytest.mark.gpu
 K, E, H = 16, 300, 7168      # 659 to 1389 tokens of 8-bit rows lie between the lines, 330 and more of 16-bit rows
 
 
-@pytest.mark.parametrize("T,quant_mode", [(658, 2), (659, 2), (659, 3), (1390, 2), (329, 0), (330, 0)])
-def test_rows_around_the_lines(gpu, oracle, T, quant_mode):
-    announce("permute stores T=%d quant=%d" % (T, quant_mode))
+@pytest.mark.parametrize("T,quant_mode,H", [(658, 2, H), (659, 2, H), (659, 3, H), (1390, 2, H), (329, 0, H), (330, 0, H),
+                                            (439, 2, 7160), (440, 2, 7160), (220, 0, 7160)])
+def test_rows_around_the_lines(gpu, oracle, T, quant_mode, H):
+    announce("permute stores T=%d H=%d quant=%d" % (T, H, quant_mode))
     rng = np.random.default_rng(T)
     ids = np.where(rng.random((T, K)) < 0.1, -1, rng.integers(0, E, size=(T, K))).astype(np.int64)
     x = synth.normal_bf16(T, H, seed=T)

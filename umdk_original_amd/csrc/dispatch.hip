@@ -47,11 +47,16 @@ __device__ __forceinline__ long long dispatch_row(const DispatchArgs &a, int t, 
 // 72 MB 37.8 / 38.3, 79 MB 40.9 / 40.1, 196 MB 89.0 / 89.3, 803 MB 346 / 341; with layout and a gather of these rows, 79 MB 53.4 / 49.7,
 // 98 MB 59.8 / 55.5, 128 MB 73.3 / 65.4, 197 MB 103.6 / 89.3, 393 MB 187 / 169.  8-bit rows with a gather of other rows, 72 MB 54.7 /
 // 54.7, 86 MB 62.5 / 61.1, 131 MB 97.3 / 94.5, 143 MB 95.9 / 92.5 (FP8 98.3 / 95.7), 172 MB 113.0 / 115.1 (115.0 / 118.2), 235 MB
-// 150.0 / 151.2 (153.3 / 157.0).
+// 150.0 / 151.2 (153.3 / 157.0).  Rows that are no whole lines of 128 bytes, dispatch with a gather of other rows: the L2 puts the two halves
+// of a line together, so they gain from less on and have no upper line: 16-bit 34 MB 25.3 / 27.8, 50 MB 32.8 / 32.0, 90 MB 56.7 / 49.4, 96
+// MB 65.5 / 57.5; int8 19 MB 25.0 / 26.9, 56 MB 48.2 / 46.1, 172 MB 130.5 / 120.7, 235 MB 176.2 / 166.0.
 bool stores_plainly(const DispatchArgs &a)
 {
-    const long long values = (long long)a.T * a.K * a.H;
-    return a.quant == 0 ? values * 2 >= 72ll << 20 : values >= 72ll << 20 && values < 152ll << 20;
+    const long long pitch = (long long)a.H * (a.quant == 0 ? 2 : 1), bytes = (long long)a.T * a.K * pitch;
+    if (pitch % 128 != 0) {
+        return bytes >= 48ll << 20;
+    }
+    return bytes >= 72ll << 20 && (a.quant == 0 || bytes < 152ll << 20);
 }
 
 // Four workgroups per CU (128 registers a lane) keep all 1024 workgroups of a 4096-token batch resident at once;
