@@ -1,0 +1,105 @@
+"""Fused layers whose quantised tokens take 2 GiB, one row more than 32-bit offsets reach: their rows are permuted, a row per
+copy, in front of a gate/up GEMM that does not gather.  What a token gets depends on no other token, so that every row has the bits
+it has in a layer of half the tokens, which gathers; a few of them are also compared with the oracle, at the tolerances of the
+ordinary layer tests."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import umdk_original_amd as cam
+from umdk_original_amd import synth
+from gpu_util import announce, assert_bits_equal, to_np
+from test_gpu_fp8 import _check_layer, _layer_inputs, _u8
+
+pytestmark = pytest.mark.gpu
+
+
+def _tokens(gpu, T, H, E, seed):
+    gen = torch.Generator(device=gpu).manual_seed(seed)
+    x = torch.empty(T, H, dtype=torch.bfloat16, device=gpu)
+    for part in x.split(1 << 18):
+        part.normal_(generator=gen)
+    ids = torch.randint(-1, E, (T, 1), generator=gen, device=gpu, dtype=torch.int32)   # some dropped
+    ids[0] = ids[T - 1] = E - 1
+    return x, ids, torch.rand(T, 1, generator=gen, device=gpu)
+
+
+def _some(T, seed):
+    edges = [0, 1, T // 2 - 1, T // 2, T - 2, T - 1]
+    return torch.tensor(edges + np.random.default_rng(seed).integers(0, T, 58).tolist())
+
+
+def _check_halves(layer, T):
+    out, etn = layer(0, T)
+    h = T // 2
+    (lo, etn_lo), (hi, etn_hi) = layer(0, h), layer(h, T)
+    assert torch.equal(etn, etn_lo + etn_hi) and 0 < int(etn.sum()) < T
+    assert torch.equal(out[:h].view(torch.int16), lo.view(torch.int16))
+    assert torch.equal(out[h:].view(torch.int16), hi.view(torch.int16))
+    return out
+
+
+def test_int8_layer(gpu, oracle):
+    T, H, E, I = (1 << 22) + 3, 512, 5, 512
+    announce("ungathered rows T=%d H=%d int8" % (T, H))
+    x, ids, gates = _tokens(gpu, T, H, E, 1)
+    w1, w1s = synth.absmax_int8_weights(E, H, 2 * I, seed=2)
+    w2, w2s = synth.absmax_int8_weights(E, I, H, seed=3)
+    dev = [[cam.prepack_weight(w1.to(gpu), True)], [w1s.to(gpu)], [cam.prepack_weight(w2.to(gpu), False)], [w2s.to(gpu)]]
+
+    def layer(t0, t1):
+        return cam.fused_deep_moe(x[t0:t1], ids[t0:t1], *dev, gates[t0:t1], None, None, "", 1, 0, E, 1, 0, 0, 0)
+
+    out = _check_halves(layer, T)
+    s = _some(T, 4).to(gpu)
+    want, _ = oracle.fused_layer(synth.bf16_bits(x[s].cpu()), ids[s].cpu().numpy().astype(np.int64), gates[s].cpu().numpy(),
+                                 w1.numpy(), w1s.numpy(), w2.numpy(), w2s.numpy())
+    assert_bits_equal(to_np(out[s]), want, "sampled tokens")
+
+
+def test_fp8_layer(gpu, oracle):
+    T, H, E, I = (1 << 21) + 1, 1024, 3, 256
+    announce("ungathered rows T=%d H=%d FP8" % (T, H))
+    x, ids, gates = _tokens(gpu, T, H, E, 5)
+    _, _, _, w1, s1, w2, s2 = _layer_inputs(8, H, E, 1, I, seed=6)
+    dev = [cam.prepack_weight(w1.to(gpu), True), s1.to(gpu), cam.prepack_weight(w2.to(gpu), False), s2.to(gpu)]
+
+    def layer(t0, t1):
+        return cam.fused_deep_moe_fp8(x[t0:t1], ids[t0:t1], *dev, gates[t0:t1])
+
+    out = _check_halves(layer, T)
+    s = _some(T, 7).to(gpu)
+    want = oracle.fp8_fused_layer(synth.bf16_bits(x[s].cpu()), ids[s].cpu().numpy().astype(np.int64), gates[s].cpu().numpy(),
+                                  _u8(w1), s1.numpy(), _u8(w2), s2.numpy())
+    _check_layer(out[s].float().cpu().numpy(), want)
+
+
+def _recorded_kernels(call):
+    """Nodes of the graph that a call records; nothing of it runs."""
+    runtime = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        keep = call()
+    n = ctypes.c_size_t()
+    status = ctypes.CDLL(runtime).hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n))
+    assert status == 0 and keep is not None
+    return n.value
+
+
+def test_schedules_take_no_launch_of_their_own(gpu):
+    H, E, I = 512, 5, 512
+    announce("launches of layers with and without gathered rows")
+    w1, w1s = synth.absmax_int8_weights(E, H, 2 * I, seed=2)
+    w2, w2s = synth.absmax_int8_weights(E, I, H, seed=3)
+    dev = [[cam.prepack_weight(w1.to(gpu), True)], [w1s.to(gpu)], [cam.prepack_weight(w2.to(gpu), False)], [w2s.to(gpu)]]
+
+    def launches(T):
+        x = torch.empty(T, H, dtype=torch.bfloat16, device=gpu)
+        ids, gates = torch.empty(T, 1, dtype=torch.int32, device=gpu), torch.empty(T, 1, device=gpu)
+        return _recorded_kernels(lambda: cam.fused_deep_moe(x, ids, *dev, gates, None, None, "", 1, 0, E, 1, 0, 0, 0))
+
+    gathered = launches(1 << 16)
+    assert gathered == 6                       # two of the plan, GMM1, re-quantisation, GMM2, combine
+    assert launches(1 << 22) == gathered + 1   # the permute

@@ -337,22 +337,7 @@ hipError_t run_grouped_gemm(cam::GemmArgs g, const int64_t *group_list, int cumu
     return cam::launch_gemm(g, s);
 }
 
-// What is in front of a layer's GEMMs: plan, quantised rows and, unless they stream, their schedules.  With row_token the rows
-// stay one per token and GMM1 gathers them.
-hipError_t layer_plan(const cam::PlanArgs &p, const cam::DispatchArgs &d, const cam::SchedSpec *specs, int32_t *row_token,
-                      bool stream, hipStream_t s)
-{
-    if (row_token != nullptr) {
-        return cam::launch_plan_quant(p, d, row_token, specs, s);
-    }
-    const hipError_t e = cam::launch_plan_dispatch(p, d, s);
-    if (e != hipSuccess || stream) {
-        return e;
-    }
-    return cam::launch_build_sched(p.tokens_per_expert, 0, p.E, d.A, 2, specs, s);
-}
-
-// The GEMMs of a fused layer: per-expert counts from its plan, g.sched filled when the permute built schedules.  A token
+// The GEMMs of a fused layer: per-expert counts from its plan, g.sched filled by launch_layer_plan unless they stream.  A token
 // names an expert once, so no expert has more than T rows.
 hipError_t layer_gemm(const cam::GemmArgs &g, const int64_t *counts, int E, int64_t A, int T, bool stream, hipStream_t s,
                       const float *products = nullptr)
@@ -1900,7 +1885,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         d.out = x1;
         d.scales = x1s;
         int32_t *token = (int32_t *)(w + o_token);
-        e = layer_plan(p, d, specs, gather ? token : nullptr, stream, s);
+        e = stream ? cam::launch_plan_dispatch(p, d, s) : cam::launch_layer_plan(p, d, gather ? token : nullptr, specs, s);
         if (e != hipSuccess) return e;
 
         cam::GemmArgs g1{};
@@ -2252,7 +2237,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         d.out = x1;
         d.scales = (float *)x1s;
         int32_t *token = (int32_t *)(w + o_token);
-        e = layer_plan(p, d, specs, gather ? token : nullptr, stream, s);
+        e = stream ? cam::launch_plan_dispatch(p, d, s) : cam::launch_layer_plan(p, d, gather ? token : nullptr, specs, s);
         if (e != hipSuccess) return e;
 
         cam::GemmArgs g1{};

@@ -124,10 +124,11 @@ struct DispatchArgs {
 hipError_t launch_dispatch(const DispatchArgs &a, hipStream_t stream);
 // launch_plan, then launch_dispatch with a.dst_row == p.dst_row; for few ids both as one launch.
 hipError_t launch_plan_dispatch(const PlanArgs &p, const DispatchArgs &a, hipStream_t stream);
-// The first part of a layer whose gate/up GEMM gathers its rows, in two launches: the plan (int32 ids), every token quantised into
-// row t of a.out ([T,H]; a.quant 2 or 3) with its scales in row t of a.scales, row_token[row] the token of a row in the order of
-// the experts (GemmArgs::a_rows), and the schedules of both GEMMs (specs), what launch_build_sched makes of the plan's counts.
-hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &a, int32_t *row_token, const SchedSpec *specs,
+// The first part of a layer whose GEMMs have schedules: the plan (int32 ids) and both schedules (specs), what launch_build_sched
+// makes of the plan's counts, in two launches.  With row_token, for a gate/up GEMM that gathers its rows, they also leave every token
+// quantised in row t of a.out ([T,H]; a.quant 2 or 3) with its scales in row t of a.scales, and in row_token[row] the token of a
+// row in the order of the experts (GemmArgs::a_rows).  Without, launch_dispatch follows (a.dst_row == p.dst_row).
+hipError_t launch_layer_plan(const PlanArgs &p, const DispatchArgs &a, int32_t *row_token, const SchedSpec *specs,
                              hipStream_t stream);
 
 // ---------------------------------------------------------------------------------------------

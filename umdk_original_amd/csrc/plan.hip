@@ -106,9 +106,9 @@ __global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 
 }
 
 // What phase 2 does besides in a layer: its first sched.nspec * sched.parts workgroups build the schedules of the GEMMs (from
-// the counts, which they add up like all the others), and the others leave the token of every row.
+// the counts, which they add up like all the others), and the others leave the token of every row where GMM1 gathers.
 struct LayerPlan {
-    int32_t *row_token;
+    int32_t *row_token;  // or null
     SchedBuild sched;
 };
 
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(kGlobalThreads) void plan_global_kernel(PlanArgs a,
             const int p = p0 + base_s[e];
             a.pos[i] = p;
             row = off_s[e] + p;
-            if (LAYER) {
+            if (LAYER && l.row_token != nullptr) {
                 l.row_token[row] = (int)((unsigned)i / (unsigned)a.K);
             }
         }
@@ -405,9 +405,22 @@ __global__ __launch_bounds__(kScanThreads) void notify_scan_kernel(const int32_t
 }
 
 template <typename IdT>
+hipError_t launch_plan_local(const PlanArgs &a, int it, int nb, int32_t *hist, hipStream_t stream)
+{
+    const dim3 grid(nb), blk(kLocalThreads);
+    switch (it) {
+        case 1: hipLaunchKernelGGL((plan_local_kernel<IdT, 1>), grid, blk, 0, stream, a, hist); break;
+        case 2: hipLaunchKernelGGL((plan_local_kernel<IdT, 2>), grid, blk, 0, stream, a, hist); break;
+        case 4: hipLaunchKernelGGL((plan_local_kernel<IdT, 4>), grid, blk, 0, stream, a, hist); break;
+        default: hipLaunchKernelGGL((plan_local_kernel<IdT, 8>), grid, blk, 0, stream, a, hist); break;
+    }
+    return hipGetLastError();
+}
+
+template <typename IdT>
 hipError_t launch_plan_t(const PlanArgs &a, int it, int nb, int32_t *hist, hipStream_t stream)
 {
-    dim3 grid(nb), blk(kLocalThreads);
+    const dim3 grid(nb), blk(kLocalThreads);
     if (nb == 1) {
         switch (it) {
             case 1: hipLaunchKernelGGL((plan_single_kernel<IdT, 1>), grid, blk, 0, stream, a); break;
@@ -416,13 +429,7 @@ hipError_t launch_plan_t(const PlanArgs &a, int it, int nb, int32_t *hist, hipSt
         }
         return hipGetLastError();
     }
-    switch (it) {
-        case 1: hipLaunchKernelGGL((plan_local_kernel<IdT, 1>), grid, blk, 0, stream, a, hist); break;
-        case 2: hipLaunchKernelGGL((plan_local_kernel<IdT, 2>), grid, blk, 0, stream, a, hist); break;
-        case 4: hipLaunchKernelGGL((plan_local_kernel<IdT, 4>), grid, blk, 0, stream, a, hist); break;
-        default: hipLaunchKernelGGL((plan_local_kernel<IdT, 8>), grid, blk, 0, stream, a, hist); break;
-    }
-    hipError_t e = hipGetLastError();
+    const hipError_t e = launch_plan_local<IdT>(a, it, nb, hist, stream);
     if (e != hipSuccess) {
         return e;
     }
@@ -485,10 +492,10 @@ hipError_t launch_plan(const PlanArgs &a, hipStream_t stream)
     return launch_plan_t<int32_t>(a, it, nb, a.hist_ws, stream);
 }
 
-hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &d, int32_t *row_token, const SchedSpec *specs,
+hipError_t launch_layer_plan(const PlanArgs &p, const DispatchArgs &d, int32_t *row_token, const SchedSpec *specs,
                              hipStream_t stream)
 {
-    if (p.hist_ws == nullptr || p.idx_is64 || row_token == nullptr || p.T <= 0 || d.T != p.T || p.E <= 0 || p.E > kMaxExperts ||
+    if (p.hist_ws == nullptr || p.idx_is64 || p.T <= 0 || d.T != p.T || p.E <= 0 || p.E > kMaxExperts ||
         d.H % 8 != 0 || d.H / 8 > kDispMaxChunks * kWave || (d.quant != 2 && d.quant != 3) ||
         (d.quant == 3 && (d.H % 128 != 0 || d.x_is_fp16))) {
         return hipErrorInvalidValue;
@@ -510,7 +517,9 @@ hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &d, int32_t *
     // most 8 builders and 64-bit divisions in their turns phase 2 took 22.1 us at 8192 tokens
     const int cap = std::max(specs[0].max_items, specs[1].max_items);
     l.sched.parts = std::min(std::max((cap + kGlobalThreads - 1) / kGlobalThreads, 1), 32);
-    if (d.quant == 3) {
+    if (row_token == nullptr) {
+        e = launch_plan_local<int32_t>(p, it, nb, p.hist_ws, stream);
+    } else if (d.quant == 3) {
         e = launch_plan_quant_as<3, 0>(p, d, it, nb, stream);
     } else {
         e = d.x_is_fp16 ? launch_plan_quant_as<2, 1>(p, d, it, nb, stream) : launch_plan_quant_as<2, 0>(p, d, it, nb, stream);
@@ -520,7 +529,8 @@ hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &d, int32_t *
     }
     hipLaunchKernelGGL((plan_global_kernel<int32_t, true>), dim3((unsigned)(nb + l.sched.nspec * l.sched.parts)),
                        dim3(kGlobalThreads), 0, stream, p, it * kLocalThreads, (const int32_t *)p.hist_ws, l);
-    return hipGetLastError();
+    e = hipGetLastError();
+    return e != hipSuccess || row_token != nullptr ? e : launch_dispatch(d, stream);
 }
 
 uint64_t layout_workspace_bytes(int64_t T, int E, int R)
