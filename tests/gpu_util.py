@@ -1,4 +1,6 @@
 """Helpers shared by the GPU parity tests (which call the HIP path through the C ABI)."""
+import ctypes
+
 import numpy as np
 import torch
 
@@ -32,3 +34,15 @@ def assert_bits_equal(got, want, what):
         bad = np.argwhere(got != want)
         raise AssertionError("%s: %d of %d elements differ; first at %s: got %s want %s" % (
             what, len(bad), got.size, bad[0].tolist(), got[tuple(bad[0])], want[tuple(bad[0])]))
+
+
+def recorded_kernels(call):
+    """Nodes of the graph that a call records; nothing of it runs."""
+    runtime = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        keep = call()
+    n = ctypes.c_size_t()
+    status = ctypes.CDLL(runtime).hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n))
+    assert status == 0 and keep is not None
+    return n.value

@@ -1,20 +1,20 @@
 """The combine on both sides of the row count up to which it finds its rows among the triples without a map (1024 rows and
-slots): rows that name no slot, several that name the same one (the last counts), rows past the receive total, more rows than
-slots, both activation types.  Bit for bit, as everywhere in the combine."""
+slots) and of what its workgroups look through between them (5 x 2^20 triples): rows that name no slot, several that name the
+same one (the last counts), rows past the receive total, more rows than slots, both activation types.  Bit for bit, as everywhere in the combine."""
 import numpy as np
 import pytest
 import torch
 
 import umdk_original_amd as cam
 from umdk_original_amd import synth
-from gpu_util import announce, assert_bits_equal
+from gpu_util import announce, assert_bits_equal, recorded_kernels
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,K,A,valid,H", [(1, 1, 1, 1, 1024), (1, 16, 1024, 1000, 7168), (64, 16, 1024, 1024, 1032),
                                            (1024, 1, 1023, 900, 1024), (128, 8, 1025, 1025, 2048), (129, 8, 1024, 1024, 2048),
-                                           (7, 3, 21, 0, 1024)])
+                                           (7, 3, 21, 0, 1024), (1024, 1, 1024, 1000, 7168)])
 @pytest.mark.parametrize("fp16", [False, True])
 def test_rows_found_by_their_triples(gpu, oracle, T, K, A, valid, H, fp16):
     announce("combine scan T=%d K=%d A=%d valid=%d H=%d fp16=%d" % (T, K, A, valid, H, fp16))
@@ -23,7 +23,7 @@ def test_rows_found_by_their_triples(gpu, oracle, T, K, A, valid, H, fp16):
     src = np.stack([np.zeros(A, np.int64), slots // K, slots % K], axis=1).astype(np.int32)
     src[rng.random(A) < 0.1, 1] = T          # no such token
     src[rng.random(A) < 0.1, 2] = -1         # no such slot
-    if A <= 1024 and T * K <= 1024 and A > 8:
+    if A <= 1024 and T * K <= 1024 and T * -(-H // 1024) * A <= 5 << 20 and A > 8:
         src[A // 2] = src[A // 4]            # (with a map it is either of them)
     elif A > T * K:
         src[T * K:, 1] = -1
@@ -38,3 +38,12 @@ def test_rows_found_by_their_triples(gpu, oracle, T, K, A, valid, H, fp16):
     counts = torch.tensor([0, valid], dtype=torch.int32, device=gpu)
     got = cam.moe_combine_normal(y.to(gpu), torch.from_numpy(src.reshape(-1)).to(gpu), counts, w.to(gpu))
     assert_bits_equal(got.view(torch.int16).cpu().numpy().view(np.uint16), want, "combined x")
+
+
+@pytest.mark.parametrize("T,K,A,H,launches", [(1024, 1, 1024, 5120, 1), (1024, 1, 1024, 5128, 2), (865, 1, 865, 7168, 1),
+                                              (866, 1, 866, 7168, 2), (128, 8, 1025, 1024, 2), (129, 8, 1024, 1024, 2)])
+def test_launches(gpu, T, K, A, H, launches):
+    announce("combine launches T=%d K=%d A=%d H=%d" % (T, K, A, H))
+    y, w = torch.empty(A, H, dtype=torch.bfloat16, device=gpu), torch.empty(T, K, device=gpu)
+    src, counts = torch.empty(3 * A, dtype=torch.int32, device=gpu), torch.empty(2, dtype=torch.int32, device=gpu)
+    assert recorded_kernels(lambda: cam.moe_combine_normal(y, src, counts, w)) == launches

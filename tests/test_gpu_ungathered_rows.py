@@ -2,15 +2,13 @@
 copy, in front of a gate/up GEMM that does not gather.  What a token gets depends on no other token, so that every row has the bits
 it has in a layer of half the tokens, which gathers; a few of them are also compared with the oracle, at the tolerances of the
 ordinary layer tests."""
-import ctypes
-
 import numpy as np
 import pytest
 import torch
 
 import umdk_original_amd as cam
 from umdk_original_amd import synth
-from gpu_util import announce, assert_bits_equal, to_np
+from gpu_util import announce, assert_bits_equal, recorded_kernels, to_np
 from test_gpu_fp8 import _check_layer, _layer_inputs, _u8
 
 pytestmark = pytest.mark.gpu
@@ -76,18 +74,6 @@ def test_fp8_layer(gpu, oracle):
     _check_layer(out[s].float().cpu().numpy(), want)
 
 
-def _recorded_kernels(call):
-    """Nodes of the graph that a call records; nothing of it runs."""
-    runtime = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
-    g = torch.cuda.CUDAGraph(keep_graph=True)
-    with torch.cuda.graph(g):
-        keep = call()
-    n = ctypes.c_size_t()
-    status = ctypes.CDLL(runtime).hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n))
-    assert status == 0 and keep is not None
-    return n.value
-
-
 def test_schedules_take_no_launch_of_their_own(gpu):
     H, E, I = 512, 5, 512
     announce("launches of layers with and without gathered rows")
@@ -98,7 +84,7 @@ def test_schedules_take_no_launch_of_their_own(gpu):
     def launches(T):
         x = torch.empty(T, H, dtype=torch.bfloat16, device=gpu)
         ids, gates = torch.empty(T, 1, dtype=torch.int32, device=gpu), torch.empty(T, 1, device=gpu)
-        return _recorded_kernels(lambda: cam.fused_deep_moe(x, ids, *dev, gates, None, None, "", 1, 0, E, 1, 0, 0, 0))
+        return recorded_kernels(lambda: cam.fused_deep_moe(x, ids, *dev, gates, None, None, "", 1, 0, E, 1, 0, 0, 0))
 
     gathered = launches(1 << 16)
     assert gathered == 6                       # two of the plan, GMM1, re-quantisation, GMM2, combine

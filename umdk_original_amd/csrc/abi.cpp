@@ -1024,7 +1024,8 @@ camStatus camMoeCombineNormalGetWorkspaceSize(const camTensor *recvX, const camT
     CAM_TRY(check_aligned(recvX, "recvX", 16));
     CAM_TRY(check_aligned(out, "out", 16));
     Carver c;
-    const bool scan = cam::combine_scans(T, K, A);
+    // (the map's place is asked for where none is made, too: a call without a workspace is refused at every size)
+    const bool scan = cam::combine_scans(T, K, A, H);
     const uint64_t o_slot = c.take((uint64_t)T * K * 4);
     cam::CombineArgs g{};
     g.y = (const uint16_t *)recvX->data;

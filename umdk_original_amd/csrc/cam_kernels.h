@@ -157,7 +157,7 @@ struct CombineArgs {
 };
 hipError_t launch_combine(const CombineArgs &a, hipStream_t stream);
 // Whether a combine of rows of the activation type needs no map (launch_invert_src_info) beside the triples of its A rows.
-bool combine_scans(int64_t T, int64_t K, int64_t A);
+bool combine_scans(int64_t T, int64_t K, int64_t A, int64_t H);
 // bf16 rows [A,H] -> wire rows [A, H + H/4] bytes: per block of 8 columns int8 values and one bf16 scale.
 // row_limit: optional device scalar; rows >= *row_limit are left untouched.
 hipError_t launch_comm_quant(const uint16_t *y, int act_fp16, int64_t A, int H, const int32_t *row_limit, uint8_t *out,

@@ -28,6 +28,8 @@ namespace {
 
 constexpr int kCombThreads = 128;
 constexpr int kCombBatch = 8;
+// Workgroups that share the columns of a token, 8 columns a thread.
+constexpr int64_t column_segments(int64_t H) { return (H / 8 + kCombThreads - 1) / kCombThreads; }
 constexpr int kScanRows = 1024;  // triples a workgroup looks through at most, 8 a thread
 
 // Rows at or beyond *row_limit (the receive total, epRecvCounts[E-1] of moe_combine_normal.h:206-207) were
@@ -377,7 +379,7 @@ static hipError_t launch_combine_as(const CombineArgs &a, hipStream_t stream)
     if (a.H % 8 != 0) {
         return hipErrorInvalidValue;
     }
-    const int segs = (a.H / 8 + kCombThreads - 1) / kCombThreads;
+    const int segs = (int)column_segments(a.H);
     const long long blocks = (long long)a.T * segs;
     if (blocks > 0x7fffffffll) {
         return hipErrorInvalidValue;
@@ -401,22 +403,25 @@ static hipError_t launch_combine_as(const CombineArgs &a, hipStream_t stream)
 // A combine of few rows is as long as its launches.  us, layout + dispatch + combine, with the map / without: one token x 4096, top-8 34.6 /
 // 30.7, 64 x 2048, top-4 31.5 / 27.8, 100 x 4096, top-6 35.1 / 31.2, 128 x 7168, top-8 50.5 / 46.8 (1024 rows), 1000 x 1024, top-1
 // 32.4 / 28.9.  A thread's triples are one round trip to the L2; with more of them, each workgroup reading all, the launch that is
-// saved costs less.
-bool combine_scans(int64_t T, int64_t K, int64_t A)
+// saved costs less.  So it does with many workgroups that hardly do anything else: combine alone in a graph, top-1, 1024 x 1024 5.0 / 3.5,
+// 1024 x 4096 6.7 / 5.9, 800 x 7168 7.8 / 7.5, 1024 x 5120 7.7 / 7.6, 1024 x 6144 8.4-8.8 / 8.6, 1024 x 7168 9.3 / 10.1; top-2, 512 x
+// 7168 7.5 / 6.9.
+bool combine_scans(int64_t T, int64_t K, int64_t A, int64_t H)
 {
-    return A > 0 && A <= kScanRows && K <= kMaxTopk && T * K <= kScanRows;
+    return A > 0 && A <= kScanRows && K <= kMaxTopk && T * K <= kScanRows &&
+           T * column_segments(H) * A <= 5ll * kScanRows * kScanRows;
 }
 
 hipError_t launch_combine(const CombineArgs &a, hipStream_t stream)
 {
     if (a.ids == nullptr && a.slot_row == nullptr) {
-        if (a.src_info == nullptr || a.wire_rows || !combine_scans(a.T, a.K, a.A) || a.H % 8 != 0) {
+        if (a.src_info == nullptr || a.wire_rows || !combine_scans(a.T, a.K, a.A, a.H) || a.H % 8 != 0) {
             return hipErrorInvalidValue;
         }
         if (a.T <= 0) {
             return hipSuccess;
         }
-        const int segs = (a.H / 8 + kCombThreads - 1) / kCombThreads;
+        const int segs = (int)column_segments(a.H);
         const dim3 grid((unsigned)(a.T * segs)), block(kCombThreads);
         if (a.act_fp16) {
             hipLaunchKernelGGL((combine_kernel<false, 1, false, true>), grid, block, 0, stream, a, segs);
