@@ -419,7 +419,7 @@ camStatus camDispatchLayoutGetWorkspaceSize(const camTensor *topkIdx, int64_t nu
         return fail(CAM_ERR_SHAPE, "DispatchLayout outputs must be [R], [E] and [T,R]");
     }
     Carver c;
-    const uint64_t o_partial = c.take(cam::layout_workspace_bytes(numTokens, (int)numExperts, (int)numRanks));
+    const uint64_t o_partial = c.take(cam::layout_workspace_bytes(numTokens, (int)numTopk, (int)numExperts, (int)numRanks));
     cam::LayoutArgs l{};
     l.idx = topkIdx->data;
     l.idx_is64 = topkIdx->dtype == CAM_DT_INT64;

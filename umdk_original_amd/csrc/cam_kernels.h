@@ -69,9 +69,9 @@ struct LayoutArgs {
     int in_rank_bytes;    // 4 or 1
     int32_t *per_expert;  // [E]
     int32_t *per_rank;    // [R]
-    int32_t *partial;     // scratch of layout_workspace_bytes(T, E, R) bytes
+    int32_t *partial;     // scratch of layout_workspace_bytes(T, K, E, R) bytes
 };
-uint64_t layout_workspace_bytes(int64_t T, int E, int R);
+uint64_t layout_workspace_bytes(int64_t T, int K, int E, int R);
 hipError_t launch_layout(const LayoutArgs &a, hipStream_t stream);
 
 // NotifyDispatch on one rank: exclusive scan + triplets.

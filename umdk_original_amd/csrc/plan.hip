@@ -364,14 +364,18 @@ __global__ __launch_bounds__(kWave) void layout_sum_kernel(LayoutArgs a, int row
     }
 }
 
-// Workgroups of a layout and tokens of each: one of kLayoutOne threads alone for a round of tokens and few flags, which saves the
-// launch that adds the counts up; else one round of tokens per workgroup up to 64 of them, whose counts are two round trips to
-// add up.  us, layout + dispatch + combine, added up / alone: 300 tokens x 4096, top-3 34.4 / 30.2, 500 x 2048, top-8 37.5 / 33.5, 1000 x
-// 4096, top-6 38.0 / 36.9, 1024 x 1024, top-8 41.1 / 38.0; with two rounds 1999 x 4096, top-6 58.7 / 64.2 (the counts of one
-// workgroup's LDS collide).
-int layout_workgroups(long long T, int R, int *span)
+// Workgroups of a layout and tokens of each: one of kLayoutOne threads alone where that is sure to save more, the launch that adds the
+// counts up, than it costs; else one round of tokens per workgroup up to 64 of them, whose counts are two round trips to add up.
+// What it costs are the counts of the tokens beyond the 256 that a workgroup has in any case, one by one where all tokens name the
+// same experts (and, of several ranks, as many ranks): the line lies where such ids are not slower.  us, added up / alone, ids
+// spread over the experts and all the same: one rank, 1024 tokens, top-1 4.4 / 3.0 and 4.4 / 3.7, 768, top-2 4.4 / 3.0 and 4.5 / 4.0, 512,
+// top-4 4.8 / 3.4 and 5.3 / 4.5, 384, top-8 5.5 / 4.3 and 6.4 / 6.0, 320, top-16 6.8 / 5.7 and 8.9 / 8.5; beyond the line 600, top-4
+// 4.8 / 3.5 and 5.1 / 4.9, 450, top-8 5.5 / 4.6 and 6.4 / 6.7, 1024, top-6 5.1 / 4.5 and 5.8 / 8.6, top-16 7.2 / 11.4 and 9.4 / 22.6.
+// Sixteen ranks, 330 tokens, top-8 6.2 / 4.8 and 8.2 / 7.7; beyond, 384, top-8 6.1 / 5.0 and 8.1 / 8.4, 290, top-16 9.1 / 7.9 and 12.3 / 13.2.
+int layout_workgroups(long long T, int K, int R, int *span)
 {
-    if (T <= kLayoutOne && T * R <= 8 * kLayoutOne) {
+    const int counts = R > 1 ? 2 * K : K;
+    if (T <= kLayoutOne && T * R <= 8 * kLayoutOne && counts <= 20 && (T - kLayoutThreads) * counts <= 1024) {
         *span = kLayoutOne;
         return 1;
     }
@@ -533,10 +537,10 @@ hipError_t launch_layer_plan(const PlanArgs &p, const DispatchArgs &d, int32_t *
     return e != hipSuccess || row_token != nullptr ? e : launch_dispatch(d, stream);
 }
 
-uint64_t layout_workspace_bytes(int64_t T, int E, int R)
+uint64_t layout_workspace_bytes(int64_t T, int K, int E, int R)
 {
     int span;
-    return (uint64_t)layout_workgroups(T, R, &span) * (uint64_t)(E + R) * sizeof(int32_t);
+    return (uint64_t)layout_workgroups(T, K, R, &span) * (uint64_t)(E + R) * sizeof(int32_t);
 }
 
 template <typename IdT, int NT>
@@ -556,7 +560,7 @@ hipError_t launch_layout(const LayoutArgs &a, hipStream_t stream)
         return hipErrorInvalidValue;
     }
     int span;
-    const int n = layout_workgroups(a.T, a.R, &span);
+    const int n = layout_workgroups(a.T, a.K, a.R, &span);
     if (n == 1 && a.T > kLayoutThreads) {
         a.idx_is64 ? launch_layout_as<int64_t, kLayoutOne>(a, n, span, stream) : launch_layout_as<int32_t, kLayoutOne>(a, n, span, stream);
     } else {
