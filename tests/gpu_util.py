@@ -36,13 +36,37 @@ def assert_bits_equal(got, want, what):
             what, len(bad), got.size, bad[0].tolist(), got[tuple(bad[0])], want[tuple(bad[0])]))
 
 
-def recorded_kernels(call):
-    """Nodes of the graph that a call records; nothing of it runs."""
-    runtime = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+def _recorded(call):
+    """The runtime, the graph that a call records and its nodes; nothing of it runs."""
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+    hip = ctypes.CDLL(path)
     g = torch.cuda.CUDAGraph(keep_graph=True)
     with torch.cuda.graph(g):
         keep = call()
-    n = ctypes.c_size_t()
-    status = ctypes.CDLL(runtime).hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n))
-    assert status == 0 and keep is not None
-    return n.value
+    raw, n = ctypes.c_void_p(g.raw_cuda_graph()), ctypes.c_size_t()
+    assert keep is not None and hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    return hip, g, nodes
+
+
+def recorded_kernels(call):
+    """How many launches a call records."""
+    return len(_recorded(call)[2])
+
+
+class _KernelNode(ctypes.Structure):   # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint * 3),
+                ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
+def recorded_names(call):
+    """The mangled names of the kernels that a call records."""
+    hip, g, nodes = _recorded(call)
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    names = []
+    for node in nodes:
+        p = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+        names.append(hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), None).decode())
+    return names

@@ -1,17 +1,18 @@
-"""The permute on both sides of the output sizes between which its rows are stored plainly (72 and, 8-bit rows, 152 MiB; rows that
-are no whole lines 48): 16-bit, int8 and FP8 rows, rows under smooth scales, ids that name no expert.  Bit for bit, as everywhere in the dispatch."""
+"""The permute on both sides of the output sizes from which its rows are stored plainly (16-bit rows 72 MiB, rows that are no whole lines
+48, 8-bit rows of whole lines never): 16-bit, int8 and FP8 rows, rows under smooth scales, ids that name no expert.  Bit for bit, as
+everywhere in the dispatch."""
 import numpy as np
 import pytest
 import torch
 
 import umdk_original_amd as cam
 from umdk_original_amd import synth
-from gpu_util import announce
+from gpu_util import announce, recorded_names
 from test_gpu_dispatch import _check_fused
 import test_gpu_shmem
 
 pytestmark = pytest.mark.gpu
-K, E, H = 16, 300, 7168      # 659 to 1389 tokens of 8-bit rows lie between the lines, 330 and more of 16-bit rows
+K, E, H = 16, 300, 7168      # 659 tokens of 8-bit rows are 72 MiB, 330 of 16-bit rows
 
 
 @pytest.mark.parametrize("T,quant_mode,H", [(658, 2, H), (659, 2, H), (659, 3, H), (1390, 2, H), (329, 0, H), (330, 0, H),
@@ -40,3 +41,14 @@ def test_fp8_rows_between_the_lines(gpu, oracle):
 
 def test_smooth_rows_between_the_lines(gpu, oracle):
     test_gpu_shmem.test_dispatch_shmem_bit_exact(gpu, oracle, 660, K, E, H, 2, True, False, 1)
+
+
+@pytest.mark.parametrize("T,quant_mode,H,plainly", [(329, 0, H, False), (330, 0, H, True), (219, 0, 7160, False), (220, 0, 7160, True),
+                                                    (439, 2, 7160, False), (440, 2, 7160, True), (659, 2, H, False), (1389, 2, H, False),
+                                                    (3000, 2, H, False), (659, 4, H, False)])
+def test_how_rows_are_stored(gpu, T, quant_mode, H, plainly):
+    announce("permute how stored T=%d H=%d quant=%d" % (T, H, quant_mode))
+    x, ids = torch.empty(T, H, dtype=torch.bfloat16, device=gpu), torch.empty(T, K, dtype=torch.int32, device=gpu)
+    permute = recorded_names(lambda: cam.moe_dispatch_fused(x, ids, E, quant_mode=quant_mode))[-1]
+    form = {0: 0, 2: 1, 4: 3}[quant_mode]    # (rows copied, quantised to int8, to FP8)
+    assert "dispatch_kernelILi%dELi0ELb%dEE" % (form, plainly) in permute

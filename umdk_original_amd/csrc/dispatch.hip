@@ -40,23 +40,26 @@ __device__ __forceinline__ long long dispatch_row(const DispatchArgs &a, int t, 
 }
 
 // How the rows are stored.  Plain stores leave the L2 (32 MB) in a better order than the waves wrote the pieces of far apart rows in,
-// and their reader finds more of them in the memory-side cache.  But what still lies in the L2 at the end of the launch has to be
-// written back before the next one, which costs more than it gains while that is most of the output; and 8-bit rows, whose
-// pieces are half as long, lose again where there are many more of them than the caches hold.  us, non-temporal / plain:
-// dispatch of 16-bit rows alone, 16 MB 9.3 / 9.5, 33 MB 14.8 / 16.3, 49 MB 16.8 / 19.0; with a gather of other rows behind it
-// 72 MB 37.8 / 38.3, 79 MB 40.9 / 40.1, 196 MB 89.0 / 89.3, 803 MB 346 / 341; with layout and a gather of these rows, 79 MB 53.4 / 49.7,
-// 98 MB 59.8 / 55.5, 128 MB 73.3 / 65.4, 197 MB 103.6 / 89.3, 393 MB 187 / 169.  8-bit rows with a gather of other rows, 72 MB 54.7 /
-// 54.7, 86 MB 62.5 / 61.1, 131 MB 97.3 / 94.5, 143 MB 95.9 / 92.5 (FP8 98.3 / 95.7), 172 MB 113.0 / 115.1 (115.0 / 118.2), 235 MB
-// 150.0 / 151.2 (153.3 / 157.0).  Rows that are no whole lines of 128 bytes, dispatch with a gather of other rows: the L2 puts the two halves
-// of a line together, so they gain from less on and have no upper line: 16-bit 34 MB 25.3 / 27.8, 50 MB 32.8 / 32.0, 90 MB 56.7 / 49.4, 96
-// MB 65.5 / 57.5; int8 19 MB 25.0 / 26.9, 56 MB 48.2 / 46.1, 172 MB 130.5 / 120.7, 235 MB 176.2 / 166.0.
+// and a reader that goes through the rows once finds more of them in the memory-side cache.  But what still lies in the L2 at the
+// end of the launch has to be written back before the next one, which costs more than it gains while that is most of the
+// output.  us, non-temporal / plain, 16-bit rows: dispatch alone, 33 MB 14.8 / 16.3, 49 MB 16.8 / 19.0, 84 MB 24.5 / 28.7, 115 MB 32.0 / 35.1, 168 MB
+// 44.1 / 45.1, 210 MB 53.8 / 52.8, 420 MB 100.3 / 98.4; with a pass over the rows behind it, 84 MB 58.8 / 53.0, 115 MB 77.7 / 63.5, 168 MB
+// 105.3 / 89.1, 210 MB 128.5 / 119.4, 420 MB 240 / 237; with a product of these rows 84 MB 181.0 / 177.9, 168 MB 420 / 414, 420 MB 763 / 757;
+// with a gather of other rows 72 MB 37.8 / 38.3, 79 MB 40.9 / 40.1, 196 MB 89.0 / 89.3, 803 MB 346 / 341.
+// 8-bit rows are there for the expert GEMMs, whose tiles read them several times over, and these are slower behind plain stores,
+// although a single pass gains as above (84 MB 61.8 / 53.3): dispatch and GMM1, int8, rows of 7168 to 32 experts 88 MB 421.5 / 437.4, 105 MB
+// 486.7 / 492.4, 126 MB 562.7 / 562.1, 155 MB 675.5 / 684.4, to 256 126 MB 239.1 / 254.8, of 4096 to 128 88 MB 256.0 / 266.5; with GMM2 and
+// combine 657.8 / 669.7, 747.8 / 760.0, 879.6 / 876.9, 1038 / 1050, 458.8 / 481.7, 429.1 / 434.8.  FP8, 7168 to 32, 88 MB 410.7 / 423.4.
+// Rows that are no whole lines of 128 bytes (no GEMM here takes 8-bit ones): the L2 puts the two halves of a line together, so they gain from
+// less on, dispatch with a gather of other rows: 16-bit 34 MB 25.3 / 27.8, 50 MB 32.8 / 32.0, 90 MB 56.7 / 49.4, 96 MB 65.5 / 57.5; int8 19 MB
+// 25.0 / 26.9, 56 MB 48.2 / 46.1, 172 MB 130.5 / 120.7, 235 MB 176.2 / 166.0.
 bool stores_plainly(const DispatchArgs &a)
 {
     const long long pitch = (long long)a.H * (a.quant == 0 ? 2 : 1), bytes = (long long)a.T * a.K * pitch;
     if (pitch % 128 != 0) {
         return bytes >= 48ll << 20;
     }
-    return bytes >= 72ll << 20 && (a.quant == 0 || bytes < 152ll << 20);
+    return a.quant == 0 && bytes >= 72ll << 20;
 }
 
 // Four workgroups per CU (128 registers a lane) keep all 1024 workgroups of a 4096-token batch resident at once;
@@ -283,11 +286,11 @@ void launch_dispatch_as(const DispatchArgs &a, hipStream_t stream)
         } else {
             hipLaunchKernelGGL((dispatch_kernel<1, 0, PLAIN>), grid, block, 0, stream, a);
         }
-    } else if (a.quant == 3) {
+    } else if (a.quant == 3) {  // (whole lines: never plainly)
         if (fp16) {
-            hipLaunchKernelGGL((dispatch_kernel<3, 1, PLAIN>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((dispatch_kernel<3, 1, false>), grid, block, 0, stream, a);
         } else {
-            hipLaunchKernelGGL((dispatch_kernel<3, 0, PLAIN>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((dispatch_kernel<3, 0, false>), grid, block, 0, stream, a);
         }
     } else {
         if (fp16) {
