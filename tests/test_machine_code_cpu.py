@@ -86,3 +86,10 @@ def test_the_build_gives_no_such_library(monkeypatch, tmp_path, fault):
 def test_the_library_as_built():
     assert os.path.exists(build.LIB_PATH)
     assert machine_code.faults(build.LIB_PATH) == []
+
+
+def test_quantised_tokens_are_stored_non_temporally():
+    """What the plan's first launch leaves for a GEMM that gathers: the tiles are slower behind plain stores."""
+    found = [[t for t in code if t.startswith("global_store_dwordx2")] for listing in machine_code.listings(build.LIB_PATH)
+             for name, code, _ in machine_code.kernels(listing) if "plan_quant_kernel" in name]
+    assert len(found) == 6 and all(len(stores) >= 8 and all(t.endswith(" nt") for t in stores) for stores in found)

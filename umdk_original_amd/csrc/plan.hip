@@ -49,11 +49,14 @@ __global__ __launch_bounds__(kLocalThreads) void plan_local_kernel(PlanArgs a, i
 }
 
 // Phase 1 of a layer whose gate/up GEMM gathers its rows: the workgroups behind the nb that rank quantise the tokens, a wave each,
-// which depends on nothing that the plan finds out.  A token's row is stored once, not once per copy, and plainly: the GEMM
-// is to find it in a cache.  HBM bound where there are many tokens.  us, ranks + their second half + permute with schedules ->
-// this + phase 2 with schedules: 8192 tokens x 4096, top-8, int8 7.6 + 6.3 + 70.9 -> 20.9 + 15.5 (layer 1512 -> 1474); 4093 in
-// FP8 5.5 + 5.8 + 45.0 -> 15.5 + 13.5 (823 -> 787); 1021 x 2048, top-6, 4.8 + 4.8 + 9.1 -> 5.0 + 7.5 (160.9 -> 158.9).  With
-// rows of 4096 columns in the registers for 7168, at 3 (FP8) and 4 waves a SIMD, FP8 took 19.2.
+// which depends on nothing that the plan finds out.  A token's row is stored once, not once per copy, and non-temporally: the tiles
+// that read it are slower behind plain stores, most where a row has few copies.  Layers, us, plain / non-temporal: 3000 tokens x
+// 4096 to 128 experts, top-1, 257.2 / 249.1, 2000, top-2, 258.5 / 252.6, 1200 x 7168 to 32, top-1, 284.3 / 278.2, 8192 x 7168 to 64, top-2
+// 421.5 / 410.3 (FP8 417.5 / 406.9), 4093 x 4096 to 128, top-8 938.6 / 932.4, 8192 1417 / 1418, but 700 x 7168 to 4, top-4 257.1 / 259.2.
+// HBM bound where there are many tokens.  us, ranks + their second half + permute with schedules -> this + phase 2 with schedules
+// (plain stores): 8192 tokens x 4096, top-8, int8 7.6 + 6.3 + 70.9 -> 20.9 + 15.5 (layer 1512 -> 1474); 4093 in FP8 5.5 + 5.8 + 45.0
+// -> 15.5 + 13.5 (823 -> 787); 1021 x 2048, top-6, 4.8 + 4.8 + 9.1 -> 5.0 + 7.5 (160.9 -> 158.9).  With rows of 4096 columns in the
+// registers for 7168, at 3 (FP8) and 4 waves a SIMD, FP8 took 19.2.
 template <int CHUNKS, int QUANT, int ACT>
 __global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 5) void plan_quant_kernel(PlanArgs a, DispatchArgs d,
                                                                                                          int it, int nb)
@@ -95,7 +98,7 @@ __global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 
     for (int j = 0; j < Row::kChunks; ++j) {
         const int c = j * kWave + lane;
         if (c < nch) {
-            dst[c] = r.q[j];
+            __builtin_nontemporal_store(r.q[j], dst + c);
         }
     }
     if (QUANT == 3) {
