@@ -49,14 +49,25 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int tid, int *scratch
     return r;
 }
 
-// Number of set mask entries (the active prefix of the batch); T when there is no mask.
+// Number of set mask entries (the active prefix of the batch); T when there is no mask.  By at least 32 threads; sixteen entries a load,
+// as the quantising workgroups of a layer's plan ask for it too, every one of them.
 __device__ __forceinline__ int count_active(const uint8_t *mask, int T, int tid, int nthreads, int *slot)
 {
     if (mask == nullptr) {
         return T;
     }
+    const int head = min((int)(-(uintptr_t)mask & 15), T);  // up to where entries are whole 16-byte words
+    const int words = (T - head) >> 4;
     int c = 0;
-    for (int t = tid; t < T; t += nthreads) {
+    for (int i = tid; i < words; i += nthreads) {
+        const v4u v = ((const v4u *)(mask + head))[i];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            c += __popc((((v[j] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | v[j]) & 0x80808080u);  // bytes that are not zero
+        }
+    }
+    const int t = tid < 16 ? tid : head + 16 * words + (tid - 16);  // the entries in front of them and behind them
+    if (t < (tid < 16 ? head : T) && tid < 32) {
         c += mask[t] != 0 ? 1 : 0;
     }
     c = wave_sum(c);
