@@ -88,8 +88,9 @@ def test_the_library_as_built():
     assert machine_code.faults(build.LIB_PATH) == []
 
 
-def test_quantised_tokens_are_stored_non_temporally():
-    """What the plan's first launch leaves for a GEMM that gathers: the tiles are slower behind plain stores."""
+@pytest.mark.parametrize("plainly", [False, True])
+def test_how_quantised_tokens_are_stored(plainly):
+    """What the plan's first launch leaves for a GEMM that gathers: tiles of few rows are slower behind plain stores."""
     found = [[t for t in code if t.startswith("global_store_dwordx2")] for listing in machine_code.listings(build.LIB_PATH)
-             for name, code, _ in machine_code.kernels(listing) if "plan_quant_kernel" in name]
-    assert len(found) == 6 and all(len(stores) >= 8 and all(t.endswith(" nt") for t in stores) for stores in found)
+             for name, code, _ in machine_code.kernels(listing) if "plan_quant_kernel" in name and "Lb%dEEE" % plainly in name]
+    assert len(found) == 6 and all(len(stores) >= 8 and all(t.endswith(" nt") != plainly for t in stores) for stores in found)

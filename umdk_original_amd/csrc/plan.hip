@@ -49,16 +49,14 @@ __global__ __launch_bounds__(kLocalThreads) void plan_local_kernel(PlanArgs a, i
 }
 
 // Phase 1 of a layer whose gate/up GEMM gathers its rows: the workgroups behind the nb that rank quantise the tokens, a wave each,
-// which depends on nothing that the plan finds out.  A token's row is stored once, not once per copy, and non-temporally: the tiles
-// that read it are slower behind plain stores, most where a row has few copies.  Layers, us, plain / non-temporal: 3000 tokens x
-// 4096 to 128 experts, top-1, 257.2 / 249.1, 2000, top-2, 258.5 / 252.6, 1200 x 7168 to 32, top-1, 284.3 / 278.2, 8192 x 7168 to 64, top-2
-// 421.5 / 410.3 (FP8 417.5 / 406.9), 4093 x 4096 to 128, top-8 938.6 / 932.4, 8192 1417 / 1418, but 700 x 7168 to 4, top-4 257.1 / 259.2.
+// which depends on nothing that the plan finds out.  A token's row is stored once, not once per copy, and non-temporally up to 256 rows
+// per expert (quantised_plainly).
 // HBM bound where there are many tokens.  us, ranks + their second half + permute with schedules -> this + phase 2 with schedules
 // (plain stores): 8192 tokens x 4096, top-8, int8 7.6 + 6.3 + 70.9 -> 20.9 + 15.5 (layer 1512 -> 1474); 4093 in FP8 5.5 + 5.8 + 45.0
 // -> 15.5 + 13.5 (823 -> 787); 1021 x 2048, top-6, 4.8 + 4.8 + 9.1 -> 5.0 + 7.5 (160.9 -> 158.9).  With rows of 4096 columns in the
 // registers for 7168, at 3 (FP8) and 4 waves a SIMD, FP8 took 19.2.
 constexpr int kMaskedTokens = 16384;  // up to where a workgroup looks through the whole mask, as long as its four tokens at 2048 columns
-template <int CHUNKS, int QUANT, int ACT>
+template <int CHUNKS, int QUANT, int ACT, bool PLAIN>
 __global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 5) void plan_quant_kernel(PlanArgs a, DispatchArgs d,
                                                                                                          int it, int nb)
 {
@@ -105,7 +103,7 @@ __global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 
     for (int j = 0; j < Row::kChunks; ++j) {
         const int c = j * kWave + lane;
         if (c < nch) {
-            __builtin_nontemporal_store(r.q[j], dst + c);
+            store_piece<PLAIN>(r.q[j], dst + c);
         }
     }
     if (QUANT == 3) {
@@ -452,17 +450,35 @@ hipError_t launch_plan_t(const PlanArgs &a, int it, int nb, int32_t *hist, hipSt
     return hipGetLastError();
 }
 
-template <int QUANT, int ACT>
+// Whether the tokens of a layer that gathers are stored plainly: tiles of experts of few rows, which stream their weights, are slower
+// behind plain stores, taller ones take as long or less.  Layers, us, plain / non-temporal, rows per expert in front: 23 3000 tokens x 4096 to 128
+// experts, top-1 257.2 / 249.1; 31 2000, top-2 258.5 / 252.6; 47 3000 x 3072, top-2 224.9 / 218.6 (FP8 220.6 / 213.6); 37 1200 x 7168 to 32,
+// top-1 284.3 / 278.2; 128 8192 x 2048 to 64, top-1 157.0 / 152.8; 187 4000 x 3072, top-3 232.8 / 226.9; 256 8192 x 7168, top-2 421.5 / 410.3
+// and 4093 x 4096 to 128, top-8 938.6 / 932.4.  312 2500 x 4096 to 16, top-2 197.3 / 197.1; 512 8192 x 4096 to 128, top-8 1417 / 1418;
+// 512 8192 x 1536 to 32, top-2 120.7 / 122.2 (FP8 113.3 / 112.9); 700 700 x 7168 to 4, top-4 257.1 / 259.2; 1024 8192 x 1024 to 16, top-2 103.6 /
+// 104.8, 8192 to 32, top-4 149.3 / 152.3; 2048 8192 x 2048 to 16, top-4 220.0 / 223.0.
+bool quantised_plainly(const PlanArgs &p) { return (long long)p.T * p.K > 256ll * p.E; }
+
+template <int QUANT, int ACT, bool PLAIN>
 hipError_t launch_plan_quant_as(const PlanArgs &p, const DispatchArgs &d, int it, int nb, hipStream_t stream)
 {
     const dim3 grid((unsigned)nb + (unsigned)((d.T + kDispWaves - 1) / kDispWaves)), block(kLocalThreads);
     // rows of up to 4096 columns in registers for 4096: more waves to a SIMD
     if (d.H <= 8 * kWave * 8) {
-        hipLaunchKernelGGL((plan_quant_kernel<8, QUANT, ACT>), grid, block, 0, stream, p, d, it, nb);
+        hipLaunchKernelGGL((plan_quant_kernel<8, QUANT, ACT, PLAIN>), grid, block, 0, stream, p, d, it, nb);
     } else {
-        hipLaunchKernelGGL((plan_quant_kernel<kDispMaxChunks, QUANT, ACT>), grid, block, 0, stream, p, d, it, nb);
+        hipLaunchKernelGGL((plan_quant_kernel<kDispMaxChunks, QUANT, ACT, PLAIN>), grid, block, 0, stream, p, d, it, nb);
     }
     return hipGetLastError();
+}
+
+template <bool PLAIN>
+hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &d, int it, int nb, hipStream_t stream)
+{
+    if (d.quant == 3) {
+        return launch_plan_quant_as<3, 0, PLAIN>(p, d, it, nb, stream);
+    }
+    return d.x_is_fp16 ? launch_plan_quant_as<2, 1, PLAIN>(p, d, it, nb, stream) : launch_plan_quant_as<2, 0, PLAIN>(p, d, it, nb, stream);
 }
 
 }  // namespace
@@ -533,10 +549,8 @@ hipError_t launch_layer_plan(const PlanArgs &p, const DispatchArgs &d, int32_t *
     l.sched.parts = std::min(std::max((cap + kGlobalThreads - 1) / kGlobalThreads, 1), 32);
     if (row_token == nullptr) {
         e = launch_plan_local<int32_t>(p, it, nb, p.hist_ws, stream);
-    } else if (d.quant == 3) {
-        e = launch_plan_quant_as<3, 0>(p, d, it, nb, stream);
     } else {
-        e = d.x_is_fp16 ? launch_plan_quant_as<2, 1>(p, d, it, nb, stream) : launch_plan_quant_as<2, 0>(p, d, it, nb, stream);
+        e = quantised_plainly(p) ? launch_plan_quant<true>(p, d, it, nb, stream) : launch_plan_quant<false>(p, d, it, nb, stream);
     }
     if (e != hipSuccess) {
         return e;
