@@ -183,15 +183,15 @@ def _layer(T, H, E, K, I, seed):
 
 @pytest.mark.parametrize("T,H,E,K,I,active,as_list,dropped", [
     (500, 512, 8, 2, 2176, None, False, False),     # 1000 ids: plan of one workgroup
-    (512, 1152, 16, 4, 1152, None, False, False),   # 2048 ids: the most that plan and permute share a launch for, were it not
-                                                    # for the schedules; ragged column blocks
+    (512, 1152, 16, 4, 1152, None, False, False),   # 2048 ids: the most that plan and permute share a launch for where
+                                                    # there are no schedules; ragged column blocks
     (513, 1024, 16, 4, 1152, None, False, True),    # 2052 ids, some dropped
     (700, 1024, 16, 4, 768, 601, True, False),      # masked tokens, a weight tensor per expert
     (2100, 512, 4, 1, 1152, 1000, False, False),    # most tokens masked
     (1021, 1024, 64, 6, 768, None, False, False),   # most experts flat
 ])
 def test_layer_bit_exact(gpu, oracle, T, H, E, K, I, active, as_list, dropped):
-    """Layers whose schedules are built beside the permute."""
+    """Layers whose schedules are built in the plan's second launch."""
     announce("tile form, layer T=%d H=%d E=%d K=%d I=%d active=%s as_list=%s dropped=%s" % (T, H, E, K, I, active, as_list,
                                                                                           dropped))
     assert T * K * 2 * I > LIMIT
@@ -325,7 +325,7 @@ def test_narrow_fp8(gpu, oracle, K):
 
 
 def test_narrow_layer_bit_exact(gpu, oracle):
-    """The narrow schedule as the permute launch builds it."""
+    """The narrow schedule as the plan's second launch builds it."""
     T, H, E, K, I = 1021, 512, 64, 6, 1152
     announce("tile form, narrow tiles, layer T=%d H=%d E=%d K=%d I=%d" % (T, H, E, K, I))
     d = _layer(T, H, E, K, I, 5)

@@ -955,7 +955,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a)
             at[j] = min(r0 + 8 * j, t.rows - 1);
         }
         // All of them in one round trip to the LDS, here and in the K loop.  Asked one by one, each beside its load: layer of 8192 tokens x
-        // 4096 1506 us, now 1499, of 4093 in FP8 800, now 796; both GEMMs of 8192 rows x 7168, which do not gather, 453, now 446.
+        // 4096 1506 us, now 1499, of 4093 in FP8 800, now 796; both GEMMs of 8192 rows x 7168, which do not gather, 453, now 446,
+        // as before there was anything to gather.
         if (gather) {
             row = rows_s[row];
 #pragma unroll

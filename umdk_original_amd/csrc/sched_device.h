@@ -99,7 +99,7 @@ struct SchedOwnTables {
 struct SchedSharedTables {
     int work_before[kMaxExperts];         // by rank: work of the tall experts ranked before
     int flat_rank[kMaxExperts];           // by rank: flat experts ranked before
-    short cfirst[kNumXcd + 1][kMaxExperts];  // by rank: the expert's groups in queues before x (tall)
+    short cfirst[kNumXcd][kMaxExperts];   // by rank: the expert's groups in queues before x (tall)
     int qbase[kNumXcd][kMaxExperts];      // by rank: items of earlier experts of its kind in queue x
     int qtall[kNumXcd], qflat[kNumXcd];
     int wtotal;
