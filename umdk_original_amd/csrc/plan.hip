@@ -8,7 +8,8 @@
 //   recv cumsum   src/cam/comm_operator/pybind/moe_dispatch_prefill.cpp:126-145
 //
 // Design.  The rank of an entry is its position among earlier flat (t,k) entries with the same
-// expert id, i.e. a stable counting sort; atomics would make the order depend on scheduling.  Two
+// expert id, i.e. a stable counting sort; atomics would make the order depend on scheduling.  Up to kExpertIds ids one
+// launch, in which a workgroup per expert looks at all of them (plan_experts_kernel); beyond, two
 // short launches, no atomics on results, no spinning, fully deterministic:
 //   1. every workgroup ranks its own contiguous chunk of the flat id sequence (wave ballots + per-wave
 //      LDS histograms) and publishes the chunk's per-expert histogram;
@@ -30,6 +31,8 @@ namespace {
 
 constexpr int kScanThreads = 1024;  // single-workgroup scan kernel (notify)
 constexpr int kGlobalThreads = 512; // phase 2: one thread per expert column
+constexpr int kExpertThreads = 1024;  // of a workgroup that looks at all ids for one expert,
+constexpr int kExpertIds = 16 * kExpertThreads;  // and up to how many there are such
 
 // Phase 1.  Workgroup b ranks the flat entries [b*chunk, (b+1)*chunk), chunk = IT*256 (rank_chunk), and
 // publishes the chunk's per-expert histogram in hist_out[b][*].
@@ -255,31 +258,61 @@ __global__ __launch_bounds__(kGlobalThreads) void plan_global_kernel(PlanArgs a,
     }
 }
 
-// Both phases in one workgroup, for id sequences that fit one chunk (at most 4 * 256 entries): the chunk's
-// histogram is the per-expert count and every base is zero, so nothing has to pass between workgroups and the
-// plan costs one launch instead of two.
+// Both phases in one launch with a workgroup per expert, each of which looks at all ids (ExpertEntries): it finds the expert's
+// offset, count and ranks by itself, so nothing passes between workgroups.  Bound by latency, and from some ten thousand ids on by
+// its instructions: every workgroup goes through all ids, which is why the two launches come back beyond kExpertIds.  us, replayed
+// from a graph, two launches (up to 1024 ids one workgroup) / this, ids spread over the experts: 64 ids to 8 experts 3.0 / 2.7, 1024 to 128
+// 5.7 / 2.9, 2400 to 64 5.7 / 2.9, 6126 to 64 5.9 / 3.3, 11994 to 64 6.5 / 4.0, 16384 to 256 6.5 / 4.4 (all the same ids 6.4 / 4.7); with 32 and
+// 64 ids a thread, 32768 to 256 7.2 / 6.7 (7.2 / 7.3), 48000 to 64 8.6 / 12.9, 64000 to 256 9.9 / 11.8, to 8 8.3 / 15.6.
 template <typename IdT, int IT>
-__global__ __launch_bounds__(kLocalThreads) void plan_single_kernel(PlanArgs a)
+__global__ __launch_bounds__(kExpertThreads, 8) void plan_experts_kernel(PlanArgs a)
 {
-    __shared__ int hist[kLocalWaves * kMaxExperts];
-    __shared__ int cnt_s[kMaxExperts];
-    __shared__ int scan_s[kLocalWaves];
-    __shared__ int total_s;
+    __shared__ int scratch[2 * kExpertThreads / kWave];
     __shared__ int active_s;
     const int tid = threadIdx.x;
-    const int E = a.E;
-    const IdT *__restrict__ idx = (const IdT *)a.idx;
-    const int t_active = count_active(a.mask, a.T, tid, kLocalThreads, &active_s);
-    const long long n = (long long)t_active * a.K;
-    const long long n_all = (long long)a.T * a.K;
-    rank_chunk<IdT, IT>(idx, 0, n, n_all, E, hist, a.pos, cnt_s);
-    __syncthreads();  // cnt_s complete; the ranks in a.pos are visible to the whole workgroup
-    write_expert_outputs<kLocalThreads>(a, cnt_s, t_active, tid, scan_s, &total_s);  // (leaves the offsets in cnt_s)
-    __syncthreads();
-    if (a.dst_row != nullptr) {
-        for (long long i = tid; i < n_all; i += kLocalThreads) {
-            const int e = i < n ? load_id(idx, i, E) : -1;
-            a.dst_row[i] = e >= 0 ? cnt_s[e] + a.pos[i] : -1;
+    const int x = blockIdx.x;
+    const int n_all = a.T * a.K;
+    ExpertEntries<kExpertThreads, IT> ids;
+    ids.load((const IdT *)a.idx, n_all);
+    const int t_active = count_active(a.mask, a.T, tid, kExpertThreads, &active_s);
+    ids.only_first(t_active * a.K);
+    ids.count(x, scratch);
+    if (tid == 0) {
+        const int end = ids.off + ids.cnt;
+        if (a.tokens_per_expert) store_count(a.tokens_per_expert + x, ids.cnt);
+        if (a.cnt) a.cnt[x] = ids.cnt;
+        if (a.off) a.off[x] = ids.off;
+        if (a.recv_off) a.recv_off[x] = ids.off;
+        if (a.recv_count) a.recv_count[x] = end;
+        if (a.group_list) a.group_list[x] = (int64_t)end;
+        if (x == a.E - 1) {
+            if (a.total) {
+                a.total[0] = end;
+            }
+            if (a.meta != nullptr) {
+                a.meta[0] = 0;
+                a.meta[1] = end;
+                a.meta[2] = t_active;
+                a.meta[3] = 0;
+            }
+        }
+    }
+    ids.ranks(x, [&](int i, int rank) {
+        a.pos[i] = rank;
+        if (a.dst_row != nullptr) {
+            a.dst_row[i] = ids.off + rank;
+        }
+    });
+    if (x == 0) {  // the entries of no expert
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int i = ids.first_entry() + it * kWave + (tid & (kWave - 1));
+            if ((unsigned)ids.e[it] >= (unsigned)a.E && i < n_all) {
+                a.pos[i] = -1;
+                if (a.dst_row != nullptr) {
+                    a.dst_row[i] = -1;
+                }
+            }
         }
     }
 }
@@ -429,18 +462,34 @@ hipError_t launch_plan_local(const PlanArgs &a, int it, int nb, int32_t *hist, h
     return hipGetLastError();
 }
 
+// f(IT), the ids a thread of a workgroup that looks at all n keeps, n <= kExpertIds.
+template <typename F>
+void with_ids_per_thread(long long n, F &&f)
+{
+    if (n <= 4 * kExpertThreads) {
+        f(std::integral_constant<int, 4>());
+    } else if (n <= 8 * kExpertThreads) {
+        f(std::integral_constant<int, 8>());
+    } else if (n <= 12 * kExpertThreads) {
+        f(std::integral_constant<int, 12>());
+    } else {
+        f(std::integral_constant<int, 16>());
+    }
+}
+
+template <typename IdT>
+hipError_t launch_plan_experts(const PlanArgs &a, hipStream_t stream)
+{
+    with_ids_per_thread((long long)a.T * a.K, [&](auto it) {
+        hipLaunchKernelGGL((plan_experts_kernel<IdT, decltype(it)::value>), dim3(a.E), dim3(kExpertThreads), 0, stream, a);
+    });
+    return hipGetLastError();
+}
+
 template <typename IdT>
 hipError_t launch_plan_t(const PlanArgs &a, int it, int nb, int32_t *hist, hipStream_t stream)
 {
     const dim3 grid(nb), blk(kLocalThreads);
-    if (nb == 1) {
-        switch (it) {
-            case 1: hipLaunchKernelGGL((plan_single_kernel<IdT, 1>), grid, blk, 0, stream, a); break;
-            case 2: hipLaunchKernelGGL((plan_single_kernel<IdT, 2>), grid, blk, 0, stream, a); break;
-            default: hipLaunchKernelGGL((plan_single_kernel<IdT, 4>), grid, blk, 0, stream, a); break;
-        }
-        return hipGetLastError();
-    }
     const hipError_t e = launch_plan_local<IdT>(a, it, nb, hist, stream);
     if (e != hipSuccess) {
         return e;
@@ -486,8 +535,6 @@ hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &d, int it, i
 void plan_geometry(long long n_all, int *it_out, int *nb_out)
 {
     int it = 1;
-    // One workgroup up to four rounds of ids (4.4-6.8 us), two launches from there on (9.6 us, where 2048 ids took one
-    // workgroup 12.2).
     if (n_all <= 4 * kLocalThreads) {
         while ((long long)it * kLocalThreads < n_all) {
             it *= 2;
@@ -513,6 +560,9 @@ hipError_t launch_plan(const PlanArgs &a, hipStream_t stream)
 {
     if (a.hist_ws == nullptr) {
         return hipErrorInvalidValue;
+    }
+    if ((long long)a.T * a.K <= kExpertIds) {
+        return a.idx_is64 ? launch_plan_experts<int64_t>(a, stream) : launch_plan_experts<int32_t>(a, stream);
     }
     int it, nb;
     plan_geometry((long long)a.T * a.K, &it, &nb);

@@ -203,6 +203,101 @@ __device__ __forceinline__ void rank_chunk(const IdT *__restrict__ idx, int b, l
     }
 }
 
+// What the ids say about one expert, found by one workgroup of NT threads that looks at all of them.  Wave w owns the IT * 64
+// entries from w * IT * 64 on and a lane keeps its ids in registers.  The number of entries that name an earlier expert is
+// the expert's offset, the number of earlier ones that name it the rank of an entry: counts of ballots, with no table and no
+// atomics, so the work does not depend on how the ids are spread.  What bounds it are its instructions, about ten for 64 ids (with
+// range checks and 64-bit addresses at every load it were forty).
+template <int NT, int IT>
+struct ExpertEntries {
+    int e[IT];     // ids, none of 0 .. E - 1 where an entry names no expert
+    int off, cnt;  // the expert's first row and its entries
+    int prior;     // of its entries, those in front of this wave's
+
+    static __device__ __forceinline__ int first_entry()
+    {
+        return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * (IT * kWave);
+    }
+
+    // (n_all <= NT * IT; entries beyond it are read as zeros, see only_first)
+    template <typename IdT>
+    __device__ __forceinline__ void load(const IdT *idx, int n_all)
+    {
+        const __amdgpu_buffer_rsrc_t rsrc =
+            __builtin_amdgcn_make_buffer_rsrc((void *)idx, 0, n_all * (int)sizeof(IdT), 0x00020000);
+        const int at = (first_entry() + (int)(threadIdx.x & (kWave - 1))) * (int)sizeof(IdT);
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            if constexpr (sizeof(IdT) == 8) {
+                const v2u v = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(rsrc, at + it * kWave * 8, 0, 0));
+                e[it] = v[1] == 0u ? (int)v[0] : -1;
+            } else {
+                e[it] = (int)__builtin_amdgcn_raw_buffer_load_b32(rsrc, at + it * kWave * 4, 0, 0);
+            }
+        }
+    }
+
+    // Entries from n on name no expert.
+    __device__ __forceinline__ void only_first(int n)
+    {
+        if (first_entry() + IT * kWave > n) {
+            const int i = first_entry() + (int)(threadIdx.x & (kWave - 1));
+#pragma unroll
+            for (int it = 0; it < IT; ++it) {
+                e[it] = i + it * kWave < n ? e[it] : -1;
+            }
+        }
+    }
+
+    // scratch: 2 * NT / 64 ints of LDS
+    __device__ __forceinline__ void count(int x, int *scratch)
+    {
+        constexpr int kWaves = NT / kWave;
+        const int lane = threadIdx.x & (kWave - 1);
+        const int w = threadIdx.x >> 6;
+        int below = 0, own = 0;
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            below += (unsigned)e[it] < (unsigned)x ? 1 : 0;
+            own += __popcll(__ballot(e[it] == x));
+        }
+        below = wave_sum(below);
+        if (lane == 0) {
+            scratch[w] = below;
+            scratch[kWaves + w] = own;
+        }
+        __syncthreads();
+        off = wave_sum(lane < kWaves ? scratch[lane] : 0);
+        const int inc = wave_inclusive_scan(lane < kWaves ? scratch[kWaves + lane] : 0);
+        cnt = wave_last(inc);
+        prior = __shfl(inc, w, kWave) - own;
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            asm volatile("" : "+v"(e[it]));  // ranks() compares anew: the masks would take two scalar registers each until then
+        }
+    }
+
+    // f(entry, rank) for every entry of the expert
+    template <typename F>
+    __device__ __forceinline__ void ranks(int x, F &&f)
+    {
+        const int lane = threadIdx.x & (kWave - 1);
+        const int base = first_entry() + lane;
+        const unsigned long long lt_mask = (1ull << lane) - 1ull;
+        int run = __builtin_amdgcn_readfirstlane(prior);
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const unsigned long long named = __ballot(e[it] == x);
+            if (named != 0) {
+                if (e[it] == x) {
+                    f(base + it * kWave, run + __popcll(named & lt_mask));
+                }
+                run += __popcll(named);
+            }
+        }
+    }
+};
+
 }  // namespace cam
 
 #endif  // CAM_RANK_DEVICE_H_
