@@ -1,0 +1,81 @@
+"""The int8 layer of a handful of tokens in its two launches, bit for bit against the oracle: one slot and the most (8, 16, 32), one row
+per expert and as many as tokens (more than are asked for at once), K steps that no wave shares evenly, the shortest and longest rows,
+both activation types, weights per expert, experts named twice by a token, ids of no expert, masks down to no token at all; and on
+which side of its lines a layer takes them."""
+import numpy as np
+import pytest
+import torch
+
+import umdk_original_amd as cam
+from umdk_original_amd import synth
+from gpu_util import announce, assert_bits_equal, recorded_kernels, to_np
+from test_gpu_fused import _check, _run
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(T, H, E, K, I, ids=None):
+    g = torch.Generator().manual_seed(T * K + H + I)
+    w1, w1s = synth.absmax_int8_weights(E, H, 2 * I, seed=5)
+    w2, w2s = synth.absmax_int8_weights(E, I, H, seed=6)
+    ids = torch.rand(T, max(E, K), generator=g).argsort(dim=1)[:, :K] % E if ids is None else torch.tensor(ids)
+    return dict(x=synth.normal_bf16(T, H, seed=7), ids=ids, gates=torch.rand(T, K, generator=g), w1=w1, w1_scale=w1s, w2=w2, w2_scale=w2s)
+
+
+@pytest.mark.parametrize("T,H,E,K,I", [
+    (1, 512, 1, 1, 512),       # one slot
+    (1, 4096, 40, 8, 1536),
+    (1, 7168, 16, 12, 640),    # the longest row
+    (1, 1152, 3, 8, 3072),     # experts named more than once, the longest products
+    (8, 1024, 2, 1, 1152),     # up to eight rows to an expert
+    (8, 640, 1, 2, 512),       # eight tokens that all name it twice
+    (2, 2048, 64, 8, 1408),
+    (4, 4096, 64, 8, 512),     # 32 slots
+    (3, 4096, 50, 7, 1024),    # 21 slots
+    (5, 2048, 9, 3, 640)])
+def test_layer_bit_exact(gpu, oracle, T, H, E, K, I):
+    announce("few tokens T=%d H=%d E=%d K=%d I=%d" % (T, H, E, K, I))
+    d = _layer(T, H, E, K, I)
+    assert _check(oracle, d, *_run(gpu, d)) == 0
+    x = d["x"].half()
+    out = cam.fused_deep_moe(x.to(gpu), d["ids"].to(torch.int32).to(gpu), [cam.prepack_weight(d["w1"].to(gpu), True)], [d["w1_scale"].to(gpu)],
+                             [cam.prepack_weight(d["w2"].to(gpu), False)], [d["w2_scale"].to(gpu)], d["gates"].to(gpu), None, None, "", 1, 0,
+                             E, 1, 0, 0, 0)[0]
+    want, _ = oracle.fused_layer_fp16(x.view(torch.int16).numpy().view(np.uint16), d["ids"].numpy(), d["gates"].numpy(), d["w1"].numpy(),
+                                      d["w1_scale"].numpy(), d["w2"].numpy(), d["w2_scale"].numpy())
+    assert_bits_equal(to_np(out.view(torch.int16)).view(np.uint16), want, "fp16 layer")
+
+
+@pytest.mark.parametrize("active", [0, 1, 3, 5])
+def test_masks_dropped_ids_and_weights_per_expert(gpu, oracle, active):
+    announce("few tokens, %d of 5 active" % active)
+    d = _layer(5, 1024, 6, 3, 512, ids=[[0, -1, 5], [6, 6, -1], [2, 2, 0], [5, 1, 2], [0, 3, -7]])
+    d["x"][2] = 0
+    mask = torch.arange(5) < active
+    out, etn = _run(gpu, d, mask=mask, per_expert=True)
+    # the oracle's layer takes ids that name experts: the others with a weight of nothing, and not counted
+    ids = d["ids"].numpy()
+    dropped = (ids < 0) | (ids >= 6)
+    ok = dict(d, ids=torch.from_numpy(np.where(dropped, 4, ids)), gates=torch.from_numpy(np.where(dropped, 0.0, d["gates"].numpy()).astype(np.float32)))
+    want, _ = oracle.fused_layer(synth.bf16_bits(ok["x"]), ok["ids"].numpy(), ok["gates"].numpy(), d["w1"].numpy(), d["w1_scale"].numpy(),
+                                 d["w2"].numpy(), d["w2_scale"].numpy(), n_active=active)
+    got = to_np(out)
+    got, want = np.where(got == 0x8000, 0, got), np.where(want == 0x8000, 0, want)   # (a weight of nothing may leave a zero's sign)
+    assert_bits_equal(got, want, "output")
+    flat = ids[:active][~dropped[:active]]
+    assert_bits_equal(to_np(etn), np.bincount(flat, minlength=6), "tokens per expert")
+
+
+@pytest.mark.parametrize("T,H,E,K,I,few", [(1, 512, 4, 8, 3072, True), (8, 1024, 4, 1, 512, True), (9, 1024, 4, 1, 512, False),
+                                           (8, 6144, 4, 1, 512, True), (8, 6272, 4, 1, 512, False),
+                                           (2, 1024, 8, 8, 1024, True), (2, 1024, 8, 8, 1152, False),
+                                           (4, 4096, 64, 8, 512, True), (4, 4096, 63, 8, 512, False), (4, 3968, 64, 8, 512, False),
+                                           (5, 4096, 64, 4, 512, False), (4, 4096, 64, 8, 1536, True), (4, 4096, 64, 8, 1664, False)])
+def test_which_layers(gpu, T, H, E, K, I, few):
+    announce("few tokens or not T=%d H=%d E=%d K=%d I=%d" % (T, H, E, K, I))
+    dev = [[cam.prepack_weight(torch.empty(E, H, 2 * I, dtype=torch.int8, device=gpu), True)], [torch.empty(E, 2 * I, device=gpu)],
+           [cam.prepack_weight(torch.empty(E, I, H, dtype=torch.int8, device=gpu), False)], [torch.empty(E, H, device=gpu)]]
+    x, ids = torch.empty(T, H, dtype=torch.bfloat16, device=gpu), torch.empty(T, K, dtype=torch.int32, device=gpu)
+    gates = torch.empty(T, K, device=gpu)
+    n = recorded_kernels(lambda: cam.fused_deep_moe(x, ids, *dev, gates, None, None, "", 1, 0, E, 1, 0, 0, 0))
+    assert n == 2 if few else n > 2

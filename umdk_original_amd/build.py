@@ -22,7 +22,7 @@ LIB_PATH = os.path.join(LIB_DIR, "libcam_mi355x.so")
 TIMELINE_LIB_PATH = os.path.join(LIB_DIR, "libcam_mi355x_timeline.so")
 CALIB_LIB_PATH = os.path.join(LIB_DIR, "libcam_calib.so")  # calibration micro-benchmarks, loaded by bench.py only
 ABI_CONSUMER_PATH = os.path.join(LIB_DIR, "abi_consumer")  # plain-C caller of the ABI (csrc/abi_consumer.c), for tests
-SOURCES = ["abi.cpp", "plan.hip", "dispatch.hip", "combine.hip", "gemm.hip", "stream_gemm.hip"]
+SOURCES = ["abi.cpp", "plan.hip", "dispatch.hip", "combine.hip", "gemm.hip", "stream_gemm.hip", "few_tokens.hip"]
 
 # -packed-fp32-ops is switched off on purpose: packed fp32 VALU forms are not used by this library.
 HIPCC_FLAGS = [

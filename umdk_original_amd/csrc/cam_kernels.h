@@ -216,6 +216,30 @@ bool stream_gemm_takes_products(int64_t max_rows, int G, int Kd, int N, int64_t 
 // rows_per_expert: the most rows one expert can have, as far as the host knows.
 hipError_t launch_stream_gemm(const StreamGemmArgs &a, int64_t rows_per_expert, hipStream_t stream);
 
+// The int8 layer of a handful of tokens (few_tokens.hip): routing, quantisation, gate/up GEMM and SwiGLU in one launch, re-quantisation,
+// down GEMM and combine in another.  w, w_scale, list are those of the launch's GEMM.
+constexpr int kFewTokens = 8;    // at most, of
+constexpr int kFewSlots = 32;    // (token, k) slots at most
+constexpr int kFewMaxH = 7168;
+struct FewTokensArgs {
+    const uint16_t *x;      // [T,H]
+    int x_is_fp16;
+    const int32_t *ids;     // [T,K]
+    const float *gates;     // [T,K]
+    const uint8_t *mask;    // optional [T]
+    int T, K, H, I, E;
+    const int8_t *w;        // packed [E,H,2I] or [E,I,H]
+    const float *w_scale;   // [E,2I] or [E,H]
+    int per_expert;         // weights given per expert through `list`
+    WeightPtrs list;
+    float *products;        // [T*K,I]: written by the first launch, read by the second
+    int64_t *tokens_per_expert;  // [E]
+    uint16_t *out;          // [T,H]
+};
+bool few_tokens_apply(int64_t T, int64_t K, int64_t E, int64_t H, int64_t I);  // whether that is the faster form
+hipError_t launch_few_tokens_up(const FewTokensArgs &a, hipStream_t stream);
+hipError_t launch_few_tokens_down(const FewTokensArgs &a, hipStream_t stream);
+
 // fp32 SwiGLU products [rows,I] -> int8 + per-row scale.  sched_for_rows: optional schedule whose header holds
 // the number of valid rows.
 hipError_t launch_requant(const float *y, int64_t max_rows, int I, const int32_t *sched_for_rows, int8_t *q,
