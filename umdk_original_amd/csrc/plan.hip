@@ -51,42 +51,14 @@ __global__ __launch_bounds__(kLocalThreads) void plan_local_kernel(PlanArgs a, i
     }
 }
 
-// Phase 1 of a layer whose gate/up GEMM gathers its rows: the workgroups behind the nb that rank quantise the tokens, a wave each,
-// which depends on nothing that the plan finds out.  A token's row is stored once, not once per copy, and non-temporally up to 256 rows
-// per expert (quantised_plainly).
-// HBM bound where there are many tokens.  us, ranks + their second half + permute with schedules -> this + phase 2 with schedules
-// (plain stores): 8192 tokens x 4096, top-8, int8 7.6 + 6.3 + 70.9 -> 20.9 + 15.5 (layer 1512 -> 1474); 4093 in FP8 5.5 + 5.8 + 45.0
-// -> 15.5 + 13.5 (823 -> 787); 1021 x 2048, top-6, 4.8 + 4.8 + 9.1 -> 5.0 + 7.5 (160.9 -> 158.9).  With rows of 4096 columns in the
-// registers for 7168, at 3 (FP8) and 4 waves a SIMD, FP8 took 19.2.
+// A wave per token: what the workgroups of a layer's plan behind those that rank do.
 constexpr int kMaskedTokens = 16384;  // up to where a workgroup looks through the whole mask, as long as its four tokens at 2048 columns
-template <int CHUNKS, int QUANT, int ACT, bool PLAIN>
-__global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 5) void plan_quant_kernel(PlanArgs a, DispatchArgs d,
-                                                                                                         int it, int nb)
+template <int CHUNKS, int QUANT, int ACT, bool PLAIN, int NT>
+__device__ __forceinline__ void quantise_token(const PlanArgs &a, const DispatchArgs &d, int block, int *active_s)
 {
     typedef TokenRow<CHUNKS, kWave> Row;
-    static_assert(kLocalThreads == kDispWaves * kWave, "both kinds of workgroups are as large");
-    __shared__ int hist[kLocalWaves * kMaxExperts];
-    __shared__ int active_s;
     const int tid = threadIdx.x;
-    const int b = blockIdx.x;
-    if (b < nb) {
-        const int t_active = count_active(a.mask, a.T, tid, kLocalThreads, &active_s);
-        auto rank = [&](auto ic) {
-            rank_chunk<int32_t, decltype(ic)::value>((const int32_t *)a.idx, b, (long long)t_active * a.K, (long long)a.T * a.K,
-                                                     a.E, hist, a.pos, a.hist_ws + (long long)b * a.E);
-        };
-        switch (it) {
-            case 1: rank(std::integral_constant<int, 1>()); break;
-            case 2: rank(std::integral_constant<int, 2>()); break;
-            case 4: rank(std::integral_constant<int, 4>()); break;
-            default: rank(std::integral_constant<int, 8>()); break;
-        }
-        if (b == 0 && tid == 0) {
-            a.hist_ws[(long long)nb * a.E] = t_active;
-        }
-        return;
-    }
-    const int t = (b - nb) * kDispWaves + (tid >> 6);
+    const int t = block * (NT / kWave) + (tid >> 6);
     const int lane = tid & (kWave - 1);
     // A token that goes nowhere, behind the active ones or without an expert, is not stored.  us, stored / not, layers of which one token
     // in sixteen goes somewhere: 8192 x 7168 to 64 experts, top-2, 229.3 / 217.0 under a mask and 240.5 / 232.0 with ids dropped, 5000 to
@@ -95,7 +67,7 @@ __global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 
     const int at = min(t, a.T - 1);
     const int id = ((const int32_t *)a.idx)[(long long)at * a.K + min(lane, a.K - 1)];  // looked at when the row is under way
     load_token_row(d.x, at, d.H, lane, r);
-    const int t_active = a.T <= kMaskedTokens ? count_active(a.mask, a.T, tid, kLocalThreads, &active_s) : a.T;
+    const int t_active = a.T <= kMaskedTokens ? count_active(a.mask, a.T, tid, NT, active_s) : a.T;
     if (t >= t_active || !__any(id >= 0 && id < a.E)) {
         return;
     }
@@ -116,12 +88,121 @@ __global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 
     }
 }
 
+// Phase 1 of a layer whose gate/up GEMM gathers its rows: the workgroups behind the nb that rank quantise the tokens, a wave each,
+// which depends on nothing that the plan finds out.  A token's row is stored once, not once per copy, and non-temporally up to 256 rows
+// per expert (quantised_plainly).
+// HBM bound where there are many tokens.  us, ranks + their second half + permute with schedules -> this + phase 2 with schedules
+// (plain stores): 8192 tokens x 4096, top-8, int8 7.6 + 6.3 + 70.9 -> 20.9 + 15.5 (layer 1512 -> 1474); 4093 in FP8 5.5 + 5.8 + 45.0
+// -> 15.5 + 13.5 (823 -> 787); 1021 x 2048, top-6, 4.8 + 4.8 + 9.1 -> 5.0 + 7.5 (160.9 -> 158.9).  With rows of 4096 columns in the
+// registers for 7168, at 3 (FP8) and 4 waves a SIMD, FP8 took 19.2.
+template <int CHUNKS, int QUANT, int ACT, bool PLAIN>
+__global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 5) void plan_quant_kernel(PlanArgs a, DispatchArgs d,
+                                                                                                         int it, int nb)
+{
+    __shared__ int hist[kLocalWaves * kMaxExperts];
+    __shared__ int active_s;
+    const int tid = threadIdx.x;
+    const int b = blockIdx.x;
+    if (b < nb) {
+        const int t_active = count_active(a.mask, a.T, tid, kLocalThreads, &active_s);
+        auto rank = [&](auto ic) {
+            rank_chunk<int32_t, decltype(ic)::value>((const int32_t *)a.idx, b, (long long)t_active * a.K, (long long)a.T * a.K,
+                                                     a.E, hist, a.pos, a.hist_ws + (long long)b * a.E);
+        };
+        switch (it) {
+            case 2: rank(std::integral_constant<int, 2>()); break;
+            case 4: rank(std::integral_constant<int, 4>()); break;
+            default: rank(std::integral_constant<int, 8>()); break;
+        }
+        if (b == 0 && tid == 0) {
+            a.hist_ws[(long long)nb * a.E] = t_active;
+        }
+        return;
+    }
+    quantise_token<CHUNKS, QUANT, ACT, PLAIN, kLocalThreads>(a, d, b - nb, &active_s);
+}
+
 // What phase 2 does besides in a layer: its first sched.nspec * sched.parts workgroups build the schedules of the GEMMs (from
 // the counts, which they add up like all the others), and the others leave the token of every row where GMM1 gathers.
 struct LayerPlan {
     int32_t *row_token;  // or null
     SchedBuild sched;
 };
+
+// All of it in one launch, up to kWholePlanIds ids: the schedule builders count the ids by themselves, a workgroup per expert ranks its
+// entries (ExpertEntries), and the workgroups behind them quantise.  Latency bound (the builders' chain) up to some thousand tokens.
+// us per layer, two launches / this; T x H, top-K of E, I: 1021 x 2048, 6 of 64, 1408 159.6 / 156.3; 700 152.2 / 148.3; 2000 x 4096, 8 of 128, 1536
+// 602.5 / 597.5; 4000 x 7168, 4 of 64, 2048 940 / 933; 300 x 7168, 8 of 16, 2048 222 / 215; 16384 x 1024, 1 of 16, 512 110 / 103.5; FP8 1400 x 2048, 3 of
+// 8, 1024 71.4 / 65.7, 2048 x 2048, 8 of 32, 768 141.6 / 137.2.  With 64 ids a thread for up to 32768 ids the registers of the ranking workgroups
+// cost the others their waves: 4093 x 4096 in FP8, 8 of 128, 782 / 797.
+constexpr int kWholeThreads = 512;
+constexpr int kWholePlanIds = 32 * kWholeThreads;
+template <int CHUNKS, int QUANT, int ACT, bool PLAIN>
+__global__ __launch_bounds__(kWholeThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 5) void whole_plan_quant_kernel(PlanArgs a, DispatchArgs d,
+                                                                                                               LayerPlan l)
+{
+    __shared__ SchedShared sched_s;
+    __shared__ int scratch[2 * kWholeThreads / kWave];
+    __shared__ int active_s;
+    const int tid = threadIdx.x;
+    const int builders = l.sched.nspec * l.sched.parts;
+    const int x = (int)blockIdx.x - builders;
+    if (x >= a.E) {
+        quantise_token<CHUNKS, QUANT, ACT, PLAIN, kWholeThreads>(a, d, x - a.E, &active_s);
+        return;
+    }
+    const int n_all = a.T * a.K;
+    auto plan = [&](auto ic) {
+        ExpertEntries<kWholeThreads, decltype(ic)::value> ids;
+        ids.load((const int32_t *)a.idx, n_all);
+        const int t_active = count_active(a.mask, a.T, tid, kWholeThreads, &active_s);
+        ids.only_first(t_active * a.K);
+        if (x < 0) {
+            for (int e = tid; e < a.E; e += kWholeThreads) {
+                sched_s.order[e] = 0;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int it = 0; it < decltype(ic)::value; ++it) {
+                // the lanes that name what the first one names are counted together: top-1 ids that are all the same one by one took
+                // a layer of 16384 tokens x 1024 from 94.5 to 97.6 us
+                const int some = __builtin_amdgcn_readfirstlane(ids.e[it]);
+                const unsigned long long alike = __ballot(ids.e[it] == some);
+                const bool first = (alike & ((1ull << (tid & (kWave - 1))) - 1ull)) == 0;
+                if ((unsigned)ids.e[it] < (unsigned)a.E && (ids.e[it] != some || first)) {
+                    atomicAdd(&sched_s.order[ids.e[it]], ids.e[it] == some ? __popcll(alike) : 1);
+                }
+            }
+            return;
+        }
+        ids.count(x, scratch);
+        if (tid == 0) {
+            a.tokens_per_expert[x] = ids.cnt;
+            if (x == a.E - 1) {
+                a.meta[0] = 0;
+                a.meta[1] = ids.off + ids.cnt;
+                a.meta[2] = t_active;
+                a.meta[3] = 0;
+            }
+        }
+        ids.ranks(x, [&](int i, int rank) {
+            a.dst_row[i] = ids.off + rank;
+            l.row_token[ids.off + rank] = (int)((unsigned)i / (unsigned)a.K);
+        });
+        if (x == 0) {
+            ids.of_no_expert(a.E, n_all, [&](int i) { a.dst_row[i] = -1; });
+        }
+    };
+    if (n_all <= 12 * kWholeThreads) {
+        plan(std::integral_constant<int, 12>());
+    } else {
+        plan(std::integral_constant<int, 32>());
+    }
+    if (x < 0) {
+        __syncthreads();
+        build_sched_part<kWholeThreads>(sched_s, l.sched, (int)blockIdx.x / l.sched.parts, (int)blockIdx.x % l.sched.parts, l.sched.parts);
+    }
+}
 
 // Phase 2.  Every workgroup sums the histogram columns (all rows for the per-expert count, the rows
 // before its own for its base), scans the counts into offsets, and finishes its own chunk:
@@ -303,17 +384,13 @@ __global__ __launch_bounds__(kExpertThreads, 8) void plan_experts_kernel(PlanArg
             a.dst_row[i] = ids.off + rank;
         }
     });
-    if (x == 0) {  // the entries of no expert
-#pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            const int i = ids.first_entry() + it * kWave + (tid & (kWave - 1));
-            if ((unsigned)ids.e[it] >= (unsigned)a.E && i < n_all) {
-                a.pos[i] = -1;
-                if (a.dst_row != nullptr) {
-                    a.dst_row[i] = -1;
-                }
+    if (x == 0) {
+        ids.of_no_expert(a.E, n_all, [&](int i) {
+            a.pos[i] = -1;
+            if (a.dst_row != nullptr) {
+                a.dst_row[i] = -1;
             }
-        }
+        });
     }
 }
 
@@ -509,6 +586,28 @@ hipError_t launch_plan_t(const PlanArgs &a, int it, int nb, int32_t *hist, hipSt
 bool quantised_plainly(const PlanArgs &p) { return (long long)p.T * p.K > 256ll * p.E; }
 
 template <int QUANT, int ACT, bool PLAIN>
+hipError_t launch_whole_plan_as(const PlanArgs &p, const DispatchArgs &d, const LayerPlan &l, hipStream_t stream)
+{
+    constexpr int kTokens = kWholeThreads / kWave;
+    const dim3 grid((unsigned)(l.sched.nspec * l.sched.parts + p.E + (d.T + kTokens - 1) / kTokens)), block(kWholeThreads);
+    if (d.H <= 8 * kWave * 8) {
+        hipLaunchKernelGGL((whole_plan_quant_kernel<8, QUANT, ACT, PLAIN>), grid, block, 0, stream, p, d, l);
+    } else {
+        hipLaunchKernelGGL((whole_plan_quant_kernel<kDispMaxChunks, QUANT, ACT, PLAIN>), grid, block, 0, stream, p, d, l);
+    }
+    return hipGetLastError();
+}
+
+template <bool PLAIN>
+hipError_t launch_whole_plan(const PlanArgs &p, const DispatchArgs &d, const LayerPlan &l, hipStream_t stream)
+{
+    if (d.quant == 3) {
+        return launch_whole_plan_as<3, 0, PLAIN>(p, d, l, stream);
+    }
+    return d.x_is_fp16 ? launch_whole_plan_as<2, 1, PLAIN>(p, d, l, stream) : launch_whole_plan_as<2, 0, PLAIN>(p, d, l, stream);
+}
+
+template <int QUANT, int ACT, bool PLAIN>
 hipError_t launch_plan_quant_as(const PlanArgs &p, const DispatchArgs &d, int it, int nb, hipStream_t stream)
 {
     const dim3 grid((unsigned)nb + (unsigned)((d.T + kDispWaves - 1) / kDispWaves)), block(kLocalThreads);
@@ -597,6 +696,9 @@ hipError_t launch_layer_plan(const PlanArgs &p, const DispatchArgs &d, int32_t *
     // most 8 builders and 64-bit divisions in their turns phase 2 took 22.1 us at 8192 tokens
     const int cap = std::max(specs[0].max_items, specs[1].max_items);
     l.sched.parts = std::min(std::max((cap + kGlobalThreads - 1) / kGlobalThreads, 1), 32);
+    if (row_token != nullptr && (long long)p.T * p.K <= kWholePlanIds) {
+        return quantised_plainly(p) ? launch_whole_plan<true>(p, d, l, stream) : launch_whole_plan<false>(p, d, l, stream);
+    }
     if (row_token == nullptr) {
         e = launch_plan_local<int32_t>(p, it, nb, p.hist_ws, stream);
     } else {

@@ -277,6 +277,19 @@ struct ExpertEntries {
         }
     }
 
+    // f(entry) for every entry of none of E experts
+    template <typename F>
+    __device__ __forceinline__ void of_no_expert(int E, int n_all, F &&f)
+    {
+        const int base = first_entry() + (int)(threadIdx.x & (kWave - 1));
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            if ((unsigned)e[it] >= (unsigned)E && base + it * kWave < n_all) {
+                f(base + it * kWave);
+            }
+        }
+    }
+
     // f(entry, rank) for every entry of the expert
     template <typename F>
     __device__ __forceinline__ void ranks(int x, F &&f)
