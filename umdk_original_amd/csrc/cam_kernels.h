@@ -209,6 +209,7 @@ struct StreamGemmArgs {
     int32_t *rows_out;          // optional: [1] receives the total row count (where launch_requant looks for it)
     const float *products;      // optional [max_rows,Kd], instead of g.a and g.a_scale: fp32 rows that the kernel quantises the
                                 // way launch_requant does, bit for bit (where stream_gemm_takes_products says so)
+    int lg_tile_rows;           // set by launch_stream_gemm
 };
 bool stream_gemm_applies(int64_t rows, int64_t N, int64_t G, bool fp8);  // whether it is the faster form
 // Whether a launch without a gate/up pair quantises its activations from fp32 rows faster than launch_requant before it.

@@ -27,7 +27,7 @@
 //   * No schedule: every workgroup derives the item list from the per-expert row counts by itself (a prefix sum over
 //     at most 512 experts) and takes items in a fixed order.  All items of a launch stream the same number of bytes,
 //     so nothing has to be balanced, and no builder runs before the GEMM.
-//   * In a layer whose tiles are a few thousand products each, the GMM2 launch quantises its activations itself (PRODUCTS):
+//   * In a layer whose tiles are some ten thousand products each, the GMM2 launch quantises its activations itself (PRODUCTS):
 //     every workgroup reads the fp32 SwiGLU products of its tile, finds the row maxima and leaves the int8 rows in LDS while
 //     its first weights are on their way.  Column blocks repeat that work, but it is a microsecond or two of latency
 //     where a launch of requant_kernel takes 3.4 (layers: one token, H 4096, I 1536: 45.9 -> 44.1 us; 128 tokens on 8
@@ -47,7 +47,8 @@ namespace {
 constexpr int kSThreads = 512;
 constexpr int R = 2;                     // 64-byte K steps in flight per wave
 constexpr int kSMaxKb = 64;              // FP8: K blocks of 128 bytes (Kd <= 8192)
-constexpr int kSBuf32 = 32768;           // activation buffer of the 32-row tiles
+constexpr int kSBuf32 = 32768;           // activation buffer of the 32-row tiles,
+constexpr int kSBuf128 = 65536;          // of the 128-row tiles
 constexpr int kProductQuads = 16;        // PRODUCTS: quads of products a thread holds, i.e. 32 K products a workgroup
 
 __device__ __forceinline__ void lds_barrier()
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
 {
     typedef typename SAcc<FP8>::v16 acc16;
     typedef typename SAcc<FP8>::v4 acc4;
-    constexpr int kABuf = MF == 1 ? kSBuf32 : 65536;  // one of the two activation buffers
+    constexpr int kABuf = MF == 1 ? kSBuf32 : kSBuf128;  // one of the two activation buffers
     constexpr int kSLds = 2 * kABuf;
     constexpr int NFR = MF == 1 ? 1 : 2;            // column fragments whose partial sums (32 KB each) fit a buffer
     const GemmArgs &a = sa.g;
@@ -153,8 +154,11 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     constexpr int quantum = S * R > 4 ? 64 * S * R : 256;  // K bytes of one turn of all S waves
     static_assert(NFR == 2 || S >= 4, "sums that pass one fragment at a time wait in registers for one block only");
     static_assert(32 * MF * quantum <= kABuf, "a turn of a full tile has to fit an activation buffer");
-    static_assert(!PRODUCTS || (MF == 1 && !FP8), "products are quantised by the 32-row tiles");
+    static_assert(!PRODUCTS || !FP8, "products are quantised to int8");
     const int kpad = (Kd + quantum - 1) / quantum * quantum;
+    // rows of a tile: with products no more than a workgroup can quantise
+    const int lg_rows = PRODUCTS && MF == 4 ? sa.lg_tile_rows : (MF == 1 ? 5 : 7);
+    const int tile_rows = 1 << lg_rows;
 
     // ---- the item list: every expert's first row and the row tiles before it.  Every wave works it out for itself, a lane an
     // expert, and stores it: the same values into the same places, so that no wave waits for another before it knows its first
@@ -187,7 +191,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
                     row += wave_last(inc);
                 }
                 rows = e < G ? rows : 0;
-                const int tiles = (rows + 32 * MF - 1) / (32 * MF);
+                const int tiles = (rows + tile_rows - 1) >> lg_rows;
                 const int inc = wave_inclusive_scan(tiles);
                 if (e < G) {
                     tile_start[e] = tile + inc - tiles;
@@ -239,8 +243,8 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
         }
         it.g = g;
         it.blk = blk;
-        it.row0 = fr + j * 32 * MF;
-        it.rows = min(er - it.row0, 32 * MF);
+        it.row0 = fr + j * tile_rows;
+        it.rows = min(er - it.row0, tile_rows);
         const int fit = kABuf / max(it.rows, 1) / quantum * quantum;
         it.ckb = min(max(fit, quantum), kpad);
         it.nch = (Kd + it.ckb - 1) / it.ckb;
@@ -769,19 +773,30 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     return sh;
 }
 
-// Whether a tile's products fit the registers of a workgroup, and its int8 rows (padded to a turn of the eight waves) an
-// activation buffer.
-bool products_fit(const StreamShape &sh, long long max_rows, int Kd)
+// log2 of the rows of a tile whose products fit the registers of a workgroup, and its int8 rows (padded to a turn of the eight waves) an
+// activation buffer; -1 where 32-row tiles are not that low.  128-row tiles are cut: a token that names an expert once makes
+// no more than one tile of it where the launch takes products, and one that names it more than once two.
+int lg_product_rows(const StreamShape &sh, long long max_rows, int Kd)
 {
-    if (!sh.small || Kd % 128 != 0) {
-        return false;
-    }
-    long long rows = 1;
-    while (rows < std::min<long long>(32, max_rows)) {
-        rows *= 2;
-    }
     const long long turn = 64 * (8 / sh.P) * R;
-    return rows * Kd <= 4ll * kProductQuads * kSThreads && rows * ((Kd + turn - 1) / turn * turn) <= kSBuf32;
+    const long long kpad = (Kd + turn - 1) / turn * turn;
+    auto fits = [&](int lg) {
+        return ((long long)Kd << lg) <= 4ll * kProductQuads * kSThreads && (kpad << lg) <= (sh.small ? kSBuf32 : kSBuf128);
+    };
+    if (Kd % 128 != 0 || !fits(0)) {
+        return -1;
+    }
+    int lg = 0;
+    if (sh.small) {
+        while ((1ll << lg) < std::min<long long>(32, max_rows)) {
+            ++lg;
+        }
+        return fits(lg) ? lg : -1;
+    }
+    while (lg < 7 && fits(lg + 1)) {
+        ++lg;
+    }
+    return sh.P == 8 ? lg : -1;   // (four groups to an item are more items than workgroups, or 32-row tiles)
 }
 
 }  // namespace
@@ -802,7 +817,9 @@ bool stream_gemm_applies(int64_t rows, int64_t N, int64_t G, bool fp8)
     return rows > 0 && (rows * N <= kMostRowsTimesColumns || (fp8 && rows <= 32 * G && rows * N <= 3 * kMostRowsTimesColumns));
 }
 
-// Where every workgroup has one item at most: with more, the quantisation of an item would interrupt the stream.
+// Where every workgroup has one item at most: with more, the quantisation of an item would interrupt the stream.  With 128-row tiles, us
+// per layer, re-quantisation as a launch / here: 16 tokens x 7168, top-8 of 16, I 2048 127.7 / 126.0, 10 x 4096, 8 of 32, 1536 108.1 /
+// 105.8, 16 x 7168, 2 of 16, 2048 115.7 / 113.4, 24 x 7168, 4 of 16, 1024 73.1 / 71.4.
 bool stream_gemm_takes_products(int64_t max_rows, int G, int Kd, int N, int64_t rows_per_expert)
 {
     int cus = 0;
@@ -810,7 +827,15 @@ bool stream_gemm_takes_products(int64_t max_rows, int G, int Kd, int N, int64_t 
         return false;
     }
     const StreamShape sh = stream_shape(G, max_rows, Kd, N, false, rows_per_expert, cus);
-    return sh.items <= (long long)sh.grid && products_fit(sh, max_rows, Kd);
+    const int lg = lg_product_rows(sh, max_rows, Kd);
+    if (lg < 0) {
+        return false;
+    }
+    if (sh.small) {
+        return sh.items <= (long long)sh.grid;
+    }
+    const long long experts = std::min<long long>(G, max_rows);
+    return rows_per_expert <= 1ll << lg && experts * ((N / 64 + sh.P - 1) / sh.P) <= cus;
 }
 
 hipError_t launch_stream_gemm(const StreamGemmArgs &sa, int64_t rows_per_expert, hipStream_t stream)
@@ -834,12 +859,21 @@ hipError_t launch_stream_gemm(const StreamGemmArgs &sa, int64_t rows_per_expert,
     }
     const StreamShape sh = stream_shape(sa.G, sa.max_rows, g.Kd, g.N, g.fp8 && g.gate_up, rows_per_expert, cus);
     if (sa.products != nullptr) {
-        if (g.fp8 || g.gate_up || !products_fit(sh, sa.max_rows, g.Kd)) {
+        const int lg = lg_product_rows(sh, sa.max_rows, g.Kd);
+        if (g.fp8 || g.gate_up || lg < 0) {
             return hipErrorInvalidValue;
         }
         // an item to a workgroup, which is what the kernel is written for
-        const unsigned grid = (unsigned)((sh.items + kNumXcd - 1) / kNumXcd * kNumXcd);
-        sh.P == 1 ? launch_kernel<1, false, 1, true>(grid, stream, sa) : launch_kernel<1, false, 2, true>(grid, stream, sa);
+        StreamGemmArgs sp = sa;
+        sp.lg_tile_rows = lg;
+        const long long items = sh.small ? sh.items
+                                         : (std::min<long long>(sa.G, sa.max_rows) + (sa.max_rows >> lg)) * ((g.N / 64 + sh.P - 1) / sh.P);
+        const unsigned grid = (unsigned)((items + kNumXcd - 1) / kNumXcd * kNumXcd);
+        if (sh.small) {
+            sh.P == 1 ? launch_kernel<1, false, 1, true>(grid, stream, sp) : launch_kernel<1, false, 2, true>(grid, stream, sp);
+        } else {
+            launch_kernel<4, false, 8, true>(grid, stream, sp);
+        }
     } else if (g.fp8) {
         launch_variant<true>(sh.small ? 1 : 4, sh.P, sh.grid, stream, sa);
     } else {
