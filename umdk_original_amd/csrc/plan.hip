@@ -51,6 +51,13 @@ __global__ __launch_bounds__(kLocalThreads) void plan_local_kernel(PlanArgs a, i
     }
 }
 
+// What phase 2 does besides in a layer: its first sched.nspec * sched.parts workgroups build the schedules of the GEMMs (from
+// the counts, which they add up like all the others), and the others leave the token of every row where GMM1 gathers.
+struct LayerPlan {
+    int32_t *row_token;  // or null
+    SchedBuild sched;
+};
+
 // A wave per token: what the workgroups of a layer's plan behind those that rank do.
 constexpr int kMaskedTokens = 16384;  // up to where a workgroup looks through the whole mask, as long as its four tokens at 2048 columns
 template <int CHUNKS, int QUANT, int ACT, bool PLAIN, int NT>
@@ -95,19 +102,33 @@ __device__ __forceinline__ void quantise_token(const PlanArgs &a, const Dispatch
 // (plain stores): 8192 tokens x 4096, top-8, int8 7.6 + 6.3 + 70.9 -> 20.9 + 15.5 (layer 1512 -> 1474); 4093 in FP8 5.5 + 5.8 + 45.0
 // -> 15.5 + 13.5 (823 -> 787); 1021 x 2048, top-6, 4.8 + 4.8 + 9.1 -> 5.0 + 7.5 (160.9 -> 158.9).  With rows of 4096 columns in the
 // registers for 7168, at 3 (FP8) and 4 waves a SIMD, FP8 took 19.2.
+//
+// Up to kWholePlanIds ids this is all of the plan (nb == 0): the schedule builders count the ids by themselves, a workgroup per expert ranks its
+// entries (ExpertEntries), and the workgroups behind them quantise.  Latency bound (the builders' chain) up to some thousand tokens.
+// us per layer, two launches / this; T x H, top-K of E, I: 1021 x 2048, 6 of 64, 1408 159.6 / 156.3; 700 152.2 / 148.3; 2000 x 4096, 8 of 128, 1536
+// 602.5 / 597.5; 4000 x 7168, 4 of 64, 2048 940 / 933; 300 x 7168, 8 of 16, 2048 222 / 215; 16384 x 1024, 1 of 16, 512 110 / 103.5; FP8 1400 x 2048, 3 of
+// 8, 1024 71.4 / 65.7, 2048 x 2048, 8 of 32, 768 141.6 / 137.2.  With 64 ids a thread for up to 32768 ids the registers of the ranking workgroups
+// cost the others their waves: 4093 x 4096 in FP8, 8 of 128, 782 / 797.
+constexpr int kWholeThreads = 512;
+constexpr int kWholePlanIds = 32 * kWholeThreads;
 template <int CHUNKS, int QUANT, int ACT, bool PLAIN>
-__global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 5) void plan_quant_kernel(PlanArgs a, DispatchArgs d,
-                                                                                                         int it, int nb)
+__global__ __launch_bounds__(kWholeThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 5) void plan_quant_kernel(PlanArgs a, DispatchArgs d,
+                                                                                                         LayerPlan l, int it, int nb)
 {
-    __shared__ int hist[kLocalWaves * kMaxExperts];
+    extern __shared__ __attribute__((aligned(16))) int lds[];   // histograms, or what the builders need
+    __shared__ int scratch[2 * kWholeThreads / kWave];
     __shared__ int active_s;
     const int tid = threadIdx.x;
-    const int b = blockIdx.x;
-    if (b < nb) {
+    if (nb > 0) {  // kLocalThreads a workgroup
+        const int b = blockIdx.x;
+        if (b >= nb) {
+            quantise_token<CHUNKS, QUANT, ACT, PLAIN, kLocalThreads>(a, d, b - nb, &active_s);
+            return;
+        }
         const int t_active = count_active(a.mask, a.T, tid, kLocalThreads, &active_s);
         auto rank = [&](auto ic) {
             rank_chunk<int32_t, decltype(ic)::value>((const int32_t *)a.idx, b, (long long)t_active * a.K, (long long)a.T * a.K,
-                                                     a.E, hist, a.pos, a.hist_ws + (long long)b * a.E);
+                                                     a.E, lds, a.pos, a.hist_ws + (long long)b * a.E);
         };
         switch (it) {
             case 2: rank(std::integral_constant<int, 2>()); break;
@@ -119,32 +140,7 @@ __global__ __launch_bounds__(kLocalThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 
         }
         return;
     }
-    quantise_token<CHUNKS, QUANT, ACT, PLAIN, kLocalThreads>(a, d, b - nb, &active_s);
-}
-
-// What phase 2 does besides in a layer: its first sched.nspec * sched.parts workgroups build the schedules of the GEMMs (from
-// the counts, which they add up like all the others), and the others leave the token of every row where GMM1 gathers.
-struct LayerPlan {
-    int32_t *row_token;  // or null
-    SchedBuild sched;
-};
-
-// All of it in one launch, up to kWholePlanIds ids: the schedule builders count the ids by themselves, a workgroup per expert ranks its
-// entries (ExpertEntries), and the workgroups behind them quantise.  Latency bound (the builders' chain) up to some thousand tokens.
-// us per layer, two launches / this; T x H, top-K of E, I: 1021 x 2048, 6 of 64, 1408 159.6 / 156.3; 700 152.2 / 148.3; 2000 x 4096, 8 of 128, 1536
-// 602.5 / 597.5; 4000 x 7168, 4 of 64, 2048 940 / 933; 300 x 7168, 8 of 16, 2048 222 / 215; 16384 x 1024, 1 of 16, 512 110 / 103.5; FP8 1400 x 2048, 3 of
-// 8, 1024 71.4 / 65.7, 2048 x 2048, 8 of 32, 768 141.6 / 137.2.  With 64 ids a thread for up to 32768 ids the registers of the ranking workgroups
-// cost the others their waves: 4093 x 4096 in FP8, 8 of 128, 782 / 797.
-constexpr int kWholeThreads = 512;
-constexpr int kWholePlanIds = 32 * kWholeThreads;
-template <int CHUNKS, int QUANT, int ACT, bool PLAIN>
-__global__ __launch_bounds__(kWholeThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 5) void whole_plan_quant_kernel(PlanArgs a, DispatchArgs d,
-                                                                                                               LayerPlan l)
-{
-    __shared__ SchedShared sched_s;
-    __shared__ int scratch[2 * kWholeThreads / kWave];
-    __shared__ int active_s;
-    const int tid = threadIdx.x;
+    SchedShared &sched_s = *(SchedShared *)lds;
     const int builders = l.sched.nspec * l.sched.parts;
     const int x = (int)blockIdx.x - builders;
     if (x >= a.E) {
@@ -176,14 +172,14 @@ __global__ __launch_bounds__(kWholeThreads, CHUNKS > 8 ? (QUANT == 3 ? 3 : 4) : 
             return;
         }
         ids.count(x, scratch);
-        if (tid == 0) {
-            a.tokens_per_expert[x] = ids.cnt;
-            if (x == a.E - 1) {
-                a.meta[0] = 0;
-                a.meta[1] = ids.off + ids.cnt;
-                a.meta[2] = t_active;
-                a.meta[3] = 0;
-            }
+        if (tid < 2) {  // 64 bits, a word a lane
+            ((int32_t *)(a.tokens_per_expert + x))[tid] = tid == 0 ? ids.cnt : 0;
+        }
+        if (tid == 0 && x == a.E - 1) {
+            a.meta[0] = 0;
+            a.meta[1] = ids.off + ids.cnt;
+            a.meta[2] = t_active;
+            a.meta[3] = 0;
         }
         ids.ranks(x, [&](int i, int rank) {
             a.dst_row[i] = ids.off + rank;
@@ -586,47 +582,29 @@ hipError_t launch_plan_t(const PlanArgs &a, int it, int nb, int32_t *hist, hipSt
 bool quantised_plainly(const PlanArgs &p) { return (long long)p.T * p.K > 256ll * p.E; }
 
 template <int QUANT, int ACT, bool PLAIN>
-hipError_t launch_whole_plan_as(const PlanArgs &p, const DispatchArgs &d, const LayerPlan &l, hipStream_t stream)
+hipError_t launch_plan_quant_as(const PlanArgs &p, const DispatchArgs &d, const LayerPlan &l, int it, int nb, hipStream_t stream)
 {
-    constexpr int kTokens = kWholeThreads / kWave;
-    const dim3 grid((unsigned)(l.sched.nspec * l.sched.parts + p.E + (d.T + kTokens - 1) / kTokens)), block(kWholeThreads);
-    if (d.H <= 8 * kWave * 8) {
-        hipLaunchKernelGGL((whole_plan_quant_kernel<8, QUANT, ACT, PLAIN>), grid, block, 0, stream, p, d, l);
-    } else {
-        hipLaunchKernelGGL((whole_plan_quant_kernel<kDispMaxChunks, QUANT, ACT, PLAIN>), grid, block, 0, stream, p, d, l);
-    }
-    return hipGetLastError();
-}
-
-template <bool PLAIN>
-hipError_t launch_whole_plan(const PlanArgs &p, const DispatchArgs &d, const LayerPlan &l, hipStream_t stream)
-{
-    if (d.quant == 3) {
-        return launch_whole_plan_as<3, 0, PLAIN>(p, d, l, stream);
-    }
-    return d.x_is_fp16 ? launch_whole_plan_as<2, 1, PLAIN>(p, d, l, stream) : launch_whole_plan_as<2, 0, PLAIN>(p, d, l, stream);
-}
-
-template <int QUANT, int ACT, bool PLAIN>
-hipError_t launch_plan_quant_as(const PlanArgs &p, const DispatchArgs &d, int it, int nb, hipStream_t stream)
-{
-    const dim3 grid((unsigned)nb + (unsigned)((d.T + kDispWaves - 1) / kDispWaves)), block(kLocalThreads);
+    const int threads = nb > 0 ? kLocalThreads : kWholeThreads, tokens = threads / kWave;
+    const int ahead = nb > 0 ? nb : l.sched.nspec * l.sched.parts + p.E;
+    const size_t lds = nb > 0 ? kLocalWaves * kMaxExperts * sizeof(int) : sizeof(SchedShared);
+    const dim3 grid((unsigned)(ahead + (d.T + tokens - 1) / tokens)), block((unsigned)threads);
     // rows of up to 4096 columns in registers for 4096: more waves to a SIMD
     if (d.H <= 8 * kWave * 8) {
-        hipLaunchKernelGGL((plan_quant_kernel<8, QUANT, ACT, PLAIN>), grid, block, 0, stream, p, d, it, nb);
+        hipLaunchKernelGGL((plan_quant_kernel<8, QUANT, ACT, PLAIN>), grid, block, lds, stream, p, d, l, it, nb);
     } else {
-        hipLaunchKernelGGL((plan_quant_kernel<kDispMaxChunks, QUANT, ACT, PLAIN>), grid, block, 0, stream, p, d, it, nb);
+        hipLaunchKernelGGL((plan_quant_kernel<kDispMaxChunks, QUANT, ACT, PLAIN>), grid, block, lds, stream, p, d, l, it, nb);
     }
     return hipGetLastError();
 }
 
 template <bool PLAIN>
-hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &d, int it, int nb, hipStream_t stream)
+hipError_t launch_plan_quant(const PlanArgs &p, const DispatchArgs &d, const LayerPlan &l, int it, int nb, hipStream_t stream)
 {
     if (d.quant == 3) {
-        return launch_plan_quant_as<3, 0, PLAIN>(p, d, it, nb, stream);
+        return launch_plan_quant_as<3, 0, PLAIN>(p, d, l, it, nb, stream);
     }
-    return d.x_is_fp16 ? launch_plan_quant_as<2, 1, PLAIN>(p, d, it, nb, stream) : launch_plan_quant_as<2, 0, PLAIN>(p, d, it, nb, stream);
+    return d.x_is_fp16 ? launch_plan_quant_as<2, 1, PLAIN>(p, d, l, it, nb, stream)
+                       : launch_plan_quant_as<2, 0, PLAIN>(p, d, l, it, nb, stream);
 }
 
 }  // namespace
@@ -696,15 +674,15 @@ hipError_t launch_layer_plan(const PlanArgs &p, const DispatchArgs &d, int32_t *
     // most 8 builders and 64-bit divisions in their turns phase 2 took 22.1 us at 8192 tokens
     const int cap = std::max(specs[0].max_items, specs[1].max_items);
     l.sched.parts = std::min(std::max((cap + kGlobalThreads - 1) / kGlobalThreads, 1), 32);
-    if (row_token != nullptr && (long long)p.T * p.K <= kWholePlanIds) {
-        return quantised_plainly(p) ? launch_whole_plan<true>(p, d, l, stream) : launch_whole_plan<false>(p, d, l, stream);
-    }
+    const bool whole = row_token != nullptr && (long long)p.T * p.K <= kWholePlanIds;
     if (row_token == nullptr) {
         e = launch_plan_local<int32_t>(p, it, nb, p.hist_ws, stream);
     } else {
-        e = quantised_plainly(p) ? launch_plan_quant<true>(p, d, it, nb, stream) : launch_plan_quant<false>(p, d, it, nb, stream);
+        const int chunks = whole ? 0 : nb;
+        e = quantised_plainly(p) ? launch_plan_quant<true>(p, d, l, it, chunks, stream)
+                                 : launch_plan_quant<false>(p, d, l, it, chunks, stream);
     }
-    if (e != hipSuccess) {
+    if (e != hipSuccess || whole) {
         return e;
     }
     hipLaunchKernelGGL((plan_global_kernel<int32_t, true>), dim3((unsigned)(nb + l.sched.nspec * l.sched.parts)),
