@@ -1807,7 +1807,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     CAM_TRY(check_aligned(output, "output", 16));
 
     const int64_t A = T * K;  // maxTokenNum of AK/fused_deep_moe/op_kernel/fused_deep_moe.h:336 for one rank
-    if (cam::few_tokens_apply(T, K, Epr, H, I)) {  // a handful of tokens: two launches
+    if (cam::few_tokens_apply(T, K, Epr, H, I, false)) {  // a handful of tokens: two launches
         Carver c;
         const uint64_t o_prod = c.take((uint64_t)A * I * 4);
         cam::FewTokensArgs f{};
@@ -2198,6 +2198,34 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
     CAM_TRY(check_aligned(output, "output", 16));
 
     const int64_t A = T * K;
+    if (cam::few_tokens_apply(T, K, E, H, I, true)) {  // a handful of tokens: two launches
+        Carver c;
+        const uint64_t o_prod = c.take((uint64_t)A * I * 4);
+        cam::FewTokensArgs f{};
+        f.x = (const uint16_t *)x->data;
+        f.ids = (const int32_t *)expertIds->data;
+        f.gates = (const float *)expertScales->data;
+        f.mask = xActiveMaskOptional ? (const uint8_t *)xActiveMaskOptional->data : nullptr;
+        f.T = (int)T;
+        f.K = (int)K;
+        f.H = (int)H;
+        f.I = (int)I;
+        f.E = (int)E;
+        f.tokens_per_expert = (int64_t *)expertTokenNums->data;
+        f.out = (uint16_t *)output->data;
+        auto run = [=](void *wsp, hipStream_t s) -> hipError_t {
+            cam::FewTokensArgs g = f;
+            g.products = (float *)((char *)wsp + o_prod);
+            g.w = w1.w;
+            g.w_scale8 = w1.s;
+            const hipError_t e = cam::launch_few_tokens_up(g, s);
+            if (e != hipSuccess) return e;
+            g.w = w2.w;
+            g.w_scale8 = w2.s;
+            return cam::launch_few_tokens_down(g, s);
+        };
+        return finish_phase1(kOpFusedFp8, c.off, run, workspaceSize, executor);
+    }
     cam::SchedSpec sp1 = sched_spec(A, E, 2 * I);
     cam::SchedSpec sp2 = sched_spec(A, E, H);
     const bool stream = cam::stream_gemm_applies(A, 2 * I, E, true);   // few rows: no schedules

@@ -217,7 +217,7 @@ bool stream_gemm_takes_products(int64_t max_rows, int G, int Kd, int N, int64_t 
 // rows_per_expert: the most rows one expert can have, as far as the host knows.
 hipError_t launch_stream_gemm(const StreamGemmArgs &a, int64_t rows_per_expert, hipStream_t stream);
 
-// The int8 layer of a handful of tokens (few_tokens.hip): routing, quantisation, gate/up GEMM and SwiGLU in one launch, re-quantisation,
+// The layer of a handful of tokens (few_tokens.hip): routing, quantisation, gate/up GEMM and SwiGLU in one launch, re-quantisation,
 // down GEMM and combine in another.  w, w_scale, list are those of the launch's GEMM.
 constexpr int kFewTokens = 8;    // at most, of
 constexpr int kFewSlots = 32;    // (token, k) slots at most
@@ -231,13 +231,14 @@ struct FewTokensArgs {
     int T, K, H, I, E;
     const int8_t *w;        // packed [E,H,2I] or [E,I,H]
     const float *w_scale;   // [E,2I] or [E,H]
+    const uint8_t *w_scale8;  // block-scaled FP8 if set: [E,H/128,2I/128] or [E,I/128,H/128]; not with fp16 or `list`
     int per_expert;         // weights given per expert through `list`
     WeightPtrs list;
     float *products;        // [T*K,I]: written by the first launch, read by the second
     int64_t *tokens_per_expert;  // [E]
     uint16_t *out;          // [T,H]
 };
-bool few_tokens_apply(int64_t T, int64_t K, int64_t E, int64_t H, int64_t I);  // whether that is the faster form
+bool few_tokens_apply(int64_t T, int64_t K, int64_t E, int64_t H, int64_t I, bool fp8);  // whether that is the faster form
 hipError_t launch_few_tokens_up(const FewTokensArgs &a, hipStream_t stream);
 hipError_t launch_few_tokens_down(const FewTokensArgs &a, hipStream_t stream);
 

@@ -1,8 +1,8 @@
-// The int8 layer for a handful of tokens in two launches: their routing and quantisation in the gate/up GEMM, the re-quantisation
+// The int8 and FP8 layers for a handful of tokens in two launches: their routing and quantisation in the gate/up GEMM, the re-quantisation
 // and the weighted sum in the down GEMM.
 //
-// Same operands and the same results, bit for bit, as the launches of dispatch.hip, stream_gemm.hip and combine.hip (the
-// reference's stages, cited there).
+// Same operands and results as the launches of dispatch.hip, stream_gemm.hip and combine.hip (the reference's stages, cited there): int8 bit
+// for bit, FP8 with the fp32 sums of a column added in another order.
 //
 // What bounds it: the weights of the experts that the tokens name, 151 MB for one token of a layer of H 4096, I 1536, top-8, which
 // take 23 us at the rate that streams reach; each of the four launches it was before (plan and permute, gate/up, down,
@@ -18,7 +18,8 @@
 // workgroup and K steps in flight per wave, layer of one token / of four: 4 and 16 36.5 / 111.9 us, 4 and 8 33.5 / 103.6, 4 and 4 32.8 / 101.9, 8 and
 // 3 32.9 / 101.7, 8 and 8 36.1 / 110.8: more workgroups to a CU beat more loads to a wave.
 // The four lanes of a column then hold the four 16-byte quarters of a 64-byte K step, which is what v_mfma_i32_16x16x64_i8 takes;
-// its sixteen rows are the expert's tokens (eight at most), the last of them repeated.
+// its sixteen rows are the expert's tokens (eight at most), the last of them repeated.  FP8 steps are 128 bytes of K, one block of scales:
+// a lane holds 32 bytes of its column, which is what v_mfma_scale_f32_16x16x128_f8f6f4 takes.
 #include <algorithm>
 
 #include "cam_device.h"
@@ -37,6 +38,29 @@ constexpr int kUpRing = 3;     // 64-byte K steps in flight per wave
 constexpr int kDownRing = 8;   // (12: layer of one token +0.6 us)
 constexpr int kFewRowBytes = 49152;  // int8 rows in LDS
 constexpr int kFewMaxI = 3072;          // products of a row in the registers of a wave
+
+template <bool FP8>
+struct Form {
+    typedef v4i Weights;    // a lane's share of a step of 16 columns
+    typedef v4i Sum;
+    typedef int One;
+    static constexpr int kStep = 64;   // K bytes
+    static __device__ __forceinline__ v4i multiply(v4i w, v4i x, v4i sum, int, int)
+    {
+        return __builtin_amdgcn_mfma_i32_16x16x64_i8(w, x, sum, 0, 0, 0);
+    }
+};
+template <>
+struct Form<true> {
+    typedef v8i Weights;
+    typedef v4f Sum;
+    typedef float One;
+    static constexpr int kStep = 128;
+    static __device__ __forceinline__ v4f multiply(v8i w, v8i x, v4f sum, int w_scale, int x_scale)
+    {
+        return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, x, sum, 0, 0, 0, w_scale, 0, x_scale);
+    }
+};
 
 __device__ __forceinline__ void lds_barrier()
 {
@@ -115,27 +139,50 @@ __device__ __forceinline__ int nth_slot(unsigned long long rows, int n)
     return __ffsll(rows) - 1;
 }
 
-// Where 16 columns of packed weights lie: lane l of a wave takes column l % 16 and quarter l / 16 of a 64-byte K step.
+// Where 16 columns of packed weights lie: lane l of a wave takes column l % 16 and quarter l / 16 of a step of K.
+template <bool FP8>
 struct WeightColumns {
     const int8_t *base;  // of the 64-column group
-    int lane_offset;     // this lane's 16 bytes in a step
+    int lane_offset;     // this lane's first 16 bytes in a step (FP8: its other 16 lie 512 bytes on)
     int step;            // bytes from one step to the next
     // 16-column part `part` (0 .. 3) of group nw of [Kd, N]
     __device__ __forceinline__ WeightColumns(const int8_t *w, int Kd, int N, int nw, int part)
     {
-        const int b8 = nw >> 3, q = lane_id() >> 4;
+        const int b8 = nw >> 3, q = lane_id() >> 4, c = (part & 1) * 16 + (lane_id() & 15);
+        const int step64 = min(8, N / 64 - 8 * b8) * 4096;
         base = w + (long long)b8 * 8 * Kd * 64 + (nw & 7) * 4096;
-        lane_offset = (q >> 1) * 2048 + (part >> 1) * 1024 + ((q & 1) * 32 + (part & 1) * 16 + (lane_id() & 15)) * 16;
-        step = min(8, N / 64 - 8 * b8) * 4096;
+        if (FP8) {
+            lane_offset = (q >> 1) * step64 + (q & 1) * 2048 + (part >> 1) * 1024 + c * 16;
+            step = 2 * step64;
+        } else {
+            lane_offset = (q >> 1) * 2048 + (part >> 1) * 1024 + ((q & 1) * 32 + c) * 16;
+            step = step64;
+        }
     }
 };
 
-template <int ACT>
+// This lane's share of step t; a step that is not there fetches nothing and gives zeros.
+template <bool FP8>
+__device__ __forceinline__ typename Form<FP8>::Weights load_weights(const int8_t *base, int lane_offset, int at, bool there)
+{
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, there ? 0x7fffffff : 0, 0x00020000);
+    const v4i lo = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_offset, at, 2));
+    if constexpr (FP8) {
+        const v4i hi = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_offset + 512, at, 2));
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    } else {
+        return lo;
+    }
+}
+
+template <bool FP8, int ACT>
 __global__ __launch_bounds__(kUpThreads, 4) void few_tokens_up_kernel(FewTokensArgs a)
 {
+    typedef Form<FP8> F;
     extern __shared__ __attribute__((aligned(16))) int8_t rows_s[];  // [T][H]
-    __shared__ __attribute__((aligned(16))) v4i part_s[kUpWaves][2][kWave];
+    __shared__ __attribute__((aligned(16))) typename F::Sum part_s[kUpWaves][2][kWave];
     __shared__ float scale_s[kFewTokens];
+    __shared__ uint8_t scale8_s[kFewTokens][kFewMaxH / 128];
     __shared__ float max_s[2][kUpWaves];
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -197,19 +244,28 @@ __global__ __launch_bounds__(kUpThreads, 4) void few_tokens_up_kernel(FewTokensA
     const int nw = c0 >> 5, half = (c0 >> 4) & 1;
     const int8_t *w = a.per_expert ? a.list.w[g] : a.w + (long long)g * H * 2 * I;
     const float *ws = a.per_expert ? a.list.s[g] : a.w_scale + (long long)g * 2 * I;
-    const WeightColumns gate(w, H, 2 * I, nw, half), up(w, H, 2 * I, nw, 2 + half);
-    const float gate_scale = ws[c0 + (tid & 15)], up_scale = ws[I + c0 + (tid & 15)];
-    const int KT = H >> 6;
-    v4i ring[kUpRing][2];
+    const WeightColumns<FP8> gate(w, H, 2 * I, nw, half), up(w, H, 2 * I, nw, 2 + half);
+    const int KT = H / F::kStep;
+    float gate_scale = 0.0f, up_scale = 0.0f;
+    int block_scales[2] = {0, 0};   // FP8: lane kb holds those of K block kb
+    if constexpr (FP8) {
+        const int nblk = (2 * I) >> 7;
+        const uint8_t *s8 = a.w_scale8 + ((long long)g * KT + min(lane, KT - 1)) * nblk;
+        block_scales[0] = s8[c0 >> 7];
+        block_scales[1] = s8[(I + c0) >> 7];
+    } else {
+        gate_scale = ws[c0 + (tid & 15)];
+        up_scale = ws[I + c0 + (tid & 15)];
+    }
+    constexpr int kRing = FP8 ? (kUpRing + 1) / 2 : kUpRing;
+    typename F::Weights ring[kRing][2];
     auto issue = [&](int i, int q) {
         const int t = wave + kUpWaves * q;
-        // (requests past the end fetch nothing and give zeros)
-        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)gate.base, 0, t < KT ? 0x7fffffff : 0, 0x00020000);
-        ring[i][0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, gate.lane_offset, t * gate.step, 2));
-        ring[i][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, up.lane_offset, t * gate.step, 2));
+        ring[i][0] = load_weights<FP8>(gate.base, gate.lane_offset, t * gate.step, t < KT);
+        ring[i][1] = load_weights<FP8>(gate.base, up.lane_offset, t * gate.step, t < KT);
     };
 #pragma unroll
-    for (int i = 0; i < kUpRing; ++i) {
+    for (int i = 0; i < kRing; ++i) {
         issue(i, i);
     }
 
@@ -236,7 +292,7 @@ __global__ __launch_bounds__(kUpThreads, 4) void few_tokens_up_kernel(FewTokensA
         for (int i = 0; i < Row::kChunks; ++i) {
             r.raw[i] = v[i];
         }
-        quant_token_row<2, ACT>(r, Max{max_s[n & 1]});  // (in turns: the maxima before have been read when a slot comes up again)
+        quant_token_row<FP8 ? 3 : 2, ACT>(r, Max{max_s[n & 1]});  // (in turns: the maxima before have been read when a slot comes up again)
 #pragma unroll
         for (int i = 0; i < Row::kChunks; ++i) {
             const int c = i * kUpThreads + tid;
@@ -244,7 +300,9 @@ __global__ __launch_bounds__(kUpThreads, 4) void few_tokens_up_kernel(FewTokensA
                 *(v2u *)(rows_s + n * H + c * 8) = r.q[i];
             }
         }
-        if (tid == 0) {
+        if (FP8) {
+            store_row_scales8(r, scale8_s[n], 0, H, tid);
+        } else if (tid == 0) {
             scale_s[n] = r.scale_out;
         }
     };
@@ -260,15 +318,23 @@ __global__ __launch_bounds__(kUpThreads, 4) void few_tokens_up_kernel(FewTokensA
     }
     lds_barrier();
 
-    v4i sum[2] = {v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}};
-    const int8_t *mine = rows_s + min(lane & 15, rows - 1) * H + (lane >> 4) * 16;
-    for (int q = 0; wave + kUpWaves * q < KT; q += kUpRing) {
+    typename F::Sum sum[2] = {typename F::Sum{}, typename F::Sum{}};
+    const int row = min(lane & 15, rows - 1);
+    const int8_t *mine = rows_s + row * H + (lane >> 4) * (F::kStep / 4);
+    for (int q = 0; wave + kUpWaves * q < KT; q += kRing) {
 #pragma unroll
-        for (int i = 0; i < kUpRing; ++i) {
-            const v4i x = *(const v4i *)(mine + min(wave + kUpWaves * (q + i), KT - 1) * 64);
-            sum[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[i][0], x, sum[0], 0, 0, 0);
-            sum[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[i][1], x, sum[1], 0, 0, 0);
-            issue(i, q + i + kUpRing);
+        for (int i = 0; i < kRing; ++i) {
+            const int t = min(wave + kUpWaves * (q + i), KT - 1);
+            const typename F::Weights x = *(const typename F::Weights *)(mine + t * F::kStep);
+            int sx = 0, sw[2] = {0, 0};
+            if constexpr (FP8) {
+                sx = scale8_s[row][t];
+                sw[0] = __builtin_amdgcn_readlane(block_scales[0], t);
+                sw[1] = __builtin_amdgcn_readlane(block_scales[1], t);
+            }
+            sum[0] = F::multiply(ring[i][0], x, sum[0], sw[0], sx);
+            sum[1] = F::multiply(ring[i][1], x, sum[1], sw[1], sx);
+            issue(i, q + i + kRing);
         }
     }
     part_s[wave][0][lane] = sum[0];
@@ -279,25 +345,32 @@ __global__ __launch_bounds__(kUpThreads, 4) void few_tokens_up_kernel(FewTokensA
     if (n >= rows) {
         return;
     }
-    int sg = 0, su = 0;
+    typename F::One sg = 0, su = 0;   // (in the order of the waves)
 #pragma unroll
     for (int v = 0; v < kUpWaves; ++v) {
-        sg += ((const int *)&part_s[v][0][(c >> 2) * 16 + n])[c & 3];
-        su += ((const int *)&part_s[v][1][(c >> 2) * 16 + n])[c & 3];
+        sg += ((const typename F::One *)&part_s[v][0][(c >> 2) * 16 + n])[c & 3];
+        su += ((const typename F::One *)&part_s[v][1][(c >> 2) * 16 + n])[c & 3];
     }
-    const float xs = scale_s[n];
-    const float tg = __fmul_rn(__fmul_rn((float)sg, gate_scale), xs);
-    const float tu = __fmul_rn(__fmul_rn((float)su, up_scale), xs);
+    float tg = sg, tu = su;
+    if constexpr (!FP8) {  // (FP8 sums carry their scales already)
+        const float xs = scale_s[n];
+        tg = __fmul_rn(__fmul_rn((float)sg, gate_scale), xs);
+        tu = __fmul_rn(__fmul_rn((float)su, up_scale), xs);
+    }
     a.products[(long long)nth_slot(row_slots, n) * I + c0 + c] = __fmul_rn(cam_silu_spec(tg), tu);
 }
 
 // RW: slots whose products a wave quantises.
-template <int ACT, int RW>
+template <bool FP8, int ACT, int RW>
 __global__ __launch_bounds__(kDownThreads, RW == 1 ? 4 : 2) void few_tokens_down_kernel(FewTokensArgs a)
 {
+    typedef Form<FP8> F;
+    constexpr int kParts = FP8 ? kDownWaves : 1;   // FP8 sums are added in the order of the waves
+    constexpr int kBlocks = kFewRowBytes / 128;
     extern __shared__ __attribute__((aligned(16))) int8_t rows_s[];  // [slots][I]
-    __shared__ int sum_s[kFewSlots][kColumns];
-    __shared__ float column_s[kFewSlots][kColumns];   // the scale of the slot's expert for each column
+    __shared__ typename F::One sum_s[kParts][kFewSlots][kColumns];
+    __shared__ float column_s[FP8 ? 1 : kFewSlots][kColumns];   // the scale of the slot's expert for each column
+    __shared__ uint8_t x_scale8_s[FP8 ? kBlocks : 1], w_scale8_s[FP8 ? kBlocks : 1];   // [slots][I / 128], of the slot's expert
     __shared__ float scale_s[kFewSlots], weight_s[kFewSlots];
     __shared__ int row_s[kFewSlots];   // the slot whose sums are this one's, -1 where it has no expert
     const int tid = threadIdx.x;
@@ -321,11 +394,31 @@ __global__ __launch_bounds__(kDownThreads, RW == 1 ? 4 : 2) void few_tokens_down
             }
         }
     };
-    // (the arithmetic of requant_kernel)
+    // (the arithmetic of requant_kernel and requant_fp8_kernel)
     auto quantise = [&](int first) {
 #pragma unroll
         for (int i = 0; i < RW; ++i) {
             const int slot = first + wave + i * kDownWaves;
+            if constexpr (FP8) {
+#pragma unroll
+                for (int q = 0; q < kQuads; ++q) {
+                    const int c = q * kWave + lane;   // a block of 128 columns to 32 lanes
+                    const v4f v = prod[i][q];
+                    const float m = group_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))), 32);
+                    const int ex = fp8_block_scale_exp(m);
+                    const float f1 = exp2_int(-(ex / 2)), f2 = exp2_int(-(ex - ex / 2));
+                    int w = 0;
+                    w = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(__fmul_rn(v[0], f1), f2), __fmul_rn(__fmul_rn(v[1], f1), f2), w, false);
+                    w = __builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(__fmul_rn(v[2], f1), f2), __fmul_rn(__fmul_rn(v[3], f1), f2), w, true);
+                    if (slot < A && c < I >> 2) {
+                        *(int *)(rows_s + slot * I + c * 4) = w;
+                        if ((lane & 31) == 0) {
+                            x_scale8_s[slot * (I >> 7) + (c >> 5)] = (uint8_t)(ex + 127);
+                        }
+                    }
+                }
+                continue;
+            }
             float m = 0.0f;
 #pragma unroll
             for (int q = 0; q < kQuads; ++q) {
@@ -362,13 +455,19 @@ __global__ __launch_bounds__(kDownThreads, RW == 1 ? 4 : 2) void few_tokens_down
         }
     }
     const Slots slots(a, loaded_id);
+    const int KT = I / F::kStep;
     float column = 0.0f, weight = 0.0f;
-    const int g = __shfl(slots.id, tid >> 4, kWave);   // (by all lanes)
-    if (tid < A * kColumns) {
-        if (g >= 0) {
-            column = (a.per_expert ? a.list.s[g] : a.w_scale + (long long)g * H)[c0 + (tid & 15)];
+    int w_scale8 = 0;
+    const int g = __shfl(slots.id, min(FP8 ? tid / KT : tid >> 4, kWave - 1), kWave);   // (by all lanes)
+    if constexpr (FP8) {
+        if (tid < A * KT && g >= 0) {
+            w_scale8 = a.w_scale8[((long long)g * KT + tid % KT) * (H >> 7) + (c0 >> 7)];
         }
-        sum_s[tid >> 4][tid & 15] = 0;
+    } else if (tid < A * kColumns && g >= 0) {
+        column = (a.per_expert ? a.list.s[g] : a.w_scale + (long long)g * H)[c0 + (tid & 15)];
+    }
+    for (int i = tid; i < kParts * kFewSlots * kColumns; i += kDownThreads) {
+        (&sum_s[0][0][0])[i] = 0;
     }
     if (tid < A) {
         weight = a.gates[tid];
@@ -376,37 +475,40 @@ __global__ __launch_bounds__(kDownThreads, RW == 1 ? 4 : 2) void few_tokens_down
     }
 
     // this wave's share of the K steps of all experts, one after the other
-    const int KT = I >> 6;
     const int steps = slots.experts() * KT, share = (steps + kDownWaves - 1) / kDownWaves;
     const int begin = wave * share, end = min(steps, begin + share);
-    v4i ring[kDownRing];
+    constexpr int kRing = FP8 ? kDownRing / 2 : kDownRing;
+    typename F::Weights ring[kRing];
     int ask_j = begin / KT, ask_t = begin - ask_j * KT;   // the next step to ask for
     const int8_t *ask_w = a.w;
     int ask_step = 0;
-    const WeightColumns none(nullptr, I, H, c0 >> 6, (c0 >> 4) & 3);
+    const WeightColumns<FP8> none(nullptr, I, H, c0 >> 6, (c0 >> 4) & 3);
     auto ask_expert = [&](int j) {
         if (j < slots.experts()) {
             const int g = slots.expert_of(slots.first_slot(j));
-            const WeightColumns wc(a.per_expert ? a.list.w[g] : a.w + (long long)g * I * H, I, H, c0 >> 6, (c0 >> 4) & 3);
+            const WeightColumns<FP8> wc(a.per_expert ? a.list.w[g] : a.w + (long long)g * I * H, I, H, c0 >> 6, (c0 >> 4) & 3);
             ask_w = wc.base;
             ask_step = wc.step;
         }
     };
     ask_expert(ask_j);
     auto issue = [&](int i, int f) {
-        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)ask_w, 0, f < end ? 0x7fffffff : 0, 0x00020000);
-        ring[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, none.lane_offset, ask_t * ask_step, 2));
+        ring[i] = load_weights<FP8>(ask_w, none.lane_offset, ask_t * ask_step, f < end);
         if (++ask_t == KT) {
             ask_t = 0;
             ask_expert(++ask_j);
         }
     };
 #pragma unroll
-    for (int i = 0; i < kDownRing; ++i) {
+    for (int i = 0; i < kRing; ++i) {
         issue(i, begin + i);
     }
 
-    if (tid < A * kColumns) {
+    if constexpr (FP8) {
+        if (tid < A * KT) {
+            w_scale8_s[tid] = (uint8_t)w_scale8;
+        }
+    } else if (tid < A * kColumns) {
         column_s[tid >> 4][tid & 15] = column;
     }
     if (tid < A) {
@@ -416,10 +518,11 @@ __global__ __launch_bounds__(kDownThreads, RW == 1 ? 4 : 2) void few_tokens_down
     lds_barrier();
 
     int j = begin / KT, t = begin - j * KT;
-    int rows = 0, slot = 0;   // of the expert, of this lane's row
-    v4i sum = {0, 0, 0, 0};
+    int rows = 0, lead = 0, slot = 0;   // of the expert, its first slot, the slot of this lane's row
+    typename F::Sum sum{};
     auto expert = [&]() {
-        const unsigned long long row_slots = slots.rows_of(slots.first_slot(j));
+        lead = slots.first_slot(j);
+        const unsigned long long row_slots = slots.rows_of(lead);
         rows = __popcll(row_slots);
         slot = nth_slot(row_slots, lane & 15);
     };
@@ -427,20 +530,30 @@ __global__ __launch_bounds__(kDownThreads, RW == 1 ? 4 : 2) void few_tokens_down
         if ((lane & 15) < rows) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                atomicAdd(&sum_s[slot][(lane >> 4) * 4 + e], sum[e]);
+                typename F::One *to = &sum_s[FP8 ? wave : 0][slot][(lane >> 4) * 4 + e];
+                if constexpr (FP8) {
+                    *to = sum[e];   // a wave has an expert's steps one after the other
+                } else {
+                    atomicAdd(to, sum[e]);
+                }
             }
         }
-        sum = v4i{0, 0, 0, 0};
+        sum = typename F::Sum{};
     };
     if (begin < end) {
         expert();
     }
-    for (int f = begin; f < end; f += kDownRing) {
+    for (int f = begin; f < end; f += kRing) {
 #pragma unroll
-        for (int i = 0; i < kDownRing; ++i) {
+        for (int i = 0; i < kRing; ++i) {
             if (f + i < end) {
-                const v4i x = *(const v4i *)(rows_s + slot * I + t * 64 + (lane >> 4) * 16);
-                sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(ring[i], x, sum, 0, 0, 0);
+                const typename F::Weights x = *(const typename F::Weights *)(rows_s + slot * I + t * F::kStep + (lane >> 4) * (F::kStep / 4));
+                int sw = 0, sx = 0;
+                if constexpr (FP8) {
+                    sw = w_scale8_s[lead * KT + t];
+                    sx = x_scale8_s[slot * KT + t];
+                }
+                sum = F::multiply(ring[i], x, sum, sw, sx);
                 ++t;
                 if (t == KT || f + i + 1 == end) {
                     leave();
@@ -450,7 +563,7 @@ __global__ __launch_bounds__(kDownThreads, RW == 1 ? 4 : 2) void few_tokens_down
                         expert();
                     }
                 }
-                issue(i, f + i + kDownRing);
+                issue(i, f + i + kRing);
             }
         }
     }
@@ -463,7 +576,16 @@ __global__ __launch_bounds__(kDownThreads, RW == 1 ? 4 : 2) void few_tokens_down
         for (int k = 0; k < a.K; ++k) {
             const int s = row_s[token * a.K + k];
             if (s >= 0) {
-                float v = __fmul_rn(__fmul_rn((float)sum_s[s][c], column_s[s][c]), scale_s[s]);
+                float v;
+                if constexpr (FP8) {
+                    v = sum_s[0][s][c];
+#pragma unroll
+                    for (int p = 1; p < kParts; ++p) {
+                        v += sum_s[p][s][c];
+                    }
+                } else {
+                    v = __fmul_rn(__fmul_rn((float)sum_s[0][s][c], column_s[s][c]), scale_s[s]);
+                }
                 if (ACT == 1) {
                     asm("" : "+v"(v));  // rounded to fp32 first, as in the GEMMs: the conversion must not swallow the product
                     v = fp16_bits_to_f32(f32_to_fp16_bits(v));
@@ -478,10 +600,26 @@ __global__ __launch_bounds__(kDownThreads, RW == 1 ? 4 : 2) void few_tokens_down
     }
 }
 
-template <int ACT, int RW>
+template <bool FP8, int ACT>
+void launch_up(dim3 grid, dim3 block, size_t lds, hipStream_t stream, const FewTokensArgs &a)
+{
+    hipLaunchKernelGGL((few_tokens_up_kernel<FP8, ACT>), grid, block, lds, stream, a);
+}
+
+template <bool FP8, int ACT>
 void launch_down(dim3 grid, dim3 block, size_t lds, hipStream_t stream, const FewTokensArgs &a)
 {
-    hipLaunchKernelGGL((few_tokens_down_kernel<ACT, RW>), grid, block, lds, stream, a);
+    if (a.T * a.K <= kDownWaves) {
+        hipLaunchKernelGGL((few_tokens_down_kernel<FP8, ACT, 1>), grid, block, lds, stream, a);
+    } else {
+        hipLaunchKernelGGL((few_tokens_down_kernel<FP8, ACT, 2>), grid, block, lds, stream, a);
+    }
+}
+
+bool few_tokens_valid(const FewTokensArgs &a)
+{
+    return few_tokens_apply(a.T, a.K, a.E, a.H, a.I, a.w_scale8 != nullptr) &&
+           (a.w_scale8 == nullptr || (a.H % 128 == 0 && a.I % 128 == 0 && !a.per_expert && !a.x_is_fp16));
 }
 
 }  // namespace
@@ -495,12 +633,19 @@ void launch_down(dim3 grid, dim3 block, size_t lds, hipStream_t stream, const Fe
 // (also 30.8 / 30.0), 48 42.8 / 54.1.  More: 4 x 4096, 8 of 128, 1536 116.5 / 102.0 (the same experts for all 65.4 / 46.2), 4 x 4096, 8 of 64, 512
 // 47.1 / 43.8, 3 x 4096, 8 of 48, 2048 111.3 / 94.0; not 8 x 4096, 4 of 8, 1536 41.9 / 46.0, 4 x 2048, 8 of 64, 1024 47.5 / 51.2, 6 x 5120, 3 of 40,
 // 1024 59.1 / 60.1.
-bool few_tokens_apply(int64_t T, int64_t K, int64_t E, int64_t H, int64_t I)
+// FP8 up to sixteen slots: 1 x 4096, 8 of 128, 1536 49.2 / 34.3, 1 of 128 38.0 / 12.7, 1 x 7168, 8 of 64, 2048 82.3 / 62.8, 2 x 4096, 8 of 64, 1536 62.7 /
+// 59.4 (the same 52.2 / 39.3), 2 x 7168, 8 of 64, 2048 127.8 / 124.2, 4 x 4096, 4 of 8, 1024 42.9 / 28.5, 2 x 1024, 8 of 64, 768 28.9 / 26.0, 1 x 1024, 8
+// of 64, 2048 28.5 / 24.3; not 1 x 1024, 8 of 64, 3072 32.1 / 33.2, 2 x 1024, 8 of 64, 1024 28.7 / 29.7, 2 x 2048, 6 of 64, 2048 39.8 / 43.0, 5 x 4096,
+// 3 of 64, 2048 69.2 / 70.5, 3 x 7168, 8 of 64, 1024 101.4 / 104.1.
+bool few_tokens_apply(int64_t T, int64_t K, int64_t E, int64_t H, int64_t I, bool fp8)
 {
     const int64_t slots = T * K;
     if (T < 1 || T > kFewTokens || K < 1 || slots > kFewSlots || E < 1 || E > kMaxExperts || H < 64 || H > kFewMaxH || I < 64 || I > kFewMaxI ||
         H % 64 != 0 || I % 64 != 0 || T * H > kFewRowBytes || slots * I > kFewRowBytes) {
         return false;
+    }
+    if (fp8) {
+        return slots <= 8 ? slots * I <= 16 * H : slots <= 16 && (slots * I <= 7 * H || slots * I <= 12288);
     }
     if (slots <= 8) {
         return true;
@@ -510,30 +655,30 @@ bool few_tokens_apply(int64_t T, int64_t K, int64_t E, int64_t H, int64_t I)
 
 hipError_t launch_few_tokens_up(const FewTokensArgs &a, hipStream_t stream)
 {
-    if (!few_tokens_apply(a.T, a.K, a.E, a.H, a.I)) {
+    if (!few_tokens_valid(a)) {
         return hipErrorInvalidValue;
     }
     const dim3 grid((unsigned)(a.T * a.K * (a.I / kColumns) + 1)), block(kUpThreads);
     const size_t lds = (size_t)a.T * a.H;
-    if (a.x_is_fp16) {
-        hipLaunchKernelGGL(few_tokens_up_kernel<1>, grid, block, lds, stream, a);
+    if (a.w_scale8 != nullptr) {
+        launch_up<true, 0>(grid, block, lds, stream, a);
     } else {
-        hipLaunchKernelGGL(few_tokens_up_kernel<0>, grid, block, lds, stream, a);
+        a.x_is_fp16 ? launch_up<false, 1>(grid, block, lds, stream, a) : launch_up<false, 0>(grid, block, lds, stream, a);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_few_tokens_down(const FewTokensArgs &a, hipStream_t stream)
 {
-    if (!few_tokens_apply(a.T, a.K, a.E, a.H, a.I)) {
+    if (!few_tokens_valid(a)) {
         return hipErrorInvalidValue;
     }
     const dim3 grid((unsigned)(a.H / kColumns)), block(kDownThreads);
     const size_t lds = (size_t)a.T * a.K * a.I;
-    if (a.T * a.K <= kDownWaves) {
-        a.x_is_fp16 ? launch_down<1, 1>(grid, block, lds, stream, a) : launch_down<0, 1>(grid, block, lds, stream, a);
+    if (a.w_scale8 != nullptr) {
+        launch_down<true, 0>(grid, block, lds, stream, a);
     } else {
-        a.x_is_fp16 ? launch_down<1, 2>(grid, block, lds, stream, a) : launch_down<0, 2>(grid, block, lds, stream, a);
+        a.x_is_fp16 ? launch_down<false, 1>(grid, block, lds, stream, a) : launch_down<false, 0>(grid, block, lds, stream, a);
     }
     return hipGetLastError();
 }
