@@ -118,13 +118,17 @@ __global__ __launch_bounds__(kDispWaves * kWave) void dispatch_smooth_kernel(Dis
 // row is what the launch takes, so it is spread over sixteen waves (four from 257 tokens on) instead of one.
 // Launches: one token x 4096 to 128 experts, top-8: 3.5 + 7.4 us -> 5.9; 64 x 4096 FP8: 6.2 + 15.6 -> 7.4; 128 x 7168 to 256
 // experts: 6.1 + 9.8 -> 7.8.
+// What bounds it beside the latencies is the counting, top-k times over a thread's ids, so an id is compared twice a time and with
+// nothing else: what lies behind the active tokens, or behind this one, is struck out beforehand.  Replayed from a graph, us, with a look
+// at the place of every id instead / this: 128 x 4096, top-8 of 128 6.44 / 5.94, 256 7.75 / 6.97, 128 x 7168, top-8 of 256 7.05 / 6.37, 341 x 4096,
+// top-6 10.44 / 9.12, 170 x 2048, top-12 8.66 / 7.49.  A wave per k that looks at all ids: 7.38, 9.97, 7.38, 11.41, 10.64.
 constexpr int kSmallIds = 2048;   // ids per launch (rows of at most 29 MB)
 template <typename IdT, int QUANT, int ACT, bool SMOOTH, int NT>
 __global__ __launch_bounds__(NT) void dispatch_small_kernel(PlanArgs p, DispatchArgs a)
 {
     constexpr int kPer = kSmallIds / NT;   // ids per thread
     constexpr int kWaves = NT / kWave;
-    __shared__ int counts[2][kMaxTopk][kWaves];  // entries before the expert's, earlier entries of it: per k and wave
+    __shared__ int counts[kWaves][kMaxTopk];  // entries before the expert's, and earlier entries of it (<< 16): per wave and k
     __shared__ int row_s[kMaxTopk];
     __shared__ float max_s[kWaves];
     __shared__ int active_s;
@@ -164,37 +168,43 @@ __global__ __launch_bounds__(NT) void dispatch_small_kernel(PlanArgs p, Dispatch
     const int t = (int)blockIdx.x - 1;
     GroupRow<NT> r;
     load_token_row(a.x, t, a.H, tid, r);
-    int id[kPer];  // entries tid, tid + NT, ...; E where none
+    int id[kPer];  // entries tid, tid + NT, ...; -1 where none
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
         const int j = tid + i * NT;
-        id[i] = E;
+        id[i] = -1;
         if (i * NT < n_all && j < n_all) {
-            const int e = load_id(idx, j, E);
-            id[i] = e >= 0 ? e : E;
+            id[i] = load_id(idx, j, E);
         }
     }
     const int own_ids = lane < K ? load_id(idx, t * K + lane, E) : -1;  // lane k: the id of entry (t,k)
     const int t_active = count_active(p.mask, p.T, tid, NT, &active_s);
     const int n = t_active * K;
+    int earlier_id[kPer];   // those of the tokens before
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int j = tid + i * NT;
+        id[i] = j < n ? id[i] : -1;
+        earlier_id[i] = j < t * K ? id[i] : -1;
+    }
+    int found = 0;   // lane k: this wave's counts for entry (t,k)
     for (int k = 0; k < K; ++k) {
-        const int own = t * K + k;
         const int e = __builtin_amdgcn_readlane(own_ids, k);
         int before = 0, earlier = 0;
-        if (own < n && e >= 0) {
 #pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                if (i * NT < n) {
-                    const int j = tid + i * NT;
-                    before += __popcll(__ballot(j < n && id[i] < e));
-                    earlier += __popcll(__ballot(j < own && id[i] == e));
-                }
+        for (int i = 0; i < kPer; ++i) {
+            if (i * NT < n) {
+                before += __popcll(__ballot((unsigned)id[i] < (unsigned)max(e, 0)));
+                earlier += __popcll(__ballot(earlier_id[i] == e));
             }
         }
-        if (lane == 0) {
-            counts[0][k][wave] = before;
-            counts[1][k][wave] = earlier;
+        if (wave == 0) {  // and in the token itself
+            earlier += __popcll(__ballot(own_ids == e) & ((1ull << k) - 1));
         }
+        found = lane == k ? before | earlier << 16 : found;
+    }
+    if (lane < K) {
+        counts[wave][lane] = found;
     }
     if (QUANT != 0 && !SMOOTH) {
         quant_token_row<QUANT, ACT>(r, GroupMax<NT>{max_s});
@@ -204,14 +214,13 @@ __global__ __launch_bounds__(NT) void dispatch_small_kernel(PlanArgs p, Dispatch
         const int own = t * K + tid;
         int row = -1, rank = -1;
         if (own < n && own_ids >= 0) {
-            rank = 0;
-            row = 0;
+            int sum = 0;   // (2048 of either at most)
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) {
-                row += counts[0][tid][w];
-                rank += counts[1][tid][w];
+                sum += counts[w][tid];
             }
-            row += rank;
+            rank = sum >> 16;
+            row = (sum & 0xffff) + rank;
         }
         row_s[tid] = row;
         p.pos[own] = rank;
