@@ -390,15 +390,78 @@ __global__ __launch_bounds__(kExpertThreads, 8) void plan_experts_kernel(PlanArg
     }
 }
 
+// The layout of up to kExpertIds ids in one launch: a workgroup per expert that looks at all ids and counts its own, and one per rank
+// that marks the tokens with an id of the rank's experts in LDS, counts them and stores their flags.  Nothing passes between
+// workgroups.  Latency bound: one round trip to the ids and, for a rank, one through LDS.  With very many flags a workgroup per rank
+// stores too many by itself.  us, replayed from a graph, two launches (up to some hundred tokens one workgroup) / this, T tokens, top-K of E, R ranks,
+// ids spread; they differ by 0.3 at most where all tokens name the same: 1, 8 of 128, 1 3.2 / 2.3; 1024, 1 of 64, 1 3.1 / 2.2; 1999, 6 of 64, 1 5.2 /
+// 3.1; 2048, 8 of 512, 1 5.9 / 4.4; 16384, 1 of 128, 1 5.9 / 4.7; 2048, 8 of 256, 16 6.6 / 4.2, 64 8.1 / 4.9; 1024, 16 of 256, 128 12.9 / 4.6; 100, 2
+// of 384, 384 7.0 / 3.7; 5000, 1 of 64, 64 (320000 flags) 6.4 / 5.6, but 16384, 1 of 128, 16 (262144) 6.1 / 7.2 and 8000, 2 of 384, 384 16.7 /
+// 21.5.  Prefill operators, 1999 tokens x 4096, top-6 of 64: 51.9 -> 49.1.
+constexpr long long kExpertFlags = 8 * kExpertIds;
+template <typename IdT, typename OutT, int IT>
+__global__ __launch_bounds__(kExpertThreads, 8) void layout_experts_kernel(LayoutArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t token_s[kExpertIds];
+    __shared__ int count_s[kExpertThreads / kWave];
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int x = blockIdx.x;
+    const int n_all = a.T * a.K;
+    ExpertEntries<kExpertThreads, IT> ids;
+    ids.load((const IdT *)a.idx, n_all);
+    int count = 0;
+    if (x < a.E) {
+        ids.only_first(n_all);
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            count += __popcll(__ballot(ids.e[it] == x));
+        }
+    } else {
+        for (int i = tid; i < (a.T + 15) >> 4; i += kExpertThreads) {
+            ((v4u *)token_s)[i] = v4u{0u, 0u, 0u, 0u};
+        }
+        __syncthreads();
+        const int rank = x - a.E;
+        const unsigned epr = (unsigned)(a.E / a.R);
+        const float inv = 1.0f / (float)a.K;
+        const int base = ids.first_entry() + lane;
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int i = base + it * kWave;
+            if (i < n_all && (unsigned)ids.e[it] - (unsigned)rank * epr < epr) {
+                token_s[(int)(((float)i + 0.5f) * inv)] = 1;   // i / K: exact below 2^15
+            }
+        }
+        __syncthreads();
+        OutT *out = (OutT *)a.in_rank + rank;
+        for (int t0 = 0; t0 < a.T; t0 += kExpertThreads) {
+            const int t = t0 + tid;
+            const int in = t < a.T ? token_s[t] : 0;
+            if (t < a.T) {
+                out[(long long)t * a.R] = (OutT)in;
+            }
+            count += __popcll(__ballot(in != 0));
+        }
+    }
+    if (lane == 0) {
+        count_s[tid >> 6] = count;
+    }
+    __syncthreads();
+    if (tid < kWave) {
+        count = wave_sum(lane < kExpertThreads / kWave ? count_s[lane] : 0);
+        if (lane == 0) {
+            (x < a.E ? a.per_expert[x] : a.per_rank[x - a.E]) = count;
+        }
+    }
+}
+
 // The layout (dispatch_layout.h:83-134): entries per expert, tokens per rank (a token counts once per rank) and
-// isTokenInRank[t,r].  Only counts are asked for, so nothing is ranked: a workgroup counts the `span` tokens from its own
-// first on in LDS and leaves its counts, experts then ranks, in a row of `partial`; layout_sum_kernel adds the rows up.  One
-// workgroup alone writes the results itself.  Latency bound: 1999 tokens x 6 ids to 64 experts, with layout, dispatch and
-// combine of 4096 columns 69.9 us when the layout was the two launches of the plan and one for the flags, 63.5 now.
+// isTokenInRank[t,r], of more ids or flags.  A workgroup counts the `span` tokens from its own first on in LDS and leaves its
+// counts, experts then ranks, in a row of `partial`; layout_sum_kernel adds the rows up.
 constexpr int kLayoutThreads = 256;
-constexpr int kLayoutOne = 1024;  // threads of a workgroup alone
-template <typename IdT, typename OutT, int NT>
-__global__ __launch_bounds__(NT) void layout_kernel(LayoutArgs a, int span)
+template <typename IdT, typename OutT>
+__global__ __launch_bounds__(kLayoutThreads) void layout_kernel(LayoutArgs a, int span)
 {
     __shared__ int count_s[kMaxExperts + kMaxRanks];
     const int tid = threadIdx.x;
@@ -407,14 +470,14 @@ __global__ __launch_bounds__(NT) void layout_kernel(LayoutArgs a, int span)
     const int E = a.E, R = a.R, K = a.K;
     const int epr = E / R;
     OutT *out = (OutT *)a.in_rank;
-    for (int c = tid; c < E + R; c += NT) {
+    for (int c = tid; c < E + R; c += kLayoutThreads) {
         count_s[c] = 0;
     }
-    for (long long i = (long long)t0 * R + tid; i < (long long)t1 * R; i += NT) {
+    for (long long i = (long long)t0 * R + tid; i < (long long)t1 * R; i += kLayoutThreads) {
         out[i] = (OutT)0;
     }
     __syncthreads();
-    for (int t = t0 + tid; t < t1; t += NT) {
+    for (int t = t0 + tid; t < t1; t += kLayoutThreads) {
         const IdT *ids = (const IdT *)a.idx + (long long)t * K;
         int e[kMaxTopk];
 #pragma unroll
@@ -440,14 +503,8 @@ __global__ __launch_bounds__(NT) void layout_kernel(LayoutArgs a, int span)
         }
     }
     __syncthreads();
-    for (int c = tid; c < E + R; c += NT) {
-        if (gridDim.x > 1) {
-            a.partial[(long long)blockIdx.x * (E + R) + c] = count_s[c];
-        } else if (c < E) {
-            a.per_expert[c] = count_s[c];
-        } else {
-            a.per_rank[c - E] = count_s[c];
-        }
+    for (int c = tid; c < E + R; c += kLayoutThreads) {
+        a.partial[(long long)blockIdx.x * (E + R) + c] = count_s[c];
     }
 }
 
@@ -478,24 +535,21 @@ __global__ __launch_bounds__(kWave) void layout_sum_kernel(LayoutArgs a, int row
     }
 }
 
-// Workgroups of a layout and tokens of each: one of kLayoutOne threads alone where that is sure to save more, the launch that adds the
-// counts up, than it costs; else one round of tokens per workgroup up to 64 of them, whose counts are two round trips to add up.
-// What it costs are the counts of the tokens beyond the 256 that a workgroup has in any case, one by one where all tokens name the
-// same experts (and, of several ranks, as many ranks): the line lies where such ids are not slower.  us, added up / alone, ids
-// spread over the experts and all the same: one rank, 1024 tokens, top-1 4.4 / 3.0 and 4.4 / 3.7, 768, top-2 4.4 / 3.0 and 4.5 / 4.0, 512,
-// top-4 4.8 / 3.4 and 5.3 / 4.5, 384, top-8 5.5 / 4.3 and 6.4 / 6.0, 320, top-16 6.8 / 5.7 and 8.9 / 8.5; beyond the line 600, top-4
-// 4.8 / 3.5 and 5.1 / 4.9, 450, top-8 5.5 / 4.6 and 6.4 / 6.7, 1024, top-6 5.1 / 4.5 and 5.8 / 8.6, top-16 7.2 / 11.4 and 9.4 / 22.6.
-// Sixteen ranks, 330 tokens, top-8 6.2 / 4.8 and 8.2 / 7.7; beyond, 384, top-8 6.1 / 5.0 and 8.1 / 8.4, 290, top-16 9.1 / 7.9 and 12.3 / 13.2.
+// Workgroups of a layout and tokens of each, 0 where a workgroup per expert and per rank does all of it in one launch: one round of
+// tokens per workgroup up to 64 of them, whose counts are two round trips to add up.  Up to 1024 tokens it is one launch where the
+// counts of the tokens beyond 256 are few, a line that one workgroup alone once set and the tests keep: beyond it two launches take 2
+// to 8 us longer (1024 tokens, top-6 of 64 5.1 / 2.5).
 int layout_workgroups(long long T, int K, int R, int *span)
 {
     const int counts = R > 1 ? 2 * K : K;
-    if (T <= kLayoutOne && T * R <= 8 * kLayoutOne && counts <= 20 && (T - kLayoutThreads) * counts <= 1024) {
-        *span = kLayoutOne;
-        return 1;
+    const bool one_launch = T <= 1024 ? T * R <= 8192 && counts <= 20 && (T - kLayoutThreads) * counts <= 1024
+                                      : T * K <= kExpertIds && T * R <= kExpertFlags;
+    if (one_launch || T <= kLayoutThreads) {
+        return 0;
     }
     const long long rounds = std::max<long long>((T + 64 * kLayoutThreads - 1) / (64 * kLayoutThreads), 1);
     *span = (int)(rounds * kLayoutThreads);
-    return (int)std::max<long long>((T + *span - 1) / *span, 1);
+    return (int)((T + *span - 1) / *span);
 }
 
 __global__ __launch_bounds__(kScanThreads) void notify_scan_kernel(const int32_t *cnt, int E, int num_tokens,
@@ -697,32 +751,47 @@ uint64_t layout_workspace_bytes(int64_t T, int K, int E, int R)
     return (uint64_t)layout_workgroups(T, K, R, &span) * (uint64_t)(E + R) * sizeof(int32_t);
 }
 
-template <typename IdT, int NT>
-void launch_layout_as(const LayoutArgs &a, int workgroups, int span, hipStream_t stream)
+template <typename IdT>
+void launch_layout_experts(const LayoutArgs &a, hipStream_t stream)
 {
-    const dim3 grid(workgroups), block(NT);
+    with_ids_per_thread((long long)a.T * a.K, [&](auto it) {
+        const dim3 grid((unsigned)(a.E + a.R)), block(kExpertThreads);
+        if (a.in_rank_bytes == 4) {
+            hipLaunchKernelGGL((layout_experts_kernel<IdT, int32_t, decltype(it)::value>), grid, block, 0, stream, a);
+        } else {
+            hipLaunchKernelGGL((layout_experts_kernel<IdT, uint8_t, decltype(it)::value>), grid, block, 0, stream, a);
+        }
+    });
+}
+
+template <typename IdT>
+void launch_layout_spans(const LayoutArgs &a, int workgroups, int span, hipStream_t stream)
+{
+    const dim3 grid((unsigned)workgroups), block(kLayoutThreads);
     if (a.in_rank_bytes == 4) {
-        hipLaunchKernelGGL((layout_kernel<IdT, int32_t, NT>), grid, block, 0, stream, a, span);
+        hipLaunchKernelGGL((layout_kernel<IdT, int32_t>), grid, block, 0, stream, a, span);
     } else {
-        hipLaunchKernelGGL((layout_kernel<IdT, uint8_t, NT>), grid, block, 0, stream, a, span);
+        hipLaunchKernelGGL((layout_kernel<IdT, uint8_t>), grid, block, 0, stream, a, span);
     }
 }
 
 hipError_t launch_layout(const LayoutArgs &a, hipStream_t stream)
 {
-    if (a.K > kMaxTopk || a.E > kMaxExperts || a.R > kMaxRanks || a.partial == nullptr) {
+    if (a.K > kMaxTopk || a.E > kMaxExperts || a.R > kMaxRanks) {
         return hipErrorInvalidValue;
     }
-    int span;
+    int span = 0;
     const int n = layout_workgroups(a.T, a.K, a.R, &span);
-    if (n == 1 && a.T > kLayoutThreads) {
-        a.idx_is64 ? launch_layout_as<int64_t, kLayoutOne>(a, n, span, stream) : launch_layout_as<int32_t, kLayoutOne>(a, n, span, stream);
-    } else {
-        a.idx_is64 ? launch_layout_as<int64_t, kLayoutThreads>(a, n, span, stream)
-                   : launch_layout_as<int32_t, kLayoutThreads>(a, n, span, stream);
+    if (n == 0) {
+        a.idx_is64 ? launch_layout_experts<int64_t>(a, stream) : launch_layout_experts<int32_t>(a, stream);
+        return hipGetLastError();
     }
+    if (a.partial == nullptr) {
+        return hipErrorInvalidValue;
+    }
+    a.idx_is64 ? launch_layout_spans<int64_t>(a, n, span, stream) : launch_layout_spans<int32_t>(a, n, span, stream);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || n == 1) {
+    if (e != hipSuccess) {
         return e;
     }
     hipLaunchKernelGGL(layout_sum_kernel, dim3((a.E + a.R + kWave - 1) / kWave), dim3(kWave), 0, stream, a, n);
