@@ -340,7 +340,7 @@ hipError_t run_grouped_gemm(cam::GemmArgs g, const int64_t *group_list, int cumu
 // The GEMMs of a fused layer: per-expert counts from its plan, g.sched filled by launch_layer_plan unless they stream.  A token
 // names an expert once, so no expert has more than T rows.
 hipError_t layer_gemm(const cam::GemmArgs &g, const int64_t *counts, int E, int64_t A, int T, bool stream, hipStream_t s,
-                      const float *products = nullptr)
+                      int32_t *queue, const float *products = nullptr)
 {
     if (!stream) {
         return cam::launch_gemm(g, s);
@@ -351,6 +351,7 @@ hipError_t layer_gemm(const cam::GemmArgs &g, const int64_t *counts, int E, int6
     sa.G = E;
     sa.max_rows = A;
     sa.products = products;
+    sa.queue = queue;
     return cam::launch_stream_gemm(sa, T, s);
 }
 
@@ -1853,6 +1854,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
     const uint64_t o_row = c.take((uint64_t)A * 4);
     const uint64_t o_token = gather ? c.take((uint64_t)A * 4) : 0;
     const uint64_t o_meta = c.take(cam::kPlanMeta * 4);
+    const uint64_t o_queue = stream ? c.take(2 * cam::kStreamQueue * 4) : 0;
     const uint64_t o_sched1 = stream ? 0 : c.take(cam::sched_bytes(A, (int)Epr, (int)(2 * I)));
     const uint64_t o_sched2 = stream ? 0 : c.take(cam::sched_bytes(A, (int)Epr, (int)H));
     const uint64_t o_hist = c.take(cam::plan_workspace_bytes(T, K, (int)Epr));
@@ -1882,6 +1884,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         int32_t *pos = (int32_t *)(w + o_pos);
         int32_t *row = (int32_t *)(w + o_row);
         int32_t *meta = (int32_t *)(w + o_meta);
+        int32_t *queue = (int32_t *)(w + o_queue);
         int8_t *x1 = (int8_t *)(w + o_x1);
         float *x1s = (float *)(w + o_x1s);
         float *prod = (float *)(w + o_prod);
@@ -1900,6 +1903,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         p.dst_row = row;
         p.tokens_per_expert = etn;
         p.meta = meta;
+        p.stream_queues = stream ? queue : nullptr;
         p.hist_ws = (int32_t *)(w + o_hist);
         hipError_t e;
         cam::SchedSpec specs[2] = {sp1, sp2};  // both GEMM schedules come from the per-expert counts of the plan
@@ -1937,7 +1941,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         g1.gate_up = 1;
         g1.epilogue = cam::kEpiSwiglu;
         g1.out = prod;
-        e = layer_gemm(g1, etn, iE, A, iT, stream, s);
+        e = layer_gemm(g1, etn, iE, A, iT, stream, s, queue);
         if (e != hipSuccess) return e;
         if (!from_products) {
             e = cam::launch_requant(prod, A, iI, stream ? meta : specs[0].sched, x2, x2s, s);  // [1] of both: rows that exist
@@ -1958,7 +1962,7 @@ camStatus camFusedDeepMoeGetWorkspaceSize(const camTensor *x, const camTensor *e
         g2.epilogue = cam::kEpiDequantBf16;
         g2.out = y;
         g2.out_fp16 = x_is_fp16;
-        e = layer_gemm(g2, etn, iE, A, iT, stream, s, from_products ? prod : nullptr);
+        e = layer_gemm(g2, etn, iE, A, iT, stream, s, queue + cam::kStreamQueue, from_products ? prod : nullptr);
         if (e != hipSuccess) return e;
 
         cam::CombineArgs cb{};
@@ -2235,6 +2239,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
     const uint64_t o_row = c.take((uint64_t)A * 4);
     const uint64_t o_token = gather ? c.take((uint64_t)A * 4) : 0;
     const uint64_t o_meta = c.take(cam::kPlanMeta * 4);
+    const uint64_t o_queue = stream ? c.take(2 * cam::kStreamQueue * 4) : 0;
     const uint64_t o_sched1 = stream ? 0 : c.take(cam::sched_bytes(A, (int)E, (int)(2 * I)));
     const uint64_t o_sched2 = stream ? 0 : c.take(cam::sched_bytes(A, (int)E, (int)H));
     const uint64_t o_hist = c.take(cam::plan_workspace_bytes(T, K, (int)E));
@@ -2262,6 +2267,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         int32_t *pos = (int32_t *)(w + o_pos);
         int32_t *row = (int32_t *)(w + o_row);
         int32_t *meta = (int32_t *)(w + o_meta);
+        int32_t *queue = (int32_t *)(w + o_queue);
         uint8_t *x1 = (uint8_t *)(w + o_x1);
         uint8_t *x1s = (uint8_t *)(w + o_x1s);
         float *prod = (float *)(w + o_prod);
@@ -2280,6 +2286,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         p.dst_row = row;
         p.tokens_per_expert = etn;
         p.meta = meta;
+        p.stream_queues = stream ? queue : nullptr;
         p.hist_ws = (int32_t *)(w + o_hist);
         hipError_t e;
         cam::SchedSpec specs[2] = {sp1, sp2};
@@ -2317,7 +2324,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         g1.epilogue = cam::kEpiSwigluFp8;  // the SwiGLU product leaves GMM1 quantised for GMM2
         g1.out = x2;
         g1.out_scale8 = x2s;
-        e = layer_gemm(g1, etn, iE, A, iT, stream, s);
+        e = layer_gemm(g1, etn, iE, A, iT, stream, s, queue);
         if (e != hipSuccess) return e;
 
         cam::GemmArgs g2{};
@@ -2332,7 +2339,7 @@ camStatus camFusedDeepMoeFp8GetWorkspaceSize(const camTensor *x, const camTensor
         g2.gate_up = 0;
         g2.epilogue = cam::kEpiDequantBf16;
         g2.out = y;
-        e = layer_gemm(g2, etn, iE, A, iT, stream, s);
+        e = layer_gemm(g2, etn, iE, A, iT, stream, s, queue + cam::kStreamQueue);
         if (e != hipSuccess) return e;
 
         cam::CombineArgs cb{};

@@ -35,6 +35,9 @@ struct SchedItem {
 };
 // Run metadata the plan kernels leave for the kernels after them: {0, total rows, active tokens, 0}.
 constexpr int kPlanMeta = 4;
+// Queues of the streaming GEMMs of a layer: a count per GEMM and XCD, each on a line of its own, that the plan clears.
+constexpr int kStreamQueueStride = 32;
+constexpr int kStreamQueue = kNumXcd * kStreamQueueStride;  // ints of a GEMM
 
 // ---------------------------------------------------------------------------------------------
 // Routing plan: counts, offsets, within-expert ranks, receive bookkeeping, GEMM tile table.
@@ -53,6 +56,7 @@ struct PlanArgs {
     int64_t *group_list;      // [E]    optional cumulative rows, int64
     int64_t *total;           // [1]    optional
     int32_t *meta;            // optional run metadata, kPlanMeta ints (see above)
+    int32_t *stream_queues;   // optional: 2 * kStreamQueue ints to clear
     int32_t *hist_ws;         // required scratch of plan_workspace_bytes(T, K, E) bytes
 };
 uint64_t plan_workspace_bytes(int64_t T, int64_t K, int E);
@@ -209,6 +213,7 @@ struct StreamGemmArgs {
     int32_t *rows_out;          // optional: [1] receives the total row count (where launch_requant looks for it)
     const float *products;      // optional [max_rows,Kd], instead of g.a and g.a_scale: fp32 rows that the kernel quantises the
                                 // way launch_requant does, bit for bit (where stream_gemm_takes_products says so)
+    int32_t *queue;             // optional: kStreamQueue cleared ints, from which workgroups then take their items
     int lg_tile_rows;           // set by launch_stream_gemm
 };
 bool stream_gemm_applies(int64_t rows, int64_t N, int64_t G, bool fp8);  // whether it is the faster form

@@ -162,6 +162,7 @@ __global__ __launch_bounds__(NT) void dispatch_small_kernel(PlanArgs p, Dispatch
         }
         __syncthreads();
         write_expert_outputs<NT>(p, hist, t_active, tid, scan_s, &total_s);
+        clear_stream_queues(p, tid, NT);
         return;
     }
 

@@ -316,6 +316,7 @@ __global__ __launch_bounds__(kGlobalThreads) void plan_global_kernel(PlanArgs a,
     if (b != 0) {
         return;
     }
+    clear_stream_queues(a, tid, kGlobalThreads);
     if (tid < E) {
         if (a.cnt) a.cnt[tid] = cnt;
         if (a.off) a.off[tid] = off;
@@ -380,6 +381,9 @@ __global__ __launch_bounds__(kExpertThreads, 8) void plan_experts_kernel(PlanArg
             a.dst_row[i] = ids.off + rank;
         }
     });
+    if (x == a.E - 1) {
+        clear_stream_queues(a, tid, kExpertThreads);
+    }
     if (x == 0) {
         ids.of_no_expert(a.E, n_all, [&](int i) {
             a.pos[i] = -1;

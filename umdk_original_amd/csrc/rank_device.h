@@ -88,6 +88,16 @@ __device__ __forceinline__ void store_count(int64_t *p, int v)
     __hip_atomic_store(p, (int64_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// (at the end of a kernel: in front of a barrier the stores would be waited for)
+__device__ __forceinline__ void clear_stream_queues(const PlanArgs &a, int tid, int nthreads)
+{
+    if (a.stream_queues != nullptr) {
+        for (int i = tid; i < 2 * kStreamQueue; i += nthreads) {
+            a.stream_queues[i] = 0;
+        }
+    }
+}
+
 // Everything the plan says about the experts, from their complete counts cnt[0..E) (LDS), by one workgroup of NT >= 256
 // threads; leaves the exclusive offsets in cnt.
 template <int NT>

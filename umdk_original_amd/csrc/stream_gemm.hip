@@ -25,14 +25,17 @@
 //     that the fragment reads are free of bank conflicts.  The matrix cores are not what it waits for (without the
 //     multiplications the decode layer's launches take the same time).
 //   * No schedule: every workgroup derives the item list from the per-expert row counts by itself (a prefix sum over
-//     at most 512 experts) and takes items in a fixed order.  All items of a launch stream the same number of bytes,
-//     so nothing has to be balanced, and no builder runs before the GEMM.
+//     at most 512 experts), and no builder runs before the GEMM.  All items of a launch stream the same number of bytes, but
+//     workgroups do not get the same share of the memory: with all items dealt out beforehand the first was done after 172 us
+//     and the last after 250, 225 on average (1.6 GB, 6 items each).  In a layer whose items make four rounds and more
+//     the last quarter of the rounds is therefore taken from queues, and the items are smaller (StreamShape).
 //   * In a layer whose tiles are some ten thousand products each, the GMM2 launch quantises its activations itself (PRODUCTS):
 //     every workgroup reads the fp32 SwiGLU products of its tile, finds the row maxima and leaves the int8 rows in LDS while
 //     its first weights are on their way.  Column blocks repeat that work, but it is a microsecond or two of latency
 //     where a launch of requant_kernel takes 3.4 (layers: one token, H 4096, I 1536: 45.9 -> 44.1 us; 128 tokens on 8
 //     experts, H 1024, I 512: 26.3 -> 25.1).
 #include <algorithm>
+#include <cmath>
 
 #include "cam_device.h"
 #include "cam_kernels.h"
@@ -120,7 +123,8 @@ struct StreamItem {     // wave-uniform
     int wstep;          // bytes from one 64-byte K step to the next
 };
 
-template <int MF, bool FP8, int P, bool PRODUCTS>
+// QUEUED: sa.queue is set.
+template <int MF, bool FP8, int P, bool PRODUCTS, bool QUEUED>
 __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel(StreamGemmArgs sa)
 {
     typedef typename SAcc<FP8>::v16 acc16;
@@ -137,6 +141,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     __shared__ __attribute__((aligned(16))) float row_scale_s[2][FP8 ? 4 : 32 * MF];
     __shared__ __attribute__((aligned(16))) uint8_t a_scale8_s[2][FP8 ? kSMaxKb * 32 * MF : 4];
     __shared__ uint8_t w_scale8_s[FP8 ? 16 * kSMaxKb : 4];
+    __shared__ int next_s;   // QUEUED: the item after the next
     __shared__ float rowmax_s[FP8 ? 8 * 32 : PRODUCTS ? 8 : 1];
 
     const int tid = threadIdx.x;
@@ -159,6 +164,16 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     // rows of a tile: with products no more than a workgroup can quantise
     const int lg_rows = PRODUCTS && MF == 4 ? sa.lg_tile_rows : (MF == 1 ? 5 : 7);
     const int tile_rows = 1 << lg_rows;
+
+    // ---- the queues: one per XCD, for its eighth of the items beyond those dealt out; the count of items handed out is a device-scope
+    // atomic, a round trip to the memory side.  Wave 0 asks in front of an item's epilogue, for the item after the next: asked earlier, the
+    // wave's weights wait behind the answer (layer of 128 tokens 391 / 397 us).  With none left in its own, a workgroup takes from the queue
+    // with most.  It ends when all are empty, or seven others were quicker in a row: these ask again after their items, so no item is left.
+    // All rounds but the first from the queues instead of the last quarter: as fast or up to 2 us slower.
+    const int xcd = (int)blockIdx.x & (kNumXcd - 1);
+    auto ask = [&](int x) {
+        return lane == 0 ? __hip_atomic_fetch_add(sa.queue + x * kStreamQueueStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    };
 
     // ---- the item list: every expert's first row and the row tiles before it.  Every wave works it out for itself, a lane an
     // expert, and stores it: the same values into the same places, so that no wave waits for another before it knows its first
@@ -215,9 +230,39 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     // Workgroup i runs on XCD i % 8.  Every XCD has an eighth of the list to itself and its workgroups walk through it side by
     // side: the row tiles and column blocks of an expert meet in one L2 instead of being fetched by all eight (the decode
     // layer's GMM1, 1024 rows over 128 experts: 261 -> 252 us; 512 rows over 16 experts with 32-row tiles: 110 -> 99 us).
-    const int xcd = (int)blockIdx.x & (kNumXcd - 1);
-    const int end_item = (int)((long long)n_items * (xcd + 1) / kNumXcd);
-    const int item_step = ((int)gridDim.x - xcd + kNumXcd - 1) / kNumXcd;
+    auto first_of = [&](int x) { return (int)((long long)n_items * x / kNumXcd); };
+    const int end_item = QUEUED ? n_items : first_of(xcd + 1);
+    const int item_step = (int)gridDim.x / kNumXcd;   // workgroups of an XCD
+    const int dealt = max(n_items / (int)gridDim.x * 3 / 4, 1);   // rounds of items that are a workgroup's without asking
+    const int dealt_items = dealt * item_step;
+    auto take = [&](int asked) -> int {
+        int i = first_of(xcd) + dealt_items + __builtin_amdgcn_readfirstlane(asked);
+        if (i < first_of(xcd + 1)) {
+            return i;
+        }
+        for (int tries = 0; tries < 7; ++tries) {
+            int left = 0;
+            if (lane < kNumXcd) {
+                left = first_of(lane + 1) - first_of(lane) - dealt_items -
+                       __hip_atomic_load(sa.queue + lane * kStreamQueueStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            int most = 0, x = 0;
+#pragma unroll
+            for (int q = 0; q < kNumXcd; ++q) {
+                const int l = __builtin_amdgcn_readlane(left, q);
+                x = l > most ? q : x;
+                most = max(most, l);
+            }
+            if (most == 0) {
+                break;
+            }
+            i = first_of(x) + dealt_items + __builtin_amdgcn_readfirstlane(ask(x));
+            if (i < first_of(x + 1)) {
+                return i;
+            }
+        }
+        return n_items;
+    };
     auto find_item = [&](int i) -> StreamItem {
         StreamItem it;
         it.g = 0; it.row0 = 0; it.rows = 0; it.blk = 0; it.ckb = quantum; it.nch = 1; it.w = nullptr; it.wstep = 0;
@@ -433,8 +478,8 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
 
     int set = 0;  // the set of scales in use, one per item in turn
     int buf = 0;  // the activation buffer in use; chunks take turns, across items too
-    int item = (int)((long long)n_items * xcd / kNumXcd) + (int)blockIdx.x / kNumXcd;
-    StreamItem cur = find_item(item);
+    int item = first_of(xcd) + (int)blockIdx.x / kNumXcd;
+    StreamItem cur = find_item(QUEUED && item >= first_of(xcd + 1) ? n_items : item);
     if (cur.rows <= 0) {
         return;
     }
@@ -451,12 +496,18 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     if constexpr (PRODUCTS) {
         quantise_products(cur, 0, 0);
     }
+    if (QUEUED && dealt == 1 && wave == 0) {
+        const int i = take(ask(xcd));
+        if (lane == 0) {
+            next_s = i;
+        }
+    }
     store_scales(cur, 0);
     a_landed();
     lds_barrier();
 
-    for (;;) {
-        item += item_step;
+    for (int turn = 0;; ++turn) {
+        item = QUEUED && turn + 1 >= dealt ? __builtin_amdgcn_readfirstlane(next_s) : item + item_step;
         StreamItem nxt{};   // PRODUCTS: a workgroup has one item
         if constexpr (!PRODUCTS) {
             nxt = find_item(item);
@@ -561,6 +612,11 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
         const int piece = lane & 7;
         const int I = N >> 1;
         const bool swiglu = a.epilogue != kEpiDequantBf16;
+        const bool asks = QUEUED && more && wave == 0 && turn + 2 >= dealt;
+        int asked = 0;
+        if (asks) {
+            asked = ask(xcd);
+        }
 #pragma unroll
         for (int mf = 0; mf < MF; ++mf) {
             if (mf > 0 && mf * 32 >= cur.rows) {   // no such rows (cur.rows is the same in every wave)
@@ -712,6 +768,12 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
         if (!more) {
             return;
         }
+        if (asks) {
+            const int i = take(asked);
+            if (lane == 0) {
+                next_s = i;
+            }
+        }
         store_scales(nxt, set ^ 1);
         lds_barrier();  // the partial sums have been read, the next item's scales are in place
         buf ^= 1;
@@ -720,17 +782,19 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     }
 }
 
-template <int MF, bool FP8, int P, bool PRODUCTS = false>
+template <int MF, bool FP8, int P, bool PRODUCTS = false, bool QUEUED = false>
 void launch_kernel(unsigned grid, hipStream_t stream, const StreamGemmArgs &sa)
 {
-    hipLaunchKernelGGL((stream_gemm_kernel<MF, FP8, P, PRODUCTS>), dim3(grid), dim3(kSThreads), 0, stream, sa);
+    hipLaunchKernelGGL((stream_gemm_kernel<MF, FP8, P, PRODUCTS, QUEUED>), dim3(grid), dim3(kSThreads), 0, stream, sa);
 }
 
 template <bool FP8>
-void launch_variant(int mf, int P, unsigned grid, hipStream_t stream, const StreamGemmArgs &sa)
+void launch_variant(int mf, int P, bool queued, unsigned grid, hipStream_t stream, const StreamGemmArgs &sa)
 {
     if (mf == 1) {
         P == 1 ? launch_kernel<1, FP8, 1>(grid, stream, sa) : launch_kernel<1, FP8, 2>(grid, stream, sa);
+    } else if (queued) {
+        P == 2 ? launch_kernel<4, FP8, 2, false, true>(grid, stream, sa) : launch_kernel<4, FP8, 4, false, true>(grid, stream, sa);
     } else if (P == 2) {
         launch_kernel<4, FP8, 2>(grid, stream, sa);
     } else {
@@ -743,29 +807,47 @@ struct StreamShape {
     int P;           // column groups per item
     long long items; // at most
     unsigned grid;
+    bool queued;     // items come from queues, if there are any
 };
 
-StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool quad, int64_t rows_per_expert, int cus)
+// `products`: for a launch that takes them (an item to a workgroup).
+StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool quad, bool products, int64_t rows_per_expert, int cus)
 {
     StreamShape sh;
     // live experts at most, and the column groups they stream
     const long long live = std::min<long long>(G, max_rows);
     const long long groups = live * (N / 64);
     const bool many = groups >= 6ll * cus;
+    // of items that the rows make, spread over the experts
+    const double reached = (double)G * (1.0 - std::pow(1.0 - 1.0 / (double)G, (double)max_rows));
+    auto rounds = [&](int P) { return reached * ((N / 64 + P - 1) / P) / cus; };
     // 32-row tiles, two workgroups per CU, while the stream is short: few column groups and no expert with more rows, or
     // all tiles resident at once.  Otherwise 128-row tiles, so that an expert's weights are read once.
     sh.small = !quad && ((rows_per_expert <= 32 && !many) || groups + max_rows / 32 * (N / 64) <= 2ll * cus);
-    // Column groups per item: as few as it takes to give every CU work, then up to a megabyte of weights per item (an
-    // item's sums and stores interrupt its stream for about two microseconds).  kEpiSwigluFp8 needs the four groups
-    // of a 128-column block together, and the fp32 products of kEpiSwiglu are the same sums in the same order (quad).
+    // Column groups per item: as few as it takes to give every CU work, then as many as make an item of about half a megabyte of
+    // weights (its sums and stores interrupt its stream for about two microseconds, and smaller items end together).
+    // kEpiSwigluFp8 needs the four groups of a 128-column block together, and the fp32 products of kEpiSwiglu are the same
+    // sums in the same order (quad).  us per layer, with up to a megabyte and no queues / this; T x H, top-K of E, I:
+    //   K over 2560 (4 / 2 groups from queues): 128 x 4096, 8 of 128, 1536 393 / 388, 64 x 3072, 6 of 128, 1536 266 / 251, 48 x 7168, 8 of 64, 2048
+    //   464 / 451; without queues 2 groups lose (400 in the first), and 24 x 4096, 8 of 128, 1536 gives 250 / 253;
+    //   K to 2560 (8 / 4): 200 x 2048, 4 of 64, 1408 139 / 131 (GMM1), 100 x 4096, 8 of 64, 2048 290 / 278 (GMM2), 500 x 1536, 2 of 64, 3072 level;
+    //   K to 1536 (8 / 4): 90 x 5120, 6 of 160, 1536, ten rounds and more 519 / 512, 64 x 5120, 6 of 32, 1536, little more than one of 8 groups
+    //   157 / 150; in between, 64 x 4096, 8 of 128, 1536, 359 / 363, and at K 512 116 / 119, so these stay;
+    //   quad, K to 2048 (8 / 4): 200 x 2048, 4 of 64, 1408 133 / 124, 700 x 1024, 8 of 256, 512 130 / 125; 4 from queues: 48 x 4096, 8 of 128, 1536 342 / 335,
+    //   256 432 / 423, level at four rounds.  More rows make sums that several waves share dearer: 500 x 2048, 8 of 128, 768 166 / 170.
     sh.P = 2;
     if (sh.small) {
         sh.P = 2 * groups >= 3ll * cus ? 2 : 1;
-    } else if (many) {
+    } else if (products) {
         sh.P = 512ll * Kd <= (1 << 20) ? 8 : 4;
     } else if (quad) {
-        sh.P = 4;
+        sh.P = many && Kd <= 2048 && max_rows > 24 * G ? 8 : 4;
+    } else if (many && Kd > 2560) {
+        sh.P = rounds(2) >= 7 ? 2 : 4;
+    } else if (many) {
+        sh.P = Kd > 1536 || (Kd > 1024 && rounds(8) < 1.3) || (Kd >= 1024 && rounds(4) >= 10) ? 4 : 8;
     }
+    sh.queued = many && !sh.small && !products && sh.P <= 4 && rounds(sh.P) >= 4;
     const long long tiles = live + max_rows / (sh.small ? 32 : 128);
     sh.items = tiles * ((N / 64 + sh.P - 1) / sh.P);
     // a multiple of eight workgroups: every XCD takes an eighth of the items
@@ -826,7 +908,7 @@ bool stream_gemm_takes_products(int64_t max_rows, int G, int Kd, int N, int64_t 
     if (max_rows <= 0 || G <= 0 || gemm_workgroups(&cus) != hipSuccess) {
         return false;
     }
-    const StreamShape sh = stream_shape(G, max_rows, Kd, N, false, rows_per_expert, cus);
+    const StreamShape sh = stream_shape(G, max_rows, Kd, N, false, true, rows_per_expert, cus);
     const int lg = lg_product_rows(sh, max_rows, Kd);
     if (lg < 0) {
         return false;
@@ -857,7 +939,8 @@ hipError_t launch_stream_gemm(const StreamGemmArgs &sa, int64_t rows_per_expert,
     if (e != hipSuccess) {
         return e;
     }
-    const StreamShape sh = stream_shape(sa.G, sa.max_rows, g.Kd, g.N, g.fp8 && g.gate_up, rows_per_expert, cus);
+    const StreamShape sh = stream_shape(sa.G, sa.max_rows, g.Kd, g.N, g.fp8 && g.gate_up, sa.products != nullptr, rows_per_expert, cus);
+    const bool queued = sh.queued && sa.queue != nullptr;
     if (sa.products != nullptr) {
         const int lg = lg_product_rows(sh, sa.max_rows, g.Kd);
         if (g.fp8 || g.gate_up || lg < 0) {
@@ -875,9 +958,9 @@ hipError_t launch_stream_gemm(const StreamGemmArgs &sa, int64_t rows_per_expert,
             launch_kernel<4, false, 8, true>(grid, stream, sp);
         }
     } else if (g.fp8) {
-        launch_variant<true>(sh.small ? 1 : 4, sh.P, sh.grid, stream, sa);
+        launch_variant<true>(sh.small ? 1 : 4, sh.P, queued, sh.grid, stream, sa);
     } else {
-        launch_variant<false>(sh.small ? 1 : 4, sh.P, sh.grid, stream, sa);
+        launch_variant<false>(sh.small ? 1 : 4, sh.P, queued, sh.grid, stream, sa);
     }
     return hipGetLastError();
 }
