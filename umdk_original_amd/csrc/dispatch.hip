@@ -39,6 +39,22 @@ __device__ __forceinline__ long long dispatch_row(const DispatchArgs &a, int t, 
     return pre + (window_row - a.recv_offset[e]);
 }
 
+// The output rows of a token's copies, that of copy k in lane k: all of them in one round trip, in front of the token's own row.  Asked
+// for one by one, each waits for the stores of the copy before (see asks_one_by_one).  us, plan and permute replayed from a graph, one by one
+// with the triples of lane 0 / this: 1999 x 4096, int8, 6 of 64 18.1 / 17.4, 2048 x 7168, 8 of 64 33.3 / 32.6, 5000 x 2048, FP8 37.3 / 35.7; 16-bit
+// rows 1999 x 4096 24.0 / 23.8.
+__device__ __forceinline__ long long own_row(const DispatchArgs &a, int t, int lane)
+{
+    const long long row = lane < a.K ? dispatch_row(a, t, lane) : -1;
+    return row < a.A ? row : -1;
+}
+
+__device__ __forceinline__ long long row_of_lane(long long own, int k)
+{
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)own, k), hi = __builtin_amdgcn_readlane((unsigned)((unsigned long long)own >> 32), k);
+    return (long long)((unsigned long long)hi << 32 | lo);
+}
+
 // How the rows are stored.  Plain stores leave the L2 (32 MB) in a better order than the waves wrote the pieces of far apart rows in,
 // and a reader that goes through the rows once finds more of them in the memory-side cache.  But what still lies in the L2 at the
 // end of the launch has to be written back before the next one, which costs more than it gains while that is most of the
@@ -62,27 +78,37 @@ bool stores_plainly(const DispatchArgs &a)
     return a.quant == 0 && bytes >= 72ll << 20;
 }
 
+// Whether a wave asks for the row of a copy behind the stores of the copy before, which spaces its stores out: very many 8-bit rows
+// lie in memory faster then, although a wave takes longer.  us, plan and permute replayed from a graph, all at once / one by one, T x H, top-K of E:
+// int8 235 MB 4096 x 7168, 8 of 256 68.1 / 64.1, 192 MB 8000 x 3000, 8 of 512 62.1 / 58.0, 172 MB 3000 x 7168, 8 of 64 50.1 / 48.3, but 131 MB 8000 x
+// 4096, 4 of 64 47.4 / 48.5, 117 MB 2048 x 7168, 8 of 64 32.4 / 33.4, 86 MB 1500 25.0 / 25.8, 12 MB 1000 x 2048, 6 of 64 10.1 / 10.3; FP8 235 MB 69.3 / 68.2;
+// 16-bit rows level, 470 MB 95.4 / 95.3.  (A wait for the stores alone does not help: 68.7 in the first.)
+bool asks_one_by_one(const DispatchArgs &a) { return a.quant != 0 && (long long)a.T * a.K * a.H >= 152ll << 20; }
+
 // Four workgroups per CU (128 registers a lane) keep all 1024 workgroups of a 4096-token batch resident at once;
 // the FP8 variant would spill at that size and stays at three.
 template <int QUANT, int ACT, bool PLAIN>
-__global__ __launch_bounds__(kDispWaves * kWave, QUANT == 3 ? 3 : 4) void dispatch_kernel(DispatchArgs a)
+__global__ __launch_bounds__(kDispWaves * kWave, QUANT == 3 ? 3 : 4) void dispatch_kernel(DispatchArgs a, bool one_by_one)
 {
-    const int t = (int)blockIdx.x * kDispWaves + (threadIdx.x >> 6);
+    const int t = (int)blockIdx.x * kDispWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & (kWave - 1);
     if (t >= a.T) {
         return;
     }
+    const long long own = own_row(a, t, lane);
     WaveRow r;
     load_token_row(a.x, t, a.H, lane, r);
     if (QUANT != 0) {
         quant_token_row<QUANT, ACT>(r, WaveMax());
     }
     for (int k = 0; k < a.K; ++k) {
-        const long long row = dispatch_row(a, t, k);
-        if (row < 0 || row >= a.A) {
-            continue;
+        const long long row = one_by_one ? dispatch_row(a, t, k) : row_of_lane(own, k);
+        if (row >= 0 && row < a.A) {
+            store_token_row<QUANT, PLAIN>(r, a.out, a.scales, row, a.H, lane);
         }
-        store_token_row<QUANT, PLAIN>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, lane);
+    }
+    if (own >= 0) {
+        store_row_origin<QUANT>(r.scale_out, a.scales, a.src_info, a.src_rank, own, t, lane);
     }
 }
 
@@ -92,21 +118,26 @@ __global__ __launch_bounds__(kDispWaves * kWave, QUANT == 3 ? 3 : 4) void dispat
 template <int ACT, bool PLAIN>
 __global__ __launch_bounds__(kDispWaves * kWave) void dispatch_smooth_kernel(DispatchArgs a)
 {
-    const int t = (int)blockIdx.x * kDispWaves + (threadIdx.x >> 6);
+    const int t = (int)blockIdx.x * kDispWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & (kWave - 1);
     if (t >= a.T) {
         return;
     }
+    const long long own = own_row(a, t, lane);
+    const int own_id = lane < a.K ? a.idx[(long long)t * a.K + lane] : -1;
     WaveRow r;
     load_token_row(a.x, t, a.H, lane, r);
     for (int k = 0; k < a.K; ++k) {
-        const long long row = dispatch_row(a, t, k);
-        const int e = a.idx[(long long)t * a.K + k];
-        if (row < 0 || row >= a.A || e < 0 || e >= a.E) {
+        const long long row = row_of_lane(own, k);
+        const int e = __builtin_amdgcn_readlane(own_id, k);
+        if (row < 0 || e < 0 || e >= a.E) {
             continue;
         }
         quant_token_row_smooth<ACT>(r, a.smooth + (long long)e * a.H, a.H, lane, WaveMax());
-        store_token_row<2, PLAIN>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, lane);
+        store_token_row<2, PLAIN>(r, a.out, a.scales, row, a.H, lane);
+        if (lane == 0) {
+            store_row_origin<2>(r.scale_out, a.scales, a.src_info, a.src_rank, row, t, k);
+        }
     }
 }
 
@@ -116,6 +147,7 @@ __global__ __launch_bounds__(kDispWaves * kWave) void dispatch_smooth_kernel(Dis
 // T * K ids (counted with ballots) gives the rows and the ranks of the K entries with no table, no scan and nothing to
 // wait for from another workgroup.  Workgroup 0 counts for the per-expert outputs.  With few tokens the latency of one
 // row is what the launch takes, so it is spread over sixteen waves (four from 257 tokens on) instead of one.
+// The triples and scales of a token's copies are stored at once, a lane each (by one thread 128 x 7168, 8 of 256 6.40 -> 6.12, 300 x 4096 8.64 -> 8.31).
 // Launches: one token x 4096 to 128 experts, top-8: 3.5 + 7.4 us -> 5.9; 64 x 4096 FP8: 6.2 + 15.6 -> 7.4; 128 x 7168 to 256
 // experts: 6.1 + 9.8 -> 7.8.
 // What bounds it beside the latencies is the counting, top-k times over a thread's ids, so an id is compared twice a time and with
@@ -239,7 +271,13 @@ __global__ __launch_bounds__(NT) void dispatch_small_kernel(PlanArgs p, Dispatch
             const int e = __builtin_amdgcn_readlane(own_ids, k);
             quant_token_row_smooth<ACT>(r, a.smooth + (long long)e * a.H, a.H, tid, GroupMax<NT>{max_s});
         }
-        store_token_row<QUANT, false>(r, a.out, a.scales, a.src_info, a.src_rank, row, t, k, a.H, tid);
+        store_token_row<QUANT, false>(r, a.out, a.scales, row, a.H, tid);
+        if (SMOOTH && tid == 0) {
+            store_row_origin<QUANT>(r.scale_out, a.scales, a.src_info, a.src_rank, row, t, k);
+        }
+    }
+    if (!SMOOTH && tid < K && row_s[tid] >= 0 && row_s[tid] < a.A) {
+        store_row_origin<QUANT>(r.scale_out, a.scales, a.src_info, a.src_rank, row_s[tid], t, tid);
     }
 }
 
@@ -281,7 +319,7 @@ template <bool PLAIN>
 void launch_dispatch_as(const DispatchArgs &a, hipStream_t stream)
 {
     const dim3 grid((a.T + kDispWaves - 1) / kDispWaves), block(kDispWaves * kWave);
-    const bool fp16 = a.x_is_fp16 != 0;
+    const bool fp16 = a.x_is_fp16 != 0, paced = asks_one_by_one(a);
     if (a.smooth != nullptr) {
         if (fp16) {
             hipLaunchKernelGGL((dispatch_smooth_kernel<1, PLAIN>), grid, block, 0, stream, a);
@@ -289,24 +327,24 @@ void launch_dispatch_as(const DispatchArgs &a, hipStream_t stream)
             hipLaunchKernelGGL((dispatch_smooth_kernel<0, PLAIN>), grid, block, 0, stream, a);
         }
     } else if (a.quant == 0) {
-        hipLaunchKernelGGL((dispatch_kernel<0, 0, PLAIN>), grid, block, 0, stream, a);  // a copy does not look at the format
+        hipLaunchKernelGGL((dispatch_kernel<0, 0, PLAIN>), grid, block, 0, stream, a, paced);  // a copy does not look at the format
     } else if (a.quant == 1) {
         if (fp16) {
-            hipLaunchKernelGGL((dispatch_kernel<1, 1, PLAIN>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((dispatch_kernel<1, 1, PLAIN>), grid, block, 0, stream, a, paced);
         } else {
-            hipLaunchKernelGGL((dispatch_kernel<1, 0, PLAIN>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((dispatch_kernel<1, 0, PLAIN>), grid, block, 0, stream, a, paced);
         }
     } else if (a.quant == 3) {  // (whole lines: never plainly)
         if (fp16) {
-            hipLaunchKernelGGL((dispatch_kernel<3, 1, false>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((dispatch_kernel<3, 1, false>), grid, block, 0, stream, a, paced);
         } else {
-            hipLaunchKernelGGL((dispatch_kernel<3, 0, false>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((dispatch_kernel<3, 0, false>), grid, block, 0, stream, a, paced);
         }
     } else {
         if (fp16) {
-            hipLaunchKernelGGL((dispatch_kernel<2, 1, PLAIN>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((dispatch_kernel<2, 1, PLAIN>), grid, block, 0, stream, a, paced);
         } else {
-            hipLaunchKernelGGL((dispatch_kernel<2, 0, PLAIN>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((dispatch_kernel<2, 0, PLAIN>), grid, block, 0, stream, a, paced);
         }
     }
 }
@@ -335,7 +373,7 @@ hipError_t launch_dispatch(const DispatchArgs &a, hipStream_t stream)
     if (a.T <= 0) {
         return hipSuccess;
     }
-    if (a.H % 8 != 0 || a.H / 8 > kDispMaxChunks * kWave || (a.quant == 3 && a.H % 128 != 0)) {
+    if (a.H % 8 != 0 || a.H / 8 > kDispMaxChunks * kWave || (a.quant == 3 && a.H % 128 != 0) || a.K > kMaxTopk) {
         return hipErrorInvalidValue;
     }
     if (a.smooth != nullptr && (a.quant != 2 || a.idx == nullptr)) {

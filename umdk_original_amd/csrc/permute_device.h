@@ -271,10 +271,23 @@ __device__ __forceinline__ void store_piece(T v, T *dst)
     }
 }
 
-// Stores the row (quantised or raw) to output row `row`, with its scale and triple.
+// The scale (of int8 rows) and the triple of output row `row`.
+template <int QUANT>
+__device__ __forceinline__ void store_row_origin(float scale, float *scales, int32_t *src_info, int src_rank, long long row, int t, int k)
+{
+    if (QUANT == 1 || QUANT == 2) {
+        scales[row] = scale;
+    }
+    if (src_info != nullptr) {
+        src_info[3 * row + 0] = src_rank;
+        src_info[3 * row + 1] = t;
+        src_info[3 * row + 2] = k;
+    }
+}
+
+// Stores the row (quantised or raw) to output row `row`, with the scales of an FP8 row.
 template <int QUANT, bool PLAIN, typename Row>
-__device__ __forceinline__ void store_token_row(const Row &r, void *out, float *scales, int32_t *src_info,
-                                                int src_rank, long long row, int t, int k, int H, int lane)
+__device__ __forceinline__ void store_token_row(const Row &r, void *out, float *scales, long long row, int H, int lane)
 {
     const int nch = H >> 3;
     if (QUANT != 0) {
@@ -298,16 +311,6 @@ __device__ __forceinline__ void store_token_row(const Row &r, void *out, float *
     }
     if (QUANT == 3) {
         store_row_scales8(r, (uint8_t *)scales, row, H, lane);
-    }
-    if (lane == 0) {
-        if (QUANT == 1 || QUANT == 2) {
-            scales[row] = r.scale_out;
-        }
-        if (src_info != nullptr) {
-            src_info[3 * row + 0] = src_rank;
-            src_info[3 * row + 1] = t;
-            src_info[3 * row + 2] = k;
-        }
     }
 }
 
