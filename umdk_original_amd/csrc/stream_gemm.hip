@@ -832,7 +832,8 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     //   464 / 451; without queues 2 groups lose (400 in the first), and 24 x 4096, 8 of 128, 1536 gives 250 / 253;
     //   K to 2560 (8 / 4): 200 x 2048, 4 of 64, 1408 139 / 131 (GMM1), 100 x 4096, 8 of 64, 2048 290 / 278 (GMM2), 500 x 1536, 2 of 64, 3072 level;
     //   K to 1536 (8 / 4): 90 x 5120, 6 of 160, 1536, ten rounds and more 519 / 512, 64 x 5120, 6 of 32, 1536, little more than one of 8 groups
-    //   157 / 150; in between, 64 x 4096, 8 of 128, 1536, 359 / 363, and at K 512 116 / 119, so these stay;
+    //   157 / 150, six rounds of a dozen rows per expert (FP8, to which int8 of so many rows does not come here) 256 x 4096, 8 of 128, 1536 422 / 409,
+    //   700 x 2048, 8 of 256, 1024 337 / 326; in between, 64 x 4096, 8 of 128, 1536, 359 / 363, and at K 512 116 / 119, so these stay;
     //   quad, K to 2048 (8 / 4): 200 x 2048, 4 of 64, 1408 133 / 124, 700 x 1024, 8 of 256, 512 130 / 125; 4 from queues: 48 x 4096, 8 of 128, 1536 342 / 335,
     //   256 432 / 423, level at four rounds.  More rows make sums that several waves share dearer: 500 x 2048, 8 of 128, 768 166 / 170.
     sh.P = 2;
@@ -845,7 +846,7 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     } else if (many && Kd > 2560) {
         sh.P = rounds(2) >= 7 ? 2 : 4;
     } else if (many) {
-        sh.P = Kd > 1536 || (Kd > 1024 && rounds(8) < 1.3) || (Kd >= 1024 && rounds(4) >= 10) ? 4 : 8;
+        sh.P = Kd > 1536 || (Kd > 1024 && rounds(8) < 1.3) || (Kd >= 1024 && (rounds(4) >= 10 || (rounds(4) >= 6 && max_rows >= 12 * G))) ? 4 : 8;
     }
     sh.queued = many && !sh.small && !products && sh.P <= 4 && rounds(sh.P) >= 4;
     const long long tiles = live + max_rows / (sh.small ? 32 : 128);
