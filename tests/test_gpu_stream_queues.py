@@ -117,6 +117,19 @@ def test_replays(gpu):
         _check(False, E, w, x, ids, gates, got)
 
 
+@pytest.mark.parametrize("H,E,I,up", [(5120, 44, 1536, 2), (5120, 48, 1536, 4), (4096, 40, 1280, 4)])
+def test_groups_of_two_rounds(gpu, H, E, I, up):
+    """Column groups of an item where there are one to two rounds of four, K over 4096 and not, and the layer with them."""
+    T, K = 40, 6
+    announce("two rounds H=%d E=%d I=%d" % (H, E, I))
+    w = _weights(gpu, False, E, H, I)
+    x, gates = torch.randn(T, H, device=gpu).to(torch.bfloat16), torch.rand(T, K, device=gpu)
+    ids = _ids(gpu, "uneven", T, E, K, E)
+    _check(False, E, w, x, ids, gates, _layer(False, E, w, x, ids, gates))
+    gemm = [n for n in recorded_names(lambda: _layer(False, E, w, x, ids, gates)) if "stream_gemm_kernel" in n][0]
+    assert "stream_gemm_kernelILi4ELb0ELi%dELb0E" % up in gemm
+
+
 @pytest.mark.parametrize("T,H,E,K,I,up,down", [(64, 3072, 128, 6, 1536, 2, 0), (4, 3072, 128, 6, 1536, 0, 0),    # few experts reached
                                                (64, 2560, 128, 6, 2048, 4, 4), (64, 2560, 60, 6, 2048, 0, 0),    # rounds of items
                                                (64, 1536, 128, 6, 2048, 0, 0), (90, 5120, 160, 6, 1536, 2, 4)])

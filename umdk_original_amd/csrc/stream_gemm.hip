@@ -830,6 +830,8 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     // sums in the same order (quad).  us per layer, with up to a megabyte and no queues / this; T x H, top-K of E, I:
     //   K over 2560 (4 / 2 groups from queues): 128 x 4096, 8 of 128, 1536 393 / 388, 64 x 3072, 6 of 128, 1536 266 / 251, 48 x 7168, 8 of 64, 2048
     //   464 / 451; without queues 2 groups lose (400 in the first), and 24 x 4096, 8 of 128, 1536 gives 250 / 253;
+    //   K over 4096, little more than one round of 4 groups (4 / 2): 30 x 5120, 6 of 44, 1536 201 / 181, 40 x 6144, 4 of 40, 1280 161 / 146, 12 x 7168, 4 of
+    //   24, 2048 161 / 146, two rounds 128 x 7168, 4 of 32, 2048 262 / 258; at 4096 40 tokens, 4 of 40, 1280 116 / 108, but 60, 2 of 36, 1408 124 / 131;
     //   K to 2560 (8 / 4): 200 x 2048, 4 of 64, 1408 139 / 131 (GMM1), 100 x 4096, 8 of 64, 2048 290 / 278 (GMM2), 500 x 1536, 2 of 64, 3072 level;
     //   K to 1536 (8 / 4): 90 x 5120, 6 of 160, 1536, ten rounds and more 519 / 512, 64 x 5120, 6 of 32, 1536, little more than one of 8 groups
     //   157 / 150, six rounds of a dozen rows per expert (FP8, to which int8 of so many rows does not come here) 256 x 4096, 8 of 128, 1536 422 / 409,
@@ -844,7 +846,7 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     } else if (quad) {
         sh.P = many && Kd <= 2048 && max_rows > 24 * G ? 8 : 4;
     } else if (many && Kd > 2560) {
-        sh.P = rounds(2) >= 7 ? 2 : 4;
+        sh.P = rounds(2) >= 7 || (Kd > 4096 && rounds(4) < 2.2) ? 2 : 4;
     } else if (many) {
         sh.P = Kd > 1536 || (Kd > 1024 && rounds(8) < 1.3) || (Kd >= 1024 && (rounds(4) >= 10 || (rounds(4) >= 6 && max_rows >= 12 * G))) ? 4 : 8;
     }
