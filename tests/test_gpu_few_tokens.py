@@ -69,7 +69,7 @@ def test_masks_dropped_ids_and_weights_per_expert(gpu, oracle, active):
 
 @pytest.mark.parametrize("T,H,E,K,I,few", [(1, 512, 4, 8, 3072, True), (8, 1024, 4, 1, 512, True), (9, 1024, 4, 1, 512, False),
                                            (2, 768, 32, 4, 3072, False), (8, 896, 32, 1, 3072, False), (4, 512, 32, 2, 2560, False),
-                                           (1, 640, 32, 8, 3072, True), (8, 1536, 32, 1, 3072, True), (8, 896, 32, 1, 2048, True),
+                                           (1, 640, 32, 8, 3072, True), (8, 1536, 32, 1, 3072, True), (8, 896, 32, 1, 2048, True), (8, 768, 8, 1, 3072, True),
                                            (8, 6144, 4, 1, 512, True), (8, 6272, 4, 1, 512, False),
                                            (2, 1024, 8, 8, 1024, True), (2, 1024, 8, 8, 1152, False),
                                            (4, 4096, 64, 8, 512, True), (4, 4096, 63, 8, 512, False), (4, 3968, 64, 8, 512, False),

@@ -625,7 +625,7 @@ bool few_tokens_valid(const FewTokensArgs &a)
 }  // namespace
 
 // Up to eight slots of one token always, of more tokens while their products, which each of the down launch's workgroups quantises first, are
-// not too many for the output columns it has; up to sixteen, and 32 of few tokens, where the down launch, whose workgroups are one for 16
+// not too many for the output columns it has, or where there are so few experts that several slots name one; up to sixteen, and 32 of few tokens, where the down launch, whose workgroups are one for 16
 // output columns, has enough of them for the length of its rows, and where the slots name different experts (a gate/up workgroup is
 // one expert's, and quantises all of its tokens).  us per layer, four launches or five / these two;
 // T x H, top-K of E, I: 1 x 4096, 8 of 128, 1536 43.0 / 32.0; 1 x 4096, 1 of 128, 1536 24.8 / 11.0; 1 x 7168, 8 of 64, 2048 74.6 / 62.3; 1 x 512, 8
@@ -637,6 +637,7 @@ bool few_tokens_valid(const FewTokensArgs &a)
 // Eight slots of few output columns (replayed from a graph), I 3072: 512 1 x 8 28.4 / 29.2, 2 x 4 26.6 / 30.3, 8 x 1 25.6 / 29.1; 768 1 x 8 30.7 / 30.5, 2 x 4
 // 29.2 / 30.4, 8 x 1 28.0 / 29.5; 1024 8 x 1 30.0 / 31.3; 1152 8 x 1 31.9 / 31.0; 2560: 512 8 x 1 24.8 / 26.3, 768 8 x 1 26.7 / 25.9; 2048: 512 2 x 4
 // 23.4 / 22.5; six slots 2 x 3 of 512, 3072 26.0 / 25.1.
+// That was 48 experts; 8 x 512, top-1, 3072 of 8 23.9 / 22.7, of 12 23.8 / 23.1, of 16 25.5 / 26.9, 2 x 512, top-4, of 8 25.6 / 24.9, of 12 25.9 / 27.2, of 16 26.4 / 27.0.
 // FP8 up to sixteen slots: 1 x 4096, 8 of 128, 1536 49.2 / 34.3, 1 of 128 38.0 / 12.7, 1 x 7168, 8 of 64, 2048 82.3 / 62.8, 2 x 4096, 8 of 64, 1536 62.7 /
 // 59.4 (the same 52.2 / 39.3), 2 x 7168, 8 of 64, 2048 127.8 / 124.2, 4 x 4096, 4 of 8, 1024 42.9 / 28.5, 2 x 1024, 8 of 64, 768 28.9 / 26.0, 1 x 1024, 8
 // of 64, 2048 28.5 / 24.3; not 1 x 1024, 8 of 64, 3072 32.1 / 33.2, 2 x 1024, 8 of 64, 1024 28.7 / 29.7, 2 x 2048, 6 of 64, 2048 39.8 / 43.0, 5 x 4096,
@@ -652,7 +653,7 @@ bool few_tokens_apply(int64_t T, int64_t K, int64_t E, int64_t H, int64_t I, boo
         return slots <= 8 ? slots * I <= 16 * H : slots <= 16 && (slots * I <= 7 * H || slots * I <= 12288);
     }
     if (slots <= 8) {
-        return T == 1 || slots * I <= 12288 + 11 * H;
+        return T == 1 || slots * I <= 12288 + 11 * H || 2 * E <= 3 * slots;
     }
     return slots * I <= 16 * H && (slots <= 16 || (T <= 4 && H >= 4096 && E >= 2 * slots));
 }
