@@ -1,7 +1,7 @@
 """Layers whose streaming GEMMs take their last items from queues: every bit as the operators one by one give it, whose items are all
 dealt out beforehand.  Spread and uneven ids, ids that leave most queues empty (fewer items than workgroups), dropped ids, inactive
 tokens, column groups that do not fill the last block; replays of a graph with other ids in between, so the counts are those of the
-replay; and which GEMMs there are queues for."""
+replay; and which GEMMs there are queues for, and how wide their items are without."""
 import pytest
 import torch
 
@@ -87,6 +87,7 @@ def test_layer_as_its_operators(gpu, fp8, shape):
         _check(fp8, E, w, x, ids, gates, _layer(fp8, E, w, x, ids, gates))
     names = recorded_names(lambda: _layer(fp8, E, w, x, ids, gates))
     gemms = [n for n in names if "stream_gemm_kernel" in n]
+    assert len(gemms) == 2
     assert [_queued(fp8, p) in n if p else "ELb0ELb0E" in n for n, p in zip(gemms, (up, down))] == [True, True], gemms
 
     active = T // 3
@@ -140,5 +141,30 @@ def test_which_gemms(gpu, T, H, E, K, I, up, down):
     x, ids = torch.empty(T, H, dtype=torch.bfloat16, device=gpu), torch.empty(T, K, dtype=torch.int32, device=gpu)
     names = recorded_names(lambda: _layer(False, E, w, x, ids, torch.empty(T, K, device=gpu)))
     gemms = [n for n in names if "stream_gemm_kernel" in n]
+    assert len(gemms) == 2
     for name, p in zip(gemms, (up, down)):
         assert ("ELb0ELb1E" in name) == (p > 0) and (p == 0 or _queued(False, p) in name), name
+
+
+# rows, experts, K, N, column groups of an item: the wider items where the workgroup with most of them streams as many columns either
+# way, the narrower where it streams fewer
+@pytest.mark.parametrize("fp8,gate_up,rows,E,kd,n,groups", [
+    (False, True, 2048, 128, 4096, 2048, 4), (False, True, 1792, 112, 5120, 1024, 4), (False, True, 1536, 96, 5120, 1024, 2),
+    (False, False, 768, 48, 1408, 2048, 8), (False, False, 768, 48, 2048, 4096, 4),
+    (True, True, 2048, 128, 1536, 2048, 8), (True, True, 2048, 96, 1280, 3072, 4), (True, False, 2048, 128, 5120, 2048, 4),
+    (True, False, 2048, 96, 5120, 1024, 2)])
+def test_items_without_queues(gpu, fp8, gate_up, rows, E, kd, n, groups):
+    announce("items without queues fp8=%d gate_up=%d rows=%d E=%d K=%d N=%d" % (fp8, gate_up, rows, E, kd, n))
+    dtype = torch.float8_e4m3fn if fp8 else torch.int8
+    w = cam.prepack_weight(torch.empty(E, kd, n, dtype=dtype, device=gpu), gate_up)
+    x, rows_to = torch.empty(rows, kd, dtype=dtype, device=gpu), torch.empty(E, dtype=torch.int64, device=gpu)
+    if fp8:
+        xs, ws = torch.empty(rows, kd // 128, dtype=torch.uint8, device=gpu), torch.empty(E, kd // 128, n // 128, dtype=torch.uint8, device=gpu)
+        out = torch.float8_e4m3fn if gate_up else torch.bfloat16
+        names = recorded_names(lambda: cam.grouped_matmul_fp8(x, xs, w, ws, rows_to, out_dtype=out))
+    else:
+        product = cam.grouped_matmul_swiglu_quant if gate_up else cam.grouped_matmul_dequant
+        xs, ws = torch.empty(rows, device=gpu), torch.empty(E, n, device=gpu)
+        names = recorded_names(lambda: product(x, xs, w, ws, rows_to))
+    gemms = [name for name in names if "stream_gemm_kernel" in name]
+    assert len(gemms) == 1 and "stream_gemm_kernelILi4ELb%dELi%dELb0ELb0E" % (fp8, groups) in gemms[0], gemms

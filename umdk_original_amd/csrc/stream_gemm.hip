@@ -810,8 +810,8 @@ struct StreamShape {
     bool queued;     // items come from queues, if there are any
 };
 
-// `products`: for a launch that takes them (an item to a workgroup).
-StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool quad, bool products, int64_t rows_per_expert, int cus)
+// `products`: for a launch that takes them (an item to a workgroup).  `queues`: the launch has queues, and its sums do not depend on P.
+StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool quad, bool products, bool queues, int64_t rows_per_expert, int cus)
 {
     StreamShape sh;
     // live experts at most, and the column groups they stream
@@ -820,35 +820,58 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     const bool many = groups >= 6ll * cus;
     // of items that the rows make, spread over the experts
     const double reached = (double)G * (1.0 - std::pow(1.0 - 1.0 / (double)G, (double)max_rows));
-    auto rounds = [&](int P) { return reached * ((N / 64 + P - 1) / P) / cus; };
+    auto rounds_of = [&](double tiles, int P) { return tiles * ((N / 64 + P - 1) / P) / cus; };
+    auto rounds = [&](int P) { return rounds_of(reached, P); };
+    // Whether the workgroup with most items, dealt out beforehand, streams fewer columns with items of P groups than of 2 P.  Skewed ids
+    // (sigmoid scores with a Zipf bias) reach fewer of the experts while there are few rows, and an expert of more than 128 has two tiles:
+    // then it is enough that it is so with those; with about one row per expert it has to be.
+    auto fewer_of = [&](double tiles, int P) { return std::ceil(rounds_of(tiles, P)) < 2 * std::ceil(rounds_of(tiles, 2 * P)); };
+    auto fewer = [&](int P) {
+        const double skewed = max_rows < 4 * G ? 0.85 : max_rows < 12 * G ? 0.94 : 1.0;
+        const bool two_tiles = queues && rows_per_expert > 128;
+        return (2 * max_rows >= 3 * G && fewer_of(reached, P)) || (!(quad && rounds(P) >= 4) && fewer_of(skewed * reached, P)) ||
+               (two_tiles && fewer_of(reached + max_rows / 256.0, P));
+    };
     // 32-row tiles, two workgroups per CU, while the stream is short: few column groups and no expert with more rows, or
     // all tiles resident at once.  Otherwise 128-row tiles, so that an expert's weights are read once.
     sh.small = !quad && ((rows_per_expert <= 32 && !many) || groups + max_rows / 32 * (N / 64) <= 2ll * cus);
-    // Column groups per item: as few as it takes to give every CU work, then as many as make an item of about half a megabyte of
-    // weights (its sums and stores interrupt its stream for about two microseconds, and smaller items end together).
-    // kEpiSwigluFp8 needs the four groups of a 128-column block together, and the fp32 products of kEpiSwiglu are the same
-    // sums in the same order (quad).  us per layer, with up to a megabyte and no queues / this; T x H, top-K of E, I:
-    //   K over 2560 (4 / 2 groups from queues): 128 x 4096, 8 of 128, 1536 393 / 388, 64 x 3072, 6 of 128, 1536 266 / 251, 48 x 7168, 8 of 64, 2048
-    //   464 / 451; without queues 2 groups lose (400 in the first), and 24 x 4096, 8 of 128, 1536 gives 250 / 253;
-    //   K over 4096, little more than one round of 4 groups (4 / 2): 30 x 5120, 6 of 44, 1536 201 / 181, 40 x 6144, 4 of 40, 1280 161 / 146, 12 x 7168, 4 of
-    //   24, 2048 161 / 146, two rounds 128 x 7168, 4 of 32, 2048 262 / 258; at 4096 40 tokens, 4 of 40, 1280 116 / 108, but 60, 2 of 36, 1408 124 / 131;
-    //   K to 2560 (8 / 4): 200 x 2048, 4 of 64, 1408 139 / 131 (GMM1), 100 x 4096, 8 of 64, 2048 290 / 278 (GMM2), 500 x 1536, 2 of 64, 3072 level;
+    // Column groups per item: as few as it takes to give every CU work, then as many as make an item of up to a megabyte of weights (its
+    // sums and stores interrupt its stream for about two microseconds), or half of them where workgroups then end closer together: dealt
+    // out beforehand, where the one with most items streams fewer columns (fewer); from queues.  kEpiSwigluFp8 needs the four groups of
+    // a 128-column block together, and the fp32 products of kEpiSwiglu are the same sums in the same order (quad).  FP8 sums depend on P,
+    // so these items are the same with queues and without.  us, twice as many groups / this; layers T x H, top-K of E, I, and
+    // products alone, which have no queue, rows x K -> N of E:
+    //   K over 4096, to two rounds of 4 groups (4 / 2): 30 x 5120, 6 of 44, 1536 201 / 184, 384 x 5120 -> 1024 of 96 92.0 / 84.7; as many columns, so it
+    //   stays at 4: 640 x 5120 -> 2560 of 40 92.4 / 100.3, 448 x 5120 -> 1024 of 112 98.0 / 101.9; over 6144 only where the last round is
+    //   not nearly full: 192 -> 2560 of 48 145.6 / 141.7, of 42 131.7 / 134.9; 40 x 6144, 4 of 40, 1280 161 / 146 with skewed ids, 168 / 175 with even ones;
+    //   K over 2560, seven rounds of 2: from queues 128 x 4096, 8 of 128, 1536 393 / 388, 64 x 3072, 6 of 128, 1536 266 / 251, 48 x 7168, 8 of 64, 2048
+    //   464 / 451; dealt out 384 x 3072 -> 3072 of 96 152.6 / 146.3, but as many columns 512 x 4096 -> 3072 of 128 249 / 252, x 5120 311 / 319;
+    //   K to 2048 (8 / 4): 200 x 2048, 4 of 64, 1408 139 / 131 (GMM1), 192 x 2048 -> 4096 of 48 68.4 / 64.8; as many columns 160 x 2048 -> 5120 of 40 72.4 /
+    //   77.4, from seven rounds of 4 on level: 512 x 1792 -> 4096 of 128 151 / 152; but experts a power of two of bytes apart, whose
+    //   workgroups may meet on the same channels, 512 x 2048 -> 4096 of 128 181.9 / 169.5, FP8 -> 2048 106 / 93, not in one round: 128 -> 4096 of 32 43.8 / 45.6;
     //   K to 1536 (8 / 4): 90 x 5120, 6 of 160, 1536, ten rounds and more 519 / 512, 64 x 5120, 6 of 32, 1536, little more than one of 8 groups
-    //   157 / 150, six rounds of a dozen rows per expert (FP8, to which int8 of so many rows does not come here) 256 x 4096, 8 of 128, 1536 422 / 409,
-    //   700 x 2048, 8 of 256, 1024 337 / 326; in between, 64 x 4096, 8 of 128, 1536, 359 / 363, and at K 512 116 / 119, so these stay;
-    //   quad, K to 2048 (8 / 4): 200 x 2048, 4 of 64, 1408 133 / 124, 700 x 1024, 8 of 256, 512 130 / 125; 4 from queues: 48 x 4096, 8 of 128, 1536 342 / 335,
-    //   256 432 / 423, level at four rounds.  More rows make sums that several waves share dearer: 500 x 2048, 8 of 128, 768 166 / 170.
+    //   157 / 150, but 192 x 1408 -> 2048 of 48 27.5 / 30.1; six rounds of a dozen rows per expert (FP8, to which int8 of so many rows does not come here)
+    //   256 x 4096, 8 of 128, 1536 422 / 409, 700 x 2048, 8 of 256, 1024 337 / 326; in between, 64 x 4096, 8 of 128, 1536, 359 / 363, and at K 512 116 / 119;
+    //   quad (8 / 4): 200 x 1280, 6 of 96, 1536 130.4 / 117.5, 4 from queues 48 x 4096, 8 of 128, 1536 342 / 335; as many columns 128 x 1536, 8 of 128, 1536
+    //   161.9 / 165.7, 768 x 1536 -> 2048 of 48 29.8 / 32.4, at K 2048, whose items are a megabyte apart, 100 x 2048, 8 of 128, 2048 300 / 273, 200, 8 of 256,
+    //   1536 413 / 396.  More rows make sums that several waves share dearer: 500 x 2048, 8 of 128, 768 166 / 170.
+    const long long expert = (long long)Kd * N;
+    const bool apart = (expert & (expert - 1)) == 0 && rounds(8) > 1;
+    const bool to2 = fewer(2) || (Kd > 6144 && std::ceil(rounds(2)) - rounds(2) < 0.35);
+    const bool to4 = fewer(4) || rounds(4) >= 7 || apart;
     sh.P = 2;
     if (sh.small) {
         sh.P = 2 * groups >= 3ll * cus ? 2 : 1;
     } else if (products) {
         sh.P = 512ll * Kd <= (1 << 20) ? 8 : 4;
     } else if (quad) {
-        sh.P = many && Kd <= 2048 && max_rows > 24 * G ? 8 : 4;
+        sh.P = many && Kd <= 2048 && (max_rows > 24 * G || !(fewer(4) || apart || (Kd == 2048 && rounds(8) > 1))) ? 8 : 4;
     } else if (many && Kd > 2560) {
-        sh.P = rounds(2) >= 7 || (Kd > 4096 && rounds(4) < 2.2) ? 2 : 4;
+        sh.P = (rounds(2) >= 7 && (queues || to2)) || (Kd > 4096 && rounds(4) < 2.2 && to2) ? 2 : 4;
+    } else if (many && Kd > 1536) {
+        sh.P = Kd > 2048 || to4 ? 4 : 8;
     } else if (many) {
-        sh.P = Kd > 1536 || (Kd > 1024 && rounds(8) < 1.3) || (Kd >= 1024 && (rounds(4) >= 10 || (rounds(4) >= 6 && max_rows >= 12 * G))) ? 4 : 8;
+        sh.P = to4 && ((Kd > 1024 && rounds(8) < 1.3) || (Kd >= 1024 && (rounds(4) >= 10 || (rounds(4) >= 6 && max_rows >= 12 * G)))) ? 4 : 8;
     }
     sh.queued = many && !sh.small && !products && sh.P <= 4 && rounds(sh.P) >= 4;
     const long long tiles = live + max_rows / (sh.small ? 32 : 128);
@@ -911,7 +934,7 @@ bool stream_gemm_takes_products(int64_t max_rows, int G, int Kd, int N, int64_t 
     if (max_rows <= 0 || G <= 0 || gemm_workgroups(&cus) != hipSuccess) {
         return false;
     }
-    const StreamShape sh = stream_shape(G, max_rows, Kd, N, false, true, rows_per_expert, cus);
+    const StreamShape sh = stream_shape(G, max_rows, Kd, N, false, true, false, rows_per_expert, cus);
     const int lg = lg_product_rows(sh, max_rows, Kd);
     if (lg < 0) {
         return false;
@@ -942,7 +965,8 @@ hipError_t launch_stream_gemm(const StreamGemmArgs &sa, int64_t rows_per_expert,
     if (e != hipSuccess) {
         return e;
     }
-    const StreamShape sh = stream_shape(sa.G, sa.max_rows, g.Kd, g.N, g.fp8 && g.gate_up, sa.products != nullptr, rows_per_expert, cus);
+    const StreamShape sh = stream_shape(sa.G, sa.max_rows, g.Kd, g.N, g.fp8 && g.gate_up, sa.products != nullptr, sa.queue != nullptr && !g.fp8,
+                                        rows_per_expert, cus);
     const bool queued = sh.queued && sa.queue != nullptr;
     if (sa.products != nullptr) {
         const int lg = lg_product_rows(sh, sa.max_rows, g.Kd);
