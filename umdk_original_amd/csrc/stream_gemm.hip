@@ -54,6 +54,9 @@ constexpr int kSBuf32 = 32768;           // activation buffer of the 32-row tile
 constexpr int kSBuf128 = 65536;          // of the 128-row tiles
 constexpr int kProductQuads = 16;        // PRODUCTS: quads of products a thread holds, i.e. 32 K products a workgroup
 
+// What the rows of a tile are padded to: the K bytes of one turn of the 8 / P waves that share the columns of an item of P groups.
+constexpr int k_quantum(int P) { return 8 / P * R > 4 ? 64 * (8 / P) * R : 256; }
+
 __device__ __forceinline__ void lds_barrier()
 {
     // LDS traffic of this wave is done, weight loads stay in flight (a __syncthreads would drain them)
@@ -156,7 +159,7 @@ __global__ __launch_bounds__(kSThreads, MF == 1 ? 4 : 2) void stream_gemm_kernel
     const int ngroups = N >> 6;
     const int blocks = (ngroups + P - 1) / P;
     const int turns = (KT + S * R - 1) / (S * R);   // turns of the ring per item
-    constexpr int quantum = S * R > 4 ? 64 * S * R : 256;  // K bytes of one turn of all S waves
+    constexpr int quantum = k_quantum(P);
     static_assert(NFR == 2 || S >= 4, "sums that pass one fragment at a time wait in registers for one block only");
     static_assert(32 * MF * quantum <= kABuf, "a turn of a full tile has to fit an activation buffer");
     static_assert(!PRODUCTS || !FP8, "products are quantised to int8");
@@ -881,13 +884,12 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     return sh;
 }
 
-// log2 of the rows of a tile whose products fit the registers of a workgroup, and its int8 rows (padded to a turn of the eight waves) an
-// activation buffer; -1 where 32-row tiles are not that low.  128-row tiles are cut: a token that names an expert once makes
-// no more than one tile of it where the launch takes products, and one that names it more than once two.
+// log2 of the rows of a tile whose products fit the registers of a workgroup, and its int8 rows, padded as the kernel pads them, an
+// activation buffer; -1 where 32-row tiles are not that low.  128-row tiles are cut: tokens that name an expert once each make
+// no more than one tile of it where the launch takes products, tokens that name it several times as many as their rows fill.
 int lg_product_rows(const StreamShape &sh, long long max_rows, int Kd)
 {
-    const long long turn = 64 * (8 / sh.P) * R;
-    const long long kpad = (Kd + turn - 1) / turn * turn;
+    const long long quantum = k_quantum(sh.P), kpad = (Kd + quantum - 1) / quantum * quantum;
     auto fits = [&](int lg) {
         return ((long long)Kd << lg) <= 4ll * kProductQuads * kSThreads && (kpad << lg) <= (sh.small ? kSBuf32 : kSBuf128);
     };
