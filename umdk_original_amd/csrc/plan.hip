@@ -585,10 +585,10 @@ hipError_t launch_plan_local(const PlanArgs &a, int it, int nb, int32_t *hist, h
 {
     const dim3 grid(nb), blk(kLocalThreads);
     switch (it) {
-        case 1: hipLaunchKernelGGL((plan_local_kernel<IdT, 1>), grid, blk, 0, stream, a, hist); break;
         case 2: hipLaunchKernelGGL((plan_local_kernel<IdT, 2>), grid, blk, 0, stream, a, hist); break;
         case 4: hipLaunchKernelGGL((plan_local_kernel<IdT, 4>), grid, blk, 0, stream, a, hist); break;
-        default: hipLaunchKernelGGL((plan_local_kernel<IdT, 8>), grid, blk, 0, stream, a, hist); break;
+        case 8: hipLaunchKernelGGL((plan_local_kernel<IdT, 8>), grid, blk, 0, stream, a, hist); break;
+        default: return hipErrorInvalidValue;  // (up to kExpertIds ids come to no second launch)
     }
     return hipGetLastError();
 }
