@@ -1,7 +1,7 @@
 """Layers of a handful of tokens in their two launches, int8 bit for bit against the oracle, FP8 within what its sums allow: one slot and the most (8, 16, 32), one row
 per expert and as many as tokens (more than are asked for at once), K steps that no wave shares evenly, the shortest and longest rows,
-both activation types, weights per expert, experts named twice by a token, ids of no expert, masks down to no token at all; and on
-which side of its lines a layer takes them."""
+both activation types, weights per expert, experts named twice by a token, ids of no expert, masks down to no token at all, the most
+that LDS holds, infinities and NaN; and on which side of its lines a layer takes them."""
 import numpy as np
 import pytest
 import torch
@@ -11,6 +11,7 @@ from umdk_original_amd import synth
 from gpu_util import announce, assert_bits_equal, recorded_kernels, to_np
 from test_gpu_fp8 import _check_layer, _layer_inputs, _u8
 from test_gpu_fused import _check, _run
+from test_gpu_stream_queues import _check as _check_bits, _ids, _layer as _run_layer, _one_by_one, _weights
 
 pytestmark = pytest.mark.gpu
 
@@ -118,3 +119,53 @@ def test_which_fp8_layers(gpu, T, H, E, K, I, few):
     gates = torch.empty(T, K, device=gpu)
     n = recorded_kernels(lambda: cam.fused_deep_moe_fp8(x, ids, *dev, gates))
     assert n == 2 if few else n > 2
+
+
+def _device_layer(gpu, fp8, T, H, E, K, I, seed):
+    w = _weights(gpu, fp8, E, H, I)
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    return w, torch.randn(T, H, generator=g, device=gpu).to(torch.bfloat16), torch.rand(T, K, generator=g, device=gpu)
+
+
+@pytest.mark.parametrize("T,H,E,K,I", [(8, 6144, 16, 2, 2048), (4, 4096, 64, 8, 1536), (2, 7168, 8, 8, 3072)])
+def test_largest_rows_in_lds(gpu, T, H, E, K, I):
+    """The most bytes of rows in either launch (48 KB, T * H and slots * I), against the operators one by one."""
+    announce("few tokens, largest T=%d H=%d E=%d K=%d I=%d" % (T, H, E, K, I))
+    w, x, gates = _device_layer(gpu, False, T, H, E, K, I, T)
+    for kind in ("spread", "one", "dropped"):
+        ids = _ids(gpu, kind, T, E, K, T)
+        assert recorded_kernels(lambda: _run_layer(False, E, w, x, ids, gates)) == 2
+        _check_bits(False, E, w, x, ids, gates, _run_layer(False, E, w, x, ids, gates))
+
+
+def test_largest_fp8_rows_in_lds(gpu, oracle):
+    """16 slots of I 3072: 48 KB of rows, whose 384 scales fill their table, beside the sums of all waves."""
+    T, H, E, K, I = 2, 7168, 8, 8, 3072
+    announce("few tokens FP8, largest")
+    ids, w, x, w1, s1, w2, s2 = _layer_inputs(T, H, E, K, I, seed=11)
+    dev = [cam.prepack_weight(w1.to(gpu), True), s1.to(gpu), cam.prepack_weight(w2.to(gpu), False), s2.to(gpu)]
+    on_gpu = [t.to(gpu) for t in (x, ids.to(torch.int32), w)]
+    assert recorded_kernels(lambda: cam.fused_deep_moe_fp8(*on_gpu[:2], *dev, on_gpu[2])) == 2
+    out, etn = cam.fused_deep_moe_fp8(*on_gpu[:2], *dev, on_gpu[2])
+    want, dbg = oracle.fp8_fused_layer(synth.bf16_bits(x), ids.numpy(), w.numpy(), _u8(w1), s1.numpy(), _u8(w2), s2.numpy(), debug=True)
+    assert np.array_equal(etn.cpu().numpy(), dbg["cnt"])
+    _check_layer(out.float().cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_infinities_and_nan(gpu, fp8):
+    """What a token holds stays in its own output: tokens with infinities and NaN are non-finite where the operators one by one make
+    them so, the others have the bits they have without them."""
+    T, H, E, K, I = 4, 2048, 8, 2, 640
+    announce("few tokens, infinities and NaN fp8=%d" % fp8)
+    w, x, gates = _device_layer(gpu, fp8, T, H, E, K, I, 5)
+    ids = torch.tensor([[0, 1], [1, 2], [0, 1], [1, 0]], dtype=torch.int32, device=gpu)   # rows of one expert side by side
+    clean = _run_layer(fp8, E, w, x, ids, gates)[0]
+    x[1, H - 1] = float("nan")
+    x[2, 0], x[2, 777] = float("inf"), float("-inf")
+    assert recorded_kernels(lambda: _run_layer(fp8, E, w, x, ids, gates)) == 2
+    got = _run_layer(fp8, E, w, x, ids, gates)[0]
+    want = _one_by_one(fp8, E, w, x, ids, gates)[0]
+    for t in (0, 3):
+        assert torch.equal(got[t].view(torch.int16), clean[t].view(torch.int16))
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())

@@ -1,13 +1,14 @@
 """The grouped GEMM's streaming form (few rows per expert) against the oracle at the sizes where it can go wrong: edges
 of its 32- and 128-row tiles and of their eight-row blocks, a K shorter than one turn of the waves or no multiple of it,
-activations in one LDS chunk and in several, column groups that do not fill the last item, both forms of group list."""
+activations in one LDS chunk and in several, column groups that do not fill the last item, the widest items of FP8 products,
+both forms of group list."""
 import numpy as np
 import pytest
 import torch
 
 import umdk_original_amd as cam
 from umdk_original_amd import synth
-from gpu_util import announce, assert_bits_equal, to_np
+from gpu_util import announce, assert_bits_equal, recorded_names, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -69,6 +70,40 @@ def test_stream_gemm_fp8_sums(gpu, oracle, sizes, K, N):
         r += n
     assert (got - want).abs().max() <= 2e-2 * want.abs().max()
     assert ((got - want).norm() / want.norm()).item() <= 5e-3
+
+
+@pytest.mark.parametrize("K,I", [(2048, 1408), (1280, 1152), (1920, 1664)])   # 5.5, 4.5 and 6.5 items of eight column groups
+def test_stream_gemm_fp8_products_of_eight_groups(gpu, K, I):
+    """Over 24 rows per expert: the fp32 products against 64-bit sums, the quantised ones bit for bit against those, an expert of three
+    row tiles and some of none among them."""
+    announce("stream fp8 products of eight groups K=%d I=%d" % (K, I))
+    G, N = 64, 2 * I
+    sizes = synth.zipf_group_sizes(G, 1700, K)
+    assert int(sizes.max()) > 256 and int((sizes == 0).sum()) == 3
+    A, g = 1700, torch.Generator(device=gpu).manual_seed(K)
+    x = torch.randn(A, K, generator=g, device=gpu).mul(4.0).to(torch.float8_e4m3fn)
+    w = torch.randn(G, K, N, generator=g, device=gpu).to(torch.float8_e4m3fn)
+    sx = torch.randint(121, 125, (A, K // 128), generator=g, dtype=torch.uint8, device=gpu)
+    sw = torch.randint(121, 125, (G, K // 128, N // 128), generator=g, dtype=torch.uint8, device=gpu)
+    wp, gl = cam.prepack_weight(w, True), torch.cumsum(sizes, 0).to(gpu)
+    for out_dtype in (torch.float32, torch.float8_e4m3fn):
+        names = recorded_names(lambda: cam.grouped_matmul_fp8(x, sx, wp, sw, gl, out_dtype=out_dtype))
+        assert any("stream_gemm_kernelILi4ELb1ELi8E" in n for n in names), names
+    got = cam.grouped_matmul_fp8(x, sx, wp, sw, gl)
+    q, s = cam.grouped_matmul_fp8(x, sx, wp, sw, gl, out_dtype=torch.float8_e4m3fn)
+    want_q, want_s = cam.quant_rows_fp8(got)
+    assert torch.equal(q.view(torch.uint8), want_q.view(torch.uint8)) and torch.equal(s, want_s)
+    r = 0
+    for e, n in enumerate(sizes.tolist()):
+        xf = x[r:r + n].double() * torch.exp2(sx[r:r + n].double() - 127).repeat_interleave(128, 1)
+        wf = w[e].double() * torch.exp2(sw[e].double() - 127).repeat_interleave(128, 0).repeat_interleave(128, 1)
+        gate, up = (xf @ wf).split(I, 1)
+        # fp32 sums of K products, the slope of SiLU at most 1.1, and the roundings of SiLU and of the product
+        eg, eu = (xf.abs() @ wf.abs()).mul(K * 2.0 ** -23).split(I, 1)
+        silu = gate * torch.sigmoid(gate)
+        bound = 1.1 * eg * (up.abs() + eu) + silu.abs() * eu + (silu * up).abs() * 2.0 ** -20
+        assert ((got[r:r + n].double() - silu * up).abs() <= bound).all()
+        r += n
 
 
 @pytest.mark.parametrize("experts", [1, 63, 64, 65, 128, 511, 512])

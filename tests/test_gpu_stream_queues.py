@@ -71,7 +71,7 @@ def _check(fp8, E, w, x, ids, gates, got):
 # T, H, E, K, I, column groups of an item in either GEMM (0: no queue)
 SHAPES = [(100, 6144, 64, 4, 2304, 2, 4), (33, 3072, 96, 8, 1920, 2, 4), (32, 2176, 250, 6, 1152, 4, 0)]
 SHAPES8 = [(100, 6144, 64, 4, 2304, 4, 4), (340, 3072, 128, 8, 2304, 4, 4), (40, 6784, 80, 8, 2688, 4, 2), (200, 3328, 128, 8, 1152, 4, 4),
-           (190, 3328, 128, 8, 1152, 4, 0)]
+           (190, 3328, 128, 8, 1152, 4, 0), (200, 2048, 64, 8, 1408, 0, 0), (200, 2048, 64, 8, 1152, 0, 0)]
 
 
 @pytest.mark.parametrize("fp8,shape", [(False, s) for s in SHAPES] + [(True, s) for s in SHAPES8])
