@@ -822,7 +822,7 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     const long long groups = live * (N / 64);
     const bool many = groups >= 6ll * cus;
     // of items that the rows make, spread over the experts
-    const double reached = (double)G * (1.0 - std::pow(1.0 - 1.0 / (double)G, (double)max_rows));
+    const double reached = many ? (double)G * (1.0 - std::pow(1.0 - 1.0 / (double)G, (double)max_rows)) : 0.0;
     auto rounds_of = [&](double tiles, int P) { return tiles * ((N / 64 + P - 1) / P) / cus; };
     auto rounds = [&](int P) { return rounds_of(reached, P); };
     // Whether the workgroup with most items, dealt out beforehand, streams fewer columns with items of P groups than of 2 P.  Skewed ids
@@ -859,22 +859,22 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     //   161.9 / 165.7, 768 x 1536 -> 2048 of 48 29.8 / 32.4, at K 2048, whose items are a megabyte apart, 100 x 2048, 8 of 128, 2048 300 / 273, 200, 8 of 256,
     //   1536 413 / 396.  More rows make sums that several waves share dearer: 500 x 2048, 8 of 128, 768 166 / 170.
     const long long expert = (long long)Kd * N;
-    const bool apart = (expert & (expert - 1)) == 0 && rounds(8) > 1;
-    const bool to2 = fewer(2) || (Kd > 6144 && std::ceil(rounds(2)) - rounds(2) < 0.35);
-    const bool to4 = fewer(4) || rounds(4) >= 7 || apart;
+    auto apart = [&] { return (expert & (expert - 1)) == 0 && rounds(8) > 1; };
+    auto to2 = [&] { return fewer(2) || (Kd > 6144 && std::ceil(rounds(2)) - rounds(2) < 0.35); };
+    auto to4 = [&] { return fewer(4) || rounds(4) >= 7 || apart(); };
     sh.P = 2;
     if (sh.small) {
         sh.P = 2 * groups >= 3ll * cus ? 2 : 1;
     } else if (products) {
         sh.P = 512ll * Kd <= (1 << 20) ? 8 : 4;
     } else if (quad) {
-        sh.P = many && Kd <= 2048 && (max_rows > 24 * G || !(fewer(4) || apart || (Kd == 2048 && rounds(8) > 1))) ? 8 : 4;
+        sh.P = many && Kd <= 2048 && (max_rows > 24 * G || !(fewer(4) || apart() || (Kd == 2048 && rounds(8) > 1))) ? 8 : 4;
     } else if (many && Kd > 2560) {
-        sh.P = (rounds(2) >= 7 && (queues || to2)) || (Kd > 4096 && rounds(4) < 2.2 && to2) ? 2 : 4;
+        sh.P = (rounds(2) >= 7 && (queues || to2())) || (Kd > 4096 && rounds(4) < 2.2 && to2()) ? 2 : 4;
     } else if (many && Kd > 1536) {
-        sh.P = Kd > 2048 || to4 ? 4 : 8;
+        sh.P = Kd > 2048 || to4() ? 4 : 8;
     } else if (many) {
-        sh.P = to4 && ((Kd > 1024 && rounds(8) < 1.3) || (Kd >= 1024 && (rounds(4) >= 10 || (rounds(4) >= 6 && max_rows >= 12 * G)))) ? 4 : 8;
+        sh.P = to4() && ((Kd > 1024 && rounds(8) < 1.3) || (Kd >= 1024 && (rounds(4) >= 10 || (rounds(4) >= 6 && max_rows >= 12 * G)))) ? 4 : 8;
     }
     sh.queued = many && !sh.small && !products && sh.P <= 4 && rounds(sh.P) >= 4;
     const long long tiles = live + max_rows / (sh.small ? 32 : 128);
