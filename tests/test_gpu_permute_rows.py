@@ -1,5 +1,5 @@
-"""The permute on both sides of the line between all rows of a token asked for at once and one by one (152 MiB of 8-bit rows), with dropped ids:
-every copy of a token in its row, with its scale and its triple.  Each token quantised once by a dispatch to one expert is the reference."""
+"""The permute on both sides of the line between all rows of a token asked for at once and one by one (152 MiB of 8-bit rows; int8 29 to 63
+MiB of tokens), with dropped ids: every copy of a token in its row, with its scale and its triple.  Each token quantised once by a dispatch to one expert is the reference."""
 import pytest
 import torch
 
@@ -11,6 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("quant", [2, 4, 0])
 @pytest.mark.parametrize("T,H,E,K", [(1389, 7168, 64, 16), (1390, 7168, 64, 16), (2222, 7168, 32, 10), (2224, 7168, 32, 10), (2501, 1024, 512, 1),
+                                     (3711, 4096, 64, 2), (3712, 4096, 64, 2), (4607, 7168, 12, 1), (4608, 7168, 12, 1),
                                      (257, 4096, 300, 8)])
 def test_copies(gpu, quant, T, H, E, K):
     announce("permute rows quant=%d T=%d H=%d E=%d K=%d" % (quant, T, H, E, K))

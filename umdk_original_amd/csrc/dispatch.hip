@@ -79,11 +79,20 @@ bool stores_plainly(const DispatchArgs &a)
 }
 
 // Whether a wave asks for the row of a copy behind the stores of the copy before, which spaces its stores out: very many 8-bit rows
-// lie in memory faster then, although a wave takes longer.  us, plan and permute replayed from a graph, all at once / one by one, T x H, top-K of E:
-// int8 235 MB 4096 x 7168, 8 of 256 68.1 / 64.1, 192 MB 8000 x 3000, 8 of 512 62.1 / 58.0, 172 MB 3000 x 7168, 8 of 64 50.1 / 48.3, but 131 MB 8000 x
-// 4096, 4 of 64 47.4 / 48.5, 117 MB 2048 x 7168, 8 of 64 32.4 / 33.4, 86 MB 1500 25.0 / 25.8, 12 MB 1000 x 2048, 6 of 64 10.1 / 10.3; FP8 235 MB 69.3 / 68.2;
+// lie in memory faster then, although a wave takes longer, and int8 rows also where their tokens begin not to stay in the L2s.  us, plan and
+// permute replayed from a graph, all at once / one by one, T x H, top-K of E:
+// int8 235 MB 4096 x 7168, 8 of 256 68.1 / 64.1, 192 MB 8000 x 3000, 8 of 512 62.1 / 58.0, 172 MB 3000 x 7168, 8 of 64 50.1 / 48.3; FP8 235 MB 69.3 / 68.2;
 // 16-bit rows level, 470 MB 95.4 / 95.3.  (A wait for the stores alone does not help: 68.7 in the first.)
-bool asks_one_by_one(const DispatchArgs &a) { return a.quant != 0 && (long long)a.T * a.K * a.H >= 152ll << 20; }
+// int8 by MiB of tokens: 28 2936 x 5000, 5 of 12 24.2 / 24.8, 4893 x 3000 28.2 / 28.6; 30 3145 x 5000, 4 of 8 27.0 / 24.1, 5242 x 3000, 6 of 64 36.1 / 33.0,
+// 3145 x 5000, 8 of 256 41.6 / 38.3, but 2194 x 7168, 8 of 256 40.2 / 40.7 and 7680 x 2048, 4 of 8 29.3 / 31.3 (8 of 256 45.5 / 45.4); 40 4194 x 5000, 6
+// of 64 44.4 / 39.6; 45 3291 x 7168, 4 of 8 35.6 / 32.0, 5760 x 4096 38.7 / 34.0; 47 3543 x 6904, 6 of 64 50.6 / 41.2; 60 4388 x 7168, 4 of 8 47.2 / 47.2,
+// 70 5120 49.5 / 50.7; FP8 level.
+bool asks_one_by_one(const DispatchArgs &a)
+{
+    const long long tokens = 2ll * a.T * a.H;
+    const bool beyond_l2 = (a.quant == 1 || a.quant == 2) && a.H > 2048 && tokens >= 29ll << 20 && tokens < 63ll << 20;
+    return a.quant != 0 && (beyond_l2 || (long long)a.T * a.K * a.H >= 152ll << 20);
+}
 
 // Four workgroups per CU (128 registers a lane) keep all 1024 workgroups of a 4096-token batch resident at once;
 // the FP8 variant would spill at that size and stays at three.
