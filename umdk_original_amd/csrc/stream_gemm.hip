@@ -827,12 +827,18 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     auto rounds = [&](int P) { return rounds_of(reached, P); };
     // Whether the workgroup with most items, dealt out beforehand, streams fewer columns with items of P groups than of 2 P.  Skewed ids
     // (sigmoid scores with a Zipf bias) reach fewer of the experts while there are few rows, and an expert of more than 128 has two tiles:
-    // then it is enough that it is so with those; with about one row per expert it has to be.
+    // then it is enough that it is so with those.  With less than a row per expert anything from half of them to all may be reached, and
+    // narrower items of K from 1536 on, which gain up to a tenth where it is so and lose a thirtieth where it is not, are taken for granted:
+    // 17 x 2048, 4 of 213, FP8, I 1664 77.7 / 71.7, 5 x 4608, 7 of 92, 2176 126.1 / 115.6, 16 x 5504, 3 of 81, 1408 86.0 / 88.5; of shorter K 12 x
+    // 1024, 6 of 233, FP8, 2816 82.8 / 88.4.
     auto fewer_of = [&](double tiles, int P) { return std::ceil(rounds_of(tiles, P)) < 2 * std::ceil(rounds_of(tiles, 2 * P)); };
     auto fewer = [&](int P) {
         const double skewed = max_rows < 4 * G ? 0.85 : max_rows < 12 * G ? 0.94 : 1.0;
         const bool two_tiles = queues && rows_per_expert > 128;
-        return (2 * max_rows >= 3 * G && fewer_of(reached, P)) || (!(quad && rounds(P) >= 4) && fewer_of(skewed * reached, P)) ||
+        if (Kd >= 1536 && (max_rows < G || (max_rows < 4 * G && fewer_of(0.7 * reached, P)))) {
+            return true;
+        }
+        return fewer_of(reached, P) || (!(quad && rounds(P) >= 4) && fewer_of(skewed * reached, P)) ||
                (two_tiles && fewer_of(reached + max_rows / 256.0, P));
     };
     // 32-row tiles, two workgroups per CU, while the stream is short: few column groups and no expert with more rows, or
@@ -849,8 +855,8 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     //   not nearly full: 192 -> 2560 of 48 145.6 / 141.7, of 42 131.7 / 134.9; 40 x 6144, 4 of 40, 1280 161 / 146 with skewed ids, 168 / 175 with even ones;
     //   K over 2560, seven rounds of 2: from queues 128 x 4096, 8 of 128, 1536 393 / 388, 64 x 3072, 6 of 128, 1536 266 / 251, 48 x 7168, 8 of 64, 2048
     //   464 / 451; dealt out 384 x 3072 -> 3072 of 96 152.6 / 146.3, but as many columns 512 x 4096 -> 3072 of 128 249 / 252, x 5120 311 / 319;
-    //   K to 2048 (8 / 4): 200 x 2048, 4 of 64, 1408 139 / 131 (GMM1), 192 x 2048 -> 4096 of 48 68.4 / 64.8; as many columns 160 x 2048 -> 5120 of 40 72.4 /
-    //   77.4, from seven rounds of 4 on level: 512 x 1792 -> 4096 of 128 151 / 152; but experts a power of two of bytes apart, whose
+    //   K to 2048 (8 / 4): 200 x 2048, 4 of 64, 1408 139 / 131 (GMM1), 192 x 2048 -> 4096 of 48 68.4 / 64.8; as many columns 560 x 2048 -> 5120 of 40 73.4 /
+    //   81.0, from seven rounds of 4 on level: 512 x 1792 -> 4096 of 128 151 / 152; but experts a power of two of bytes apart, whose
     //   workgroups may meet on the same channels, 512 x 2048 -> 4096 of 128 181.9 / 169.5, FP8 -> 2048 106 / 93, not in one round: 128 -> 4096 of 32 43.8 / 45.6;
     //   K to 1536 (8 / 4): 90 x 5120, 6 of 160, 1536, ten rounds and more 519 / 512, 64 x 5120, 6 of 32, 1536, little more than one of 8 groups
     //   157 / 150, but 192 x 1408 -> 2048 of 48 27.5 / 30.1; six rounds of a dozen rows per expert (FP8, to which int8 of so many rows does not come here)
