@@ -191,7 +191,7 @@ def _layer(T, H, E, K, I, seed):
     (1021, 1024, 64, 6, 768, None, False, False),   # most experts flat
 ])
 def test_layer_bit_exact(gpu, oracle, T, H, E, K, I, active, as_list, dropped):
-    """Layers whose schedules are built in the plan's second launch."""
+    """Layers whose schedules are built in the plan."""
     announce("tile form, layer T=%d H=%d E=%d K=%d I=%d active=%s as_list=%s dropped=%s" % (T, H, E, K, I, active, as_list,
                                                                                           dropped))
     assert T * K * 2 * I > LIMIT
@@ -325,7 +325,7 @@ def test_narrow_fp8(gpu, oracle, K):
 
 
 def test_narrow_layer_bit_exact(gpu, oracle):
-    """The narrow schedule as the plan's second launch builds it."""
+    """The narrow schedule as the plan builds it."""
     T, H, E, K, I = 1021, 512, 64, 6, 1152
     announce("tile form, narrow tiles, layer T=%d H=%d E=%d K=%d I=%d" % (T, H, E, K, I))
     d = _layer(T, H, E, K, I, 5)

@@ -8,15 +8,15 @@
 // take 23 us at the rate that streams reach; each of the four launches it was before (plan and permute, gate/up, down,
 // combine) began and ended with several microseconds in which no weight moved.  With so few (token, k) slots every workgroup can
 // find out by itself what the launches in front of it and behind it were for:
-//   * gate/up: a workgroup of four waves is 16 gate and 16 up columns of one expert.  It reads the ids (at most 16), asks for its
+//   * gate/up: a workgroup of eight waves is 16 gate and 16 up columns of one expert.  It reads the ids (at most 32), asks for its
 //     first weights as soon as it knows its expert, and quantises the expert's tokens to LDS while they are on their way.
 //   * down: a workgroup of eight waves is 16 output columns of ALL slots, so the weighted sum over a token's slots needs no other
-//     workgroup.  It quantises the fp32 products of every slot (96 KB at most, out of L2) while its first weights are on
+//     workgroup.  It quantises the fp32 products of every slot (192 KB at most, out of L2) while its first weights are on
 //     their way.
 // 16 columns, half of what the weights are packed by, because the shapes leave few workgroups otherwise: 768 and 256 in the example, whose
 // launches take 20.0 and 13.0 us under the tracer (four before: 5.0 + 19.7 + 13.0 + 4.5), the layer 32.0 us (43.0).  Waves per gate/up
 // workgroup and K steps in flight per wave, layer of one token / of four: 4 and 16 36.5 / 111.9 us, 4 and 8 33.5 / 103.6, 4 and 4 32.8 / 101.9, 8 and
-// 3 32.9 / 101.7, 8 and 8 36.1 / 110.8: more workgroups to a CU beat more loads to a wave.
+// 8 36.1 / 110.8, 8 and 3, as built, 32.9 / 101.7: few loads to a wave, which leave room for more waves to a CU, beat many.
 // The four lanes of a column then hold the four 16-byte quarters of a 64-byte K step, which is what v_mfma_i32_16x16x64_i8 takes;
 // its sixteen rows are the expert's tokens (eight at most), the last of them repeated.  FP8 steps are 128 bytes of K, one block of scales:
 // a lane holds 32 bytes of its column, which is what v_mfma_scale_f32_16x16x128_f8f6f4 takes.

@@ -1,5 +1,5 @@
 // Device code that builds the work-item schedule of the grouped GEMM: used by the stand-alone builder kernel and, in a layer,
-// by workgroups of the plan's second launch.
+// by workgroups of the plan: of its one launch up to 16384 ids, of its second beyond.
 #ifndef CAM_SCHED_DEVICE_H_
 #define CAM_SCHED_DEVICE_H_
 
