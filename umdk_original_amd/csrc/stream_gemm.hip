@@ -830,12 +830,12 @@ StreamShape stream_shape(long long G, long long max_rows, int Kd, int N, bool qu
     // then it is enough that it is so with those.  With less than a row per expert anything from half of them to all may be reached, and
     // narrower items of K from 1536 on, which gain up to a tenth where it is so and lose a thirtieth where it is not, are taken for granted:
     // 17 x 2048, 4 of 213, FP8, I 1664 77.7 / 71.7, 5 x 4608, 7 of 92, 2176 126.1 / 115.6, 16 x 5504, 3 of 81, 1408 86.0 / 88.5; of shorter K 12 x
-    // 1024, 6 of 233, FP8, 2816 82.8 / 88.4.
+    // 1024, 6 of 233, FP8, 2816 82.8 / 88.4, quad 8 x 1664, 2 of 70, 3072 55.2 / 59.8.
     auto fewer_of = [&](double tiles, int P) { return std::ceil(rounds_of(tiles, P)) < 2 * std::ceil(rounds_of(tiles, 2 * P)); };
     auto fewer = [&](int P) {
         const double skewed = max_rows < 4 * G ? 0.85 : max_rows < 12 * G ? 0.94 : 1.0;
         const bool two_tiles = queues && rows_per_expert > 128;
-        if (Kd >= 1536 && (max_rows < G || (max_rows < 4 * G && fewer_of(0.7 * reached, P)))) {
+        if (!quad && Kd >= 1536 && (max_rows < G || (max_rows < 4 * G && fewer_of(0.7 * reached, P)))) {
             return true;
         }
         return fewer_of(reached, P) || (!(quad && rounds(P) >= 4) && fewer_of(skewed * reached, P)) ||
