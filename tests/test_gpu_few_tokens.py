@@ -71,6 +71,7 @@ def test_masks_dropped_ids_and_weights_per_expert(gpu, oracle, active):
 @pytest.mark.parametrize("T,H,E,K,I,few", [(1, 512, 4, 8, 3072, True), (8, 1024, 4, 1, 512, True), (9, 1024, 4, 1, 512, False),
                                            (2, 768, 32, 4, 3072, False), (8, 896, 32, 1, 3072, False), (4, 512, 32, 2, 2560, False),
                                            (1, 640, 32, 8, 3072, True), (8, 1536, 32, 1, 3072, True), (8, 896, 32, 1, 2048, True), (8, 768, 8, 1, 3072, True),
+                                           (4, 5120, 64, 8, 512, False), (4, 4352, 64, 4, 2048, False), (4, 5120, 64, 4, 2048, True),
                                            (8, 6144, 4, 1, 512, True), (8, 6272, 4, 1, 512, False),
                                            (2, 1024, 8, 8, 1024, True), (2, 1024, 8, 8, 1152, False),
                                            (4, 4096, 64, 8, 512, True), (4, 4096, 63, 8, 512, False), (4, 3968, 64, 8, 512, False),
@@ -109,7 +110,7 @@ def test_fp8_layer(gpu, oracle, T, H, E, K, I, active):
 
 @pytest.mark.parametrize("T,H,E,K,I,few", [(1, 1024, 4, 8, 2048, True), (1, 1024, 4, 8, 2176, False), (2, 4096, 4, 8, 1792, True),
                                            (2, 4096, 4, 8, 1920, False), (4, 1024, 4, 4, 768, True), (4, 1024, 4, 4, 896, False),
-                                           (4, 4096, 64, 8, 512, False)])
+                                           (4, 4096, 64, 8, 512, False), (4, 5120, 64, 4, 1536, False), (2, 5120, 64, 5, 1024, True)])
 def test_which_fp8_layers(gpu, T, H, E, K, I, few):
     announce("few tokens or not, FP8 T=%d H=%d E=%d K=%d I=%d" % (T, H, E, K, I))
     f8 = torch.float8_e4m3fn

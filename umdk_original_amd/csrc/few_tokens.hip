@@ -642,6 +642,11 @@ bool few_tokens_valid(const FewTokensArgs &a)
 // 59.4 (the same 52.2 / 39.3), 2 x 7168, 8 of 64, 2048 127.8 / 124.2, 4 x 4096, 4 of 8, 1024 42.9 / 28.5, 2 x 1024, 8 of 64, 768 28.9 / 26.0, 1 x 1024, 8
 // of 64, 2048 28.5 / 24.3; not 1 x 1024, 8 of 64, 3072 32.1 / 33.2, 2 x 1024, 8 of 64, 1024 28.7 / 29.7, 2 x 2048, 6 of 64, 2048 39.8 / 43.0, 5 x 4096,
 // 3 of 64, 2048 69.2 / 70.5, 3 x 7168, 8 of 64, 1024 101.4 / 104.1.
+// Over eight slots the down launch has one workgroup to a CU, and from 4224 to 6144 output columns 264 to 384 of them: a second round of a
+// few.  Times as fast as the launches before (replayed from a graph; of 64 experts): FP8, 16 slots of 1536 4224 0.82, 5120 0.94, 6144 1.00, 12 of 2560
+// 4608 0.91, 5632 0.93; little or very much to quantise gains all the same, 16 of 1024 4608 1.00 and, skewed, 1.15, 12 of 3072 5888 1.13, 6144
+// 1.17.  int8, 16 slots of 2048 4224 0.91, 4608 0.97, 5120 0.98, 12 of 1536 4224 1.06; 32 of 512 4224 0.80, 5120 0.89, 6144 0.90, 24 of 1536 4608 0.95, 6144
+// 1.11, of 2048 5120 1.04.
 bool few_tokens_apply(int64_t T, int64_t K, int64_t E, int64_t H, int64_t I, bool fp8)
 {
     const int64_t slots = T * K;
@@ -649,11 +654,18 @@ bool few_tokens_apply(int64_t T, int64_t K, int64_t E, int64_t H, int64_t I, boo
         H % 64 != 0 || I % 64 != 0 || T * H > kFewRowBytes || slots * I > kFewRowBytes) {
         return false;
     }
+    const bool second_round = slots > 8 && H > 4096 && H <= 6144;
     if (fp8) {
+        if (second_round && 10 * slots * I > 37 * H && slots * I < 36000) {
+            return false;
+        }
         return slots <= 8 ? slots * I <= 16 * H : slots <= 16 && (slots * I <= 7 * H || slots * I <= 12288);
     }
     if (slots <= 8) {
         return T == 1 || slots * I <= 12288 + 11 * H || 2 * E <= 3 * slots;
+    }
+    if (second_round && (slots <= 16 ? H < 4608 && slots * I > 24000 : slots * I < 40960 && (H < 5632 || I <= 512))) {
+        return false;
     }
     return slots * I <= 16 * H && (slots <= 16 || (T <= 4 && H >= 4096 && E >= 2 * slots));
 }
